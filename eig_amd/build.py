@@ -26,6 +26,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 UNITS = {
     "ctx.hip": False,
     "syrk.hip": True,
+    "xdigit.hip": False,
     "eigh.hip": True,
     "project.hip": False,
     "serve.hip": False,

@@ -63,6 +63,8 @@ struct eig_ctx {
 
   // XTX (normalised, row-major nrows x nrows) and partial sums
   DevBuf xtx, part;
+  // FP64 form on the integer matrix cores: digit planes, tables, INT32 sums, pair list
+  DevBuf xdplanes, xdtab, xdpart, xdmisc;
   bool have_xtx = false;
 
   // eigensolver
@@ -120,6 +122,7 @@ __device__ __host__ inline float eig_bf16_to_f32(uint16_t h) {
 }
 
 // internal launchers implemented in the kernel translation units
+int eig_syrk_digits(eig_ctx *ctx, double *dst, int *done);
 int eig_run_syrk(eig_ctx *ctx, int form, int bf16_block, double *trace_scale);
 // builds ctx->selg: per sample tile st, 64-SNP group g and sample i, 16 bytes at
 // [(st * ceil(M/64) + g) * 128 + i]; word 2h + (s >> 1), bits 16 (s & 1) + 2 j hold the

@@ -6,7 +6,9 @@
 // fly from the 2-bit tile layout; nothing but packed codes and a 4-entry level
 // table per SNP is read from HBM.
 //
-//  form FP64   : levels in FP64, v_mfma_f64_16x16x4 accumulation in FP64.
+//  form FP64   : exact integer sums over fixed-point digits of the levels (xdigit.hip);
+//                where that workspace does not fit, levels in FP64 with
+//                v_mfma_f64_16x16x4 accumulation (k_syrk_f64).
 //  form BF16X3 : each level split into bf16 hi + lo; hi*hi + hi*lo + lo*hi on
 //                v_mfma_f32_32x32x16_bf16 into FP32 accumulators, which are
 //                added into FP64 accumulators every `blk` SNPs.
@@ -543,61 +545,73 @@ int eig_run_syrk(eig_ctx *ctx, int form, int bf16_block, double *trace_scale) {
     if (bf16_block <= 0) bf16_block = 4096;
     if (bf16_block % 16 != 0) return eig_set_err(ctx, EIG_E_ARG, "bf16_block % 16 != 0");
   }
-  // Split the SNP range (split-K).  Every block of one launch runs equally long, so
-  // the launch takes ceil(P*s / slots) rounds of M/s SNPs each, slots being the
-  // blocks the chip holds at once: choose s to minimise that, plus a small charge
-  // per split for the partial tiles it writes and the finaliser reads.  Chunks are
-  // multiples of the FP32 block (bf16) or of 256 SNPs and hold at least 2048 SNPs.
-  const int64_t align = split ? std::lcm<int64_t>(bf16_block, kGrp) : 256;
-  const bool grpblk = split && bf16_block % kGrp == 0;
-  typedef void (*bf16_kernel)(const uint4 *, int64_t, int64_t, const uint32_t *, int32_t, int64_t,
-                              int32_t, double *);
-  bf16_kernel kb = nullptr;
-  if (form == EIG_FORM_BF16X3)
-    kb = grpblk ? k_syrk_bf16<false, true> : k_syrk_bf16<false, false>;
-  else if (form == EIG_FORM_BF16X4)
-    kb = grpblk ? k_syrk_bf16<true, true> : k_syrk_bf16<true, false>;
-  int occ = 0;
-  if (form == EIG_FORM_FP64)
-    EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_syrk_f64, 256, 0));
-  else
-    EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kb, 256, 0));
-  const int64_t slots = (int64_t)std::max(occ, 1) * std::max(ctx->num_cu, 1);
-  const int64_t smax = std::max<int64_t>(1, std::min<int64_t>(32, M / std::max<int64_t>(align, 2048)));
-  int64_t chunk = M, best = -1;
-  double best_cost = 0.0;
-  for (int64_t s = 1; s <= smax; ++s) {
-    int64_t c = (M + s - 1) / s;
-    c = ((c + align - 1) / align) * align;
-    const int64_t ns = (M + c - 1) / c;
-    if (ns != s) continue;  // alignment merged two splits: s is not reachable
-    const double rounds = (double)((P * ns + slots - 1) / slots);
-    const double cost = rounds * (double)c / (double)M + 0.001 * (double)ns;
-    if (best < 0 || cost < best_cost - 1e-12) {
-      best = s;
-      best_cost = cost;
-      chunk = c;
+  const size_t tile = (size_t)kTileS * kTileS;
+  EIG_TRY(eig_ensure(ctx, ctx->xtx, sizeof(double) * (size_t)n * n));
+  int32_t nsplit = 1;
+  int done = 0;
+  if (form == EIG_FORM_FP64) {
+    // the digit planes at every size (198 x 2,000: 0.10 against 0.46 ms of k_syrk_f64;
+    // 1,000 x 50,000: 0.58 against 1.37; 5,000 x 600,000: 99 against 343), k_syrk_f64
+    // where their workspace does not fit the card
+    EIG_TRY(eig_ensure(ctx, ctx->part, sizeof(double) * (tile * P + 64 + T)));
+    eig_time_begin(ctx);
+    EIG_TRY(eig_syrk_digits(ctx, (double *)ctx->part.p, &done));
+  }
+  if (!done) {
+    // Split the SNP range (split-K).  Every block of one launch runs equally long, so
+    // the launch takes ceil(P*s / slots) rounds of M/s SNPs each, slots being the
+    // blocks the chip holds at once: choose s to minimise that, plus a small charge
+    // per split for the partial tiles it writes and the finaliser reads.  Chunks are
+    // multiples of the FP32 block (bf16) or of 256 SNPs and hold at least 2048 SNPs.
+    const int64_t align = split ? std::lcm<int64_t>(bf16_block, kGrp) : 256;
+    const bool grpblk = split && bf16_block % kGrp == 0;
+    typedef void (*bf16_kernel)(const uint4 *, int64_t, int64_t, const uint32_t *, int32_t, int64_t,
+                                int32_t, double *);
+    bf16_kernel kb = nullptr;
+    if (form == EIG_FORM_BF16X3)
+      kb = grpblk ? k_syrk_bf16<false, true> : k_syrk_bf16<false, false>;
+    else if (form == EIG_FORM_BF16X4)
+      kb = grpblk ? k_syrk_bf16<true, true> : k_syrk_bf16<true, false>;
+    int occ = 0;
+    if (form == EIG_FORM_FP64)
+      EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_syrk_f64, 256, 0));
+    else
+      EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kb, 256, 0));
+    const int64_t slots = (int64_t)std::max(occ, 1) * std::max(ctx->num_cu, 1);
+    const int64_t smax = std::max<int64_t>(1, std::min<int64_t>(32, M / std::max<int64_t>(align, 2048)));
+    int64_t chunk = M, best = -1;
+    double best_cost = 0.0;
+    for (int64_t s = 1; s <= smax; ++s) {
+      int64_t c = (M + s - 1) / s;
+      c = ((c + align - 1) / align) * align;
+      const int64_t ns = (M + c - 1) / c;
+      if (ns != s) continue;  // alignment merged two splits: s is not reachable
+      const double rounds = (double)((P * ns + slots - 1) / slots);
+      const double cost = rounds * (double)c / (double)M + 0.001 * (double)ns;
+      if (best < 0 || cost < best_cost - 1e-12) {
+        best = s;
+        best_cost = cost;
+        chunk = c;
+      }
+    }
+    nsplit = (int32_t)((M + chunk - 1) / chunk);
+    // after the partial tiles: the trace, then the T per-tile diagonal sums
+    EIG_TRY(eig_ensure(ctx, ctx->part, sizeof(double) * (tile * P * nsplit + 64 + T)));
+    const unsigned grid = (unsigned)(P * nsplit);
+    const int64_t G64 = (M + kGrp - 1) / kGrp;
+    if (split) EIG_TRY(eig_ensure_selb(ctx));
+    eig_time_begin(ctx);
+    if (form == EIG_FORM_FP64) {
+      hipLaunchKernelGGL(k_syrk_f64, dim3(grid), dim3(256), 0, ctx->stream,
+                         (const uint32_t *)ctx->sel.p, M, (const double *)ctx->lev.p, P, chunk,
+                         (double *)ctx->part.p);
+    } else {
+      hipLaunchKernelGGL(kb, dim3(grid), dim3(256), 0, ctx->stream, (const uint4 *)ctx->selb.p,
+                         G64, M, (const uint32_t *)ctx->levbf.p, P, chunk, bf16_block,
+                         (double *)ctx->part.p);
     }
   }
-  int32_t nsplit = (int32_t)((M + chunk - 1) / chunk);
-  size_t tile = (size_t)kTileS * kTileS;
-  // after the partial tiles: the trace, then the T per-tile diagonal sums
-  EIG_TRY(eig_ensure(ctx, ctx->part, sizeof(double) * (tile * P * nsplit + 64 + T)));
-  EIG_TRY(eig_ensure(ctx, ctx->xtx, sizeof(double) * (size_t)n * n));
   double *d_tr = (double *)ctx->part.p + tile * P * nsplit;
-  unsigned grid = (unsigned)(P * nsplit);
-  const int64_t G64 = (M + kGrp - 1) / kGrp;
-  if (split) EIG_TRY(eig_ensure_selb(ctx));
-  eig_time_begin(ctx);
-  if (form == EIG_FORM_FP64) {
-    hipLaunchKernelGGL(k_syrk_f64, dim3(grid), dim3(256), 0, ctx->stream,
-                       (const uint32_t *)ctx->sel.p, M, (const double *)ctx->lev.p, P, chunk,
-                       (double *)ctx->part.p);
-  } else {
-    hipLaunchKernelGGL(kb, dim3(grid), dim3(256), 0, ctx->stream, (const uint4 *)ctx->selb.p,
-                       G64, M, (const uint32_t *)ctx->levbf.p, P, chunk, bf16_block,
-                       (double *)ctx->part.p);
-  }
   EIG_HIP(ctx, hipGetLastError());
   eig_time_end(ctx, "syrk");
   eig_time_begin(ctx);

@@ -31,7 +31,8 @@ extern "C" {
 #define EIG_E_CONVERGE (-6)/* eigensolver did not converge                          */
 
 /* XTX accumulation forms */
-#define EIG_FORM_FP64 0   /* FP64 end to end (MFMA f64)                             */
+#define EIG_FORM_FP64 0   /* FP64: levels in fixed point with at least FP64's accuracy,
+                             summed exactly (digit planes on the integer MFMA)       */
 #define EIG_FORM_BF16X3 1 /* split-BF16 hi+lo, 3 MFMA products (hi.hi, hi.lo, lo.hi),
                              FP32 per SNP block, FP64 across blocks                 */
 #define EIG_FORM_BF16X4 2 /* as BF16X3 plus the lo.lo product                       */
