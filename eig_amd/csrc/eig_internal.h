@@ -130,7 +130,7 @@ int eig_run_syrk(eig_ctx *ctx, int form, int bf16_block, double *trace_scale);
 constexpr int kGrp = 64;  // SNPs per group of the grouped code layout
 int eig_ensure_selg(eig_ctx *ctx);
 // internal: a helper's own small problem -- the context's published eigenvectors
-// (used by the loadings) and its cached tridiagonal graph are left untouched
+// (used by the loadings) and its stage times are left untouched
 int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, double *evals,
                  double *evecs,
                  bool internal = false);

@@ -19,8 +19,7 @@
 //     Cross-block sums are per-block partials reduced in a fixed order (same
 //     bits in every block, independent of scheduling).  After each panel
 //     k_syr2k applies A -= V W^T + W V^T to the trailing matrix.  The reflector of
-//     row c is left in A[c][c+1:], with tau[c].  The launch sequence for one n is
-//     captured once into a hipGraph and replayed.
+//     row c is left in A[c][c+1:], with tau[c].
 //  2. All eigenvalues of the tridiagonal T: Sturm counts on a shared grid of the
 //     Gershgorin interval, then 9-way multisection (8 lanes per eigenvalue, one
 //     count each).
@@ -34,7 +33,6 @@
 //  Wave-level sums exchange lanes by DPP and permlane swaps (xlane), not through LDS.
 #include <cmath>
 #include <cstring>
-#include <mutex>
 #include <vector>
 
 #include "eig_internal.h"
@@ -1455,14 +1453,6 @@ static void launch_tridiag(EigWs ws, int32_t n, int32_t clock_khz, hipStream_t s
   }
 }
 
-struct TridiagGraph {
-  int32_t n = -1;
-  void *a = nullptr;
-  hipGraphExec_t exec = nullptr;
-  std::mutex mu;  // every context on the device shares the cached graph
-};
-static TridiagGraph g_graph[16];  // per device
-
 int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, double *evals,
                  double *evecs, bool internal) {
   if (n <= 0) return eig_set_err(ctx, EIG_E_ARG, "eigh: n <= 0");
@@ -1491,7 +1481,6 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
          o_X = add((size_t)kMaxVec * N), o_lu = add((size_t)kMaxVec * kLuF * N),
          o_Z = add(kNB * kMaxVec), o_T = add((size_t)npanel * kNB * kNB),
          o_pw = add((size_t)2 * maxw * kPW), o_ps = add((size_t)maxblk), o_sync = add(8);
-  void *old = ctx->ework.p;
   EIG_TRY(eig_ensure(ctx, ctx->ework, need));
   char *base = (char *)ctx->ework.p;
   EigWs ws;
@@ -1528,30 +1517,14 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
   EIG_HIP(ctx, hipMemsetAsync(ws.W, 0, sizeof(double) * kNB * N, st));
   EIG_HIP(ctx, hipMemsetAsync(ws.xtmp, 0, sizeof(double) * lda, st));
 
-  // ---- tridiagonalisation (graph replay for n above a few hundred)
+  // ---- tridiagonalisation: plain launches.  The host queues a launch in ~3 us, less than
+  // the shortest column takes on the device, so a captured graph of the ~2 N launches
+  // replays no faster (n = 1,000: 9.54 against 9.59 ms, n = 5,000: 97.5 against 96.4) and
+  // capturing it costs every first solve of an order or a context 1.5 and 12.5 ms.
   int32_t clock_khz = 0;
   EIG_HIP(ctx, hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, ctx->device));
   tbeg();
-  const bool use_graph = !internal && n >= 256 && getenv("EIG_NO_GRAPH") == nullptr;
-  if (use_graph) {
-    TridiagGraph &G = g_graph[ctx->device & 15];
-    std::lock_guard<std::mutex> lock(G.mu);
-    if (G.exec == nullptr || G.n != n || G.a != (void *)ws.a || old != ctx->ework.p) {
-      if (G.exec) hipGraphExecDestroy(G.exec);
-      G.exec = nullptr;
-      hipGraph_t graph;
-      EIG_HIP(ctx, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-      launch_tridiag(ws, n, clock_khz, st);
-      EIG_HIP(ctx, hipStreamEndCapture(st, &graph));
-      EIG_HIP(ctx, hipGraphInstantiate(&G.exec, graph, nullptr, nullptr, 0));
-      hipGraphDestroy(graph);
-      G.n = n;
-      G.a = ws.a;
-    }
-    EIG_HIP(ctx, hipGraphLaunch(G.exec, st));
-  } else {
-    launch_tridiag(ws, n, clock_khz, st);
-  }
+  launch_tridiag(ws, n, clock_khz, st);
   EIG_HIP(ctx, hipGetLastError());
   tend("tridiag");
   // ---- eigenvalues
