@@ -947,8 +947,8 @@ constexpr int kInvB = 16;  // recurrence steps per batch of loads
 // (the pivoted LU of T - lambda I), kInvStart (start vectors), kInvSolve and kInvGs (per
 // iteration: the two triangular solves, then Gram-Schmidt against the batch's earlier
 // vectors of the same cluster and normalisation), for `iters` iterations.  A single
-// batch runs all stages in one launch; longer runs of vectors go in batches with the
-// Gram-Schmidt against earlier batches between a launch's solves and its GS.
+// batch of at most kMaxVec vectors runs all stages in one launch (k_invit); more vectors
+// run the first three per batch (k_invit_batches).
 enum { kInvFactor = 1, kInvStart = 2, kInvSolve = 4, kInvGs = 8, kInvAll = 15 };
 // The LU factors are interleaved over the vectors, so that one recurrence step's
 // accesses of all lanes share a cache line: field f of step i of vector kv sits at
@@ -959,8 +959,8 @@ struct LuCol {
   double *p;  // lu + f * kMaxVec + kv
   __device__ double &operator[](int32_t i) const { return p[(int64_t)i * (kLuF * kMaxVec)]; }
 };
-__global__ __launch_bounds__(256) void k_invit(EigWs ws, int32_t n, int32_t nvec, int32_t j0,
-                                               int32_t flags, int32_t iters) {
+__device__ __forceinline__ void invit_part(const EigWs &ws, int32_t n, int32_t nvec, int32_t j0,
+                                           int32_t flags, int32_t iters) {
   __shared__ double red[4];
   __shared__ double dots[2];
   const double tnorm = ws.sc[S_TNORM];
@@ -1141,6 +1141,137 @@ __global__ __launch_bounds__(256) void k_invit(EigWs ws, int32_t n, int32_t nvec
       __syncthreads();
     }
   }
+}
+
+__global__ __launch_bounds__(256) void k_invit(EigWs ws, int32_t n, int32_t nvec) {
+  // two iterations: the eigenvalues are accurate to a few ulps, so one solve already
+  // leaves contamination of order eps ||T|| / gap from outside a cluster, and the
+  // second squares it (the parity tests pass with one; two keep a margin)
+  invit_part(ws, n, nvec, 0, kInvAll, 2);
+}
+
+// ---- more than kMaxVec vectors ----
+// One block per batch of kMaxVec vectors (vector j of the call's list at XT + j n): LU,
+// start vectors and two solves, each followed by a normalisation (a wave per vector).  The
+// batches of a launch do not depend on each other; the vectors are orthogonalised
+// afterwards.
+__global__ __launch_bounds__(256) void k_invit_batches(EigWs ws, int32_t n, int32_t nvec,
+                                                       int32_t b0, double *__restrict__ XT,
+                                                       double *__restrict__ lu) {
+  const int32_t j0 = (b0 + (int32_t)blockIdx.x) * kMaxVec;
+  const int32_t nb = min(kMaxVec, nvec - j0);
+  ws.X = XT + (int64_t)j0 * n;
+  ws.lu = lu + (int64_t)blockIdx.x * kMaxVec * kLuF * n;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int it = 0; it < 2; ++it) {
+    invit_part(ws, n, nb, j0, (it == 0 ? kInvFactor | kInvStart : 0) | kInvSolve, 1);
+    for (int32_t v = wv; v < nb; v += 4) {
+      double *x = ws.X + (int64_t)v * n;
+      double s = 0.0;
+      for (int32_t i = lane; i < n; i += 64) s += x[i] * x[i];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) s += xlane(s, o);
+      const double inv = 1.0 / sqrt(s);
+      for (int32_t i = lane; i < n; i += 64) x[i] *= inv;
+    }
+    __syncthreads();
+  }
+}
+
+// Orthonormalisation of a batch of nb <= 64 vectors (X, vector v at X + v n) among
+// themselves by its Gram matrix: X <- X R^-1 with G = R^T R (Cholesky), the same vectors
+// as Gram-Schmidt in order.  Its error grows with the square of the batch's condition
+// number, so the caller runs it twice.  Three launches on many blocks instead of 2,016
+// dot products and updates in turn by one block (4 ms an iteration at n = 1,203; all three
+// take 0.085).
+constexpr int kGsRows = 64;
+__global__ __launch_bounds__(256) void k_gs_gram(const double *__restrict__ X, int32_t n, int32_t nb,
+                                                 double *__restrict__ part) {
+  __shared__ double sx[kMaxVec][kGsRows + 1];
+  const int t = threadIdx.x, r0 = blockIdx.x * kGsRows;
+  for (int e = t; e < kMaxVec * kGsRows; e += 256) {
+    const int v = e / kGsRows, i = e % kGsRows;
+    sx[v][i] = (v < nb && r0 + i < n) ? X[(int64_t)v * n + r0 + i] : 0.0;
+  }
+  __syncthreads();
+  const int v0 = (t >> 4) * 4, u0 = (t & 15) * 4;
+  double g[4][4] = {};
+  for (int i = 0; i < kGsRows; ++i)
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) g[a][b] += sx[v0 + a][i] * sx[u0 + b][i];
+  double *out = part + (int64_t)blockIdx.x * kMaxVec * kMaxVec;
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) out[(v0 + a) * kMaxVec + u0 + b] = g[a][b];
+}
+// Rinv (upper triangular, [u][v]) from the nblk partial Gram matrices, summed in order.
+// A vector that depends on the earlier ones to rounding gets a pivot of at least 1e-30 of
+// its square norm, so that the factor stays finite.
+__global__ __launch_bounds__(1024) void k_gs_chol(const double *__restrict__ part, int32_t nblk,
+                                                  int32_t nb, double *__restrict__ Rinv) {
+  __shared__ double G[kMaxVec][kMaxVec + 1], E[kMaxVec][kMaxVec + 1], d0[kMaxVec], d[kMaxVec];
+  const int t = threadIdx.x, c = t & 63, q = t >> 6;
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const int r = q + 16 * h;
+    G[r][c] = sum_strided(part + r * kMaxVec + c, kMaxVec * kMaxVec, 0, 1, nblk);
+    E[r][c] = r == c ? 1.0 : 0.0;
+    if (r == c) d0[r] = G[r][c];
+  }
+  __syncthreads();
+  // elimination of [G | I] without square roots: step k changes the rows below k only,
+  // right of column k in G and up to column k in the inverse, so one barrier a step
+  // separates it from the next (54 us; a Cholesky factor and a back substitution took 103)
+  for (int k = 0; k < nb; ++k) {
+    const double dk = fmax(G[k][k], 1e-30 * d0[k]);
+    if (t == 0) d[k] = dk;
+    const double gk = G[k][c], ek = E[k][c], rk = 1.0 / dk;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const int r = q + 16 * h;
+      if (r > k) {
+        const double m = G[r][k] * rk;
+        if (c > k) G[r][c] -= m * gk;
+        else E[r][c] -= m * ek;
+      }
+    }
+    __syncthreads();
+  }
+  // rows of the inverse over the pivots' roots are L^-1; R^-1 is its transpose
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const int v = q + 16 * h;
+    Rinv[c * kMaxVec + v] = (v < nb && c <= v) ? E[v][c] / sqrt(d[v]) : 0.0;
+  }
+}
+__global__ __launch_bounds__(256) void k_gs_apply(double *__restrict__ X, int32_t n, int32_t nb,
+                                                  const double *__restrict__ Rinv) {
+  __shared__ double sx[kMaxVec][kGsRows + 1], sr[kMaxVec][kMaxVec];
+  const int t = threadIdx.x, r0 = blockIdx.x * kGsRows;
+  for (int e = t; e < kMaxVec * kGsRows; e += 256) {
+    const int v = e / kGsRows, i = e % kGsRows;
+    sx[v][i] = (v < nb && r0 + i < n) ? X[(int64_t)v * n + r0 + i] : 0.0;
+    sr[e / kMaxVec][e % kMaxVec] = Rinv[e];
+  }
+  __syncthreads();
+  const int i = t & 63;
+  for (int v = t >> 6; v < nb; v += 4) {
+    double s = 0.0;
+    for (int u = 0; u <= v; ++u) s += sx[u][i] * sr[u][v];
+    if (r0 + i < n) X[(int64_t)v * n + r0 + i] = s;
+  }
+}
+
+// zeros in place of what the matrix held left of each reflector's first entry within its
+// panel (rows c0 .. c0 + q of reflector q), so that a panel is a plain n x 32 operand
+__global__ void k_bt_clean(EigWs ws, int32_t n, int32_t last) {
+  const int32_t c = blockIdx.x * 8 + (threadIdx.x >> 5), i = threadIdx.x & 31;
+  if (c > last) return;
+  const int32_t c0 = c / kNB * kNB;
+  if (c0 + i <= c) ws.a[(int64_t)c * ws.lda + c0 + i] = 0.0;
 }
 
 // ---------------------------------------------------------------- back-transform
@@ -1544,11 +1675,11 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
   }
   EIG_HIP(ctx, hipGetLastError());
   tend("bisect");
-  // ---- eigenvectors: one batch of at most kMaxVec (inverse iteration, back-transform,
-  // sign rule), or, for more vectors, batches of kMaxVec in eigenvalue order with
-  // each iteration's vectors orthogonalised against the earlier batches' vectors of
-  // the same cluster (classical Gram-Schmidt, twice, as FP64 MFMA products) between
-  // the solves and the batch's own Gram-Schmidt
+  // ---- eigenvectors: one batch of at most kMaxVec (inverse iteration with Gram-Schmidt,
+  // back-transform, sign rule); more vectors run in batches of kMaxVec in eigenvalue
+  // order: every batch's solves, then batch by batch the Gram-Schmidt against the earlier
+  // vectors and within the batch, then the back-transform of all
+  // vectors together as FP64 MFMA products
   const int32_t last = n - 2;  // last reflector row
   const int32_t p_last = last >= 0 ? last / kNB : -1;
   auto back_transform = [&](int32_t nb) -> int {
@@ -1570,10 +1701,7 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
   };
   tbeg();
   if (nvec > 0 && nvec <= kMaxVec) {
-    // two iterations: the eigenvalues are accurate to a few ulps, so one solve already
-    // leaves contamination of order eps ||T|| / gap from outside a cluster, and the
-    // second squares it (the parity tests pass with one; two keep a margin)
-    hipLaunchKernelGGL(k_invit, dim3(1), dim3(256), 0, st, ws, n, nvec, 0, (int32_t)kInvAll, 2);
+    hipLaunchKernelGGL(k_invit, dim3(1), dim3(256), 0, st, ws, n, nvec);
     tend("invit");
     tbeg();
     if (last >= 0) {
@@ -1583,52 +1711,68 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
     }
     EIG_TRY(back_transform(nvec));
   } else if (nvec > kMaxVec) {
-    // the T-basis vectors of all batches (vector j at j*N) and the CGS coefficients
-    EIG_TRY(eig_ensure(ctx, ctx->evall, sizeof(double) * ((size_t)N * nvec + (size_t)kMaxVec * nvec)));
-    double *XT = (double *)ctx->evall.p, *Cc = XT + (size_t)N * nvec;
-    std::vector<double> ev(N);
-    double sc[S_COUNT];
-    EIG_HIP(ctx, hipMemcpyAsync(ev.data(), ws.eval, sizeof(double) * N, hipMemcpyDeviceToHost, st));
-    EIG_HIP(ctx, hipMemcpyAsync(sc, ws.sc, sizeof(sc), hipMemcpyDeviceToHost, st));
-    EIG_HIP(ctx, hipStreamSynchronize(st));
-    const double tol = 1e-3 * sc[S_TNORM];  // the cluster criterion of k_invit
+    // all vectors (vector j at j N), the Gram-Schmidt and back-transform coefficients, the
+    // partial Gram matrices, R^-1, and the LU factors of as many batches as 2 GiB hold
+    const int32_t nbatch = (nvec + kMaxVec - 1) / kMaxVec, nblk = (n + kGsRows - 1) / kGsRows;
+    const size_t lub = (size_t)kMaxVec * kLuF * N;
+    const int32_t group = (int32_t)std::max<size_t>(1, std::min<size_t>(nbatch, ((size_t)1 << 28) / lub));
+    const size_t sq = (size_t)kMaxVec * kMaxVec;
+    EIG_TRY(eig_ensure(ctx, ctx->evall, sizeof(double) * ((size_t)N * nvec + (size_t)kMaxVec * nvec +
+                                                          sq * nblk + sq + lub * group)));
+    double *XT = (double *)ctx->evall.p, *Cc = XT + (size_t)N * nvec, *gp = Cc + (size_t)kMaxVec * nvec,
+           *Ri = gp + sq * nblk, *lu = Ri + sq;
+    for (int32_t b = 0; b < nbatch; b += group)
+      hipLaunchKernelGGL(k_invit_batches, dim3((unsigned)std::min(group, nbatch - b)), dim3(256), 0, st,
+                         ws, n, nvec, b, XT, lu);
+    EIG_HIP(ctx, hipGetLastError());
+    // against every earlier vector, not only those of close eigenvalues: the products are
+    // a small part, and vectors a few 1e-3 ||T|| apart stay orthogonal to the last ulps
+    for (int32_t j0 = 0; j0 < nvec; j0 += kMaxVec) {
+      const int32_t nb = std::min<int32_t>(kMaxVec, nvec - j0), nc = j0;
+      double *X = XT + (size_t)j0 * N;
+      const double *P = XT;
+      for (int rep = 0; rep < 2; ++rep) {
+        if (nc > 0) {
+          EIG_TRY(eig_gemm_f64(ctx, st, true, false, nc, nb, N, 1.0, P, N, 0, X, N, 0, 0.0, Cc, nc, 0, 1));
+          EIG_TRY(eig_gemm_f64(ctx, st, false, false, N, nb, nc, -1.0, P, N, 0, Cc, nc, 0, 1.0, X, N, 0, 1));
+        }
+        hipLaunchKernelGGL(k_gs_gram, dim3((unsigned)nblk), dim3(256), 0, st, (const double *)X, n, nb, gp);
+        hipLaunchKernelGGL(k_gs_chol, dim3(1), dim3(1024), 0, st, (const double *)gp, nblk, nb, Ri);
+        hipLaunchKernelGGL(k_gs_apply, dim3((unsigned)nblk), dim3(256), 0, st, X, n, nb, (const double *)Ri);
+      }
+    }
+    EIG_HIP(ctx, hipGetLastError());
+    tend("invit");
+    tbeg();
     if (last >= 0) {
       hipLaunchKernelGGL(k_bt_gram, dim3((unsigned)(p_last + 1), kBtSplit), dim3(256), 0, st, ws, n,
                          last);
       hipLaunchKernelGGL(k_bt_prep, dim3((unsigned)(p_last + 1)), dim3(256), 0, st, ws, n, last);
-    }
-    for (int32_t j0 = 0; j0 < nvec; j0 += kMaxVec) {
-      const int32_t nb = std::min<int32_t>(kMaxVec, nvec - j0);
-      int32_t c0 = j0;  // earlier vectors within tol of eigenvalue j0 (descending order)
-      while (c0 > 0 && std::fabs(ev[N - 1 - (c0 - 1)] - ev[N - 1 - j0]) <= tol) --c0;
-      const int32_t nc = j0 - c0;
-      for (int it = 0; it < 3; ++it) {
-        const int32_t f = (it == 0 ? (kInvFactor | kInvStart) : 0) | kInvSolve;
-        hipLaunchKernelGGL(k_invit, dim3(1), dim3(256), 0, st, ws, n, nb, j0, f, 1);
-        for (int rep = 0; rep < 2 && nc > 0; ++rep) {
-          const double *P = XT + (size_t)c0 * N;
-          EIG_TRY(eig_gemm_f64(ctx, st, true, false, nc, nb, N, 1.0, P, N, 0, ws.X, N, 0, 0.0, Cc,
-                               nc, 0, 1));
-          EIG_TRY(eig_gemm_f64(ctx, st, false, false, N, nb, nc, -1.0, P, N, 0, Cc, nc, 0, 1.0,
-                               ws.X, N, 0, 1));
-        }
-        hipLaunchKernelGGL(k_invit, dim3(1), dim3(256), 0, st, ws, n, nb, j0, (int32_t)kInvGs, 1);
+      hipLaunchKernelGGL(k_bt_clean, dim3((unsigned)(last / 8 + 1)), dim3(256), 0, st, ws, n, last);
+      double *Z = Cc + (size_t)kNB * nvec;
+      for (int32_t p = p_last; p >= 0; --p) {
+        const int32_t c0 = p * kNB, np = std::min(kNB, last - c0 + 1);
+        const int64_t rows = N - c0 - 1;
+        const double *Vp = ws.a + (size_t)c0 * lda + c0 + 1;
+        EIG_TRY(eig_gemm_f64(ctx, st, true, false, np, nvec, rows, 1.0, Vp, lda, 0, XT + c0 + 1, N, 0,
+                             0.0, Cc, kNB, 0, 1));
+        EIG_TRY(eig_gemm_f64(ctx, st, true, false, np, nvec, np, 1.0, ws.Tall + (size_t)p * kNB * kNB,
+                             kNB, 0, Cc, kNB, 0, 0.0, Z, kNB, 0, 1));
+        EIG_TRY(eig_gemm_f64(ctx, st, false, false, rows, nvec, np, -1.0, Vp, lda, 0, Z, kNB, 0, 1.0,
+                             XT + c0 + 1, N, 0, 1));
       }
-      EIG_HIP(ctx, hipMemcpyAsync(XT + (size_t)j0 * N, ws.X, sizeof(double) * N * nb,
+    }
+    EigWs wx = ws;
+    wx.X = XT;
+    hipLaunchKernelGGL(k_finish_vec, dim3((unsigned)nvec), dim3(256), 0, st, wx, n);
+    EIG_HIP(ctx, hipGetLastError());
+    if (evecs)
+      EIG_HIP(ctx, hipMemcpyAsync(evecs, XT, sizeof(double) * N * nvec, hipMemcpyDeviceToHost, st));
+    if (!internal) {
+      EIG_TRY(eig_ensure(ctx, ctx->evecs_dev, sizeof(double) * N * kMaxVec));
+      EIG_HIP(ctx, hipMemcpyAsync(ctx->evecs_dev.p, XT, sizeof(double) * N * kMaxVec,
                                   hipMemcpyDeviceToDevice, st));
-      EIG_TRY(back_transform(nb));
-      if (evecs)
-        EIG_HIP(ctx, hipMemcpyAsync(evecs + (size_t)j0 * N, ws.X, sizeof(double) * N * nb,
-                                    hipMemcpyDeviceToHost, st));
-      if (!internal && j0 == 0) {
-        EIG_TRY(eig_ensure(ctx, ctx->evecs_dev, sizeof(double) * N * kMaxVec));
-        EIG_HIP(ctx, hipMemcpyAsync(ctx->evecs_dev.p, ws.X, sizeof(double) * N * kMaxVec,
-                                    hipMemcpyDeviceToDevice, st));
-      }
     }
-    EIG_HIP(ctx, hipStreamSynchronize(st));
-    tend("invit");
-    tbeg();
   } else {
     tend("invit");
     tbeg();
