@@ -27,6 +27,7 @@ UNITS = {
     "ctx.hip": False,
     "syrk.hip": True,
     "xdigit.hip": False,
+    "codes.hip": False,
     "eigh.hip": True,
     "project.hip": False,
     "serve.hip": False,

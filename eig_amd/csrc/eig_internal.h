@@ -149,3 +149,48 @@ int eig_gemm_f64(eig_ctx *ctx, hipStream_t st, bool ta, bool tb, int64_t m, int6
 // no data), *d_itype = the types on the device.
 int eig_lsq_filltab(eig_ctx *ctx, const int32_t *use, const int32_t *itype, int32_t npop,
                     int32_t K, double **fill, const int32_t **d_itype);
+
+// ---- products of packed codes with FP64 columns (codes.hip) ------------------
+// The code words of a set of rows: row r's words pairs q = 0..3 of stage b (128 codes)
+// at row base + b * KB + (q >> 1) * QH + (q & 1) * 8; row base = rows[r], or base +
+// (r >> 7) * RT + (r & 127) * RS.  nword 16-code words per row are valid.
+enum { kCodeLinear = 0, kCodeGrouped = 1, kCodeBytes = 2 };
+struct CodeView {
+  const uint8_t *base;
+  const uint8_t *const *rows;
+  int64_t RT, RS, KB, QH;
+  int64_t nrow, nword;
+  int32_t layout;
+};
+// columns: what kind of values, and where they are (see col_value)
+enum { kColPanel, kColAxes, kColLevB, kColFx, kColLsqR, kColLsqG };
+struct CodeCols {
+  int kind;
+  const double *a;
+  int64_t ld, n;
+  const double *lev = nullptr, *fancy = nullptr, *xmean = nullptr;
+  const uint8_t *ignore = nullptr;
+  const double *fxscal = nullptr;
+  int32_t K = 0;
+};
+enum { kCdPair, kCdSum, kCdMiss };
+struct CodesPlan {
+  int mode;
+  int32_t C, ngroup, Cg, NT, nrowblk, nsplit;
+  int64_t nblk, per, rowpad;
+  size_t head_bytes, dig_bytes, part_bytes;
+};
+// one INT32 sum holds this many terms (digit 128, code 3)
+constexpr int64_t kCodesMaxK = (int64_t)5 << 20;
+CodesPlan eig_codes_plan(const eig_ctx *ctx, int mode, int32_t C, int64_t nrow, int64_t nblk,
+                         int32_t smax);
+int eig_codes_scales(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, void *head, hipStream_t st);
+int eig_codes_restart(eig_ctx *ctx, const CodesPlan &P, void *head, hipStream_t st);
+int eig_codes_mul(eig_ctx *ctx, const CodesPlan &P, const CodeView &v, const CodeCols &cols, int64_t b0,
+                  void *head, void *dig, void *part, bool accum, hipStream_t st);
+int eig_codes_out_sum(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void *head, const void *part,
+                      double scale, double *out, int64_t ldr, int64_t ldc, int32_t Cpad, bool add,
+                      hipStream_t st);
+int eig_codes_out_pair(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void *head, const void *part,
+                       const double *lev, const uint8_t *ignore, double scale, double *out, int64_t ldr,
+                       int64_t ldc, hipStream_t st);

@@ -12,27 +12,21 @@
 // singular vectors of B (from the eigen-decomposition of B^T B) are the
 // eigenvectors, S^2 / ncols the eigenvalues (kjg_fpca.c:79-95).
 //
-// The two panel products read X straight from the 2-bit sample-tile layout and
-// multiply on FP64 MFMA (16x16x4), or, in the split-BF16 form, on BF16 MFMA
-// (32x32x16) over hi/lo splits; both are persistent kernels whose grid and
-// split-K factor are picked by a timing tuner on the first call for a shape, and
-// the 2I+1 products of the power iteration are replayed as one captured graph.
-// The instances of up to 32 columns load each step's operands while the previous
-// step's MFMAs run (two LDS buffers, one barrier per step).  The tall-skinny Gram
-// and basis products run on the library's FP64 MFMA GEMM (gemm.hip).
+// The two panel products read X straight from packed codes: in the FP64 form as exact
+// integer products with fixed-point digits of the panel (codes.hip), in the split-BF16
+// form on BF16 MFMA (32x32x16) over hi/lo splits.  The BF16 instances of up to 32 columns
+// load each step's operands while the previous step's MFMAs run (two LDS buffers, one
+// barrier per step).  The tall-skinny Gram and basis products run on the library's FP64
+// MFMA GEMM (gemm.hip).
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <mutex>
 #include <vector>
 
 #include "eig_internal.h"
 
-typedef __attribute__((__vector_size__(4 * sizeof(double)))) double f64x4;
-
 namespace {
-constexpr int kKC = 32;       // samples (X A) or SNPs (X^T B) per LDS stage
 constexpr int kMaxCT = 16;    // column tiles of 16 -> at most 256 columns
 constexpr int kJacMax = 256;  // order limit of the one-block Jacobi eigensolver
 }  // namespace
@@ -89,355 +83,6 @@ __global__ void k_fpca_gauss(double *__restrict__ A, int32_t npad, int32_t lda, 
     z = sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
   }
   A[idx] = z;
-}
-
-// ---------------------------------------------------------------- Y = X A
-// Persistent over SNP tiles of 128 (4 waves x 32 SNPs); each wave holds a
-// 32 x 16CT FP64 accumulator.  A: npad x lda (rows = samples, zero padded);
-// Y rows m, columns [0, C) at Y[m * ldy + c].
-template <int CT>
-__global__ __launch_bounds__(256) void k_fpca_xa(const uint32_t *__restrict__ sel, int64_t M,
-                                                 int32_t nst, const double *__restrict__ lf,
-                                                 const double *__restrict__ A, int32_t lda,
-                                                 double *__restrict__ Y, int64_t ldy, int32_t C) {
-  __shared__ double sA[kKC][16 * CT];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t ntiles = (M + 127) / 128;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t mb = tile * 128 + 32 * w;
-    int64_t r[2];
-    double lv[2][3];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      r[t] = mb + 16 * t + (lane & 15);
-      const bool ok = r[t] < M;
-#pragma unroll
-      for (int g = 0; g < 3; ++g) lv[t][g] = ok ? lf[4 * r[t] + g] : 0.0;
-    }
-    f64x4 acc[2][CT];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c) acc[t][c] = f64x4{0.0, 0.0, 0.0, 0.0};
-    for (int32_t st = 0; st < nst; ++st) {
-      for (int kc = 0; kc < kTileS; kc += kKC) {
-        __syncthreads();
-        const double *src = A + (int64_t)(st * kTileS + kc) * lda;
-        for (int idx = threadIdx.x; idx < kKC * 16 * CT; idx += 256) {
-          const int k = idx / (16 * CT), c = idx % (16 * CT);
-          sA[k][c] = src[(int64_t)k * lda + c];
-        }
-        __syncthreads();
-        uint32_t wd[2][2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          if (r[t] < M) {
-            const uint2 v = *(const uint2 *)(sel + ((int64_t)st * M + r[t]) * kTileWords + kc / 16);
-            wd[t][0] = v.x;
-            wd[t][1] = v.y;
-          } else {
-            wd[t][0] = wd[t][1] = ~0u;
-          }
-        }
-#pragma unroll
-        for (int ks = 0; ks < kKC / 4; ++ks) {
-          const int sh = 2 * ((ks & 3) * 4 + (lane >> 4));
-          double a[2];
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            const uint32_t code = (wd[t][ks >> 2] >> sh) & 3u;
-            a[t] = code == 0 ? lv[t][0] : (code == 1 ? lv[t][1] : (code == 2 ? lv[t][2] : 0.0));
-          }
-#pragma unroll
-          for (int c = 0; c < CT; ++c) {
-            const double b = sA[4 * ks + (lane >> 4)][16 * c + (lane & 15)];
-            acc[0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], b, acc[0][c], 0, 0, 0);
-            acc[1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], b, acc[1][c], 0, 0, 0);
-          }
-        }
-      }
-    }
-    // accumulator layout: lane l, element e -> row l/16 + 4e, column l%16
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t row = mb + 16 * t + (lane >> 4) + 4 * e;
-          const int col = 16 * c + (lane & 15);
-          if (row < M && col < C) Y[row * ldy + col] = acc[t][c][e];
-        }
-  }
-}
-
-// The same Y = X A with the next sample stage's loads (the panel rows and each
-// lane's genotype words) issued before the current stage's MFMAs: the panel stage
-// goes global -> registers -> one of two LDS buffers, one barrier per stage.  For
-// CT <= 2, as k_fpca_xtb_pf.
-template <int CT>
-__global__ __launch_bounds__(256, 4) void k_fpca_xa_pf(const uint32_t *__restrict__ sel,
-                                                       int64_t M, int32_t nst,
-                                                       const double *__restrict__ lf,
-                                                       const double *__restrict__ A, int32_t lda,
-                                                       double *__restrict__ Y, int64_t ldy,
-                                                       int32_t C) {
-  constexpr int kAE = kKC * 16 * CT / 256;  // panel elements per thread per stage
-  constexpr int kStT = kTileS / kKC;        // stages per sample tile
-  __shared__ double sA[2][kKC][16 * CT];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int64_t ntiles = (M + 127) / 128;
-  const int32_t nstage = nst * kStT;
-  double ra[kAE];
-  uint2 rw[2];
-  int buf = 0;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t mb = tile * 128 + 32 * w;
-    int64_t r[2];
-    double lv[2][3];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      r[t] = mb + 16 * t + (lane & 15);
-      const bool ok = r[t] < M;
-#pragma unroll
-      for (int g = 0; g < 3; ++g) lv[t][g] = ok ? lf[4 * r[t] + g] : 0.0;
-    }
-    auto fetch = [&](int32_t q) {
-      const int32_t st = q / kStT, kc = (q % kStT) * kKC;
-      const double *src = A + (int64_t)(st * kTileS + kc) * lda;
-#pragma unroll
-      for (int j = 0; j < kAE; ++j) {
-        const int idx = tid + 256 * j;
-        ra[j] = src[(int64_t)(idx / (16 * CT)) * lda + idx % (16 * CT)];
-      }
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-        rw[t] = r[t] < M ? *(const uint2 *)(sel + ((int64_t)st * M + r[t]) * kTileWords + kc / 16)
-                         : make_uint2(~0u, ~0u);
-    };
-    f64x4 acc[2][CT];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c) acc[t][c] = f64x4{0.0, 0.0, 0.0, 0.0};
-    fetch(0);
-    for (int32_t q = 0; q < nstage; ++q) {
-#pragma unroll
-      for (int j = 0; j < kAE; ++j) {
-        const int idx = tid + 256 * j;
-        sA[buf][idx / (16 * CT)][idx % (16 * CT)] = ra[j];
-      }
-      const uint32_t wd[2][2] = {{rw[0].x, rw[0].y}, {rw[1].x, rw[1].y}};
-      // the other buffer was last read before this barrier's previous instance
-      __syncthreads();
-      if (q + 1 < nstage) fetch(q + 1);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < kKC / 4; ++ks) {
-        const int sh = 2 * ((ks & 3) * 4 + (lane >> 4));
-        double a[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const uint32_t code = (wd[t][ks >> 2] >> sh) & 3u;
-          a[t] = code == 0 ? lv[t][0] : (code == 1 ? lv[t][1] : (code == 2 ? lv[t][2] : 0.0));
-        }
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-          const double b = sA[buf][4 * ks + (lane >> 4)][16 * c + (lane & 15)];
-          acc[0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], b, acc[0][c], 0, 0, 0);
-          acc[1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], b, acc[1][c], 0, 0, 0);
-        }
-      }
-      buf ^= 1;
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t row = mb + 16 * t + (lane >> 4) + 4 * e;
-          const int col = 16 * c + (lane & 15);
-          if (row < M && col < C) Y[row * ldy + col] = acc[t][c][e];
-        }
-  }
-}
-
-// ---------------------------------------------------------------- partial X^T B
-// Persistent over (sample tile, SNP split) items; a block covers one sample tile
-// (4 waves x 32 samples) and SNPs [s*mchunk, min(M, (s+1)*mchunk)).  B: rows m,
-// columns [0, C) at B[m * ldb + c] (columns >= C read as 0).  part[s][i][c],
-// i < nst*128, c < 16CT (row stride ldp).
-template <int CT>
-__global__ __launch_bounds__(256) void k_fpca_xtb(const uint32_t *__restrict__ sel, int64_t M,
-                                                  int32_t nst, const double *__restrict__ lf,
-                                                  const double *__restrict__ B, int64_t ldb,
-                                                  int32_t C, int32_t S, int64_t mchunk,
-                                                  double *__restrict__ part, int32_t ldp) {
-  __shared__ double sB[kKC][16 * CT];
-  __shared__ double sL[kKC][4];
-  __shared__ uint32_t sW[kKC][kTileWords];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t items = (int64_t)nst * S;
-  const int64_t npad = (int64_t)nst * kTileS;
-  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
-    const int32_t st = (int32_t)(it % nst), s = (int32_t)(it / nst);
-    const int64_t m0 = (int64_t)s * mchunk, m1 = min(M, m0 + mchunk);
-    f64x4 acc[2][CT];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c) acc[t][c] = f64x4{0.0, 0.0, 0.0, 0.0};
-    for (int64_t mb = m0; mb < m1; mb += kKC) {
-      __syncthreads();
-      for (int idx = threadIdx.x; idx < kKC * 16 * CT; idx += 256) {
-        const int k = idx / (16 * CT), c = idx % (16 * CT);
-        const int64_t m = mb + k;
-        sB[k][c] = (m < m1 && c < C) ? B[m * ldb + c] : 0.0;
-      }
-      if (threadIdx.x < kKC * 4) {
-        const int k = threadIdx.x >> 2, g = threadIdx.x & 3;
-        const int64_t m = mb + k;
-        sL[k][g] = m < m1 ? lf[4 * m + g] : 0.0;
-      } else if (threadIdx.x < kKC * 4 + kKC * kTileWords / 2) {
-        const int q = threadIdx.x - kKC * 4;  // one uint2 of one SNP's tile record
-        const int k = q >> 2, wv = (q & 3) * 2;
-        const int64_t m = mb + k;
-        uint2 v = make_uint2(~0u, ~0u);
-        if (m < m1) v = *(const uint2 *)(sel + ((int64_t)st * M + m) * kTileWords + wv);
-        sW[k][wv] = v.x;
-        sW[k][wv + 1] = v.y;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int ks = 0; ks < kKC / 4; ++ks) {
-        const int k = 4 * ks + (lane >> 4);
-        double a[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int sl = 32 * w + 16 * t + (lane & 15);  // sample within the tile
-          const uint32_t code = (sW[k][sl >> 4] >> (2 * (sl & 15))) & 3u;
-          a[t] = sL[k][code];
-        }
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-          const double b = sB[k][16 * c + (lane & 15)];
-          acc[0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], b, acc[0][c], 0, 0, 0);
-          acc[1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], b, acc[1][c], 0, 0, 0);
-        }
-      }
-    }
-    double *out = part + ((int64_t)s * npad + (int64_t)st * kTileS) * ldp;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = 32 * w + 16 * t + (lane >> 4) + 4 * e;
-          out[(int64_t)row * ldp + 16 * c + (lane & 15)] = acc[t][c][e];
-        }
-  }
-}
-
-// The same partial X^T B with the next SNP stage's loads issued before the current
-// stage's MFMAs: the stage goes global -> registers -> one of two LDS buffers, so
-// one barrier per stage suffices and the load latency hides behind 8 MFMA steps.
-// For CT <= 2, whose prefetch registers fit beside the accumulators at four waves
-// per SIMD (wider instances spill there).
-template <int CT>
-__global__ __launch_bounds__(256, 4) void k_fpca_xtb_pf(const uint32_t *__restrict__ sel, int64_t M,
-                                                     int32_t nst, const double *__restrict__ lf,
-                                                     const double *__restrict__ B, int64_t ldb,
-                                                     int32_t C, int32_t S, int64_t mchunk,
-                                                     double *__restrict__ part, int32_t ldp) {
-  constexpr int kBE = kKC * 16 * CT / 256;  // B elements per thread per stage
-  static_assert(kKC * 4 == 128 && kKC * kTileWords / 2 == 128, "stage loads take 256 threads");
-  __shared__ double sB[2][kKC][16 * CT];
-  __shared__ double sL[2][kKC][4];
-  __shared__ uint32_t sW[2][kKC][kTileWords];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int64_t items = (int64_t)nst * S;
-  const int64_t npad = (int64_t)nst * kTileS;
-  double rb[kBE];
-  double rl = 0.0;
-  uint2 rw = make_uint2(~0u, ~0u);
-  int buf = 0;
-  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
-    const int32_t st = (int32_t)(it % nst), s = (int32_t)(it / nst);
-    const int64_t m0 = (int64_t)s * mchunk, m1 = min(M, m0 + mchunk);
-    // threads 0..127: level (k, g) = (tid/4, tid%4); 128..255: uint2 q of SNP k's record
-    auto fetch = [&](int64_t mb) {
-#pragma unroll
-      for (int j = 0; j < kBE; ++j) {
-        const int idx = tid + 256 * j;
-        const int k = idx / (16 * CT), c = idx % (16 * CT);
-        const int64_t m = mb + k;
-        rb[j] = (m < m1 && c < C) ? B[m * ldb + c] : 0.0;
-      }
-      if (tid < 128) {
-        const int64_t m = mb + (tid >> 2);
-        rl = m < m1 ? lf[4 * m + (tid & 3)] : 0.0;
-      } else {
-        const int q = tid - 128;
-        const int64_t m = mb + (q >> 2);
-        rw = make_uint2(~0u, ~0u);
-        if (m < m1) rw = *(const uint2 *)(sel + ((int64_t)st * M + m) * kTileWords + (q & 3) * 2);
-      }
-    };
-    f64x4 acc[2][CT];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c) acc[t][c] = f64x4{0.0, 0.0, 0.0, 0.0};
-    if (m0 < m1) fetch(m0);
-    for (int64_t mb = m0; mb < m1; mb += kKC) {
-#pragma unroll
-      for (int j = 0; j < kBE; ++j) {
-        const int idx = tid + 256 * j;
-        sB[buf][idx / (16 * CT)][idx % (16 * CT)] = rb[j];
-      }
-      if (tid < 128) {
-        sL[buf][tid >> 2][tid & 3] = rl;
-      } else {
-        const int q = tid - 128;
-        sW[buf][q >> 2][(q & 3) * 2] = rw.x;
-        sW[buf][q >> 2][(q & 3) * 2 + 1] = rw.y;
-      }
-      // the other buffer was last read before this barrier's previous instance
-      __syncthreads();
-      if (mb + kKC < m1) fetch(mb + kKC);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < kKC / 4; ++ks) {
-        const int k = 4 * ks + (lane >> 4);
-        double a[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int sl = 32 * w + 16 * t + (lane & 15);  // sample within the tile
-          const uint32_t code = (sW[buf][k][sl >> 4] >> (2 * (sl & 15))) & 3u;
-          a[t] = sL[buf][k][code];
-        }
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-          const double b = sB[buf][k][16 * c + (lane & 15)];
-          acc[0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], b, acc[0][c], 0, 0, 0);
-          acc[1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], b, acc[1][c], 0, 0, 0);
-        }
-      }
-      buf ^= 1;
-    }
-    double *out = part + ((int64_t)s * npad + (int64_t)st * kTileS) * ldp;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = 32 * w + 16 * t + (lane >> 4) + 4 * e;
-          out[(int64_t)row * ldp + 16 * c + (lane & 15)] = acc[t][c][e];
-        }
-  }
 }
 
 // out[i][c] = scale * sum_s part[s][i][c] (splits in order) for c < min(ldp, ldo);
@@ -989,43 +634,6 @@ __global__ __launch_bounds__(1024) void k_jacobi(double *__restrict__ A, int32_t
 }
 
 // ---------------------------------------------------------------- host side
-struct FpcaTune {
-  int64_t M = -1;
-  int32_t nst = -1, CT = -1;
-  int32_t grid = 0, S = 0;
-};
-
-struct FpcaState {
-  hipGraphExec_t gexec = nullptr;
-  // everything the captured power-iteration graph bakes in: buffer addresses (the
-  // workspace base and every offset in it), shape, form, launch shapes and the 1/ncols
-  // scale; a call whose signature differs re-captures
-  std::vector<int64_t> gsig;
-  FpcaTune xa[kMaxCT + 1], xtb[kMaxCT + 1];
-  // held for the whole call: the graph and the tuners are shared by
-  // every context on the device
-  std::mutex mu;
-};
-static FpcaState g_fpca[16];
-
-#define FP_KCASE(n, ...) \
-  case n: {              \
-    constexpr int CT = n; \
-    __VA_ARGS__;         \
-  } break;
-#define FP_CTSWITCH(ctx, ct, ...)                                                            \
-  switch (ct) {                                                                              \
-    FP_KCASE(1, __VA_ARGS__) FP_KCASE(2, __VA_ARGS__) FP_KCASE(3, __VA_ARGS__)               \
-    FP_KCASE(4, __VA_ARGS__) FP_KCASE(5, __VA_ARGS__) FP_KCASE(6, __VA_ARGS__)               \
-    FP_KCASE(7, __VA_ARGS__) FP_KCASE(8, __VA_ARGS__) FP_KCASE(9, __VA_ARGS__)               \
-    FP_KCASE(10, __VA_ARGS__) FP_KCASE(11, __VA_ARGS__) FP_KCASE(12, __VA_ARGS__)            \
-    FP_KCASE(13, __VA_ARGS__) FP_KCASE(14, __VA_ARGS__) FP_KCASE(15, __VA_ARGS__)            \
-    FP_KCASE(16, __VA_ARGS__)                                                                \
-    default:                                                                                 \
-      return eig_set_err(ctx, EIG_E_ARG, "fpca: column count out of range");                 \
-  }
-
-
 namespace {
 struct Plan {
   int64_t M;
@@ -1034,100 +642,6 @@ struct Plan {
   const double *lf;
 };
 }  // namespace
-
-static int launch_xa(eig_ctx *ctx, const Plan &P, int CT, int grid, const double *A, int32_t lda,
-                     double *Y, int64_t ldy, int32_t C, hipStream_t st) {
-  FP_CTSWITCH(ctx, CT,
-              if constexpr (CT <= 2) hipLaunchKernelGGL((k_fpca_xa_pf<CT>), dim3(grid), dim3(256),
-                                                        0, st, P.sel, P.M, P.nst, P.lf, A, lda, Y,
-                                                        ldy, C);
-              else hipLaunchKernelGGL((k_fpca_xa<CT>), dim3(grid), dim3(256), 0, st, P.sel, P.M,
-                                      P.nst, P.lf, A, lda, Y, ldy, C));
-  return EIG_OK;
-}
-
-static int launch_xtb(eig_ctx *ctx, const Plan &P, int CT, int grid, int S, const double *B,
-                      int64_t ldb, int32_t C, double *part, double *out, int32_t ldo, double scale,
-                      hipStream_t st) {
-  const int64_t mchunk = ((P.M + S - 1) / S + kKC - 1) / kKC * kKC;
-  const int32_t ldp = 16 * CT;
-  FP_CTSWITCH(ctx, CT,
-              if constexpr (CT <= 2) hipLaunchKernelGGL((k_fpca_xtb_pf<CT>), dim3(grid), dim3(256),
-                                                        0, st, P.sel, P.M, P.nst, P.lf, B, ldb, C,
-                                                        S, mchunk, part, ldp);
-              else hipLaunchKernelGGL((k_fpca_xtb<CT>), dim3(grid), dim3(256), 0, st, P.sel, P.M,
-                                      P.nst, P.lf, B, ldb, C, S, mchunk, part, ldp));
-  const int64_t tot = (int64_t)P.npad * ldp;
-  hipLaunchKernelGGL(k_fpca_reduce, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st,
-                     (const double *)part, S, (int64_t)P.npad, ldp, scale, out, ldo);
-  return EIG_OK;
-}
-
-template <class Fn>
-static int time_launch(eig_ctx *ctx, Fn &&fn, float &ms) {
-  hipStream_t st = ctx->stream;
-  EIG_HIP(ctx, hipEventRecord(ctx->ev0, st));
-  int rc = fn();
-  if (rc != EIG_OK) return rc;
-  EIG_HIP(ctx, hipEventRecord(ctx->ev1, st));
-  EIG_HIP(ctx, hipEventSynchronize(ctx->ev1));
-  EIG_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-  return EIG_OK;
-}
-
-// Timing tuner for X A: persistent grid for this shape (A: npad x 16CT, Y scratch).
-static int tune_xa(eig_ctx *ctx, FpcaState &F, const Plan &P, int CT, const double *A,
-                   int32_t lda, double *Y, int64_t ldy) {
-  FpcaTune &ta = F.xa[CT];
-  hipStream_t st = ctx->stream;
-  const int cu = ctx->num_cu;
-  if (ta.M != P.M || ta.nst != P.nst) {
-    float best = 1e30f;
-    for (int gm : {1, 2, 4}) {
-      const int grid = (int)std::min<int64_t>((int64_t)gm * cu, (P.M + 127) / 128);
-      float ms = 0.f;
-      EIG_TRY(time_launch(
-          ctx, [&] { return launch_xa(ctx, P, CT, grid, A, lda, Y, ldy, 16 * CT, st); }, ms));
-      if (ms < best) {
-        best = ms;
-        ta.grid = grid;
-      }
-    }
-    ta.M = P.M;
-    ta.nst = P.nst;
-  }
-  return EIG_OK;
-}
-
-// Timing tuner for X^T B: persistent grid and split count (B: M x >= 16CT, out scratch).
-static int tune_xtb(eig_ctx *ctx, FpcaState &F, const Plan &P, int CT, const double *B,
-                    int64_t ldb, double *part, int32_t Smax, double *out, int32_t ldo) {
-  FpcaTune &tb = F.xtb[CT];
-  hipStream_t st = ctx->stream;
-  const int cu = ctx->num_cu;
-  if (tb.M != P.M || tb.nst != P.nst) {
-    float best = 1e30f;
-    for (int S : {1, 2, 4, 8}) {
-      if (S > Smax) continue;
-      for (int gm : {1, 2, 4}) {
-        const int grid = (int)std::min<int64_t>((int64_t)gm * cu, (int64_t)P.nst * S);
-        float ms = 0.f;
-        EIG_TRY(time_launch(
-            ctx,
-            [&] { return launch_xtb(ctx, P, CT, grid, S, B, ldb, 16 * CT, part, out, ldo, 1.0, st); },
-            ms));
-        if (ms < best) {
-          best = ms;
-          tb.grid = grid;
-          tb.S = S;
-        }
-      }
-    }
-    tb.M = P.M;
-    tb.nst = P.nst;
-  }
-  return EIG_OK;
-}
 
 // Eigen-decomposition of the n x n symmetric device matrix G (column-major, ld n):
 // eigenvalues descending in w (host), eigenvectors in the columns of V (device,
@@ -1404,8 +918,6 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
                        kJacMax);
   if (!ctx->have_stats) return eig_set_err(ctx, EIG_E_STATE, "eig_fpca before eig_snpstats");
   EIG_HIP(ctx, hipSetDevice(ctx->device));
-  FpcaState &F = g_fpca[ctx->device & 15];
-  std::lock_guard<std::mutex> lock(F.mu);
   hipStream_t st = ctx->stream;
   const int64_t M = ctx->nsnp;
   const int32_t n = ctx->nrows, nst = ctx->nst, npad = nst * kTileS;
@@ -1416,7 +928,7 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   for (int64_t m = 0; m < M; ++m) ncols += status[m] != EIG_SNP_DEAD;
   if (ncols == 0) return eig_set_err(ctx, EIG_E_ARG, "eig_fpca: no SNPs");
 
-  const int CTL = (L + 15) / 16, lda = 16 * CTL;
+  const int lda = 16 * ((L + 15) / 16);
   const int64_t ldq = ((Ctot + 15) / 16) * 16;
   const int Smax = 8;
   // workspace: lf | Omega x2 | Q | part | G | V | Vwork | U | B | small
@@ -1446,7 +958,30 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   const size_t o_lbf = bf ? add(sizeof(uint32_t) * 4 * M) : 0;
   const size_t o_ta = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxa * npad) : 0;
   const size_t o_tb = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxb * Mpad) : 0;
-  void *old = ctx->scratch2.p;
+  // FP64 form: the code products' digit operands and INT32 sums (codes.hip), one area for
+  // the X A, X^T B and finishing X^T U products
+  if (!bf) EIG_TRY(eig_ensure_selg(ctx));
+  const int64_t G64 = Mpad / kGrp;
+  const CodeView vm{(const uint8_t *)ctx->sel.p, nullptr, 128 * 32, 32, M * 32, 16, M, (int64_t)nst * 8,
+                    kCodeLinear};
+  const CodeView vs{(const uint8_t *)ctx->selg.p, nullptr, G64 * 2048, 16, 4096, 2048, npad, G64 * 4,
+                    kCodeGrouped};
+  CodesPlan pa{}, pb{}, pu{};
+  size_t o_cw = 0;
+  if (!bf) {
+    // splits whose sums stay within 2 GiB
+    auto smax = [](size_t one) { return (int32_t)std::max<size_t>(1, std::min<size_t>(32, ((size_t)2 << 30) / one)); };
+    pa = eig_codes_plan(ctx, kCdPair, L, M, nst, 1);
+    pa = eig_codes_plan(ctx, kCdPair, L, M, nst, smax(pa.part_bytes));
+    pb = eig_codes_plan(ctx, kCdSum, L, npad, (G64 + 1) / 2, 1);
+    pb = eig_codes_plan(ctx, kCdSum, L, npad, (G64 + 1) / 2, smax(pb.part_bytes / pb.nsplit));
+    pu = eig_codes_plan(ctx, kCdSum, Ctot, npad, (G64 + 1) / 2, 1);
+    pu = eig_codes_plan(ctx, kCdSum, Ctot, npad, (G64 + 1) / 2, smax(pu.part_bytes / pu.nsplit));
+    size_t cw = 0;
+    for (const CodesPlan *q : {&pa, &pb, &pu})
+      cw = std::max(cw, q->head_bytes + up(q->dig_bytes) + q->part_bytes);
+    o_cw = add(cw);
+  }
   EIG_TRY(eig_ensure(ctx, ctx->scratch2, off));
   char *base = (char *)ctx->scratch2.p;
   double *lf = (double *)(base + o_lf), *A0 = (double *)(base + o_a0), *A1 = (double *)(base + o_a1);
@@ -1494,36 +1029,38 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
     occ = 0;
     EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_fpca_xa_bf16<2>, 256, 0));
     bxa_grid = (int)std::min<int64_t>((M + 127) / 128, (int64_t)std::max(occ, 1) * ctx->num_cu);
-  } else {
-    // the tuners write scratch outputs (U and Bm), never Q or the panels in use
-    EIG_TRY(tune_xa(ctx, F, P, CTL, A0, lda, U, ldq));
-    EIG_TRY(tune_xtb(ctx, F, P, CTL, U, ldq, part, Smax, Bm, lda));
   }
+  // X A and X^T B of the FP64 form: `plan`'s product of the codes with cols, its INT32 sums
+  // left in the work area
+  char *cw = base + o_cw;
+  auto code_mul = [&](const CodesPlan &plan, const CodeView &v, const CodeCols &cols) -> int {
+    EIG_TRY(eig_codes_scales(ctx, plan, cols, cw, st));
+    return eig_codes_mul(ctx, plan, v, cols, 0, cw, cw + plan.head_bytes,
+                         cw + plan.head_bytes + up(plan.dig_bytes), false, st);
+  };
+  auto code_xtb = [&](const CodesPlan &plan, const double *B_, double scale, double *out, int64_t ldo,
+                      int32_t Cpad) -> int {
+    CodeCols c{kColLevB, B_, ldq, M};
+    c.lev = lf;
+    EIG_TRY(code_mul(plan, vs, c));
+    return eig_codes_out_sum(ctx, plan, npad, cw, cw + plan.head_bytes + up(plan.dig_bytes), scale, out,
+                             ldo, 1, Cpad, false, st);
+  };
   auto xa = [&](const double *A_, double *Y_) -> int {
     if (bf)
       return launch_xa_bf16(ctx, P, lbf, tah, tal, cxa, A_, lda, Y_, ldq, L, bxa_grid, st);
-    return launch_xa(ctx, P, CTL, F.xa[CTL].grid, A_, lda, Y_, ldq, L, st);
+    EIG_TRY(code_mul(pa, vm, CodeCols{kColPanel, A_, lda, n}));
+    return eig_codes_out_pair(ctx, pa, M, cw, cw + pa.head_bytes + up(pa.dig_bytes), lf, nullptr, 1.0,
+                              Y_, ldq, 1, st);
   };
   auto xtb = [&](const double *B_, double *out_) -> int {
     if (bf)
       return launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, lbf, tbh, tbl, Mpad, B_, ldq, L,
                              part, part_doubles, out_, lda, 1.0 / (double)ncols, bslots, st);
-    return launch_xtb(ctx, P, CTL, F.xtb[CTL].grid, F.xtb[CTL].S, B_, ldq, L, part, out_, lda,
-                      1.0 / (double)ncols, st);
+    return code_xtb(pb, B_, 1.0 / (double)ncols, out_, lda, lda);
   };
-  // ---- power iterations (captured once per shape and buffer set, then replayed)
-  double inv_ncols = 1.0 / (double)ncols;
-  int64_t inv_bits;
-  std::memcpy(&inv_bits, &inv_ncols, sizeof inv_bits);
-  const std::vector<int64_t> sig = {
-      (int64_t)(uintptr_t)ctx->sel.p, (int64_t)(uintptr_t)ctx->selg.p, (int64_t)(uintptr_t)base,
-      (int64_t)off, (int64_t)o_lf, (int64_t)o_a0, (int64_t)o_a1, (int64_t)o_q, (int64_t)o_part,
-      (int64_t)o_lbf, (int64_t)o_ta, (int64_t)o_tb, M, nst, K, L, I, (int64_t)bf, inv_bits,
-      bf ? ((int64_t)bslots[0] * 100000 + bslots[1]) * 100000 + bxa_grid
-         : (int64_t)F.xa[CTL].grid * 1000 + F.xtb[CTL].S};
-  (void)old;
-  const bool same = F.gexec && F.gsig == sig;
-  auto power = [&]() -> int {
+  // ---- power iterations
+  {
     double *cur = A0, *nxt = A1;
     for (int32_t i = 0; i < I; ++i) {
       EIG_TRY(xa(cur, Q + (size_t)i * L));
@@ -1531,26 +1068,6 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
       std::swap(cur, nxt);
     }
     EIG_TRY(xa(cur, Q + (size_t)I * L));
-    return EIG_OK;
-  };
-  if (getenv("EIG_NO_GRAPH")) {
-    EIG_TRY(power());
-  } else {
-    if (!same) {
-      if (F.gexec) hipGraphExecDestroy(F.gexec);
-      F.gexec = nullptr;
-      hipGraph_t graph;
-      EIG_HIP(ctx, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-      int rc = power();
-      hipError_t e = hipStreamEndCapture(st, &graph);
-      if (rc != EIG_OK) return rc;
-      if (e != hipSuccess) return eig_set_err(ctx, EIG_E_HIP, "fpca capture: %s", hipGetErrorString(e));
-      e = hipGraphInstantiate(&F.gexec, graph, nullptr, nullptr, 0);
-      hipGraphDestroy(graph);
-      if (e != hipSuccess) return eig_set_err(ctx, EIG_E_HIP, "fpca graph: %s", hipGetErrorString(e));
-      F.gsig = sig;
-    }
-    EIG_HIP(ctx, hipGraphLaunch(F.gexec, st));
   }
   EIG_HIP(ctx, hipGetLastError());
   eig_time_end(ctx, "fpca_power");
@@ -1629,17 +1146,10 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
                               ldq, r - r64, part, part_doubles, Bm + r64, (int32_t)ldq, 1.0, bslots,
                               st));
   } else {
-    // in 32-column pieces: the wide instances hold all r columns' accumulators and run
-    // one wave per SIMD, at about half the FP64 rate of k_fpca_xtb<2> (four waves per
-    // SIMD), which the power iteration has tuned already when L <= 32.  A last piece
-    // whose 32 columns would pass ldq (a multiple of 16 >= r) takes 16.
-    for (int32_t c0 = 0; c0 < r; c0 += 32) {
-      const int32_t cw = std::min<int32_t>(32, r - c0);
-      const int ct = c0 + 32 <= ldq ? 2 : 1;
-      EIG_TRY(tune_xtb(ctx, F, P, ct, src + c0, ldq, part, Smax, Bm + c0, (int32_t)ldq));
-      EIG_TRY(launch_xtb(ctx, P, ct, F.xtb[ct].grid, F.xtb[ct].S, src + c0, ldq, cw, part,
-                         Bm + c0, (int32_t)ldq, 1.0, st));
-    }
+    // the plan made for every column serves a basis of fewer (r <= Ctot): the missing
+    // ones have no digits
+    CodesPlan pr = eig_codes_plan(ctx, kCdSum, r, npad, (G64 + 1) / 2, pu.nsplit);
+    EIG_TRY(code_xtb(pr, src, 1.0, Bm, ldq, r));
   }
   EIG_TRY(gemm_nt_long(ctx, r, r, npad, Bm, ldq, Bm, ldq, G, r, part, part_doubles, st));
   // top-K eigenpairs of B^T B (order r up to 256) by the FP64 eigensolver: all

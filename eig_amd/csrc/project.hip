@@ -1,15 +1,15 @@
 // SNP loadings, projection scales and lsqproject on the device.
 //
-//  loadings : ffvecs[j][m] = sum_i 10 v_j[i] z_m[i].  z takes three values per
-//             SNP, so each (sample tile, SNP) first bins the eigenvector entries
-//             by genotype code: S_g[j] = sum_{i: g_i = g} v_j[i]; then
-//             ffvecs[j][m] = 10 * sum_g level_g S_g[j].
+//  loadings : ffvecs[j][m] = sum_i 10 v_j[i] z_m[i], a product of the samples' codes with
+//             the axes (codes.hip).
 //  fxscal   : fxvecs[j][i] = sum_m x_i[m] ffvecs[j][m] with the reference's row
-//             fix-up x = g*fancy - mean*fancy (missing or ignored -> 0).
+//             fix-up x = g*fancy - mean*fancy (missing or ignored -> 0), a product of
+//             the SNPs' codes with the loadings.
 //  lsqproject: per individual, over observed SNPs, the K x K Gram of
-//             e_m = fxscal .* ffvecs[:,m] and the right-hand side sum_m e_m x_m,
-//             reduced over fixed SNP chunks in chunk order, then the Cholesky
-//             solve of nicksrc/linsubs.c (choldc/cholsl) per individual.
+//             e_m = fxscal .* ffvecs[:,m] and the right-hand side sum_m e_m x_m, as
+//             products of the codes and the missing bits with the e_m e_m^T and e_m (with
+//             usepopsformissing's fill: FP64 sums over fixed SNP chunks in chunk order),
+//             then the Cholesky solve of nicksrc/linsubs.c (choldc/cholsl) per individual.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -38,127 +38,24 @@ constexpr int kLsqChunk = 4096;  // SNPs per lsqproject partial
   }
 
 // ---------------------------------------------------------------- loadings
-// block = 256 threads handles 64 SNPs; thread (m = t>>2, part = t&3) covers
-// samples 32*part .. 32*part+31 of each sample tile.
-template <int K>
-__global__ __launch_bounds__(256) void k_loadings(const uint32_t *__restrict__ sel, int64_t M,
-                                                  int32_t nst, int32_t nrows,
-                                                  const double *__restrict__ ev,
-                                                  const double *__restrict__ lev,
-                                                  const uint8_t *__restrict__ ignore,
-                                                  double *__restrict__ ff) {
-  __shared__ double fv[kMaxK][kTileS];
-  __shared__ double red[4][64][kMaxK];
-  const int t = threadIdx.x, ml = t >> 2, part = t & 3;
-  const int64_t m = (int64_t)blockIdx.x * 64 + ml;
-  double S[3][K];
-#pragma unroll
-  for (int g = 0; g < 3; ++g)
-#pragma unroll
-    for (int j = 0; j < K; ++j) S[g][j] = 0.0;
-  for (int32_t st = 0; st < nst; ++st) {
-    __syncthreads();
-    for (int idx = t; idx < K * kTileS; idx += 256) {
-      int j = idx / kTileS, i = idx % kTileS;
-      int32_t gi = st * kTileS + i;
-      fv[j][i] = gi < nrows ? ev[(int64_t)j * nrows + gi] : 0.0;
-    }
-    __syncthreads();
-    if (m < M) {
-      const uint32_t *wp = sel + ((int64_t)st * M + m) * kTileWords + 2 * part;
-      uint32_t w0 = wp[0], w1 = wp[1];
-      for (int s = 0; s < 32; ++s) {
-        uint32_t code = ((s < 16 ? w0 : w1) >> (2 * (s & 15))) & 3u;
-        int i = 32 * part + s;
-        if (code < 3) {
-#pragma unroll
-          for (int j = 0; j < K; ++j) {
-            double v = fv[j][i];
-            S[0][j] += code == 0 ? v : 0.0;
-            S[1][j] += code == 1 ? v : 0.0;
-            S[2][j] += code == 2 ? v : 0.0;
-          }
-        }
-      }
-    }
-  }
-  // combine the 4 parts of each SNP in fixed order
-  double out[K];
-  const double *L = lev + 4 * (m < M ? m : 0);
-#pragma unroll
-  for (int j = 0; j < K; ++j) out[j] = L[0] * S[0][j] + L[1] * S[1][j] + L[2] * S[2][j];
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < K; ++j) red[part][ml][j] = out[j];
-  __syncthreads();
-  if (part == 0 && m < M) {
-    bool ign = ignore[m] != 0;
-    for (int j = 0; j < K; ++j) {
-      double s = ((red[0][ml][j] + red[1][ml][j]) + red[2][ml][j]) + red[3][ml][j];
-      ff[(int64_t)j * M + m] = ign ? 0.0 : 10.0 * s;
-    }
-  }
+// ignore[m] (status not kept, unless the caller gave a mask) and xmean = mean * fancy
+__global__ void k_load_prep(const int32_t *__restrict__ status, const double *__restrict__ mean,
+                            const double *__restrict__ fancy, int64_t M, int32_t mask,
+                            uint8_t *__restrict__ ignore, double *__restrict__ xmean) {
+  const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (m >= M) return;
+  if (mask) ignore[m] = status[m] != EIG_SNP_KEPT;
+  xmean[m] = mean[m] * fancy[m];
 }
 
-// ---------------------------------------------------------------- fxvecs
-// block (sample tile st, SNP chunk): thread i < 128 -> sample st*128+i.
-constexpr int kFxChunk = 2048;
-template <int K>
-__global__ __launch_bounds__(128) void k_fxvecs(const uint32_t *__restrict__ sel, int64_t M,
-                                                int32_t nst, int32_t nrows,
-                                                const double *__restrict__ ff,
-                                                const double *__restrict__ fancy,
-                                                const double *__restrict__ xmean,
-                                                const uint8_t *__restrict__ ignore,
-                                                double *__restrict__ partial) {
-  __shared__ double sf[64][kMaxK + 2];
-  const int i = threadIdx.x;
-  const int32_t st = blockIdx.x % nst;
-  const int64_t chunk = blockIdx.x / nst;
-  const int64_t m0 = chunk * kFxChunk, m1 = min(M, m0 + kFxChunk);
-  double acc[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) acc[j] = 0.0;
-  for (int64_t mb = m0; mb < m1; mb += 64) {
-    __syncthreads();
-    for (int idx = i; idx < 64 * (K + 2); idx += 128) {
-      int r = idx / (K + 2), c = idx % (K + 2);
-      int64_t m = mb + r;
-      double v = 0.0;
-      if (m < m1) {
-        if (c < K) v = ff[(int64_t)c * M + m];
-        else if (c == K) v = ignore[m] ? 0.0 : fancy[m];
-        else v = ignore[m] ? 0.0 : xmean[m];
-      }
-      sf[r][c] = v;
-    }
-    __syncthreads();
-    const int64_t lim = min((int64_t)64, m1 - mb);
-    for (int r = 0; r < lim; ++r) {
-      uint32_t wv = sel[((int64_t)st * M + mb + r) * kTileWords + (i >> 4)];
-      uint32_t code = (wv >> (2 * (i & 15))) & 3u;
-      double g = (code == 3u) ? -1.0 : (double)code;
-      double y = g * sf[r][K];
-      double x = (y < -0.001) ? 0.0 : y - sf[r][K + 1];
-#pragma unroll
-      for (int j = 0; j < K; ++j) acc[j] += x * sf[r][j];
-    }
-  }
-  const int32_t gi = st * kTileS + i;
-  if (gi < nrows)
-#pragma unroll
-    for (int j = 0; j < K; ++j) partial[(chunk * K + j) * (int64_t)nrows + gi] = acc[j];
-}
-
-__global__ void k_fxscal(const double *__restrict__ partial, int64_t nchunk, int32_t nrows,
-                         int32_t K, double *__restrict__ fxvecs, double *__restrict__ fxscal) {
+// fxscal[j] = 1 / sqrt(sum_i fxvecs[j][i]^2)
+__global__ void k_fxscal(const double *__restrict__ fxvecs, int32_t nrows,
+                         double *__restrict__ fxscal) {
   __shared__ double red[256];
   const int j = blockIdx.x;
   double s2 = 0.0;
   for (int32_t i = threadIdx.x; i < nrows; i += 256) {
-    double s = 0.0;
-    for (int64_t c = 0; c < nchunk; ++c) s += partial[(c * K + j) * (int64_t)nrows + i];
-    fxvecs[(int64_t)j * nrows + i] = s;
+    const double s = fxvecs[(int64_t)j * nrows + i];
     s2 += s * s;
   }
   red[threadIdx.x] = s2;
@@ -183,12 +80,11 @@ __global__ __launch_bounds__(64) void k_lsq_gram(const uint8_t *__restrict__ gen
                                                  const uint8_t *__restrict__ ignore,
                                                  const double *__restrict__ fill,
                                                  const int32_t *__restrict__ itype, int32_t npop,
-                                                 double *__restrict__ partial, int32_t nblk,
-                                                 int64_t chunk0) {
+                                                 double *__restrict__ partial, int32_t nblk) {
   __shared__ double se[64][kMaxK + 2];
   const int li = threadIdx.x;
   const int32_t q = (blockIdx.x % nblk) * 64 + li;
-  const int64_t chunk = chunk0 + blockIdx.x / nblk;
+  const int64_t chunk = blockIdx.x / nblk;
   const int64_t m0 = chunk * kLsqChunk, m1 = min(M, m0 + kLsqChunk);
   constexpr int nP = K * (K + 1) / 2;
   double G[nP];
@@ -198,7 +94,7 @@ __global__ __launch_bounds__(64) void k_lsq_gram(const uint8_t *__restrict__ gen
 #pragma unroll
   for (int j = 0; j < K; ++j) r[j] = 0.0;
   double kk = 0.0, nobs = 0.0;
-  const int32_t ty = (fill && q < nind) ? itype[q] : -1;
+  const int32_t ty = q < nind ? itype[q] : -1;
   for (int64_t mb = m0; mb < m1; mb += 64) {
     __syncthreads();
     {
@@ -243,7 +139,7 @@ __global__ __launch_bounds__(64) void k_lsq_gram(const uint8_t *__restrict__ gen
     }
   }
   if (q < nind) {
-    double *out = partial + ((chunk - chunk0) * (int64_t)nind + q) * (nP + K + 2);
+    double *out = partial + (chunk * (int64_t)nind + q) * (nP + K + 2);
 #pragma unroll
     for (int p = 0; p < nP; ++p) out[p] = G[p];
 #pragma unroll
@@ -335,43 +231,52 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
   const int64_t M = ctx->nsnp;
   const int32_t n = ctx->nrows;
   hipStream_t st = ctx->stream;
-  // ignore mask (host), xmean = mean*fancy (device, computed here)
-  std::vector<uint8_t> ign(M);
-  if (ignore) {
-    std::memcpy(ign.data(), ignore, M);
-  } else {
-    std::vector<int32_t> s(M);
-    EIG_HIP(ctx, hipMemcpy(s.data(), ctx->status.p, 4 * M, hipMemcpyDeviceToHost));
-    for (int64_t m = 0; m < M; ++m) ign[m] = s[m] != EIG_SNP_KEPT;
-  }
-  std::vector<double> mean(M), fancy(M), xm(M);
-  EIG_HIP(ctx, hipMemcpy(mean.data(), ctx->mean.p, 8 * M, hipMemcpyDeviceToHost));
-  EIG_HIP(ctx, hipMemcpy(fancy.data(), ctx->fancy.p, 8 * M, hipMemcpyDeviceToHost));
-  for (int64_t m = 0; m < M; ++m) xm[m] = mean[m] * fancy[m];
   EIG_TRY(eig_ensure(ctx, ctx->ignore_dev, M));
   EIG_TRY(eig_ensure(ctx, ctx->ffvecs, 8 * (size_t)K * M));
   EIG_TRY(eig_ensure(ctx, ctx->fxscal, 8 * (size_t)(kMaxK + M)));  // fxscal | xmean
-  EIG_TRY(eig_ensure(ctx, ctx->projw, 8 * (size_t)K * n));
+  EIG_TRY(eig_ensure(ctx, ctx->projw, 8 * (size_t)K * n * 2));     // axes | fxvecs
+  EIG_TRY(eig_ensure_selg(ctx));
   double *d_fx = (double *)ctx->fxscal.p, *d_xm = d_fx + kMaxK;
-  EIG_HIP(ctx, hipMemcpyAsync(ctx->ignore_dev.p, ign.data(), M, hipMemcpyHostToDevice, st));
-  EIG_HIP(ctx, hipMemcpyAsync(d_xm, xm.data(), 8 * M, hipMemcpyHostToDevice, st));
-  EIG_HIP(ctx, hipMemcpyAsync(ctx->projw.p, evecs, 8 * (size_t)K * n, hipMemcpyHostToDevice, st));
+  double *d_ev = (double *)ctx->projw.p, *d_fxv = d_ev + (size_t)K * n;
+  double *d_ff = (double *)ctx->ffvecs.p;
+  uint8_t *d_ign = (uint8_t *)ctx->ignore_dev.p;
+  if (ignore) EIG_HIP(ctx, hipMemcpyAsync(d_ign, ignore, M, hipMemcpyHostToDevice, st));
+  EIG_HIP(ctx, hipMemcpyAsync(d_ev, evecs, 8 * (size_t)K * n, hipMemcpyHostToDevice, st));
+  // ffvecs = 10 Z^T v as a product over the samples (rows = SNPs), fxvecs = X ff as one
+  // over the SNPs (rows = samples), on the code planes (codes.hip).  At 5,000 x 600,000,
+  // K = 10, both read the codes once: 19.6 ms with per-code bins and FP64 sums on the
+  // vector units, LOADMS now.
+  const int64_t G64 = (M + kGrp - 1) / kGrp;
+  const CodeView vm{(const uint8_t *)ctx->sel.p, nullptr, 128 * 32, 32, M * 32, 16, M,
+                    (int64_t)ctx->nst * 8, kCodeLinear};
+  const CodeView vs{(const uint8_t *)ctx->selg.p, nullptr, G64 * 2048, 16, 4096, 2048,
+                    (int64_t)ctx->nst * kTileS, G64 * 4, kCodeGrouped};
+  CodeCols ax{kColAxes, d_ev, n, n};
+  CodeCols fc{kColFx, d_ff, M, M};
+  fc.fancy = (const double *)ctx->fancy.p;
+  fc.xmean = d_xm;
+  fc.ignore = d_ign;
+  const CodesPlan pl = eig_codes_plan(ctx, kCdPair, K, M, ctx->nst, 16);
+  const CodesPlan pf = eig_codes_plan(ctx, kCdSum, K, vs.nrow, (G64 + 1) / 2, 32);
+  const size_t need = std::max(pl.head_bytes + pl.dig_bytes + pl.part_bytes,
+                               pf.head_bytes + pf.dig_bytes + pf.part_bytes);
+  EIG_TRY(eig_ensure(ctx, ctx->scratch2, need));
+  char *ws = (char *)ctx->scratch2.p;
   eig_time_begin(ctx);
-  EIG_KSWITCH(K, hipLaunchKernelGGL((k_loadings<KC>), dim3((unsigned)((M + 63) / 64)), dim3(256),
-                                    0, st, (const uint32_t *)ctx->sel.p, M, ctx->nst, n,
-                                    (const double *)ctx->projw.p, (const double *)ctx->lev.p,
-                                    (const uint8_t *)ctx->ignore_dev.p, (double *)ctx->ffvecs.p));
-  EIG_HIP(ctx, hipGetLastError());
-  const int64_t nchunk = (M + kFxChunk - 1) / kFxChunk;
-  EIG_TRY(eig_ensure(ctx, ctx->scratch2, 8 * (size_t)(nchunk * K * n + (size_t)K * n)));
-  double *d_part = (double *)ctx->scratch2.p, *d_fxv = d_part + nchunk * K * n;
-  EIG_KSWITCH(K, hipLaunchKernelGGL((k_fxvecs<KC>), dim3((unsigned)(nchunk * ctx->nst)), dim3(128),
-                                    0, st, (const uint32_t *)ctx->sel.p, M, ctx->nst, n,
-                                    (const double *)ctx->ffvecs.p, (const double *)ctx->fancy.p,
-                                    (const double *)d_xm, (const uint8_t *)ctx->ignore_dev.p,
-                                    d_part));
-  hipLaunchKernelGGL(k_fxscal, dim3((unsigned)K), dim3(256), 0, st, (const double *)d_part,
-                     nchunk, n, K, d_fxv, d_fx);
+  hipLaunchKernelGGL(k_load_prep, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, st,
+                     (const int32_t *)ctx->status.p, (const double *)ctx->mean.p,
+                     (const double *)ctx->fancy.p, M, ignore ? 0 : 1, d_ign, d_xm);
+  EIG_TRY(eig_codes_scales(ctx, pl, ax, ws, st));
+  EIG_TRY(eig_codes_mul(ctx, pl, vm, ax, 0, ws, ws + pl.head_bytes, ws + pl.head_bytes + pl.dig_bytes,
+                        false, st));
+  EIG_TRY(eig_codes_out_pair(ctx, pl, M, ws, ws + pl.head_bytes + pl.dig_bytes,
+                             (const double *)ctx->lev.p, d_ign, 10.0, d_ff, 1, M, st));
+  EIG_TRY(eig_codes_scales(ctx, pf, fc, ws, st));
+  EIG_TRY(eig_codes_mul(ctx, pf, vs, fc, 0, ws, ws + pf.head_bytes, ws + pf.head_bytes + pf.dig_bytes,
+                        false, st));
+  EIG_TRY(eig_codes_out_sum(ctx, pf, n, ws, ws + pf.head_bytes + pf.dig_bytes, 1.0, d_fxv, 1, n, K,
+                            false, st));
+  hipLaunchKernelGGL(k_fxscal, dim3((unsigned)K), dim3(256), 0, st, (const double *)d_fxv, n, d_fx);
   EIG_HIP(ctx, hipGetLastError());
   eig_time_end(ctx, "loadings");
   if (ffvecs)
@@ -380,6 +285,122 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
   EIG_HIP(ctx, hipStreamSynchronize(st));
   ctx->last_K = K;
   ctx->have_load = true;
+  return EIG_OK;
+}
+
+// ---------------------------------------------------------------- normal equations
+// GENO rows of SNPs m0 .. (64 per group) and individuals q0 .. (128 per tile) as the
+// grouped codes of eig_ensure_selg: 16 bytes per (tile, group, individual).  SNPs past M
+// and individuals past nind read as missing.
+__global__ __launch_bounds__(256) void k_regroup_geno(const uint8_t *__restrict__ geno, int64_t rlen,
+                                                      int64_t M, int32_t nind, int64_t m0, int32_t q0,
+                                                      int64_t G64, int64_t ngroups,
+                                                      uint4 *__restrict__ out) {
+  __shared__ uint8_t by[2][kGrp][36];
+  const int half = threadIdx.x >> 7, i = threadIdx.x & 127;
+  const int64_t gid = (int64_t)blockIdx.x * 2 + half;  // tile * G64 + group
+  const bool live = gid < ngroups;
+  const int64_t tile = live ? gid / G64 : 0, g = live ? gid % G64 : 0;
+  const int64_t b0 = q0 / 4 + tile * 32;  // first byte of the tile's 128 individuals
+  const int64_t nby = (nind + 3) / 4;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int idx = i + 128 * e, r = idx >> 5, b = idx & 31;
+    const int64_t m = m0 + g * kGrp + r;
+    by[half][r][b] = (live && m < M && b0 + b < nby) ? geno[m * rlen + b0 + b] : 0xFF;
+  }
+  __syncthreads();
+  if (!live) return;
+  const bool in = q0 + tile * 128 + i < nind;
+  const int sh = 6 - 2 * (i & 3);
+  uint32_t o[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t c = ((uint32_t)by[half][16 * s + 8 * h + j][i >> 2] >> sh) & 3u;
+        o[2 * h + (s >> 1)] |= c << (16 * (s & 1) + 2 * j);
+      }
+  out[gid * kTileS + i] = in ? make_uint4(o[0], o[1], o[2], o[3]) : make_uint4(~0u, ~0u, ~0u, ~0u);
+}
+
+// The normal equations of every individual, acc[q][W]: the Gram's upper triangle, the
+// right-hand side and the observed count, from the current loadings, in a workspace of
+// `bytes` at ws.  The Gram is the sum of e e^T over all kept SNPs minus that over the
+// individual's missing ones, so it needs the missing bits alone.  Individuals run in
+// chunks of whole tiles and SNPs in chunks of whole stages, as the workspace holds; the
+// sums within kLsqRange stages are exact, so the chunks do not change the result.
+constexpr int64_t kLsqRange = kCodesMaxK / 128 / 2;  // whole chunks of it stay within kCodesMaxK
+static int lsq_normal(eig_ctx *ctx, double *acc, char *ws, size_t bytes) {
+  const int64_t M = ctx->nsnp;
+  const int32_t nind = ctx->nind, K = ctx->last_K, nP = K * (K + 1) / 2, W = nP + K + 2;
+  hipStream_t st = ctx->stream;
+  const double *d_fx = (const double *)ctx->fxscal.p, *d_xm = d_fx + kMaxK;
+  CodeCols cr{kColLsqR, (const double *)ctx->ffvecs.p, M, M};
+  cr.fancy = (const double *)ctx->fancy.p;
+  cr.xmean = d_xm;
+  cr.ignore = (const uint8_t *)ctx->ignore_dev.p;
+  cr.fxscal = d_fx;
+  cr.K = K;
+  CodeCols cg = cr;
+  cg.kind = kColLsqG;
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const int64_t nblk_all = (M + 127) / 128;
+  int64_t nr = (nind + 255) / 256 * 256, nb = std::min(nblk_all, kLsqRange);
+  int32_t smax = 32;
+  CodesPlan pr, pg;
+  size_t codes = 0;
+  for (;;) {
+    pr = eig_codes_plan(ctx, kCdSum, K + 1, std::min<int64_t>(nr, nind), nb, smax);
+    pg = eig_codes_plan(ctx, kCdMiss, nP, std::min<int64_t>(nr, nind), nb, smax);
+    codes = up((size_t)nr * nb * 32);
+    const size_t need = pr.head_bytes + pg.head_bytes + up(pr.dig_bytes) + up(pg.dig_bytes) +
+                        up(pr.part_bytes) + up(pg.part_bytes) + codes;
+    if (need <= bytes) break;
+    if (nb > 512) nb = (nb + 1) / 2;
+    else if (smax > 4) smax /= 2;
+    else if (nb > 64) nb = (nb + 1) / 2;
+    else if (smax > 1) smax /= 2;
+    else if (nr > 256) nr = std::max<int64_t>(256, nr / 2 / 256 * 256);
+    else return eig_set_err(ctx, EIG_E_NOMEM, "lsqproject: workspace too small");
+  }
+  char *p = ws;
+  auto take = [&](size_t b) {
+    char *q = p;
+    p += up(b);
+    return q;
+  };
+  void *hr = take(pr.head_bytes), *hg = take(pg.head_bytes);
+  void *dr = take(pr.dig_bytes), *dg = take(pg.dig_bytes);
+  void *sr = take(pr.part_bytes), *sg = take(pg.part_bytes);
+  uint4 *cd = (uint4 *)take(codes);
+  EIG_TRY(eig_codes_scales(ctx, pr, cr, hr, st));
+  EIG_TRY(eig_codes_scales(ctx, pg, cg, hg, st));
+  for (int64_t q0 = 0; q0 < nind; q0 += nr) {
+    const int64_t rows = std::min<int64_t>(nr, nind - q0), tiles = (rows + 127) / 128;
+    for (int64_t s0 = 0; s0 < nblk_all; s0 += kLsqRange) {
+      EIG_TRY(eig_codes_restart(ctx, pr, hr, st));
+      EIG_TRY(eig_codes_restart(ctx, pg, hg, st));
+      const int64_t s1 = std::min(nblk_all, s0 + kLsqRange);
+      // a last, shorter chunk keeps the plan: SNPs past s1 have no digits
+      cr.n = cg.n = std::min(M, s1 * 128);
+      for (int64_t b0 = s0; b0 < s1; b0 += nb) {
+        const int64_t G64 = 2 * nb;
+        hipLaunchKernelGGL(k_regroup_geno, dim3((unsigned)((tiles * G64 + 1) / 2)), dim3(256), 0, st,
+                           (const uint8_t *)ctx->geno.p, ctx->rlen, M, nind, b0 * 128, (int32_t)q0,
+                           G64, tiles * G64, cd);
+        const CodeView v{(const uint8_t *)cd, nullptr, G64 * 2048, 16, 4096, 2048, tiles * 128, G64 * 4,
+                         kCodeGrouped};
+        EIG_TRY(eig_codes_mul(ctx, pr, v, cr, b0, hr, dr, sr, b0 > s0, st));
+        EIG_TRY(eig_codes_mul(ctx, pg, v, cg, b0, hg, dg, sg, b0 > s0, st));
+      }
+      double *a = acc + q0 * W;
+      EIG_TRY(eig_codes_out_sum(ctx, pg, rows, hg, sg, 1.0, a, W, 1, nP, s0 > 0, st));
+      EIG_TRY(eig_codes_out_sum(ctx, pr, rows, hr, sr, 1.0, a + nP, W, 1, K + 1, s0 > 0, st));
+    }
+  }
   return EIG_OK;
 }
 
@@ -395,24 +416,35 @@ static int lsqproject(eig_ctx *ctx, const int32_t *use, const int32_t *itype, in
   double *d_fill = nullptr;
   const int32_t *d_itype = nullptr;
   if (itype) EIG_TRY(eig_lsq_filltab(ctx, use, itype, npop, K, &d_fill, &d_itype));
-  const int64_t nchunk = (M + kLsqChunk - 1) / kLsqChunk;
-  const int32_t nblk = (nind + 63) / 64;
-  size_t part_b = 8 * (size_t)nchunk * nind * W;
   size_t out_b = 8 * (size_t)2 * K * nind + 4 * (size_t)nind * 2 + 256;
-  EIG_TRY(eig_ensure(ctx, ctx->scratch2, part_b));
   EIG_TRY(eig_ensure(ctx, ctx->proj_out, out_b));
   double *d_ans = (double *)ctx->proj_out.p, *d_rhs = d_ans + (size_t)K * nind;
   int32_t *d_st = (int32_t *)(d_rhs + (size_t)K * nind), *d_use = d_st + nind;
   EIG_HIP(ctx, hipMemcpyAsync(d_use, use, 4 * (size_t)nind, hipMemcpyHostToDevice, st));
   EIG_HIP(ctx, hipMemsetAsync(d_ans, 0, 8 * (size_t)K * nind, st));
   const double *d_fx = (const double *)ctx->fxscal.p, *d_xm = d_fx + kMaxK;
-  eig_time_begin(ctx);
-  EIG_KSWITCH(K, hipLaunchKernelGGL((k_lsq_gram<KC>), dim3((unsigned)(nchunk * nblk)), dim3(64),
-                                    0, st, (const uint8_t *)ctx->geno.p, ctx->rlen, M, nind,
-                                    (const double *)ctx->ffvecs.p, d_fx,
-                                    (const double *)ctx->fancy.p, d_xm,
-                                    (const uint8_t *)ctx->ignore_dev.p, (const double *)d_fill,
-                                    d_itype, npop, (double *)ctx->scratch2.p, nblk, (int64_t)0));
+  int64_t nchunk = 1;
+  if (!itype) {
+    // the normal equations from the code planes (5,000 x 600,000, K = 10: LSQMS against
+    // 25.6 ms of FP64 sums per individual); the workspace holds up to 1 GiB of it at once
+    const size_t acc_b = (8 * (size_t)nind * W + 255) & ~(size_t)255;
+    const size_t work = std::min((size_t)1 << 30, ((size_t)nind + 4096) * (M + 4096) + ((size_t)64 << 20));
+    EIG_TRY(eig_ensure(ctx, ctx->scratch2, acc_b + work));
+    eig_time_begin(ctx);
+    EIG_TRY(lsq_normal(ctx, (double *)ctx->scratch2.p, (char *)ctx->scratch2.p + acc_b, work));
+  } else {
+    // a fill's genotypes are FP64 values of their own: sums per individual
+    nchunk = (M + kLsqChunk - 1) / kLsqChunk;
+    const int32_t nblk = (nind + 63) / 64;
+    EIG_TRY(eig_ensure(ctx, ctx->scratch2, 8 * (size_t)nchunk * nind * W));
+    eig_time_begin(ctx);
+    EIG_KSWITCH(K, hipLaunchKernelGGL((k_lsq_gram<KC>), dim3((unsigned)(nchunk * nblk)), dim3(64),
+                                      0, st, (const uint8_t *)ctx->geno.p, ctx->rlen, M, nind,
+                                      (const double *)ctx->ffvecs.p, d_fx,
+                                      (const double *)ctx->fancy.p, d_xm,
+                                      (const uint8_t *)ctx->ignore_dev.p, (const double *)d_fill,
+                                      d_itype, npop, (double *)ctx->scratch2.p, nblk));
+  }
   hipLaunchKernelGGL(k_lsq_solve, dim3((unsigned)((nind + 127) / 128)), dim3(128), 0, st,
                      (const double *)ctx->scratch2.p, nchunk, nind, K, (const int32_t *)d_use,
                      d_itype, d_ans, d_rhs, d_st);
@@ -455,20 +487,9 @@ extern "C" int eig_lsqproject_fill(eig_ctx *ctx, const int32_t *use, const int32
 
 // ---------------------------------------------------------------- allocation-free lsqproject
 namespace {
-__global__ void k_zero(double *__restrict__ p, int64_t n) {
+__global__ void k_lsq_clear(double *__restrict__ p, int64_t n) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e < n) p[e] = 0.0;
-}
-
-// acc[q][p] += part[c][q][p] for the group's chunks c in order: the same sequence of
-// additions as k_lsq_solve's loop over all chunks
-__global__ void k_lsq_accum(double *__restrict__ acc, const double *__restrict__ part,
-                            int64_t nchunk, int64_t per) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (e >= per) return;
-  double v = acc[e];
-  for (int64_t c = 0; c < nchunk; ++c) v += part[c * per + e];
-  acc[e] = v;
 }
 
 // the stale-answer rule of the reference, in individual order, one thread per axis j:
@@ -497,13 +518,11 @@ extern "C" int eig_lsqproject_noalloc(eig_ctx *ctx, const int32_t *use, double *
     return eig_set_err(ctx, EIG_E_STATE, "eig_lsqproject_noalloc before eig_loadings");
   if (!ctx->noalloc) return eig_set_err(ctx, EIG_E_STATE, "eig_lsqproject_noalloc: no workspace");
   EIG_HIP(ctx, hipSetDevice(ctx->device));
-  const int64_t M = ctx->nsnp;
   const int32_t nind = ctx->nind, K = ctx->last_K;
   hipStream_t st = ctx->stream;
   const int nP = K * (K + 1) / 2, W = nP + K + 2;
-  const int64_t nchunk = (M + kLsqChunk - 1) / kLsqChunk;
-  const int32_t nblk = (nind + 63) / 64;
-  // workspace: acc | ans | rhs | A | B | status | use | partials of G chunks
+  // workspace: acc | ans | rhs | A | B | status | use | the products' work area (at least the
+  // size of acc, which holds chunks of it at every K)
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t per = (size_t)nind * W;
   const size_t o_acc = 0, o_ans = up(8 * per), o_rhs = o_ans + up(8 * (size_t)K * nind),
@@ -514,33 +533,19 @@ extern "C" int eig_lsqproject_noalloc(eig_ctx *ctx, const int32_t *use, double *
     return eig_set_err(ctx, EIG_E_ARG,
                        "eig_lsqproject_noalloc: %d individuals x K=%d need more than the %zu-byte "
                        "static workspace", nind, K, ctx->noalloc_bytes);
-  const int64_t G = std::min<int64_t>(nchunk, (int64_t)((ctx->noalloc_bytes - o_part) / (8 * per)));
   char *base = (char *)ctx->noalloc;
   double *d_acc = (double *)(base + o_acc), *d_ans = (double *)(base + o_ans),
          *d_rhs = (double *)(base + o_rhs), *d_A = (double *)(base + o_A),
-         *d_B = (double *)(base + o_B), *d_part = (double *)(base + o_part);
+         *d_B = (double *)(base + o_B);
   int32_t *d_st = (int32_t *)(base + o_st), *d_use = (int32_t *)(base + o_use);
   const size_t kn = (size_t)K * nind;
   EIG_HIP(ctx, hipMemcpyAsync(d_use, use, 4 * (size_t)nind, hipMemcpyHostToDevice, st));
   // the caller's current outputs go in, so entries the rule leaves alone come back as they were
   if (acoeffs) EIG_HIP(ctx, hipMemcpyAsync(d_A, acoeffs, 8 * kn, hipMemcpyHostToDevice, st));
   if (bcoeffs) EIG_HIP(ctx, hipMemcpyAsync(d_B, bcoeffs, 8 * kn, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_zero, dim3((unsigned)((per + 255) / 256)), dim3(256), 0, st, d_acc,
-                     (int64_t)per);
-  hipLaunchKernelGGL(k_zero, dim3((unsigned)((kn + 255) / 256)), dim3(256), 0, st, d_ans,
+  hipLaunchKernelGGL(k_lsq_clear, dim3((unsigned)((kn + 255) / 256)), dim3(256), 0, st, d_ans,
                      (int64_t)kn);
-  const double *d_fx = (const double *)ctx->fxscal.p, *d_xm = d_fx + kMaxK;
-  for (int64_t c0 = 0; c0 < nchunk; c0 += G) {
-    const int64_t gc = std::min<int64_t>(G, nchunk - c0);
-    EIG_KSWITCH(K, hipLaunchKernelGGL((k_lsq_gram<KC>), dim3((unsigned)(gc * nblk)), dim3(64), 0,
-                                      st, (const uint8_t *)ctx->geno.p, ctx->rlen, M, nind,
-                                      (const double *)ctx->ffvecs.p, d_fx,
-                                      (const double *)ctx->fancy.p, d_xm,
-                                      (const uint8_t *)ctx->ignore_dev.p, (const double *)nullptr,
-                                      (const int32_t *)nullptr, 0, d_part, nblk, c0));
-    hipLaunchKernelGGL(k_lsq_accum, dim3((unsigned)((per + 255) / 256)), dim3(256), 0, st, d_acc,
-                       (const double *)d_part, gc, (int64_t)per);
-  }
+  EIG_TRY(lsq_normal(ctx, d_acc, base + o_part, ctx->noalloc_bytes - o_part));
   hipLaunchKernelGGL(k_lsq_solve, dim3((unsigned)((nind + 127) / 128)), dim3(128), 0, st,
                      (const double *)d_acc, (int64_t)1, nind, K, (const int32_t *)d_use,
                      (const int32_t *)nullptr, d_ans, d_rhs, d_st);
