@@ -166,7 +166,7 @@ __device__ __forceinline__ double col_quantum(u64 mx) {
 }
 
 // Digit operands of one stage (128 k from word 8 (b0 + blockIdx.x)) and column group:
-// dst[(group * nblk + blk) * planes * NT + plane * NT + tile][step a][1024]; lane l's 16
+// dst[(((group * nblk + blk) * 2 + step a) * planes + plane) * NT + tile][1024]; lane l's 16
 // bytes of a step's operand: digit column l % 16 of the tile, word 2 (l / 16) + a, byte
 // 4 t + b = code slot 4 b + t.  Digit column s * Cg + c holds digit s (highest first) of the
 // group's column c.  sums[2 c], [2 c + 1]: the sums of v3 on the grid, in two parts of 28
@@ -186,36 +186,49 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
   for (int e = t * 16; e < bytes; e += 256 * 16) *(uint4 *)&img[e] = make_uint4(0, 0, 0, 0);
   if (t < 2 * kMaxCols) ssum[t] = 0;
   __syncthreads();
-  for (int e = t; e < kSt * nc; e += 256) {
-    const int p = rowmajor ? e / nc : e & (kSt - 1), c = rowmajor ? e % nc : e / kSt;
-    const int jl = p >> 4, i = p & 15;
-    const int64_t k = code_elem(layout, 8 * (b0 + blk) + jl, i);
+  // an item is one dword of an operand: the code slots u, u + 4, u + 8, u + 12 of a word
+  for (int e = t; e < 32 * nc; e += 256) {
+    const int p = rowmajor ? e / nc : e & 31, c = rowmajor ? e % nc : e >> 5;
+    const int jl = p >> 2, u = p & 3;
     const u64 m = mx[c0 + c];
     if ((m >> 52) >= 0x7FF) continue;
     const int sh = col_shift(m);
-    const Col3 v = col_value<KIND>(A, k, c0 + c);
-    const int at = (jl & 1) * kFragB + (jl >> 1) * 256 + (i & 3) * 4 + (i >> 2);
-    auto put = [&](double x, int plane) {
-      int64_t q = llrint(scalbn(x, sh));
+    Col3 v[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      v[b] = col_value<KIND>(A, code_elem(layout, 8 * (b0 + blk) + jl, 4 * b + u), c0 + c);
+    const int at = (jl >> 1) * 256 + u * 4;
+    auto put = [&](double x0, double x1, double x2, double x3, int plane) {
+      int64_t q[4] = {llrint(scalbn(x0, sh)), llrint(scalbn(x1, sh)), llrint(scalbn(x2, sh)),
+                      llrint(scalbn(x3, sh))};
 #pragma unroll
       for (int s = kDig - 1; s >= 0; --s) {
-        const int32_t d = (int8_t)(q & 0xFF);
-        q = (q - d) >> 8;
+        uint32_t w = 0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int32_t d = (int8_t)(q[b] & 0xFF);
+          q[b] = (q[b] - d) >> 8;
+          w |= ((uint32_t)d & 0xFFu) << (8 * b);
+        }
         const int dc = s * Cg + c;
-        img[(plane * NT + (dc >> 4)) * 2 * kFragB + (dc & 15) * 16 + at] = (uint8_t)d;
+        *(uint32_t *)&img[((jl & 1) * planes * NT + plane * NT + (dc >> 4)) * kFragB + (dc & 15) * 16 + at] = w;
       }
     };
     if (MODE == kCdMiss) {
-      put(v.v2, 0);
+      put(v[0].v2, v[1].v2, v[2].v2, v[3].v2, 0);
     } else {
-      put(v.v1, 0);
-      if (MODE == kCdSum) put(v.v2, 1);
+      put(v[0].v1, v[1].v1, v[2].v1, v[3].v1, 0);
+      if (MODE == kCdSum) put(v[0].v2, v[1].v2, v[2].v2, v[3].v2, 1);
     }
-    const int64_t q3 = llrint(scalbn(v.v3, sh));
-    if (q3 != 0) {
-      atomicAdd(&ssum[2 * c], (u64)(q3 & ((1 << 28) - 1)));
-      atomicAdd(&ssum[2 * c + 1], (u64)(q3 >> 28));
+    int64_t lo = 0, hi = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int64_t q3 = llrint(scalbn(v[b].v3, sh));
+      lo += q3 & ((1 << 28) - 1);
+      hi += q3 >> 28;
     }
+    if (lo != 0) atomicAdd(&ssum[2 * c], (u64)lo);
+    if (hi != 0) atomicAdd(&ssum[2 * c + 1], (u64)hi);
   }
   __syncthreads();
   uint8_t *out = dst + ((int64_t)blockIdx.y * gridDim.x + blk) * bytes;
@@ -224,6 +237,10 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
 }
 
 // ------------------------------------------------------------------ the product
+// rows of a block: four waves of R row tiles of 16
+constexpr int cd_rows(int mode, int NT) {
+  return 64 * (mode == kCdPair ? 2 : mode == kCdSum && NT == kMaxNT ? 3 : 4);
+}
 struct MulArgs {
   CodeView v;
   const uint8_t *dig;
@@ -237,16 +254,17 @@ struct MulArgs {
 
 // One block per (row block, split, group): four waves of R row tiles of 16.  MODE kCdPair
 // multiplies one digit set with the codes and with the missing bits into two sums, kCdSum
-// two sets into one, kCdMiss one set with the missing bits.  A stage's digits (NT tiles x
-// planes x 2 KB) go through one of two LDS buffers, loaded into registers a stage ahead;
-// the codes come straight from memory, a word pair per lane and row tile.  R = 4 (two
-// for kCdPair, whose operands feed twice the products) keeps an operand read from LDS in
-// use for 64 cycles of MFMA, half the LDS' rate.
+// two sets into one, kCdMiss one set with the missing bits.  A half stage's digits (64 k:
+// NT tiles x planes x 1 KB) go through one of two LDS buffers, loaded into registers half a
+// stage ahead; the codes come straight from memory, a word pair per lane and row tile.
+// R = 4 (two for kCdPair, whose operands feed twice the products) keeps an operand read
+// from LDS in use for 64 cycles of MFMA, half the LDS' rate; nine tiles of two planes take
+// R = 3, whose sums leave registers for both planes' operands (R = 4 spilled 14 to 50).
 template <int NT, int MODE, int R>
 __global__ __launch_bounds__(256, 2) void k_cd_mul(MulArgs A) {
   constexpr int planes = MODE == kCdSum ? 2 : 1, nacc = MODE == kCdPair ? 2 : 1;
-  constexpr int bytes = planes * NT * 2 * kFragB, nld = bytes / 4096;
-  constexpr int tail = bytes % 4096;  // 0 or 2048: the last 128 threads' worth
+  constexpr int bytes = planes * NT * kFragB, nld = bytes / 4096;  // of a half stage
+  constexpr int tail = bytes % 4096 / 16;  // threads with one more piece
   __shared__ __align__(16) uint8_t lds[2][bytes];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane >> 4;
   const int64_t item = blockIdx.x;
@@ -254,7 +272,7 @@ __global__ __launch_bounds__(256, 2) void k_cd_mul(MulArgs A) {
   const int32_t rb = (int32_t)((item / A.ngroup) % A.nrowblk);
   const int32_t split = (int32_t)(item / ((int64_t)A.ngroup * A.nrowblk));
   const int64_t k0 = split * A.per, k1 = min(A.nblk, k0 + A.per);
-  const uint8_t *dig = A.dig + ((int64_t)grp * A.nblk) * bytes;
+  const uint8_t *dig = A.dig + ((int64_t)grp * A.nblk) * (2 * bytes) + t * 16;
   const int64_t r0 = ((int64_t)rb * 4 + w) * (16 * R);
   const uint8_t *rp[R];
 #pragma unroll
@@ -273,108 +291,131 @@ __global__ __launch_bounds__(256, 2) void k_cd_mul(MulArgs A) {
     }
   };
   i32x4 st[nld + 1];
-  auto load = [&](int64_t k) {
-    const uint8_t *s = dig + min(k, k1 - 1) * bytes + t * 16;
+  auto load = [&](int64_t h) {  // half stage h, or the last one again past the end
+    const uint8_t *s = dig + min(h, 2 * k1 - 1) * bytes;
 #pragma unroll
     for (int u = 0; u < nld; ++u) st[u] = *(const i32x4 *)(s + u * 4096);
-    if (tail && t < 128) st[nld] = *(const i32x4 *)(s + nld * 4096);
+    if (tail && t < tail) st[nld] = *(const i32x4 *)(s + nld * 4096);
   };
   auto store = [&](int buf) {
 #pragma unroll
     for (int u = 0; u < nld; ++u) *(i32x4 *)&lds[buf][t * 16 + u * 4096] = st[u];
-    if (tail && t < 128) *(i32x4 *)&lds[buf][t * 16 + nld * 4096] = st[nld];
+    if (tail && t < tail) *(i32x4 *)&lds[buf][t * 16 + nld * 4096] = st[nld];
   };
   i32x4 acc[nacc][NT][R];
-  int32_t *out = A.part + (((int64_t)grp * A.nsplit + split) * nacc) * A.rowpad * (NT * 16);
 #pragma unroll
   for (int a = 0; a < nacc; ++a)
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        acc[a][n][r] = i32x4{0, 0, 0, 0};
-        if (A.accum)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            acc[a][n][r][e] = out[(a * A.rowpad + r0 + 16 * r + 4 * q + e) * (NT * 16) + 16 * n + (lane & 15)];
-      }
+      for (int r = 0; r < R; ++r) acc[a][n][r] = i32x4{0, 0, 0, 0};
   uint2 cw[R], cn[R];
-  load(k0);
+  load(2 * k0);
   codes(k0, cw);
   store(0);
   __syncthreads();
-  int buf = 0;
   for (int64_t k = k0; k < k1; ++k) {
-    load(k + 1);
     codes(k + 1, cn);
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
-      i32x4 fc[R], fm[R];
+      load(2 * k + a + 1);
+      auto code_op = [&](i32x4 (&f)[R]) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const uint32_t x = a ? cw[r].y : cw[r].x;
-        const uint32_t ms = x & (x >> 1) & 0x55555555u;
+        for (int r = 0; r < R; ++r) {
+          const uint32_t x = a ? cw[r].y : cw[r].x;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          fc[r][u] = (int)((x >> (2 * u)) & 0x03030303u);
-          fm[r][u] = (int)((ms >> (2 * u)) & 0x01010101u);
+          for (int u = 0; u < 4; ++u) f[r][u] = (int)((x >> (2 * u)) & 0x03030303u);
         }
-      }
+      };
+      auto miss_op = [&](i32x4 (&f)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint32_t x = a ? cw[r].y : cw[r].x, ms = x & (x >> 1) & 0x55555555u;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) f[r][u] = (int)((ms >> (2 * u)) & 0x01010101u);
+        }
+      };
+      auto dig_op = [&](int n) { return *(const i32x4 *)&lds[a][n * kFragB + lane * 16]; };
+      auto mul = [&](const i32x4 (&f)[R], const i32x4 &d, i32x4 (&c)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) c[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[r], d, c[r], 0, 0, 0);
+      };
+      i32x4 fc[R], fm[R];
+      if constexpr (MODE != kCdMiss) code_op(fc);
+      miss_op(fm);
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
-        const i32x4 d0 = *(const i32x4 *)&lds[buf][(2 * n + a) * kFragB + lane * 16];
+        const i32x4 d = dig_op(n);
         if constexpr (MODE == kCdPair) {
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            acc[0][n][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fc[r], d0, acc[0][n][r], 0, 0, 0);
-            acc[1][n][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fm[r], d0, acc[1][n][r], 0, 0, 0);
-          }
+          mul(fc, d, acc[0][n]);
+          mul(fm, d, acc[nacc - 1][n]);
         } else if constexpr (MODE == kCdSum) {
-          const i32x4 d1 = *(const i32x4 *)&lds[buf][(2 * (NT + n) + a) * kFragB + lane * 16];
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-            acc[0][n][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fc[r], d0, acc[0][n][r], 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-            acc[0][n][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fm[r], d1, acc[0][n][r], 0, 0, 0);
+          mul(fc, d, acc[0][n]);
+          mul(fm, dig_op(NT + n), acc[0][n]);
         } else {
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-            acc[0][n][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fm[r], d0, acc[0][n][r], 0, 0, 0);
+          mul(fm, d, acc[0][n]);
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
+      store(a ^ 1);
+      __syncthreads();
     }
-    store(buf ^ 1);
 #pragma unroll
     for (int r = 0; r < R; ++r) cw[r] = cn[r];
-    __syncthreads();
-    buf ^= 1;
   }
   // v_mfma_i32_16x16x64: lane l, result e holds D[4 (l / 16) + e][l % 16]
+  int32_t *out = A.part + (((int64_t)grp * A.nsplit + split) * nacc) * A.rowpad * (NT * 16) +
+                 (r0 + 4 * q) * (NT * 16) + (lane & 15);
+  const bool more = A.accum != 0;
+#pragma unroll 1
+  for (int a = 0; a < nacc; ++a) {
 #pragma unroll
-  for (int a = 0; a < nacc; ++a)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          out[(a * A.rowpad + r0 + 16 * r + 4 * q + e) * (NT * 16) + 16 * n + (lane & 15)] = acc[a][n][r][e];
+        for (int n = 0; n < NT; ++n) {
+          int32_t *o = out + (16 * r + e) * (NT * 16) + 16 * n;
+          const int v = nacc == 2 && a == 1 ? acc[nacc - 1][n][r][e] : acc[0][n][r][e];
+          *o = more ? *o + v : v;
+        }
+    out += A.rowpad * (NT * 16);
+  }
 }
 
 // ------------------------------------------------------------------ results
-// column j (of its group's Cg) of one row: the digits' sum over the splits, in units of
-// the column's grid, as hi * 2^24 + lo, both exact
-__device__ __forceinline__ void digit_sum(const int32_t *__restrict__ p, int64_t step, int32_t nsplit,
-                                          int32_t Cg, int64_t &hi, int64_t &lo) {
+// kOutRows rows of one group's sums, over the splits, in LDS: a block reads them in whole
+// lines (a thread per result reading its digits from memory took 1.3 ms for 600,000 rows
+// of ten columns stored by column, now 0.19, and 0.13 for 100,000 of twenty, now 0.10)
+constexpr int kOutRows = 16;
+template <int NACC>
+__device__ __forceinline__ void out_rows(const int32_t *__restrict__ part, int32_t NTc, int64_t rowpad,
+                                         int32_t nsplit, int64_t row0, int64_t *sm) {
+  const int64_t plane = rowpad * NTc;
+#pragma unroll
+  for (int a = 0; a < NACC; ++a) {
+    const int32_t *p = part + a * plane + row0 * NTc;
+    for (int e = threadIdx.x * 4; e < kOutRows * NTc; e += 1024) {
+      int64_t v[4] = {0, 0, 0, 0};
+#pragma unroll 4
+      for (int32_t sp = 0; sp < nsplit; ++sp) {
+        const i32x4 x = *(const i32x4 *)(p + sp * (NACC * plane) + e);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] += x[u];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sm[a * kOutRows * NTc + e + u] = v[u];
+    }
+  }
+  __syncthreads();
+}
+// a column's digits in units of its grid, as hi * 2^24 + lo, both exact
+__device__ __forceinline__ void digit_sum(const int64_t *p, int32_t Cg, int64_t &hi, int64_t &lo) {
   hi = lo = 0;
 #pragma unroll
   for (int s = 0; s < kDig; ++s) {
-    int64_t v = 0;
-#pragma unroll 8
-    for (int32_t sp = 0; sp < nsplit; ++sp) v += p[sp * step + s * Cg];
-    if (s < 4) hi = hi * 256 + v;
-    else lo = lo * 256 + v;
+    if (s < 4) hi = hi * 256 + p[s * Cg];
+    else lo = lo * 256 + p[s * Cg];
   }
 }
 __device__ __forceinline__ double two_parts(int64_t hi, int64_t lo) {
@@ -390,24 +431,28 @@ __global__ __launch_bounds__(256) void k_cd_out_sum(const int32_t *__restrict__ 
                                                     const u64 *__restrict__ sums, double scale,
                                                     double *__restrict__ out, int64_t ldr, int64_t ldc,
                                                     int32_t add) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t row = e / Cpad;
-  const int32_t c = (int32_t)(e % Cpad);
-  if (row >= nrow) return;
-  double v = 0.0;
-  if (c < C) {
-    const int32_t g = c / Cg, j = c % Cg;
-    const int64_t step = rowpad * NTc;
-    int64_t hi, lo;
-    digit_sum(part + (int64_t)g * nsplit * step + row * NTc + j, step, nsplit, Cg, hi, lo);
-    // the sums' parts split at 28 bits, the digits' at 24
-    const int64_t s0 = (int64_t)sums[2 * c], s1 = (int64_t)sums[2 * c + 1];
-    hi += 16 * s1;
-    lo += s0;
-    v = two_parts(hi, lo) * col_quantum(mx[c]) * scale;
+  __shared__ int64_t sm[kOutRows * kMaxNT * 16];
+  const int64_t row0 = (int64_t)blockIdx.x * kOutRows;
+  const int32_t g = blockIdx.y, c0 = g * Cg, c1 = g + 1 == (int32_t)gridDim.y ? Cpad : c0 + Cg;
+  out_rows<1>(part + (int64_t)g * nsplit * rowpad * NTc, NTc, rowpad, nsplit, row0, sm);
+  const int32_t w = c1 - c0;
+  for (int e = threadIdx.x; e < kOutRows * w; e += 256) {
+    const int r = ldc == 1 ? e / w : e % kOutRows, j = ldc == 1 ? e % w : e / kOutRows;
+    const int64_t row = row0 + r;
+    const int32_t c = c0 + j;
+    if (row >= nrow) continue;
+    double v = 0.0;
+    if (c < C) {
+      int64_t hi, lo;
+      digit_sum(sm + r * NTc + j, Cg, hi, lo);
+      // the sums' parts split at 28 bits, the digits' at 24
+      hi += 16 * (int64_t)sums[2 * c + 1];
+      lo += (int64_t)sums[2 * c];
+      v = two_parts(hi, lo) * col_quantum(mx[c]) * scale;
+    }
+    double *o = out + row * ldr + c * ldc;
+    *o = add ? *o + v : v;
   }
-  double *o = out + row * ldr + c * ldc;
-  *o = add ? *o + v : v;
 }
 
 // rows = SNPs: f (C - 3 M) + l0 (S - M) times `scale`, C and M the sums over the codes and
@@ -420,37 +465,32 @@ __global__ __launch_bounds__(256) void k_cd_out_pair(const int32_t *__restrict__
                                                      const double *__restrict__ lev,
                                                      const uint8_t *__restrict__ ignore, double scale,
                                                      double *__restrict__ out, int64_t ldr, int64_t ldc) {
-  int64_t row;
-  int32_t c;
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (ldc == 1) {
-    row = e / C;
-    c = (int32_t)(e % C);
-  } else {
-    row = e % nrow;
-    c = (int32_t)(e / nrow);
-    if (c >= C) return;
+  __shared__ int64_t sm[2 * kOutRows * kMaxNT * 16];
+  const int64_t row0 = (int64_t)blockIdx.x * kOutRows;
+  const int32_t g = blockIdx.y, c0 = g * Cg, w = min(Cg, C - c0);
+  out_rows<2>(part + (int64_t)g * nsplit * 2 * rowpad * NTc, NTc, rowpad, nsplit, row0, sm);
+  for (int e = threadIdx.x; e < kOutRows * w; e += 256) {
+    const int r = ldc == 1 ? e / w : e % kOutRows, j = ldc == 1 ? e % w : e / kOutRows;
+    const int64_t row = row0 + r;
+    const int32_t c = c0 + j;
+    if (row >= nrow) continue;
+    double v = 0.0;
+    if (!ignore || !ignore[row]) {
+      int64_t ch, cl, mh, ml;
+      digit_sum(sm + r * NTc + j, Cg, ch, cl);
+      digit_sum(sm + (kOutRows + r) * NTc + j, Cg, mh, ml);
+      const double l0 = lev[4 * row], f = 0.5 * (lev[4 * row + 2] - l0);
+      const double x = two_parts(ch - 3 * mh, cl - 3 * ml);
+      const double y = two_parts(16 * (int64_t)sums[2 * c + 1] - mh, (int64_t)sums[2 * c] - ml);
+      v = (f * x + l0 * y) * col_quantum(mx[c]) * scale;
+    }
+    out[row * ldr + c * ldc] = v;
   }
-  if (row >= nrow) return;
-  double v = 0.0;
-  if (!ignore || !ignore[row]) {
-    const int32_t g = c / Cg, j = c % Cg;
-    const int64_t plane = rowpad * NTc, step = 2 * plane;
-    const int32_t *p = part + (int64_t)g * nsplit * step + row * NTc + j;
-    int64_t ch, cl, mh, ml;
-    digit_sum(p, step, nsplit, Cg, ch, cl);
-    digit_sum(p + plane, step, nsplit, Cg, mh, ml);
-    const double l0 = lev[4 * row], f = 0.5 * (lev[4 * row + 2] - l0);
-    const double x = two_parts(ch - 3 * mh, cl - 3 * ml);
-    const double y = two_parts(16 * (int64_t)sums[2 * c + 1] - mh, (int64_t)sums[2 * c] - ml);
-    v = (f * x + l0 * y) * col_quantum(mx[c]) * scale;
-  }
-  out[row * ldr + c * ldc] = v;
 }
 
 template <int KIND, int MODE, int NT>
 void launch_mul(const MulArgs &A, hipStream_t st) {
-  constexpr int R = MODE == kCdPair ? 2 : 4;
+  constexpr int R = cd_rows(MODE, NT) / 64;
   hipLaunchKernelGGL((k_cd_mul<NT, MODE, R>), dim3((unsigned)((int64_t)A.nrowblk * A.ngroup * A.nsplit)),
                      dim3(256), 0, st, A);
 }
@@ -470,7 +510,7 @@ CodesPlan eig_codes_plan(const eig_ctx *ctx, int mode, int32_t C, int64_t nrow, 
   P.C = C;
   P.nblk = nblk;
   cd_groups(C, P.ngroup, P.Cg, P.NT);
-  const int32_t rows = mode == kCdPair ? 128 : 256;
+  const int32_t rows = cd_rows(mode, P.NT);
   P.nrowblk = (int32_t)((nrow + rows - 1) / rows);
   P.rowpad = (int64_t)P.nrowblk * rows;
   // splits: rounds of the blocks the chip holds (two per CU) times stages each, plus the
@@ -565,7 +605,8 @@ int eig_codes_out_sum(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void
                       double scale, double *out, int64_t ldr, int64_t ldc, int32_t Cpad, bool add,
                       hipStream_t st) {
   const u64 *mx = (const u64 *)head;
-  hipLaunchKernelGGL(k_cd_out_sum, dim3((unsigned)((nrow * Cpad + 255) / 256)), dim3(256), 0, st,
+  hipLaunchKernelGGL(k_cd_out_sum, dim3((unsigned)((nrow + kOutRows - 1) / kOutRows), (unsigned)P.ngroup),
+                     dim3(256), 0, st,
                      (const int32_t *)part, P.NT * 16, P.rowpad, P.nsplit, P.Cg, P.C, Cpad, nrow, mx,
                      mx + P.C, scale, out, ldr, ldc, add ? 1 : 0);
   EIG_HIP(ctx, hipGetLastError());
@@ -576,7 +617,8 @@ int eig_codes_out_pair(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const voi
                        const double *lev, const uint8_t *ignore, double scale, double *out, int64_t ldr,
                        int64_t ldc, hipStream_t st) {
   const u64 *mx = (const u64 *)head;
-  hipLaunchKernelGGL(k_cd_out_pair, dim3((unsigned)((nrow * P.C + 255) / 256)), dim3(256), 0, st,
+  hipLaunchKernelGGL(k_cd_out_pair, dim3((unsigned)((nrow + kOutRows - 1) / kOutRows), (unsigned)P.ngroup),
+                     dim3(256), 0, st,
                      (const int32_t *)part, P.NT * 16, P.rowpad, P.nsplit, P.Cg, P.C, nrow, mx, mx + P.C,
                      lev, ignore, scale, out, ldr, ldc);
   EIG_HIP(ctx, hipGetLastError());

@@ -358,6 +358,7 @@ extern "C" int eig_select(eig_ctx *ctx, const int32_t *xindex, int32_t nrows) {
   ctx->nrows = nrows;
   ctx->nst = nst;
   ctx->have_sel = true;
+  ctx->sel_all = ident && nrows == ctx->nind;
   ctx->have_selg = ctx->have_selb = ctx->have_stats = ctx->have_xtx = ctx->have_load = false;
   return EIG_OK;
 }

@@ -41,6 +41,7 @@ struct eig_ctx {
   DevBuf xindex, sel;
   int32_t nrows = 0, nst = 0;
   bool have_sel = false;
+  bool sel_all = false;  // every loaded individual, in order
   // the same codes regrouped per 64-SNP group for the split-BF16 XTX (built on
   // first use after each selection)
   DevBuf selg;

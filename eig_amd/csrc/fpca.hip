@@ -643,44 +643,52 @@ struct Plan {
 };
 }  // namespace
 
-// Eigen-decomposition of the n x n symmetric device matrix G (column-major, ld n):
-// eigenvalues descending in w (host), eigenvectors in the columns of V (device,
-// ld n) in the same order.
-// The same cyclic Jacobi for orders up to kJacLds, with A and V held in LDS (the
-// global-memory version pays an L2 round trip per rotation round).
+// The orthonormalising factor of a block of n <= kJacLds columns from their Gram matrix G
+// (column-major, ld n): with G = D S D (D the columns' norms) and S = Z diag(w) Z^T,
+// w descending, the columns k of V = D^-1 Z diag(w)^-1/2 whose w_k > 1e-13 w_0; *keep their
+// number (0 when S has no positive eigenvalue, -1 when the Jacobi sweeps ran out).  One
+// block, everything in LDS: cyclic Jacobi in which a thread owns a 2 x 2 block of (row
+// pair, column pair) and applies both rotations to it, two barriers a round (the
+// column and row passes one by one took five more); the scaling, the order and the cut,
+// with their copies and waits, were the host's (2.9 of the 18 ms that a basis of 11 x 20
+// columns of 100,003 takes).
 constexpr int kJacLds = 48;
-__global__ __launch_bounds__(256) void k_jacobi_lds(double *__restrict__ A, int32_t lda,
-                                                    double *__restrict__ V, int32_t ldv, int32_t n,
-                                                    int32_t max_sweeps, double tol,
-                                                    int32_t *__restrict__ sweeps_out) {
-  __shared__ double sA[kJacLds][kJacLds + 1], sV[kJacLds][kJacLds + 1];
-  __shared__ int32_t idx[kJacLds];
-  __shared__ int32_t pp[kJacLds / 2], pq[kJacLds / 2];
+__global__ __launch_bounds__(256) void k_orth_lds(const double *__restrict__ G, double *__restrict__ V,
+                                                  int32_t n, int32_t max_sweeps, double tol,
+                                                  int32_t *__restrict__ keep) {
+  __shared__ double sA[kJacLds][kJacLds + 1], sV[kJacLds][kJacLds + 1], dsc[kJacLds];
   __shared__ double cs[kJacLds / 2], sn[kJacLds / 2];
-  __shared__ int rotated;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int np = n + (n & 1);
+  __shared__ int32_t pp[kJacLds / 2], pq[kJacLds / 2], rank[kJacLds];
+  __shared__ int rotated, nkeep;
+  const int tid = threadIdx.x;
+  const int np = n + (n & 1);  // an odd order gets a dummy index n
   const int half = np / 2;
-  // sA[j][i] = A[j * lda + i] (column j), sV likewise
-  for (int e = tid; e < n * n; e += nt) {
+  if (tid < n) {
+    const double g = G[(int64_t)tid * n + tid];
+    dsc[tid] = g > 0.0 ? sqrt(g) : 1.0;
+  }
+  if (tid == 0) nkeep = 0;
+  __syncthreads();
+  for (int e = tid; e < n * n; e += 256) {  // sA[j][i] = column j, row i
     const int i = e % n, j = e / n;
-    sA[j][i] = A[(int64_t)j * lda + i];
+    sA[j][i] = G[e] / (dsc[i] * dsc[j]);
     sV[j][i] = (i == j) ? 1.0 : 0.0;
   }
   __syncthreads();
   int sweep = 0;
   for (; sweep < max_sweeps; ++sweep) {
     if (tid == 0) rotated = 0;
-    for (int e = tid; e < np; e += nt) idx[e] = e;
     __syncthreads();
     for (int round = 0; round < np - 1; ++round) {
-      for (int k = tid; k < half; k += nt) {
-        int p = idx[k], q = idx[np - 1 - k];
-        if (p > q) {
-          const int t = p;
-          p = q;
-          q = t;
-        }
+      if (tid < half) {
+        // round robin: slot 0 holds index 0, slot s index 1 + (s - 1 - round) mod (np - 1)
+        const int s0 = tid, s1 = np - 1 - tid;
+        auto at = [&](int s) {
+          const int v = s - 1 - round;
+          return s == 0 ? 0 : 1 + (v < 0 ? v + np - 1 : v);
+        };
+        const int x = at(s0), y = at(s1);
+        const int p = x < y ? x : y, q = x < y ? y : x;
         double c = 1.0, s = 0.0;
         if (q < n) {
           const double apq = sA[q][p], app = sA[p][p], aqq = sA[q][q];
@@ -692,57 +700,63 @@ __global__ __launch_bounds__(256) void k_jacobi_lds(double *__restrict__ A, int3
             rotated = 1;
           }
         }
-        pp[k] = p;
-        pq[k] = q < n ? q : p;
-        cs[k] = c;
-        sn[k] = q < n ? s : 0.0;
+        pp[tid] = p;
+        pq[tid] = q;
+        cs[tid] = c;
+        sn[tid] = s;
       }
       __syncthreads();
-      for (int e = tid; e < n * half; e += nt) {  // columns: A <- A J, V <- V J
-        const int i = e % n, k = e / n;
-        const double c = cs[k], s = sn[k];
-        if (s == 0.0) continue;
-        const int p = pp[k], q = pq[k];
-        const double x = sA[p][i], y = sA[q][i];
-        sA[p][i] = c * x - s * y;
-        sA[q][i] = s * x + c * y;
-        const double u = sV[p][i], v = sV[q][i];
-        sV[p][i] = c * u - s * v;
-        sV[q][i] = s * u + c * v;
-      }
-      __syncthreads();
-      for (int e = tid; e < n * half; e += nt) {  // rows: A <- J^T A
-        const int j = e % n, k = e / n;
-        const double c = cs[k], s = sn[k];
-        if (s == 0.0) continue;
-        const int p = pp[k], q = pq[k];
-        const double x = sA[j][p], y = sA[j][q];
-        sA[j][p] = c * x - s * y;
-        sA[j][q] = s * x + c * y;
-      }
-      __syncthreads();
-      for (int k = tid; k < half; k += nt)
-        if (sn[k] != 0.0) {
-          sA[pq[k]][pp[k]] = 0.0;
-          sA[pp[k]][pq[k]] = 0.0;
+      // A <- J^T A J, block (row pair k, column pair l)
+      for (int l = tid >> 4; l < half; l += 16)
+        for (int k = tid & 15; k < half; k += 16) {
+          const double ck = cs[k], sk = sn[k], cl = cs[l], sl = sn[l];
+          if (sk == 0.0 && sl == 0.0) continue;
+          const int p = pp[k], q = pq[k], r = pp[l], u = pq[l];
+          const bool hq = q < n, hu = u < n;
+          const double a00 = sA[r][p], a10 = hq ? sA[r][q] : 0.0, a01 = hu ? sA[u][p] : 0.0,
+                       a11 = hq && hu ? sA[u][q] : 0.0;
+          // columns first: (r, u) <- (cl r - sl u, sl r + cl u), then rows likewise
+          const double b00 = cl * a00 - sl * a01, b01 = sl * a00 + cl * a01;
+          const double b10 = cl * a10 - sl * a11, b11 = sl * a10 + cl * a11;
+          const bool diag = k == l && sk != 0.0;  // the annihilated pair: exact zeros
+          sA[r][p] = ck * b00 - sk * b10;
+          if (hu) sA[u][p] = diag ? 0.0 : ck * b01 - sk * b11;
+          if (hq) sA[r][q] = diag ? 0.0 : sk * b00 + ck * b10;
+          if (hq && hu) sA[u][q] = sk * b01 + ck * b11;
         }
-      {
-        const int e = tid + 1;
-        int v = 0;
-        if (e < np) v = (e == 1) ? idx[np - 1] : idx[e - 1];
-        __syncthreads();
-        if (e < np) idx[e] = v;
-        __syncthreads();
-      }
+      for (int k = tid >> 5; k < half; k += 8)  // V <- V J
+        for (int i = tid & 31; i < n; i += 32) {
+          const double c = cs[k], s = sn[k];
+          if (s == 0.0) continue;
+          const int p = pp[k], q = pq[k];
+          const double u = sV[p][i], v = sV[q][i];
+          sV[p][i] = c * u - s * v;
+          sV[q][i] = s * u + c * v;
+        }
+      __syncthreads();
     }
     if (!rotated) break;
+    __syncthreads();
   }
-  for (int e = tid; e < n * n; e += nt) {
+  // descending order, ties by index
+  if (tid < n) {
+    const double w = sA[tid][tid];
+    double w0 = w;
+    int r = 0;
+    for (int j = 0; j < n; ++j) {
+      const double x = sA[j][j];
+      w0 = fmax(w0, x);
+      r += x > w || (x == w && j < tid);
+    }
+    rank[tid] = r;
+    if (w0 > 0.0 && w > 1e-13 * w0) atomicAdd(&nkeep, 1);
+  }
+  __syncthreads();
+  for (int e = tid; e < n * n; e += 256) {
     const int i = e % n, j = e / n;
-    A[(int64_t)j * lda + i] = sA[j][i];
-    V[(int64_t)j * ldv + i] = sV[j][i];
+    V[(int64_t)rank[j] * n + i] = sV[j][i] / (sqrt(sA[j][j]) * dsc[i]);
   }
-  if (tid == 0) sweeps_out[0] = sweep;
+  if (tid == 0) *keep = sweep >= max_sweeps ? -1 : nkeep;
 }
 
 // V column k = work column ord[k] (n x n, column-major)
@@ -754,26 +768,45 @@ __global__ void k_gather_cols(double *__restrict__ V, const double *__restrict__
   V[e] = work[(int64_t)ord[k] * n + i];
 }
 
-// C (m x n, column-major, ld ldc) = sum over s of part[s] (m x n, ld m), in order
-__global__ void k_sum_parts(const double *__restrict__ part, int32_t S, int32_t m, int32_t n,
-                            double *__restrict__ C, int32_t ldc) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t mn = (int64_t)m * n;
-  if (e >= mn) return;
+// C (m x n, column-major, ld ldc) = sum over s of part[s] (m x n, ld m): 256 / T elements
+// a block, T threads each summing every T-th part, then those sums in order
+template <int T>
+__global__ __launch_bounds__(256) void k_sum_parts(const double *__restrict__ part, int32_t S,
+                                                   int32_t m, int32_t n, double *__restrict__ C,
+                                                   int32_t ldc) {
+  constexpr int E = 256 / T;
+  __shared__ double sm[T][E];
+  const int l = threadIdx.x % E, g = threadIdx.x / E;
+  const int64_t e = (int64_t)blockIdx.x * E + l, mn = (int64_t)m * n;
   double v = 0.0;
-  for (int32_t sp = 0; sp < S; ++sp) v += part[(int64_t)sp * mn + e];
-  C[(e / m) * ldc + (e % m)] = v;
+  if (e < mn) {
+#pragma unroll 8
+    for (int32_t sp = g; sp < S; sp += T) v += part[(int64_t)sp * mn + e];
+  }
+  sm[g][l] = v;
+  __syncthreads();
+  if (g == 0 && e < mn) {
+    for (int u = 1; u < T; ++u) v += sm[u][l];
+    C[(e / m) * ldc + (e % m)] = v;
+  }
 }
 
 // C (m x n, column-major, ld ldc) = A B^T, A m x k (ld lda) and B n x k (ld ldb) column-major,
 // for a long k: k is cut into S equal chunks (one batched product) and a remainder,
-// whose partial products are summed in chunk order.  A single product of these shapes
-// has only a few output tiles to spread a long k over.
-static int gemm_nt_long(eig_ctx *ctx, int32_t m, int32_t n, int64_t k, const double *A,
+// whose partial products are summed.  A single product of these shapes has only a few
+// output tiles to spread a long k over.  `fine`: chunks for 1,024 blocks, of at least 256 k
+// (k = 100,003: 27 us a product against 140 in up to 64 chunks of at least 4,096, 24 to 96
+// blocks).  The split-BF16 form keeps the coarse chunks and their order of summation: it
+// rounds the basis to BF16 pairs, so a basis that differs in the last bits moves its
+// eigenvectors by that form's own error over their gaps (1.6e-5 on a panel of twelve
+// populations of like drift).
+static int gemm_nt_long(eig_ctx *ctx, bool fine, int32_t m, int32_t n, int64_t k, const double *A,
                         int64_t lda, const double *B, int64_t ldb, double *C, int32_t ldc,
                         double *part, size_t part_doubles, hipStream_t st) {
   const int64_t mn = (int64_t)m * n;
-  int64_t S = std::min<int64_t>(64, k / 4096);
+  const int64_t tiles = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
+  int64_t S = fine ? std::min<int64_t>(std::max<int64_t>(1, 1024 / tiles), k / 256)
+                   : std::min<int64_t>(64, k / 4096);
   S = std::min<int64_t>(S, (int64_t)(part_doubles / std::max<int64_t>(mn, 1)) - 1);
   if (S < 2)
     return eig_gemm_f64(ctx, st, false, true, m, n, k, 1.0, A, lda, 0, B, ldb, 0, 0.0, C, ldc, 0, 1);
@@ -786,22 +819,24 @@ static int gemm_nt_long(eig_ctx *ctx, int32_t m, int32_t n, int64_t k, const dou
                          B + S * kc * ldb, ldb, 0, 0.0, part + S * mn, m, 0, 1));
     ++nparts;
   }
-  hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st,
-                     (const double *)part, nparts, m, n, C, ldc);
+  if (fine)
+    hipLaunchKernelGGL(k_sum_parts<4>, dim3((unsigned)((mn + 63) / 64)), dim3(256), 0, st,
+                       (const double *)part, nparts, m, n, C, ldc);
+  else
+    hipLaunchKernelGGL(k_sum_parts<1>, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st,
+                       (const double *)part, nparts, m, n, C, ldc);
   EIG_HIP(ctx, hipGetLastError());
   return EIG_OK;
 }
 
+// Eigen-decomposition of the n x n symmetric device matrix G (column-major, ld n) of more
+// than kJacLds columns: eigenvalues descending in w (host), eigenvectors in the columns of
+// V (device, ld n) in the same order.
 static int small_eigh(eig_ctx *ctx, double *G, int32_t n, double *V, std::vector<double> &w,
                       double *work, int32_t *d_sweeps) {
   if (n > kJacMax) return eig_set_err(ctx, EIG_E_ARG, "fpca: basis larger than %d", kJacMax);
   hipStream_t st = ctx->stream;
-  if (n <= kJacLds)
-    hipLaunchKernelGGL(k_jacobi_lds, dim3(1), dim3(256), 0, st, G, n, work, n, n, 30, 1e-15,
-                       d_sweeps);
-  else
-    hipLaunchKernelGGL(k_jacobi, dim3(1), dim3(1024), 0, st, G, n, work, n, n, 30, 1e-15,
-                       d_sweeps);
+  hipLaunchKernelGGL(k_jacobi, dim3(1), dim3(1024), 0, st, G, n, work, n, n, 30, 1e-15, d_sweeps);
   EIG_HIP(ctx, hipGetLastError());
   std::vector<double> a((size_t)n * n);
   int32_t sweeps = 0;
@@ -1083,7 +1118,7 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   // W (nc columns, column-major nc x M at Wp, ld ldq) -= U_r (U_r^T W)
   auto project = [&](double *Wp, int32_t nc) -> int {
     if (r == 0) return EIG_OK;
-    EIG_TRY(gemm_nt_long(ctx, r, nc, M, U, ldq, Wp, ldq, Cb, r, part, part_doubles, st));
+    EIG_TRY(gemm_nt_long(ctx, !bf, r, nc, M, U, ldq, Wp, ldq, Cb, r, part, part_doubles, st));
     EIG_TRY(eig_gemm_f64(ctx, st, true, false, nc, M, r, -1.0, Cb, r, 0, U, ldq, 0, 1.0, Wp, ldq,
                          0, 1));
     return EIG_OK;
@@ -1091,7 +1126,19 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   // Out (keep columns) = orthonormal basis of the nc columns at Wp
   auto orth = [&](const double *Wp, int32_t nc, double *Out, int32_t &keep) -> int {
     keep = 0;
-    EIG_TRY(gemm_nt_long(ctx, nc, nc, M, Wp, ldq, Wp, ldq, G, nc, part, part_doubles, st));
+    EIG_TRY(gemm_nt_long(ctx, !bf, nc, nc, M, Wp, ldq, Wp, ldq, G, nc, part, part_doubles, st));
+    if (nc <= kJacLds) {
+      hipLaunchKernelGGL(k_orth_lds, dim3(1), dim3(256), 0, st, (const double *)G, V, nc, 30, 1e-15,
+                         d_sweeps);
+      EIG_HIP(ctx, hipGetLastError());
+      EIG_HIP(ctx, hipMemcpyAsync(&keep, d_sweeps, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+      EIG_HIP(ctx, hipStreamSynchronize(st));
+      if (keep < 0) return eig_set_err(ctx, EIG_E_CONVERGE, "fpca: Jacobi did not converge");
+      if (keep > 0)
+        EIG_TRY(eig_gemm_f64(ctx, st, true, false, keep, M, nc, 1.0, V, nc, 0, Wp, ldq, 0, 0.0, Out,
+                             ldq, 0, 1));
+      return EIG_OK;
+    }
     std::vector<double> g((size_t)nc * nc), dsc(nc);
     EIG_HIP(ctx, hipMemcpyAsync(g.data(), G, sizeof(double) * g.size(), hipMemcpyDeviceToHost, st));
     EIG_HIP(ctx, hipStreamSynchronize(st));
@@ -1151,7 +1198,7 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
     CodesPlan pr = eig_codes_plan(ctx, kCdSum, r, npad, (G64 + 1) / 2, pu.nsplit);
     EIG_TRY(code_xtb(pr, src, 1.0, Bm, ldq, r));
   }
-  EIG_TRY(gemm_nt_long(ctx, r, r, npad, Bm, ldq, Bm, ldq, G, r, part, part_doubles, st));
+  EIG_TRY(gemm_nt_long(ctx, !bf, r, r, npad, Bm, ldq, Bm, ldq, G, r, part, part_doubles, st));
   // top-K eigenpairs of B^T B (order r up to 256) by the FP64 eigensolver: all
   // eigenvalues, K eigenvectors into V (column-major r x K)
   {

@@ -152,19 +152,24 @@ __global__ __launch_bounds__(64) void k_lsq_gram(const uint8_t *__restrict__ gen
 // reduce chunks in order, Cholesky solve (choldc/cholsl order of operations)
 // itype (may be NULL): with the fill, an individual of type >= 0 is also ignored when
 // its observed genotypes alone number <= K (lsqproj's first loop, smartpca.c:4637-4651).
-__global__ void k_lsq_solve(const double *__restrict__ partial, int64_t nchunk, int32_t nind,
-                            int32_t K, const int32_t *__restrict__ use,
-                            const int32_t *__restrict__ itype, double *__restrict__ ans,
-                            double *__restrict__ rhs_out, int32_t *__restrict__ st) {
+template <int K>
+__global__ __launch_bounds__(64) void k_lsq_solve(const double *__restrict__ partial, int64_t nchunk,
+                                                  int32_t nind, const int32_t *__restrict__ use,
+                                                  const int32_t *__restrict__ itype,
+                                                  double *__restrict__ ans, double *__restrict__ rhs_out,
+                                                  int32_t *__restrict__ st) {
   const int32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= nind) return;
-  const int nP = K * (K + 1) / 2, W = nP + K + 2;
-  double acc[kMaxK * (kMaxK + 1) / 2 + kMaxK + 2];
+  constexpr int nP = K * (K + 1) / 2, W = nP + K + 2;
+  double acc[W];
+#pragma unroll
   for (int p = 0; p < W; ++p) acc[p] = 0.0;
   for (int64_t c = 0; c < nchunk; ++c) {
     const double *pp = partial + (c * (int64_t)nind + q) * W;
+#pragma unroll
     for (int p = 0; p < W; ++p) acc[p] += pp[p];
   }
+#pragma unroll
   for (int j = 0; j < K; ++j) rhs_out[(int64_t)j * nind + q] = acc[nP + j];
   if (!use[q]) {
     st[q] = 3;
@@ -174,33 +179,25 @@ __global__ void k_lsq_solve(const double *__restrict__ partial, int64_t nchunk, 
     st[q] = 1;
     return;
   }
-  double a[kMaxK][kMaxK], p[kMaxK], x[kMaxK];
-  {
-    int idx = 0;
-    for (int i = 0; i < K; ++i)
-      for (int j = i; j < K; ++j) {
-        a[i][j] = acc[idx];
-        a[j][i] = acc[idx];
-        ++idx;
-      }
-  }
+  // the upper triangle at (i, j), j >= i, holds a[i][j] until step (i, j) puts the factor's
+  // [j][i] there: constant indices, so everything stays in registers
+  auto at = [&](int i, int j) -> double & { return acc[i * K - i * (i - 1) / 2 + (j - i)]; };
+  double p[K], x[K];
   bool bad = false;
-  for (int i = 0; i < K * K; ++i)
-    if (isnan(a[i / K][i % K])) bad = true;
-  for (int i = 0; i < K; ++i)
-    if (isnan(acc[nP + i])) bad = true;
-  for (int i = 0; i < K && !bad; ++i) {
+#pragma unroll
+  for (int i = 0; i < nP + K; ++i) bad |= isnan(acc[i]);
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+#pragma unroll
     for (int j = i; j < K; ++j) {
-      double s = a[i][j];
-      for (int k = i - 1; k >= 0; --k) s -= a[i][k] * a[j][k];
+      double s = at(i, j);
+#pragma unroll
+      for (int k = i - 1; k >= 0; --k) s -= at(k, i) * at(k, j);
       if (i == j) {
-        if (s <= 0.0) {
-          bad = true;
-          break;
-        }
-        p[i] = sqrt(s);
+        bad |= s <= 0.0;
+        p[i] = sqrt(s > 0.0 ? s : 1.0);
       } else {
-        a[j][i] = s / p[i];
+        at(i, j) = s / p[i];
       }
     }
   }
@@ -208,16 +205,21 @@ __global__ void k_lsq_solve(const double *__restrict__ partial, int64_t nchunk, 
     st[q] = 2;
     return;
   }
+#pragma unroll
   for (int i = 0; i < K; ++i) {
     double s = acc[nP + i];
-    for (int k = i - 1; k >= 0; --k) s -= a[i][k] * x[k];
+#pragma unroll
+    for (int k = i - 1; k >= 0; --k) s -= at(k, i) * x[k];
     x[i] = s / p[i];
   }
+#pragma unroll
   for (int i = K - 1; i >= 0; --i) {
     double s = x[i];
-    for (int k = i + 1; k < K; ++k) s -= a[k][i] * x[k];
+#pragma unroll
+    for (int k = i + 1; k < K; ++k) s -= at(i, k) * x[k];
     x[i] = s / p[i];
   }
+#pragma unroll
   for (int j = 0; j < K; ++j) ans[(int64_t)j * nind + q] = x[j];
   st[q] = 0;
 }
@@ -245,7 +247,7 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
   // ffvecs = 10 Z^T v as a product over the samples (rows = SNPs), fxvecs = X ff as one
   // over the SNPs (rows = samples), on the code planes (codes.hip).  At 5,000 x 600,000,
   // K = 10, both read the codes once: 19.6 ms with per-code bins and FP64 sums on the
-  // vector units, LOADMS now.
+  // vector units, 1.45 now.
   const int64_t G64 = (M + kGrp - 1) / kGrp;
   const CodeView vm{(const uint8_t *)ctx->sel.p, nullptr, 128 * 32, 32, M * 32, 16, M,
                     (int64_t)ctx->nst * 8, kCodeLinear};
@@ -296,18 +298,30 @@ __global__ __launch_bounds__(256) void k_regroup_geno(const uint8_t *__restrict_
                                                       int64_t M, int32_t nind, int64_t m0, int32_t q0,
                                                       int64_t G64, int64_t ngroups,
                                                       uint4 *__restrict__ out) {
-  __shared__ uint8_t by[2][kGrp][36];
+  __shared__ __align__(4) uint8_t by[2][kGrp][36];
   const int half = threadIdx.x >> 7, i = threadIdx.x & 127;
   const int64_t gid = (int64_t)blockIdx.x * 2 + half;  // tile * G64 + group
   const bool live = gid < ngroups;
   const int64_t tile = live ? gid / G64 : 0, g = live ? gid % G64 : 0;
   const int64_t b0 = q0 / 4 + tile * 32;  // first byte of the tile's 128 individuals
   const int64_t nby = (nind + 3) / 4;
+  // four bytes a load (rows start at any byte; the hardware takes unaligned words), single
+  // ones where a row's last word would pass its end
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int idx = i + 128 * e, r = idx >> 5, b = idx & 31;
+  for (int e = 0; e < 4; ++e) {
+    const int idx = i + 128 * e, r = idx >> 3, b = (idx & 7) * 4;
     const int64_t m = m0 + g * kGrp + r;
-    by[half][r][b] = (live && m < M && b0 + b < nby) ? geno[m * rlen + b0 + b] : 0xFF;
+    const uint8_t *src = geno + m * rlen + b0 + b;
+    uint32_t word = ~0u;
+    if (live && m < M) {
+      if (b0 + b + 4 <= nby) {
+        __builtin_memcpy(&word, src, 4);
+      } else {
+        for (int u = 0; u < 4; ++u)
+          if (b0 + b + u < nby) word = (word & ~(0xFFu << (8 * u))) | ((uint32_t)src[u] << (8 * u));
+      }
+    }
+    *(uint32_t *)&by[half][r][b] = word;
   }
   __syncthreads();
   if (!live) return;
@@ -350,12 +364,15 @@ static int lsq_normal(eig_ctx *ctx, double *acc, char *ws, size_t bytes) {
   const int64_t nblk_all = (M + 127) / 128;
   int64_t nr = (nind + 255) / 256 * 256, nb = std::min(nblk_all, kLsqRange);
   int32_t smax = 32;
+  // with every individual selected, the selection's grouped codes are the individuals'
+  const bool shared = ctx->sel_all && ctx->have_selg;
+  const int64_t Gall = (M + kGrp - 1) / kGrp;
   CodesPlan pr, pg;
   size_t codes = 0;
   for (;;) {
     pr = eig_codes_plan(ctx, kCdSum, K + 1, std::min<int64_t>(nr, nind), nb, smax);
     pg = eig_codes_plan(ctx, kCdMiss, nP, std::min<int64_t>(nr, nind), nb, smax);
-    codes = up((size_t)nr * nb * 32);
+    codes = shared ? 0 : up((size_t)nr * nb * 32);
     const size_t need = pr.head_bytes + pg.head_bytes + up(pr.dig_bytes) + up(pg.dig_bytes) +
                         up(pr.part_bytes) + up(pg.part_bytes) + codes;
     if (need <= bytes) break;
@@ -388,11 +405,17 @@ static int lsq_normal(eig_ctx *ctx, double *acc, char *ws, size_t bytes) {
       cr.n = cg.n = std::min(M, s1 * 128);
       for (int64_t b0 = s0; b0 < s1; b0 += nb) {
         const int64_t G64 = 2 * nb;
-        hipLaunchKernelGGL(k_regroup_geno, dim3((unsigned)((tiles * G64 + 1) / 2)), dim3(256), 0, st,
-                           (const uint8_t *)ctx->geno.p, ctx->rlen, M, nind, b0 * 128, (int32_t)q0,
-                           G64, tiles * G64, cd);
-        const CodeView v{(const uint8_t *)cd, nullptr, G64 * 2048, 16, 4096, 2048, tiles * 128, G64 * 4,
-                         kCodeGrouped};
+        CodeView v{(const uint8_t *)cd, nullptr, G64 * 2048, 16, 4096, 2048, tiles * 128, G64 * 4,
+                   kCodeGrouped};
+        if (shared) {
+          v.base = (const uint8_t *)ctx->selg.p + ((q0 >> 7) * Gall + 2 * b0) * 2048;
+          v.RT = Gall * 2048;
+          v.nword = (Gall - 2 * b0) * 4;
+        } else {
+          hipLaunchKernelGGL(k_regroup_geno, dim3((unsigned)((tiles * G64 + 1) / 2)), dim3(256), 0, st,
+                             (const uint8_t *)ctx->geno.p, ctx->rlen, M, nind, b0 * 128, (int32_t)q0,
+                             G64, tiles * G64, cd);
+        }
         EIG_TRY(eig_codes_mul(ctx, pr, v, cr, b0, hr, dr, sr, b0 > s0, st));
         EIG_TRY(eig_codes_mul(ctx, pg, v, cg, b0, hg, dg, sg, b0 > s0, st));
       }
@@ -425,7 +448,7 @@ static int lsqproject(eig_ctx *ctx, const int32_t *use, const int32_t *itype, in
   const double *d_fx = (const double *)ctx->fxscal.p, *d_xm = d_fx + kMaxK;
   int64_t nchunk = 1;
   if (!itype) {
-    // the normal equations from the code planes (5,000 x 600,000, K = 10: LSQMS against
+    // the normal equations from the code planes (5,000 x 600,000, K = 10: 2.3 against
     // 25.6 ms of FP64 sums per individual); the workspace holds up to 1 GiB of it at once
     const size_t acc_b = (8 * (size_t)nind * W + 255) & ~(size_t)255;
     const size_t work = std::min((size_t)1 << 30, ((size_t)nind + 4096) * (M + 4096) + ((size_t)64 << 20));
@@ -445,9 +468,9 @@ static int lsqproject(eig_ctx *ctx, const int32_t *use, const int32_t *itype, in
                                       (const uint8_t *)ctx->ignore_dev.p, (const double *)d_fill,
                                       d_itype, npop, (double *)ctx->scratch2.p, nblk));
   }
-  hipLaunchKernelGGL(k_lsq_solve, dim3((unsigned)((nind + 127) / 128)), dim3(128), 0, st,
-                     (const double *)ctx->scratch2.p, nchunk, nind, K, (const int32_t *)d_use,
-                     d_itype, d_ans, d_rhs, d_st);
+  EIG_KSWITCH(K, hipLaunchKernelGGL((k_lsq_solve<KC>), dim3((unsigned)((nind + 63) / 64)), dim3(64), 0,
+                                    st, (const double *)ctx->scratch2.p, nchunk, nind,
+                                    (const int32_t *)d_use, d_itype, d_ans, d_rhs, d_st));
   EIG_HIP(ctx, hipGetLastError());
   eig_time_end(ctx, "lsqproject");
   std::vector<double> ans((size_t)K * nind), rhs((size_t)K * nind);
@@ -546,9 +569,10 @@ extern "C" int eig_lsqproject_noalloc(eig_ctx *ctx, const int32_t *use, double *
   hipLaunchKernelGGL(k_lsq_clear, dim3((unsigned)((kn + 255) / 256)), dim3(256), 0, st, d_ans,
                      (int64_t)kn);
   EIG_TRY(lsq_normal(ctx, d_acc, base + o_part, ctx->noalloc_bytes - o_part));
-  hipLaunchKernelGGL(k_lsq_solve, dim3((unsigned)((nind + 127) / 128)), dim3(128), 0, st,
-                     (const double *)d_acc, (int64_t)1, nind, K, (const int32_t *)d_use,
-                     (const int32_t *)nullptr, d_ans, d_rhs, d_st);
+  EIG_KSWITCH(K, hipLaunchKernelGGL((k_lsq_solve<KC>), dim3((unsigned)((nind + 63) / 64)), dim3(64), 0,
+                                    st, (const double *)d_acc, (int64_t)1, nind,
+                                    (const int32_t *)d_use, (const int32_t *)nullptr, d_ans, d_rhs,
+                                    d_st));
   hipLaunchKernelGGL(k_lsq_stale, dim3(1), dim3(64), 0, st, (const double *)d_ans,
                      (const double *)d_rhs, (const int32_t *)d_st, nind, K, acoeffs ? d_A : nullptr,
                      bcoeffs ? d_B : nullptr);
