@@ -237,9 +237,9 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
 }
 
 // ------------------------------------------------------------------ the product
-// rows of a block: four waves of R row tiles of 16
-constexpr int cd_rows(int mode, int NT) {
-  return 64 * (mode == kCdPair ? 2 : mode == kCdSum && NT == kMaxNT ? 3 : 4);
+// row tiles of 16 per wave at most (a block is four waves)
+constexpr int cd_tiles(int mode, int NT) {
+  return mode == kCdPair ? 2 : mode == kCdSum && NT == kMaxNT ? 3 : 4;
 }
 struct MulArgs {
   CodeView v;
@@ -383,6 +383,67 @@ __global__ __launch_bounds__(256, 2) void k_cd_mul(MulArgs A) {
   }
 }
 
+// ---- up to 16 rows: one row tile, so the digits are read once and bound the product.
+// A wave streams the digit operands of its range of stages straight from memory, a half
+// stage (NT x planes KB) ahead of its MFMAs; nothing is shared between waves.
+// part[grp][split][row < nrow][NT * 16].
+template <int NT, int MODE>
+__global__ __launch_bounds__(256) void k_cd_stream(const uint8_t *__restrict__ dig_, int32_t *__restrict__ part,
+                                                   CodeRows rows, int64_t nword, int64_t nblk, int64_t per,
+                                                   int32_t ngroup, int32_t nsplit) {
+  constexpr int planes = MODE == kCdSum ? 2 : 1, F = planes * NT, bytes = F * kFragB;
+  const int lane = threadIdx.x & 63, q = lane >> 4;
+  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (item >= (int64_t)ngroup * nsplit) return;
+  const int32_t grp = (int32_t)(item % ngroup), split = (int32_t)(item / ngroup);
+  const int64_t k0 = split * per, k1 = min(nblk, k0 + per);
+  const uint8_t *rp = rows.row[min(lane & 15, rows.n - 1)] + q * 8;
+  const uint8_t *dig = dig_ + (grp * nblk) * (2 * bytes) + lane * 16;
+  i32x4 acc[NT], f[F], g[F];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = i32x4{0, 0, 0, 0};
+  auto load = [&](int64_t h, i32x4 (&d)[F]) {
+    const uint8_t *s = dig + min(h, 2 * k1 - 1) * bytes;
+#pragma unroll
+    for (int n = 0; n < F; ++n) d[n] = *(const i32x4 *)(s + n * kFragB);
+  };
+  auto codes = [&](int64_t k) {
+    uint2 c = make_uint2(~0u, ~0u);
+    if (k < k1 && 8 * k + 2 * q < nword) c = *(const uint2 *)(rp + k * 32);
+    return c;
+  };
+  auto mul = [&](uint32_t x, const i32x4 (&d)[F]) {
+    const uint32_t ms = x & (x >> 1) & 0x55555555u;
+    i32x4 fc, fm;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      fc[u] = (int)((x >> (2 * u)) & 0x03030303u);
+      fm[u] = (int)((ms >> (2 * u)) & 0x01010101u);
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      if (MODE == kCdSum) acc[n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fc, d[n], acc[n], 0, 0, 0);
+      acc[n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fm, d[(planes - 1) * NT + n], acc[n], 0, 0, 0);
+    }
+  };
+  load(2 * k0, f);
+  uint2 cw = codes(k0);
+  for (int64_t k = k0; k < k1; ++k) {
+    load(2 * k + 1, g);
+    const uint2 cn = codes(k + 1);
+    mul(cw.x, f);
+    load(2 * k + 2, f);
+    mul(cw.y, g);
+    cw = cn;
+  }
+  int32_t *out = part + ((int64_t)grp * nsplit + split) * rows.n * (NT * 16) + (lane & 15);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (4 * q + e < rows.n)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) out[(4 * q + e) * (NT * 16) + 16 * n] = acc[n][e];
+}
+
 // ------------------------------------------------------------------ results
 // kOutRows rows of one group's sums, over the splits, in LDS: a block reads them in whole
 // lines (a thread per result reading its digits from memory took 1.3 ms for 600,000 rows
@@ -455,6 +516,40 @@ __global__ __launch_bounds__(256) void k_cd_out_sum(const int32_t *__restrict__ 
   }
 }
 
+// The results of kCdSum and kCdMiss over many splits: one block per (row, group), seven
+// slices of the splits side by side (part[grp][split][rowpad][NTc])
+__global__ __launch_bounds__(1024) void k_cd_out_small(const int32_t *__restrict__ part, int32_t NTc,
+                                                       int64_t rowpad, int32_t nsplit, int32_t Cg, int32_t C,
+                                                       const u64 *__restrict__ mx,
+                                                       const u64 *__restrict__ sums,
+                                                       double *__restrict__ out, int64_t ldr) {
+  __shared__ int64_t sl[7][kMaxNT * 16], sm[kMaxNT * 16];
+  const int32_t row = blockIdx.x, g = blockIdx.y;
+  const int t = threadIdx.x, j = t % NTc, s = t / NTc;
+  if (s < 7) {
+    int64_t v = 0;
+    const int32_t *p = part + ((int64_t)g * nsplit * rowpad + row) * NTc + j;
+#pragma unroll 8
+    for (int32_t sp = s; sp < nsplit; sp += 7) v += p[sp * rowpad * NTc];
+    sl[s][j] = v;
+  }
+  __syncthreads();
+  if (t < NTc) {
+    int64_t v = 0;
+#pragma unroll
+    for (int u = 0; u < 7; ++u) v += sl[u][t];
+    sm[t] = v;
+  }
+  __syncthreads();
+  const int32_t c = g * Cg + t;
+  if (t < Cg && c < C) {
+    int64_t hi, lo;
+    digit_sum(sm + t, Cg, hi, lo);
+    out[row * ldr + c] = two_parts(hi + 16 * (int64_t)sums[2 * c + 1], lo + (int64_t)sums[2 * c]) *
+                         col_quantum(mx[c]);
+  }
+}
+
 // rows = SNPs: f (C - 3 M) + l0 (S - M) times `scale`, C and M the sums over the codes and
 // the missing bits, S the column's own; zero where ignore (may be null) is set
 __global__ __launch_bounds__(256) void k_cd_out_pair(const int32_t *__restrict__ part, int32_t NTc,
@@ -488,11 +583,13 @@ __global__ __launch_bounds__(256) void k_cd_out_pair(const int32_t *__restrict__
   }
 }
 
-template <int KIND, int MODE, int NT>
-void launch_mul(const MulArgs &A, hipStream_t st) {
-  constexpr int R = cd_rows(MODE, NT) / 64;
-  hipLaunchKernelGGL((k_cd_mul<NT, MODE, R>), dim3((unsigned)((int64_t)A.nrowblk * A.ngroup * A.nsplit)),
-                     dim3(256), 0, st, A);
+template <int MODE, int NT>
+void launch_mul(const MulArgs &A, int R, hipStream_t st) {
+  constexpr int RX = cd_tiles(MODE, NT);
+  const dim3 grid((unsigned)((int64_t)A.nrowblk * A.ngroup * A.nsplit));
+  if (R == 1) hipLaunchKernelGGL((k_cd_mul<NT, MODE, 1>), grid, dim3(256), 0, st, A);
+  else if (R == 2) hipLaunchKernelGGL((k_cd_mul<NT, MODE, 2>), grid, dim3(256), 0, st, A);
+  else hipLaunchKernelGGL((k_cd_mul<NT, MODE, RX>), grid, dim3(256), 0, st, A);
 }
 }  // namespace
 
@@ -503,19 +600,21 @@ static void cd_groups(int32_t C, int32_t &ngroup, int32_t &Cg, int32_t &NT) {
   NT = Cg * kDig <= 80 ? 5 : 9;
 }
 
-CodesPlan eig_codes_plan(const eig_ctx *ctx, int mode, int32_t C, int64_t nrow, int64_t nblk,
-                         int32_t smax) {
+CodesPlan eig_codes_plan(int num_cu, int mode, int32_t C, int64_t nrow, int64_t nblk, int32_t smax) {
   CodesPlan P;
   P.mode = mode;
   P.C = C;
   P.nblk = nblk;
   cd_groups(C, P.ngroup, P.Cg, P.NT);
-  const int32_t rows = cd_rows(mode, P.NT);
+  // fewer row tiles a wave where the rows fill no more (three run as the most)
+  P.R = (int32_t)std::min<int64_t>(cd_tiles(mode, P.NT), (nrow + 63) / 64);
+  if (P.R > 2) P.R = cd_tiles(mode, P.NT);
+  const int32_t rows = 64 * P.R;
   P.nrowblk = (int32_t)((nrow + rows - 1) / rows);
   P.rowpad = (int64_t)P.nrowblk * rows;
   // splits: rounds of the blocks the chip holds (two per CU) times stages each, plus the
   // sums' way to memory and back, worth about two stages a block
-  const int64_t slots = 2 * (int64_t)std::max(ctx->num_cu, 1);
+  const int64_t slots = 2 * (int64_t)std::max(num_cu, 1);
   double best = 0.0;
   P.nsplit = 1;
   P.per = nblk;
@@ -576,10 +675,9 @@ int eig_codes_restart(eig_ctx *ctx, const CodesPlan &P, void *head, hipStream_t 
   return EIG_OK;
 }
 
-// digit operands of stages b0 .. b0 + P.nblk - 1 and the product of the view's codes with
-// them, into part (added to it with accum)
-int eig_codes_mul(eig_ctx *ctx, const CodesPlan &P, const CodeView &v, const CodeCols &cols, int64_t b0,
-                  void *head, void *dig, void *part, bool accum, hipStream_t st) {
+// digit operands of stages b0 .. b0 + P.nblk - 1 (and the sums of v3 there, added to head's)
+int eig_codes_build(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, int32_t layout, int64_t b0,
+                    void *head, void *dig, hipStream_t st) {
   const ColArgs A = col_args(cols);
   const u64 *mx = (const u64 *)head;
   u64 *sums = (u64 *)head + P.C;
@@ -588,28 +686,55 @@ int eig_codes_mul(eig_ctx *ctx, const CodesPlan &P, const CodeView &v, const Cod
            constexpr int MODE = KIND == kColPanel || KIND == kColAxes ? kCdPair
                                 : KIND == kColLsqG                    ? kCdMiss
                                                                       : kCdSum;
-           hipLaunchKernelGGL((k_cd_build<KIND, MODE>), grid, dim3(256), 0, st, A, v.layout, b0, P.C, P.Cg,
+           hipLaunchKernelGGL((k_cd_build<KIND, MODE>), grid, dim3(256), 0, st, A, layout, b0, P.C, P.Cg,
                               P.NT, mx, (uint8_t *)dig, sums));
-  MulArgs m{v, (const uint8_t *)dig, (int32_t *)part, P.nblk, P.per, P.nrowblk, P.ngroup, P.nsplit,
-            P.rowpad, accum ? 1 : 0};
-  CD_KINDS(cols.kind,
-           constexpr int MODE = KIND == kColPanel || KIND == kColAxes ? kCdPair
-                                : KIND == kColLsqG                    ? kCdMiss
-                                                                      : kCdSum;
-           if (P.NT == 5) launch_mul<KIND, MODE, 5>(m, st); else launch_mul<KIND, MODE, 9>(m, st));
   EIG_HIP(ctx, hipGetLastError());
   return EIG_OK;
+}
+
+// the product of the view's codes with P.nblk stages of digits, into part (added to it
+// with accum)
+hipError_t eig_codes_product(const CodesPlan &P, const CodeView &v, const void *dig, void *part,
+                             bool accum, hipStream_t st) {
+  MulArgs m{v, (const uint8_t *)dig, (int32_t *)part, P.nblk, P.per, P.nrowblk, P.ngroup, P.nsplit,
+            P.rowpad, accum ? 1 : 0};
+  if (P.mode == kCdPair) {
+    if (P.NT == 5) launch_mul<kCdPair, 5>(m, P.R, st); else launch_mul<kCdPair, 9>(m, P.R, st);
+  } else if (P.mode == kCdSum) {
+    if (P.NT == 5) launch_mul<kCdSum, 5>(m, P.R, st); else launch_mul<kCdSum, 9>(m, P.R, st);
+  } else {
+    if (P.NT == 5) launch_mul<kCdMiss, 5>(m, P.R, st); else launch_mul<kCdMiss, 9>(m, P.R, st);
+  }
+  return hipGetLastError();
+}
+
+int eig_codes_mul(eig_ctx *ctx, const CodesPlan &P, const CodeView &v, const CodeCols &cols, int64_t b0,
+                  void *head, void *dig, void *part, bool accum, hipStream_t st) {
+  EIG_TRY(eig_codes_build(ctx, P, cols, v.layout, b0, head, dig, st));
+  EIG_HIP(ctx, eig_codes_product(P, v, dig, part, accum, st));
+  return EIG_OK;
+}
+
+hipError_t eig_codes_sum(const CodesPlan &P, int64_t nrow, const void *head, const void *part, double scale,
+                         double *out, int64_t ldr, int64_t ldc, int32_t Cpad, bool add, hipStream_t st) {
+  const u64 *mx = (const u64 *)head;
+  // a block per row where the splits are many: 16 rows a block add them one after another
+  if (P.nsplit > 8 && nrow <= 4096 && ldc == 1 && Cpad == P.C && scale == 1.0 && !add) {
+    hipLaunchKernelGGL(k_cd_out_small, dim3((unsigned)nrow, (unsigned)P.ngroup), dim3(1024), 0, st,
+                       (const int32_t *)part, P.NT * 16, P.rowpad, P.nsplit, P.Cg, P.C, mx, mx + P.C, out,
+                       ldr);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(k_cd_out_sum, dim3((unsigned)((nrow + kOutRows - 1) / kOutRows), (unsigned)P.ngroup),
+                     dim3(256), 0, st, (const int32_t *)part, P.NT * 16, P.rowpad, P.nsplit, P.Cg, P.C,
+                     Cpad, nrow, mx, mx + P.C, scale, out, ldr, ldc, add ? 1 : 0);
+  return hipGetLastError();
 }
 
 int eig_codes_out_sum(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void *head, const void *part,
                       double scale, double *out, int64_t ldr, int64_t ldc, int32_t Cpad, bool add,
                       hipStream_t st) {
-  const u64 *mx = (const u64 *)head;
-  hipLaunchKernelGGL(k_cd_out_sum, dim3((unsigned)((nrow + kOutRows - 1) / kOutRows), (unsigned)P.ngroup),
-                     dim3(256), 0, st,
-                     (const int32_t *)part, P.NT * 16, P.rowpad, P.nsplit, P.Cg, P.C, Cpad, nrow, mx,
-                     mx + P.C, scale, out, ldr, ldc, add ? 1 : 0);
-  EIG_HIP(ctx, hipGetLastError());
+  EIG_HIP(ctx, eig_codes_sum(P, nrow, head, part, scale, out, ldr, ldc, Cpad, add, st));
   return EIG_OK;
 }
 
@@ -623,4 +748,30 @@ int eig_codes_out_pair(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const voi
                      lev, ignore, scale, out, ldr, ldc);
   EIG_HIP(ctx, hipGetLastError());
   return EIG_OK;
+}
+
+// the product of up to 16 rows (kCodeBytes layout, nword words each) and its results in
+// one go: out[row * ldr + c]; kCdSum and kCdMiss.  part: eig_codes_small_bytes(P).
+constexpr int32_t kSmallSplits = 512;  // waves per group: ten stages each at 600,000 SNPs
+size_t eig_codes_small_bytes(const CodesPlan &P) {
+  return (size_t)P.ngroup * kSmallSplits * 16 * P.NT * 16 * 4;
+}
+hipError_t eig_codes_small(const CodesPlan &P, const CodeRows &rows, int64_t nword, const void *head,
+                           const void *dig, void *part, double *out, int64_t ldr, hipStream_t st) {
+  const u64 *mx = (const u64 *)head;
+  int64_t per = (P.nblk + kSmallSplits - 1) / kSmallSplits;
+  const int32_t ns = (int32_t)((P.nblk + per - 1) / per);
+  const dim3 grid((unsigned)(((int64_t)P.ngroup * ns + 3) / 4));
+  const uint8_t *d = (const uint8_t *)dig;
+  int32_t *p = (int32_t *)part;
+  if (P.mode == kCdSum) {
+    if (P.NT == 5) hipLaunchKernelGGL((k_cd_stream<5, kCdSum>), grid, dim3(256), 0, st, d, p, rows, nword, P.nblk, per, P.ngroup, ns);
+    else hipLaunchKernelGGL((k_cd_stream<9, kCdSum>), grid, dim3(256), 0, st, d, p, rows, nword, P.nblk, per, P.ngroup, ns);
+  } else {
+    if (P.NT == 5) hipLaunchKernelGGL((k_cd_stream<5, kCdMiss>), grid, dim3(256), 0, st, d, p, rows, nword, P.nblk, per, P.ngroup, ns);
+    else hipLaunchKernelGGL((k_cd_stream<9, kCdMiss>), grid, dim3(256), 0, st, d, p, rows, nword, P.nblk, per, P.ngroup, ns);
+  }
+  hipLaunchKernelGGL(k_cd_out_small, dim3((unsigned)rows.n, (unsigned)P.ngroup), dim3(1024), 0, st,
+                     (const int32_t *)part, P.NT * 16, (int64_t)rows.n, ns, P.Cg, P.C, mx, mx + P.C, out, ldr);
+  return hipGetLastError();
 }

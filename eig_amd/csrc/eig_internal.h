@@ -177,16 +177,28 @@ struct CodeCols {
 enum { kCdPair, kCdSum, kCdMiss };
 struct CodesPlan {
   int mode;
-  int32_t C, ngroup, Cg, NT, nrowblk, nsplit;
+  int32_t C, ngroup, Cg, NT, R, nrowblk, nsplit;
   int64_t nblk, per, rowpad;
   size_t head_bytes, dig_bytes, part_bytes;
 };
 // one INT32 sum holds this many terms (digit 128, code 3)
 constexpr int64_t kCodesMaxK = (int64_t)5 << 20;
-CodesPlan eig_codes_plan(const eig_ctx *ctx, int mode, int32_t C, int64_t nrow, int64_t nblk,
-                         int32_t smax);
+CodesPlan eig_codes_plan(int num_cu, int mode, int32_t C, int64_t nrow, int64_t nblk, int32_t smax);
 int eig_codes_scales(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, void *head, hipStream_t st);
 int eig_codes_restart(eig_ctx *ctx, const CodesPlan &P, void *head, hipStream_t st);
+int eig_codes_build(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, int32_t layout, int64_t b0,
+                    void *head, void *dig, hipStream_t st);
+hipError_t eig_codes_product(const CodesPlan &P, const CodeView &v, const void *dig, void *part,
+                             bool accum, hipStream_t st);
+hipError_t eig_codes_sum(const CodesPlan &P, int64_t nrow, const void *head, const void *part, double scale,
+                         double *out, int64_t ldr, int64_t ldc, int32_t Cpad, bool add, hipStream_t st);
+struct CodeRows {
+  const uint8_t *row[16];
+  int32_t n;
+};
+size_t eig_codes_small_bytes(const CodesPlan &P);
+hipError_t eig_codes_small(const CodesPlan &P, const CodeRows &rows, int64_t nword, const void *head,
+                           const void *dig, void *part, double *out, int64_t ldr, hipStream_t st);
 int eig_codes_mul(eig_ctx *ctx, const CodesPlan &P, const CodeView &v, const CodeCols &cols, int64_t b0,
                   void *head, void *dig, void *part, bool accum, hipStream_t st);
 int eig_codes_out_sum(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void *head, const void *part,

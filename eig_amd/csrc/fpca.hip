@@ -1006,12 +1006,12 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   if (!bf) {
     // splits whose sums stay within 2 GiB
     auto smax = [](size_t one) { return (int32_t)std::max<size_t>(1, std::min<size_t>(32, ((size_t)2 << 30) / one)); };
-    pa = eig_codes_plan(ctx, kCdPair, L, M, nst, 1);
-    pa = eig_codes_plan(ctx, kCdPair, L, M, nst, smax(pa.part_bytes));
-    pb = eig_codes_plan(ctx, kCdSum, L, npad, (G64 + 1) / 2, 1);
-    pb = eig_codes_plan(ctx, kCdSum, L, npad, (G64 + 1) / 2, smax(pb.part_bytes / pb.nsplit));
-    pu = eig_codes_plan(ctx, kCdSum, Ctot, npad, (G64 + 1) / 2, 1);
-    pu = eig_codes_plan(ctx, kCdSum, Ctot, npad, (G64 + 1) / 2, smax(pu.part_bytes / pu.nsplit));
+    pa = eig_codes_plan(ctx->num_cu, kCdPair, L, M, nst, 1);
+    pa = eig_codes_plan(ctx->num_cu, kCdPair, L, M, nst, smax(pa.part_bytes));
+    pb = eig_codes_plan(ctx->num_cu, kCdSum, L, npad, (G64 + 1) / 2, 1);
+    pb = eig_codes_plan(ctx->num_cu, kCdSum, L, npad, (G64 + 1) / 2, smax(pb.part_bytes / pb.nsplit));
+    pu = eig_codes_plan(ctx->num_cu, kCdSum, Ctot, npad, (G64 + 1) / 2, 1);
+    pu = eig_codes_plan(ctx->num_cu, kCdSum, Ctot, npad, (G64 + 1) / 2, smax(pu.part_bytes / pu.nsplit));
     size_t cw = 0;
     for (const CodesPlan *q : {&pa, &pb, &pu})
       cw = std::max(cw, q->head_bytes + up(q->dig_bytes) + q->part_bytes);
@@ -1195,7 +1195,7 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   } else {
     // the plan made for every column serves a basis of fewer (r <= Ctot): the missing
     // ones have no digits
-    CodesPlan pr = eig_codes_plan(ctx, kCdSum, r, npad, (G64 + 1) / 2, pu.nsplit);
+    CodesPlan pr = eig_codes_plan(ctx->num_cu, kCdSum, r, npad, (G64 + 1) / 2, pu.nsplit);
     EIG_TRY(code_xtb(pr, src, 1.0, Bm, ldq, r));
   }
   EIG_TRY(gemm_nt_long(ctx, !bf, r, r, npad, Bm, ldq, Bm, ldq, G, r, part, part_doubles, st));

@@ -258,8 +258,8 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
   fc.fancy = (const double *)ctx->fancy.p;
   fc.xmean = d_xm;
   fc.ignore = d_ign;
-  const CodesPlan pl = eig_codes_plan(ctx, kCdPair, K, M, ctx->nst, 16);
-  const CodesPlan pf = eig_codes_plan(ctx, kCdSum, K, vs.nrow, (G64 + 1) / 2, 32);
+  const CodesPlan pl = eig_codes_plan(ctx->num_cu, kCdPair, K, M, ctx->nst, 16);
+  const CodesPlan pf = eig_codes_plan(ctx->num_cu, kCdSum, K, vs.nrow, (G64 + 1) / 2, 32);
   const size_t need = std::max(pl.head_bytes + pl.dig_bytes + pl.part_bytes,
                                pf.head_bytes + pf.dig_bytes + pf.part_bytes);
   EIG_TRY(eig_ensure(ctx, ctx->scratch2, need));
@@ -370,8 +370,8 @@ static int lsq_normal(eig_ctx *ctx, double *acc, char *ws, size_t bytes) {
   CodesPlan pr, pg;
   size_t codes = 0;
   for (;;) {
-    pr = eig_codes_plan(ctx, kCdSum, K + 1, std::min<int64_t>(nr, nind), nb, smax);
-    pg = eig_codes_plan(ctx, kCdMiss, nP, std::min<int64_t>(nr, nind), nb, smax);
+    pr = eig_codes_plan(ctx->num_cu, kCdSum, K + 1, std::min<int64_t>(nr, nind), nb, smax);
+    pg = eig_codes_plan(ctx->num_cu, kCdMiss, nP, std::min<int64_t>(nr, nind), nb, smax);
     codes = shared ? 0 : up((size_t)nr * nb * 32);
     const size_t need = pr.head_bytes + pg.head_bytes + up(pr.dig_bytes) + up(pg.dig_bytes) +
                         up(pr.part_bytes) + up(pg.part_bytes) + codes;

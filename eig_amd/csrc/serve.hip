@@ -1,22 +1,21 @@
 // lsqproject serving: a request loop over a device-resident reference panel.
 //
-// The panel (per SNP: the K projection rows e_m = fxscal .* ffvecs[:,m], the
-// fancy scale, -1 for an ignored SNP, and xmean = mean*fancy) is built once on
-// the device from a context whose loadings are current.  Requests of 1..max_batch
-// query samples arrive as sample-major packed rows (SNP m of a sample at byte m/4,
-// bits 7-6, 5-4, 3-2, 1-0 for m%4 = 0..3, code 3 = missing).  A worker thread
-// admits pending requests into free lanes: each lane is a stream with its own
-// descriptor, row, partial-sum and output memory and a captured graph of three
-// persistent kernels.  Requests that arrive while other lanes are on the device
-// are batched into the next free lane, so their work overlaps.
+// The panel is the digit operands (codes.hip) of the projection rows e_m = fxscal .*
+// ffvecs[:,m] times the fancy scale and xmean = mean*fancy, for the right-hand sides, and
+// of the products e_m e_m^T, for the normal matrices, built once on the device from a
+// context whose loadings are current.  Requests of 1..max_batch query samples arrive as
+// sample-major packed rows (SNP m of a sample at byte m/4, bits 7-6, 5-4, 3-2, 1-0 for
+// m%4 = 0..3, code 3 = missing).  A worker thread admits pending requests into free lanes:
+// each lane is a stream with its own descriptor, row, partial-sum and output memory.
+// Requests that arrive while other lanes are on the device are batched into the next free
+// lane, so their work overlaps.
 //
 // Per sample the arithmetic is lsqproj + regressit + solvit (smartpca.c:4606-4757,
 // regsubs.c:8-74, linsubs.c:296-393): over the sample's observed, kept SNPs the
 // Gram co = sum e_m e_m^T and rhs rr = sum e_m x_m with x = g*fancy - xmean
-// (fixxrow, qpsubs.c:338-349), then Cholesky (choldc/cholsl order).  The SNP
-// range is cut into fixed chunks of `chunk` SNPs, each summed in SNP order, and
-// the chunk sums are added in chunk order: a sample's result depends on its own
-// row and the server's chunk only, never on the other samples of its batch.
+// (fixxrow, qpsubs.c:338-349), then Cholesky (choldc/cholsl order).  The sums are exact
+// integers on the panel's grid, whatever kernel and splits a batch takes, so a sample's
+// result depends on its own row only, never on the other samples of its batch.
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -36,158 +35,26 @@ constexpr int kSrvMaxBatch = 1024;  // samples per lane (descriptor capacity)
 constexpr int kSrvMaxLanes = 8;
 
 struct SrvDesc {
-  int32_t n;
-  int32_t pad_[3];
   const uint8_t *rows[kSrvMaxBatch];
 };
 
-constexpr int panel_stride(int K) { return (K + 3) & ~1; }  // K + 2 rounded up to even
-
 // ------------------------------------------------------------------ kernels
-__global__ void k_srv_panel(const double *__restrict__ ff, const double *__restrict__ fxscal,
-                            const double *__restrict__ fancy, const double *__restrict__ xmean,
-                            const uint8_t *__restrict__ ignore, int64_t M, int32_t K, int32_t S,
-                            double *__restrict__ panel) {
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M) return;
-  double *p = panel + m * S;
-  for (int j = 0; j < K; ++j) p[j] = fxscal[j] * ff[(int64_t)j * M + m];
-  p[K] = ignore[m] ? -1.0 : fancy[m];
-  p[K + 1] = xmean[m];
-  for (int j = K + 2; j < S; ++j) p[j] = 0.0;
-}
-
-// Random query rows for the launch-shape tuner (any byte is a valid row).
-__global__ void k_srv_fill(uint8_t *__restrict__ rows, int64_t bytes, uint64_t seed) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= bytes) return;
-  uint64_t x = seed + (uint64_t)i * 0x9E3779B97F4A7C15ull;
-  x ^= x >> 31;
-  x *= 0xBF58476D1CE4E5B9ull;
-  x ^= x >> 29;
-  rows[i] = (uint8_t)(x >> 24);
-}
-
-// Per (64-sample block, SNP chunk) work item: the Gram upper triangle, the rhs
-// and the observed count of each sample over the chunk.  Persistent: a fixed
-// grid strides over the n-dependent item count read from the descriptor.
-// partial layout: [(c * W + p) * nmax + q].
-template <int K, bool kGuard>
-__device__ __forceinline__ void srv_group(uint4 w, const double *__restrict__ pm, int64_t mg,
-                                          int64_t m1, double *G, double *r, double &kk) {
-  // built without contraction: x = g*fancy - xmean rounds as the reference's two
-  // operations; the Gram and rhs accumulations are explicit fused multiply-adds
-  constexpr int S = panel_stride(K);
-#pragma unroll 1
-  for (int wi = 0; wi < 4; ++wi) {
-    const uint32_t wv = wi == 0 ? w.x : (wi == 1 ? w.y : (wi == 2 ? w.z : w.w));
-#pragma unroll 2
-    for (int t = 0; t < 16; ++t) {
-      const int s = 16 * wi + t;
-      if (kGuard && mg + s >= m1) break;
-      const uint32_t code = (wv >> (8 * (t >> 2) + 2 * (3 - (t & 3)))) & 3u;
-      const double *pe = pm + (int64_t)s * S;
-      const double fz = pe[K], xm = pe[K + 1];
-      const bool obs = code != 3u && fz >= 0.0;
-      const double wobs = obs ? 1.0 : 0.0;
-      const double y = (double)code * fz;
-      const double xv = obs ? y - xm : 0.0;
-      // e * 1 = e and e * 0 = +-0 exactly: the masked row adds nothing to G
-      double e[K], ew[K];
-#pragma unroll
-      for (int a = 0; a < K; ++a) {
-        e[a] = pe[a];
-        ew[a] = e[a] * wobs;
-      }
-#pragma unroll
-      for (int a = 0; a < K; ++a) r[a] = fma(ew[a], xv, r[a]);
-#pragma unroll
-      for (int a = 0; a < K; ++a)
-#pragma unroll
-        for (int c = a; c < K; ++c) {
-          double &g = G[a * K - a * (a - 1) / 2 + (c - a)];
-          g = fma(ew[a], e[c], g);
-        }
-      kk += wobs;
-    }
-  }
-}
-
-template <int K>
-__global__ __launch_bounds__(64) void k_srv_gram(const SrvDesc *__restrict__ desc,
-                                                 const double *__restrict__ panel, int64_t M,
-                                                 int32_t chunk, int32_t nchunk, int32_t nmax,
-                                                 double *__restrict__ partial) {
-  constexpr int S = panel_stride(K);
-  constexpr int nP = K * (K + 1) / 2, W = nP + K + 1;
-  const int32_t n = desc->n;
-  const int32_t nsb = (n + 63) >> 6;
-  const int64_t items = (int64_t)nsb * nchunk;
-  const int lane = threadIdx.x;
-  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
-    const int32_t sb = (int32_t)(it % nsb), c = (int32_t)(it / nsb);
-    const int32_t q = sb * 64 + lane;
-    const bool act = q < n;
-    const uint8_t *row = desc->rows[act ? q : 0];
-    double G[nP], r[K], kk = 0.0;
-#pragma unroll
-    for (int p = 0; p < nP; ++p) G[p] = 0.0;
-#pragma unroll
-    for (int a = 0; a < K; ++a) r[a] = 0.0;
-    const int64_t m0 = (int64_t)c * chunk, m1 = min(M, m0 + chunk);
-    for (int64_t mg = m0; mg < m1; mg += 64) {
-      uint4 w = make_uint4(~0u, ~0u, ~0u, ~0u);  // inactive lanes read as all missing
-      if (act) w = *(const uint4 *)(row + (mg >> 2));
-      const double *pm = panel + mg * S;
-      if (mg + 64 <= m1)
-        srv_group<K, false>(w, pm, mg, m1, G, r, kk);
-      else
-        srv_group<K, true>(w, pm, mg, m1, G, r, kk);
-    }
-    if (act) {
-      double *out = partial + (int64_t)c * W * nmax + q;
-#pragma unroll
-      for (int p = 0; p < nP; ++p) out[(int64_t)p * nmax] = G[p];
-#pragma unroll
-      for (int a = 0; a < K; ++a) out[(int64_t)(nP + a) * nmax] = r[a];
-      out[(int64_t)(nP + K) * nmax] = kk;
-    }
-  }
-}
-
-// sums[p * nmax + q] = sum over chunks in chunk order; one thread per (p, q).
-__global__ __launch_bounds__(256) void k_srv_reduce(const SrvDesc *__restrict__ desc,
-                                                    const double *__restrict__ partial,
-                                                    int32_t nchunk, int32_t W, int32_t nmax,
-                                                    double *__restrict__ sums) {
-  const int32_t n = desc->n;
-  const int64_t total = (int64_t)W * n;
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t p = (int32_t)(idx / n), q = (int32_t)(idx % n);
-    const double *src = partial + (int64_t)p * nmax + q;
-    double s = 0.0;
-    for (int32_t c = 0; c < nchunk; ++c) s += src[(int64_t)c * W * nmax];
-    sums[(int64_t)p * nmax + q] = s;
-  }
-}
-
 // Cholesky solve per sample (choldc + cholsl order) on the packed triangle.
 // out[q * (K + 2) + j]: coefficients, then status (0 solved, 1 <= K observed,
 // 2 Cholesky failed or NaN), then the observed-SNP count.
 template <int K>
-__global__ __launch_bounds__(64) void k_srv_solve(const SrvDesc *__restrict__ desc,
-                                                  const double *__restrict__ sums, int32_t nmax,
+// sums: per sample the triangle, the right-hand side and the observed count.  out is host
+// memory: the few results leave with the kernel, without a copy of their own behind it.
+__global__ __launch_bounds__(64) void k_srv_solve(int32_t n, const double *__restrict__ sums,
                                                   double *__restrict__ out) {
-  constexpr int nP = K * (K + 1) / 2;
-  const int32_t n = desc->n;
+  constexpr int nP = K * (K + 1) / 2, W = nP + K + 1;
   for (int32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
     double A[nP], b[K], p[K], x[K];
 #pragma unroll
-    for (int i = 0; i < nP; ++i) A[i] = sums[(int64_t)i * nmax + q];
+    for (int i = 0; i < nP; ++i) A[i] = sums[(int64_t)q * W + i];
 #pragma unroll
-    for (int i = 0; i < K; ++i) b[i] = sums[(int64_t)(nP + i) * nmax + q];
-    const double kk = sums[(int64_t)(nP + K) * nmax + q];
+    for (int i = 0; i < K; ++i) b[i] = sums[(int64_t)q * W + nP + i];
+    const double kk = sums[(int64_t)q * W + nP + K];
     double *o = out + (int64_t)q * (K + 2);
     o[K + 1] = kk;
     if (kk <= (double)K) {
@@ -258,10 +125,10 @@ struct SrvReq {
 struct SrvLane {
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
-  hipGraphExec_t gexec = nullptr;
   SrvDesc *desc_h = nullptr, *desc_d = nullptr;
   uint8_t *rows_d = nullptr;
-  double *partial_d = nullptr, *sums_d = nullptr, *out_d = nullptr, *out_h = nullptr;
+  char *partial_d = nullptr;
+  double *sums_d = nullptr, *out_h = nullptr;
   std::vector<std::shared_ptr<SrvReq>> reqs;
   std::vector<int32_t> offs;
   bool busy = false;
@@ -269,13 +136,17 @@ struct SrvLane {
 
 struct eig_server {
   int device = 0;
-  int32_t K = 0, S = 0, nP = 0, W = 0;
+  int32_t K = 0, nP = 0, W = 0;
   int64_t M = 0, rowbytes = 0, rowpad = 0;
   int32_t nlanes = 0, max_batch = 0;
-  int32_t chunk = 0, nchunk = 0, grid_gram = 0, grid_red = 0, grid_solve = 0;
+  int32_t chunk = 0, smax = 1;
   int num_cu = 0;
   double eigscale[kSrvMaxK];
-  double *panel_d = nullptr;
+  // the panel: scales and digit operands of the right-hand sides and of the normal matrices
+  CodesPlan pr, pg;
+  char *panel_d = nullptr;
+  void *head_r = nullptr, *head_g = nullptr, *dig_r = nullptr, *dig_g = nullptr;
+  size_t part_bytes = 0;  // of a lane
   SrvLane lane[kSrvMaxLanes];
 
   std::mutex mu;
@@ -307,6 +178,16 @@ static int srv_err(eig_server *s, int code, const char *fmt, ...) {
                      hipGetErrorString(e_));                                                  \
   } while (0)
 
+// a batch's plan: splits of at least `chunk` SNPs, as many as help and 32 MiB of sums hold
+static CodesPlan srv_plan(const eig_server *s, int mode, int32_t n) {
+  const int32_t C = mode == kCdSum ? s->K + 1 : s->nP;
+  const int64_t nblk = (s->M + 127) / 128;
+  const CodesPlan one = eig_codes_plan(s->num_cu, mode, C, n, nblk, 1);
+  const size_t per = one.part_bytes / one.nsplit;
+  return eig_codes_plan(s->num_cu, mode, C, n, nblk,
+                        (int32_t)std::min<int64_t>(s->smax, std::max<int64_t>(1, ((int64_t)32 << 20) / (int64_t)per)));
+}
+
 #define SRV_KCASE(n, ...) \
   case n: {               \
     constexpr int KC = n; \
@@ -324,92 +205,37 @@ static int srv_err(eig_server *s, int code, const char *fmt, ...) {
       return srv_err(s, EIG_E_ARG, "K out of range");                                       \
   }
 
-// The three kernels of one batch on `st`, reading the batch from desc_d.
-static int srv_launch(eig_server *s, hipStream_t st, const SrvDesc *desc_d, double *partial_d,
-                      double *sums_d, double *out_d, int32_t chunk, int32_t nchunk,
-                      int32_t grid_gram) {
-  const int32_t nmax = s->max_batch;
-  SRV_KSWITCH(s, s->K,
-              hipLaunchKernelGGL((k_srv_gram<KC>), dim3(grid_gram), dim3(64), 0, st, desc_d,
-                                 (const double *)s->panel_d, s->M, chunk, nchunk, nmax,
-                                 partial_d));
-  hipLaunchKernelGGL(k_srv_reduce, dim3(s->grid_red), dim3(256), 0, st, desc_d,
-                     (const double *)partial_d, nchunk, s->W, nmax, sums_d);
-  SRV_KSWITCH(s, s->K,
-              hipLaunchKernelGGL((k_srv_solve<KC>), dim3(s->grid_solve), dim3(64), 0, st, desc_d,
-                                 (const double *)sums_d, nmax, out_d));
-  SRV_HIP(s, hipGetLastError());
-  return EIG_OK;
-}
-
-// Launch-shape tuner: times (chunk, persistent grid) candidates on random rows at
-// a small and a large batch and keeps the fastest weighted sum.  The chunk it
-// picks stays fixed for the server's lifetime (results depend on it).
-static int srv_autotune(eig_server *s, int32_t chunk_req) {
-  static const int32_t kChunks[] = {1024, 2048, 4096, 8192};
-  static const int32_t kGridMul[] = {2, 4, 8};
-  SrvLane &L = s->lane[0];
+// A batch's normal equations and solutions on its lane's stream.  Up to 16 samples fill one
+// row tile: the digits, 355 MB at 600,000 SNPs and K = 10, stream through once
+// (k_cd_stream: 76 us, and 0.11 ms from submit to result, where FP64 sums of a lane per
+// sample took 0.82).  More share each digit operand through LDS (k_cd_mul: 112 samples in
+// 0.19 ms, 586 in 0.49).
+static int srv_launch(eig_server *s, SrvLane &L, int32_t n) {
   hipStream_t st = L.stream;
-  const int32_t ntest[2] = {32, std::min(512, s->max_batch)};
-  const double weight[2] = {1.0, 0.25};
-  uint8_t *rows = L.rows_d;
-  hipLaunchKernelGGL(k_srv_fill, dim3((unsigned)((ntest[1] * s->rowpad + 255) / 256)), dim3(256),
-                     0, st, rows, (int64_t)ntest[1] * s->rowpad, (uint64_t)0xE16);
-  hipEvent_t e0, e1;
-  SRV_HIP(s, hipEventCreate(&e0));
-  SRV_HIP(s, hipEventCreate(&e1));
-  double best = 1e30;
-  int32_t best_c = chunk_req > 0 ? chunk_req : 2048, best_g = 4 * s->num_cu;
-  for (int32_t ch : kChunks) {
-    if (chunk_req > 0 && ch != chunk_req) continue;
-    const int32_t nch = (int32_t)((s->M + ch - 1) / ch);
-    if ((int64_t)nch > s->nchunk) continue;  // partial memory sized for the smallest chunk
-    for (int32_t gm : kGridMul) {
-      const int32_t g = gm * s->num_cu;
-      double score = 0.0;
-      for (int t = 0; t < 2; ++t) {
-        L.desc_h->n = ntest[t];
-        for (int32_t q = 0; q < ntest[t]; ++q) L.desc_h->rows[q] = rows + (int64_t)q * s->rowpad;
-        SRV_HIP(s, hipMemcpyAsync(L.desc_d, L.desc_h, sizeof(SrvDesc), hipMemcpyHostToDevice, st));
-        double tmin = 1e30;
-        for (int rep = 0; rep < 3; ++rep) {
-          SRV_HIP(s, hipEventRecord(e0, st));
-          int rc = srv_launch(s, st, L.desc_d, L.partial_d, L.sums_d, L.out_d, ch, nch, g);
-          if (rc != EIG_OK) return rc;
-          SRV_HIP(s, hipEventRecord(e1, st));
-          SRV_HIP(s, hipEventSynchronize(e1));
-          float ms = 0.f;
-          SRV_HIP(s, hipEventElapsedTime(&ms, e0, e1));
-          if (rep > 0) tmin = std::min(tmin, (double)ms);
-        }
-        score += weight[t] * tmin;
-      }
-      if (score < best) {
-        best = score;
-        best_c = ch;
-        best_g = g;
-      }
-    }
+  const int64_t nword = s->rowpad / 4;
+  if (n <= 16) {
+    CodeRows rows;
+    rows.n = n;
+    for (int32_t i = 0; i < 16; ++i) rows.row[i] = L.desc_h->rows[i < n ? i : 0];
+    char *sg = L.partial_d + eig_codes_small_bytes(s->pr);
+    SRV_HIP(s, eig_codes_small(s->pg, rows, nword, s->head_g, s->dig_g, sg, L.sums_d, s->W, st));
+    SRV_HIP(s, eig_codes_small(s->pr, rows, nword, s->head_r, s->dig_r, L.partial_d, L.sums_d + s->nP,
+                               s->W, st));
+  } else {
+    SRV_HIP(s, hipMemcpyAsync(L.desc_d, L.desc_h, sizeof(void *) * (size_t)n, hipMemcpyHostToDevice, st));
+    const CodeView v{nullptr, L.desc_d->rows, 0, 0, 32, 16, n, nword, kCodeBytes};
+    const CodesPlan pr = srv_plan(s, kCdSum, n), pg = srv_plan(s, kCdMiss, n);
+    char *sg = L.partial_d + (pr.part_bytes + 255) / 256 * 256;
+    SRV_HIP(s, eig_codes_product(pg, v, s->dig_g, sg, false, st));
+    SRV_HIP(s, eig_codes_product(pr, v, s->dig_r, L.partial_d, false, st));
+    SRV_HIP(s, eig_codes_sum(pg, n, s->head_g, sg, 1.0, L.sums_d, s->W, 1, s->nP, false, st));
+    SRV_HIP(s, eig_codes_sum(pr, n, s->head_r, L.partial_d, 1.0, L.sums_d + s->nP, s->W, 1, s->K + 1,
+                             false, st));
   }
-  hipEventDestroy(e0);
-  hipEventDestroy(e1);
-  s->chunk = best_c;
-  s->nchunk = (int32_t)((s->M + best_c - 1) / best_c);
-  s->grid_gram = best_g;
-  return EIG_OK;
-}
-
-static int srv_capture(eig_server *s, SrvLane &L) {
-  hipGraph_t graph = nullptr;
-  SRV_HIP(s, hipStreamBeginCapture(L.stream, hipStreamCaptureModeThreadLocal));
-  int rc = srv_launch(s, L.stream, L.desc_d, L.partial_d, L.sums_d, L.out_d, s->chunk, s->nchunk,
-                      s->grid_gram);
-  hipError_t e = hipStreamEndCapture(L.stream, &graph);
-  if (rc != EIG_OK) return rc;
-  if (e != hipSuccess) return srv_err(s, EIG_E_HIP, "capture: %s", hipGetErrorString(e));
-  e = hipGraphInstantiate(&L.gexec, graph, nullptr, nullptr, 0);
-  hipGraphDestroy(graph);
-  if (e != hipSuccess) return srv_err(s, EIG_E_HIP, "graph: %s", hipGetErrorString(e));
+  SRV_KSWITCH(s, s->K,
+              hipLaunchKernelGGL((k_srv_solve<KC>), dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, n,
+                                 (const double *)L.sums_d, L.out_h));
+  SRV_HIP(s, hipGetLastError());
   return EIG_OK;
 }
 
@@ -430,12 +256,8 @@ static int srv_dispatch(eig_server *s, SrvLane &L) {
     }
     off += r->nq;
   }
-  L.desc_h->n = off;
-  SRV_HIP(s, hipMemcpyAsync(L.desc_d, L.desc_h, 16 + sizeof(void *) * (size_t)off,
-                            hipMemcpyHostToDevice, st));
-  SRV_HIP(s, hipGraphLaunch(L.gexec, st));
-  SRV_HIP(s, hipMemcpyAsync(L.out_h, L.out_d, sizeof(double) * (size_t)off * (s->K + 2),
-                            hipMemcpyDeviceToHost, st));
+  int rc = srv_launch(s, L, off);
+  if (rc != EIG_OK) return rc;
   SRV_HIP(s, hipEventRecord(L.done, st));
   return EIG_OK;
 }
@@ -511,9 +333,13 @@ static void srv_worker(eig_server *s) {
     for (int l = 0; l < s->nlanes; ++l) any_busy |= s->lane[l].busy;
     if (s->stopping && !any_busy && s->pending.empty()) break;
     if (progressed) continue;
-    if (any_busy)
-      s->cv_work.wait_for(lk, std::chrono::microseconds(20));
-    else
+    if (any_busy) {
+      // a batch takes 0.1 to a few tenths of a millisecond; a timed wait of 20 us returns
+      // after 70 to 80
+      lk.unlock();
+      std::this_thread::yield();
+      lk.lock();
+    } else
       s->cv_work.wait(lk, [s] { return s->stopping || !s->pending.empty(); });
   }
 }
@@ -521,7 +347,6 @@ static void srv_worker(eig_server *s) {
 static void srv_free(eig_server *s) {
   for (int l = 0; l < kSrvMaxLanes; ++l) {
     SrvLane &L = s->lane[l];
-    if (L.gexec) hipGraphExecDestroy(L.gexec);
     if (L.done) hipEventDestroy(L.done);
     if (L.stream) hipStreamDestroy(L.stream);
     if (L.desc_h) hipHostFree(L.desc_h);
@@ -530,13 +355,12 @@ static void srv_free(eig_server *s) {
     if (L.rows_d) hipFree(L.rows_d);
     if (L.partial_d) hipFree(L.partial_d);
     if (L.sums_d) hipFree(L.sums_d);
-    if (L.out_d) hipFree(L.out_d);
   }
   if (s->panel_d) hipFree(s->panel_d);
   delete s;
 }
 
-static int srv_alloc_lane(eig_server *s, SrvLane &L, size_t partial_bytes) {
+static int srv_alloc_lane(eig_server *s, SrvLane &L) {
   SRV_HIP(s, hipStreamCreateWithFlags(&L.stream, hipStreamNonBlocking));
   SRV_HIP(s, hipEventCreateWithFlags(&L.done, hipEventDisableTiming));
   SRV_HIP(s, hipHostMalloc((void **)&L.desc_h, sizeof(SrvDesc), hipHostMallocDefault));
@@ -544,9 +368,8 @@ static int srv_alloc_lane(eig_server *s, SrvLane &L, size_t partial_bytes) {
                            hipHostMallocDefault));
   SRV_HIP(s, hipMalloc((void **)&L.desc_d, sizeof(SrvDesc)));
   SRV_HIP(s, hipMalloc((void **)&L.rows_d, (size_t)s->max_batch * s->rowpad));
-  SRV_HIP(s, hipMalloc((void **)&L.partial_d, partial_bytes));
+  SRV_HIP(s, hipMalloc((void **)&L.partial_d, s->part_bytes));
   SRV_HIP(s, hipMalloc((void **)&L.sums_d, sizeof(double) * s->W * s->max_batch));
-  SRV_HIP(s, hipMalloc((void **)&L.out_d, sizeof(double) * s->max_batch * (s->K + 2)));
   std::memset(L.desc_h, 0, sizeof(SrvDesc));
   return EIG_OK;
 }
@@ -570,7 +393,6 @@ extern "C" int eig_server_start(eig_ctx *ctx, const double *eigscale, int32_t nl
   s->device = ctx->device;
   s->num_cu = ctx->num_cu;
   s->K = ctx->last_K;
-  s->S = panel_stride(s->K);
   s->nP = s->K * (s->K + 1) / 2;
   s->W = s->nP + s->K + 1;
   s->M = ctx->nsnp;
@@ -578,39 +400,69 @@ extern "C" int eig_server_start(eig_ctx *ctx, const double *eigscale, int32_t nl
   s->rowpad = ((s->M + 63) / 64) * 16;
   s->nlanes = nlanes;
   s->max_batch = max_batch;
-  s->grid_red = 4 * s->num_cu;
-  s->grid_solve = (max_batch + 63) / 64;
   for (int j = 0; j < kSrvMaxK; ++j) s->eigscale[j] = (eigscale && j < s->K) ? eigscale[j] : 1.0;
-  // partial sums sized for the smallest chunk the tuner may pick
-  const int32_t min_chunk = chunk > 0 ? chunk : 1024;
-  s->nchunk = (int32_t)((s->M + min_chunk - 1) / min_chunk);
+  // splits of a batch: at least `chunk` SNPs each; 4,096 when the caller leaves it (at
+  // 600,000 SNPs, K = 10, 112 samples alone and a burst of 963 in 24 requests take 0.17 and
+  // 0.85 ms with 1,024, 0.19 and 0.74 with 4,096, 0.45 and 0.85 with 16,384)
+  s->chunk = chunk > 0 ? chunk : 4096;
+  s->smax = (int32_t)std::min<int64_t>(512, std::max<int64_t>(1, s->M / std::max(s->chunk, 128)));
   auto fail = [&](int rc) {
     ctx->err = s->err;
     srv_free(s);
     return rc;
   };
-  if (hipMalloc((void **)&s->panel_d, sizeof(double) * s->S * s->M) != hipSuccess)
-    return fail(srv_err(s, EIG_E_NOMEM, "panel allocation"));
   {
     const double *fx = (const double *)ctx->fxscal.p;
-    hipLaunchKernelGGL(k_srv_panel, dim3((unsigned)((s->M + 255) / 256)), dim3(256), 0, ctx->stream,
-                       (const double *)ctx->ffvecs.p, fx, (const double *)ctx->fancy.p, fx + kMaxK,
-                       (const uint8_t *)ctx->ignore_dev.p, s->M, s->K, s->S, s->panel_d);
+    CodeCols cr{kColLsqR, (const double *)ctx->ffvecs.p, s->M, s->M};
+    cr.fancy = (const double *)ctx->fancy.p;
+    cr.xmean = fx + kMaxK;
+    cr.ignore = (const uint8_t *)ctx->ignore_dev.p;
+    cr.fxscal = fx;
+    cr.K = s->K;
+    CodeCols cg = cr;
+    cg.kind = kColLsqG;
+    s->pr = srv_plan(s, kCdSum, 16);
+    s->pg = srv_plan(s, kCdMiss, 16);
+    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    if (hipMalloc((void **)&s->panel_d, s->pr.head_bytes + s->pg.head_bytes + up(s->pr.dig_bytes) +
+                                            s->pg.dig_bytes) != hipSuccess)
+      return fail(srv_err(s, EIG_E_NOMEM, "panel allocation"));
+    s->head_r = s->panel_d;
+    s->head_g = s->panel_d + s->pr.head_bytes;
+    s->dig_r = (char *)s->head_g + s->pg.head_bytes;
+    s->dig_g = (char *)s->dig_r + up(s->pr.dig_bytes);
+    for (int g = 0; g < 2; ++g) {
+      const CodesPlan &P = g ? s->pg : s->pr;
+      const CodeCols &c = g ? cg : cr;
+      void *head = g ? s->head_g : s->head_r, *dig = g ? s->dig_g : s->dig_r;
+      int rc = eig_codes_scales(ctx, P, c, head, ctx->stream);
+      if (rc == EIG_OK) rc = eig_codes_build(ctx, P, c, kCodeBytes, 0, head, dig, ctx->stream);
+      if (rc != EIG_OK) return fail(srv_err(s, rc, "panel build failed"));
+    }
     if (hipStreamSynchronize(ctx->stream) != hipSuccess)
       return fail(srv_err(s, EIG_E_HIP, "panel build failed"));
-  }
-  // lane 0 first with the largest partial buffer (tuner), the rest after tuning
-  int rc = srv_alloc_lane(s, s->lane[0], sizeof(double) * s->nchunk * s->W * (size_t)max_batch);
-  if (rc != EIG_OK) return fail(rc);
-  rc = srv_autotune(s, chunk);
-  if (rc != EIG_OK) return fail(rc);
-  for (int l = 1; l < nlanes; ++l) {
-    rc = srv_alloc_lane(s, s->lane[l], sizeof(double) * s->nchunk * s->W * (size_t)max_batch);
-    if (rc != EIG_OK) return fail(rc);
+    // a lane's partial sums: the small product's, or any batch's
+    s->part_bytes = eig_codes_small_bytes(s->pr) + eig_codes_small_bytes(s->pg);
+    for (int32_t n = 17; n <= max_batch; ++n)
+      s->part_bytes = std::max(s->part_bytes, up(srv_plan(s, kCdSum, n).part_bytes) +
+                                                  up(srv_plan(s, kCdMiss, n).part_bytes));
   }
   for (int l = 0; l < nlanes; ++l) {
-    rc = srv_capture(s, s->lane[l]);
+    SrvLane &L = s->lane[l];
+    int rc = srv_alloc_lane(s, L);
     if (rc != EIG_OK) return fail(rc);
+    // a batch of each kind on the lane, so that the first request does not pay for the
+    // stream's queue and the first touch of its memory (any byte is a valid row)
+    const int32_t nw = std::min(32, max_batch);
+    if (hipMemsetAsync(L.rows_d, 0, (size_t)nw * s->rowpad, L.stream) != hipSuccess)
+      return fail(srv_err(s, EIG_E_HIP, "lane start"));
+    for (int32_t i = 0; i < nw; ++i) L.desc_h->rows[i] = L.rows_d + (int64_t)i * s->rowpad;
+    for (int32_t n : {1, nw}) {
+      rc = srv_launch(s, L, n);
+      if (rc != EIG_OK) return fail(rc);
+    }
+    if (hipEventRecord(L.done, L.stream) != hipSuccess || hipStreamSynchronize(L.stream) != hipSuccess)
+      return fail(srv_err(s, EIG_E_HIP, "lane start"));
   }
   s->worker = std::thread(srv_worker, s);
   *out = s;
@@ -677,7 +529,7 @@ extern "C" int eig_server_info(eig_server *s, int32_t *K, int64_t *nsnp, int64_t
   if (nsnp) *nsnp = s->M;
   if (rowpad) *rowpad = s->rowpad;
   if (chunk) *chunk = s->chunk;
-  if (grid) *grid = s->grid_gram;
+  if (grid) *grid = 2 * s->num_cu;
   if (batches) *batches = s->nbatches;
   if (samples) *samples = s->nsamples;
   return EIG_OK;
