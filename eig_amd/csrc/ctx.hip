@@ -99,7 +99,7 @@ extern "C" void eig_close(eig_ctx *ctx) {
                     &ctx->evecs_dev, &ctx->ffvecs, &ctx->fxscal,   &ctx->projw,    &ctx->proj_out,
                     &ctx->use_dev, &ctx->ignore_dev, &ctx->scratch, &ctx->scratch2,
                     &ctx->selg,   &ctx->selb,   &ctx->fill,     &ctx->evall,
-                    &ctx->xdplanes, &ctx->xdtab, &ctx->xdpart, &ctx->xdmisc};
+                    &ctx->tribuf, &ctx->xdplanes, &ctx->xdtab, &ctx->xdpart, &ctx->xdmisc};
   for (DevBuf *b : bufs) free_buf(*b);
   if (ctx->hostpin.p) hipHostFree(ctx->hostpin.p);
   hipEventDestroy(ctx->ev0);

@@ -70,6 +70,7 @@ struct eig_ctx {
 
   // eigensolver
   DevBuf ework;
+  DevBuf tribuf;     // the tridiagonalisation's exchange words
   DevBuf evecs_dev;  // nvec x nrows of the last eig_eigh_xtx
   DevBuf evall;      // all-vector eigensolves: every batch's tridiagonal-basis vectors
   int32_t last_nvec = 0;

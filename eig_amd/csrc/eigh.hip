@@ -12,10 +12,9 @@
 //              known up front from w.v = tau (y.v - 2 p.q); in the same pass the
 //              next row x = A[c+1] - (V W^T + W V^T)[c+1] and per-block partials
 //              of its norm and of the next column's panel dots V^T x, W^T x.
-//     Trailing orders of 1,000 and more run the parts as two kernels (k_symv,
-//     k_wcol); shorter ones run them in one launch, k_column, whose w-column
-//     blocks load what they can up front and wait on a ticket counter for the
-//     symv blocks.
+//     Both are launches of their own (k_symv, k_wcol).  Once the trailing matrix fits the
+//     register files (order 2,048) one resident launch per range of orders runs all its
+//     columns (k_tri).
 //     Cross-block sums are per-block partials reduced in a fixed order (same
 //     bits in every block, independent of scheduling).  After each panel
 //     k_syr2k applies A -= V W^T + W V^T to the trailing matrix.  The reflector of
@@ -32,7 +31,9 @@
 //     per vector sums them in block order into Z_p = T_p V_p^T X.
 //  Wave-level sums exchange lanes by DPP and permlane swaps (xlane), not through LDS.
 #include <cmath>
+#include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "eig_internal.h"
@@ -56,7 +57,7 @@ struct EigWs {
   double *part1;          // per-block partial dots of the back-transform
   double *pw;             // [2][maxw][kPW] column hand-off partials (by column parity)
   double *ps;             // [maxblk] per-block y.v of the symv part
-  int32_t *sync;          // [0] hand-off ticket counter, [1] hand-off timeout flag
+  int32_t *sync;          // [1] set if a resident launch gave up waiting
   int32_t maxw;
   double *eval;           // ascending
   double *X;              // nvec x n eigenvectors
@@ -216,24 +217,14 @@ __global__ __launch_bounds__(256) void k_col0(EigWs ws, int32_t n) {
     ws.d[0] = ws.a[0];
     ws.pw[0] = s;
     ws.pw[1] = n > 1 ? ws.a[1] : 0.0;
-    ws.sync[0] = 0;
-    ws.sync[1] = 0;
   }
 }
 
-// a store that is coherent device-wide once the wave's vmcnt has drained (it
-// writes through the XCD's L2), for the values the wcol part of the same launch
-// reads (y and the y.v partials)
-__device__ inline void store_dev(double *p, double v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // ---------------------------------------------------------------- symv part
-constexpr int kSymvRows = 8;      // symv rows per block in k_column
-constexpr int kSymvRowsLong = 4;  // in k_symv (long columns): 106 VGPRs, 4 waves/SIMD;
-                                  // 2 ms less than 8 rows at n = 5,000 (measured)
-template <int R>
+constexpr int kSymvRows = 4;  // symv rows per block: 106 VGPRs, 4 waves/SIMD; 2 ms less
+                              // than 8 rows at n = 5,000
 __device__ inline void symv_part(const EigWs &ws, int32_t n, int32_t c, int32_t j, int32_t blk) {
+  constexpr int R = kSymvRows;
   __shared__ double red[4][R];
   __shared__ double sscale;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -324,12 +315,15 @@ __device__ inline void symv_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
   // butterfly transpose-reduce of the R row sums: after the exchanges at offsets
   // R/2, ..., 1 lane l holds row (l & (R-1)) summed over its group of R lanes; the
   // exchanges at R, 2R, ..., 32 sum the groups
-  static_assert(R == 4 || R == 8, "R rows per block: 4 or 8");
 #pragma unroll
   for (int o = R / 2; o > 0; o >>= 1) {
     const bool b = (lane & o) != 0;
 #pragma unroll
-    for (int k = 0; k < o; ++k) acc[k] = (b ? acc[k + o] : acc[k]) + xlane(b ? acc[k] : acc[k + o], o);
+    for (int k = 0; k < o; ++k) {
+      // values first: a select between array elements becomes one of their indices
+      const double x = acc[k], y = acc[k + o];
+      acc[k] = (b ? y : x) + xlane(b ? x : y, o);
+    }
   }
   {
     double a = acc[0];
@@ -349,14 +343,14 @@ __device__ inline void symv_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
         const double vr = (r == c + 1) ? 1.0 : xown * scale;
         const double yr = (red[0][rr] + red[1][rr]) + (red[2][rr] + red[3][rr]);
         val = yr * vr;
-        store_dev(ws.y + r, yr);
+        ws.y[r] = yr;
         ws.V[(int64_t)r * kNB + j] = vr;
         ws.a[(int64_t)c * lda + r] = vr;
       }
     }
 #pragma unroll
     for (int o = R / 2; o > 0; o >>= 1) val += xlane(val, o);
-    if (lane == 0) store_dev(ws.ps + blk, val);
+    if (lane == 0) ws.ps[blk] = val;
   }
 }
 
@@ -364,12 +358,8 @@ __device__ inline void symv_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
 // Panel vectors are stored row-major, V[r * kNB + q], so a thread loads its row's
 // coefficients in one batch; entries of columns not yet in this panel are stale
 // but always meet a zero coefficient.
-// kEarly (a launch after the symv part's): y and the y.v partials are final before
-// the launch starts, so their loads go out with the others and the part runs on one
-// round of memory latency instead of two.
-template <bool kEarly, class Wait>
 __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t j, int32_t blk,
-                                 int32_t nps, Wait &&wait) {
+                                 int32_t nps) {
   __shared__ double red[4][4];
   __shared__ double pqr[4][2 * kNB];  // raw panel dots per wave
   __shared__ double pq[2 * kNB];      // p_q = V_q . v, q_q = W_q . v (zero for q >= j)
@@ -380,9 +370,9 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
   const int32_t lda = ws.lda;
   const double *pwc = ws.pw + (int64_t)(c & 1) * ws.maxw * kPW;
   const int32_t nw = wcol_blocks(n, c);
-  // ---- loads of data from earlier launches go out before the hand-off wait: this
-  // row's quarter of the panel vectors (column j, written by this launch's symv part,
-  // is rebuilt from x below) and its entry of the trailing row c+1, its x, row c+1's
+  // ---- all loads go out first, so the part runs on one round of memory latency: this
+  // row's quarter of the panel vectors (column j is
+  // rebuilt from x below) and its entry of the trailing row c+1, its x, row c+1's
   // panel coefficients, and the panel-dot and norm partials
   const int32_t r = c1 + blk * kWRows + (int32_t)(threadIdx.x >> 2);
   const bool inr = r < n;
@@ -415,12 +405,10 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
     const int q = threadIdx.x & (kNB - 1);
     atc = (threadIdx.x < kNB) ? ws.V[(int64_t)c1 * kNB + q] : ws.W[(int64_t)c1 * kNB + q];
   }
-  double ye = 0.0, yc1e = 0.0, ype[8];
-  if constexpr (kEarly) {
-    ye = ws.y[rs];
-    yc1e = ws.y[c1];
-    load8(ws.ps, 1, threadIdx.x, 256, nps, ype);
-  }
+  double yy = ws.y[rs];
+  const double yc1 = ws.y[c1];
+  double yp[8];
+  load8(ws.ps, 1, threadIdx.x, 256, nps, yp);
   double praw = 0.0;
   {
     const int comp = lane;  // 0..31 V dots, 32..63 W dots
@@ -442,12 +430,7 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
     col_scalars_sums(sum_rest(pwc, kPW, lane, 64, nw, ln0), sum_rest(pwc + 1, kPW, lane, 64, nw, ln1),
                      tau, scale, beta);
   }
-  if (!wait()) return;
-  // ---- the symv part's outputs: y and the per-block partials of y.v
-  double yy = kEarly ? ye : ws.y[rs];
-  const double yc1 = kEarly ? yc1e : ws.y[c1];
-  double yv = kEarly ? sum_rest(ws.ps, 1, threadIdx.x, 256, nps, ype)
-                     : sum_strided(ws.ps, 1, threadIdx.x, 256, nps);
+  double yv = sum_rest(ws.ps, 1, threadIdx.x, 256, nps, yp);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) yv += xlane(yv, o);
   if (lane == 0) red[wv][0] = yv;
@@ -553,7 +536,10 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
       const bool bsel = (lane & off) != 0;
 #pragma unroll
       for (int k = 0; k < half; ++k)
-        t[k] = (bsel ? t[k + half] : t[k]) + xlane(bsel ? t[k] : t[k + half], off);
+      {
+        const double p0 = t[k], p1 = t[k + half];
+        t[k] = (bsel ? p1 : p0) + xlane(bsel ? p0 : p1, off);
+      }
     }
     const int i = (lane >> 2) & 15;
     const int comp = (i < 8) ? 8 * sub + i : kNB + 8 * sub + (i - 8);
@@ -571,74 +557,11 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
   }
 }
 
-// The two parts as kernels of their own, for long columns: there the symv part
-// streams a large trailing matrix and a launch boundary costs less than holding
-// w-column blocks and draining device-coherent stores inside one launch.
-template <int R>
 __global__ __launch_bounds__(256) void k_symv(EigWs ws, int32_t n, int32_t c, int32_t j) {
-  symv_part<R>(ws, n, c, j, (int32_t)blockIdx.x);
+  symv_part(ws, n, c, j, (int32_t)blockIdx.x);
 }
 __global__ __launch_bounds__(256) void k_wcol(EigWs ws, int32_t n, int32_t c, int32_t j, int32_t nps) {
-  wcol_part<true>(ws, n, c, j, (int32_t)blockIdx.x, nps, []() { return true; });
-}
-
-// ---------------------------------------------------------------- k_column
-// One launch per column with gw + gsym blocks (gw = ceil((n-c-1)/64) w-column
-// chunks, gsym = ceil((n-c-1)/8) symv row groups).  Blocks gw .. gw+gsym-1 run the
-// symv part for their 8 rows and then add one to a ticket counter once their y and
-// ps stores (device-coherent stores) have completed.  Blocks 0 .. gw-1 run the
-// w-column part for one 64-row chunk each: they issue their loads of data from
-// earlier launches at once, then wait until all gsym tickets are in, then read y
-// and the y.v partials.  The waiters never hold up a symv block (k_column runs for
-// trailing orders below kMergeBelow, so there are at most 16 of them, far fewer than
-// the blocks the device holds at once), so the launch cannot deadlock; the wait is
-// bounded anyway, and a timeout sets sync[1] for the host to report.  The waiters
-// first sleep for quiet_ticks of the device's wall clock (most of the symv part's
-// expected duration), then poll.  The counter is cleared by k_col0 and grows
-// monotonically over the columns: column c's tickets are base .. base + gsym - 1.
-// Ordering rests on the ISA, not on a release: the y and partial stores write through
-// the XCD's L2 (sc1) and are drained (vmcnt 0) before the ticket is added, and the
-// waiter polls with sc1 loads and runs an agent-scope acquire (L2 invalidate) before
-// reading them.  A release would write back the whole L2 once per block.
-constexpr int64_t kHandoffSpin = 1 << 22;
-__global__ __launch_bounds__(256) void k_column(EigWs ws, int32_t n, int32_t c, int32_t j,
-                                                int32_t base, int64_t quiet_ticks) {
-  __shared__ int32_t ok_sh;
-  const int32_t gw = (n - c - 1 + kWRows - 1) / kWRows;
-  const int32_t gsym = (int32_t)gridDim.x - gw;
-  if ((int32_t)blockIdx.x >= gw) {
-    symv_part<kSymvRows>(ws, n, c, j, (int32_t)blockIdx.x - gw);
-    // each wave drains its own device-coherent stores, then one thread adds the ticket
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0)
-      __hip_atomic_fetch_add(ws.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return;
-  }
-  const uint64_t t_start = wall_clock64();
-  auto wait = [&]() -> bool {
-    if (threadIdx.x == 0) {
-      // no polling for most of the symv part's expected time: polls are device-
-      // coherent loads and slow down the symv blocks' stream of the matrix
-      while ((int64_t)(wall_clock64() - t_start) < quiet_ticks) __builtin_amdgcn_s_sleep(32);
-      int32_t ok = 0;
-      for (int64_t s = 0; s < kHandoffSpin; ++s) {
-        if (__hip_atomic_load(ws.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= base + gsym) {
-          ok = 1;
-          break;
-        }
-        if (__hip_atomic_load(ws.sync + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
-        __builtin_amdgcn_s_sleep(1);
-      }
-      if (!ok) __hip_atomic_store(ws.sync + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      ok_sh = ok;
-    }
-    __syncthreads();
-    if (!ok_sh) return false;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    return true;
-  };
-  wcol_part<false>(ws, n, c, j, (int32_t)blockIdx.x, gsym, wait);
+  wcol_part(ws, n, c, j, (int32_t)blockIdx.x, nps);
 }
 
 // A[r][s] -= sum_q V[r][q] W[s][q] + W[r][q] V[s][q] for r, s >= k0: one FP64 MFMA
@@ -762,6 +685,285 @@ __global__ __launch_bounds__(256) void k_syr2k(EigWs ws, int32_t n, int32_t k0, 
         const int32_t c = cb + 32 * wc + 16 * b + (lane & 15);
         if (r < n && c < n) ws.a[(int64_t)r * lda + c] = old[a][b][e] - acc[a][b][e];
       }
+}
+
+// ---------------------------------------------------------------- resident part
+// Tridiagonalisation of a trailing matrix that the register files hold: columns c0 .. c1-1
+// in one launch, block b holding rows c0 + b RS .. in registers (thread t: columns c0 + t +
+// T k of every row).  Per column c every block forms the same reflector v from x = row c
+// and the products of its own rows with it; they and the owner's copy of row c+1 go to
+// memory, every block reads all of them back and forms w = tau y + alpha v and the next x
+// = row c+1 - w - w_{c+1} v for itself, and each applies the rank-2 update to its own rows
+// while it forms the next products.  So a column is one exchange between blocks, three
+// barriers within them, and no pass over memory.
+//
+// Every word exchanged is its own flag: the buffers hold kTriNone, a NaN that no
+// arithmetic produces, until the word's one store of the launch (device-coherent, 8 bytes
+// at once), and a reader polls the words it needs with device-coherent loads until none is
+// kTriNone.  No order between words is assumed.  A block whose rows are all done leaves.
+// The blocks have to run at the same time: there is one per CU at most (host side), and
+// the host runs one such launch at a time on a device (two that each held part of the CUs
+// would wait for each other).  Should some not be scheduled (the
+// device shared with other programs), each wait ends after kTriLimit ticks of the wall
+// clock and sets sync[1]; the host then starts over without this kernel.
+constexpr uint64_t kTriNone = 0xFFF4E1D2C3B4A596ull;
+constexpr int64_t kTriLimit = 50000000;  // 0.5 s at 100 MHz
+__global__ __launch_bounds__(256) void k_tri_fill(uint64_t *__restrict__ p, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+    p[i] = kTriNone;
+}
+__device__ __forceinline__ void store_dev(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double load_dev(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Sums over the wave of the row values that lanes hold, four rows at a time as they come
+// (few registers live at once), then over the groups: lane l ends with row l % R2's sum
+// (R2 = 8 or 16).  rows4 leaves row l % 4 summed over the lanes' groups of four.
+__device__ __forceinline__ double xpick(bool b, double x, double y, int o) {
+  return (b ? y : x) + xlane(b ? x : y, o);
+}
+__device__ __forceinline__ double rows4(const double (&v)[4]) {
+  const int lane = threadIdx.x & 63;
+  const bool b2 = (lane & 2) != 0, b1 = (lane & 1) != 0;
+  return xpick(b1, xpick(b2, v[0], v[2], 2), xpick(b2, v[1], v[3], 2), 1);
+}
+template <int G>
+__device__ __forceinline__ double rows_sum(const double (&z)[G]) {
+  const int lane = threadIdx.x & 63;
+  const bool b4 = (lane & 4) != 0, b8 = (lane & 8) != 0;
+  double a;
+  if constexpr (G == 1) {
+    a = z[0];
+    a += xlane(a, 4);
+    a += xlane(a, 8);
+  } else if constexpr (G == 2) {
+    a = xpick(b4, z[0], z[1], 4);
+    a += xlane(a, 8);
+  } else {
+    const double z3 = G == 4 ? z[G - 1] : 0.0;
+    a = xpick(b4, xpick(b8, z[0], z[2], 8), xpick(b8, z[1], z3, 8), 4);
+  }
+  a += xlane(a, 16);
+  a += xlane(a, 32);
+  return a;
+}
+__device__ __forceinline__ double tri_rcp(double a) {
+  double r = __builtin_amdgcn_rcp(a);
+  r = fma(r, fma(-a, r, 1.0), r);
+  return fma(r, fma(-a, r, 1.0), r);
+}
+// Indices are local to the stage: column and row i of the kernel are c0 + i of the matrix.
+template <int T, int K, int RS>
+__global__ __launch_bounds__(T) void k_tri(EigWs ws, int32_t n, int32_t c0, int32_t c1,
+                                           double *__restrict__ yb, double *__restrict__ rb,
+                                           int64_t ldb) {
+  constexpr int W = T / 64;
+  constexpr int G = RS / 4;  // rows are summed in groups of four
+  static_assert(RS % 4 == 0 && RS <= 16, "rows per block");
+  __shared__ double sv[2][T * K], sw[T * K];
+  __shared__ double red[W][16], rdot[W], rnrm[W], sy1, sal;
+  __shared__ int32_t dead;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int32_t nl = n - c0, cols = c1 - c0, r0 = (int32_t)blockIdx.x * RS;  // first row
+  const int64_t lda = ws.lda;
+  double *const A = ws.a + (int64_t)c0 * lda + c0;
+  // thread t's columns are t + T k: with the uniform part in scalars, one offset serves all
+  // of a thread's addresses, and comparisons are with t
+  double a[RS][K], x[K], v[K], w[K];
+#pragma unroll
+  for (int s = 0; s < RS; ++s)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double *p = A + (int64_t)min(r0 + s, nl - 1) * lda + T * k;
+      a[s][k] = (r0 + s < nl && t < nl - T * k) ? p[t] : 0.0;
+    }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const double *p = A + T * k;
+    x[k] = t < nl - T * k ? p[t] : 0.0;
+    v[k] = w[k] = 0.0;
+    sv[0][t + T * k] = sv[1][t + T * k] = sw[t + T * k] = 0.0;
+  }
+  if (t == 0) dead = 0;
+  if (blockIdx.x == 0 && t == 0) ws.d[c0] = x[0];
+  // row c is overwritten by its reflector only after an exchange that every block took part
+  // in, so each has read row c0 and its own rows by then
+  // norm of x beyond c + 1, and x_{c+1}
+  auto norm = [&](int32_t c) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      s = fma(x[k], t >= c + 2 - T * k ? x[k] : 0.0, s);
+      if (t == c + 1 - T * k) sal = x[k];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += xlane(s, o);
+    if (lane == 0) rnrm[wv] = s;
+  };
+  norm(0);
+  __syncthreads();
+  for (int32_t c = 0; c < cols; ++c) {
+    if (r0 + RS - 1 <= c) return;  // no live rows: nothing to give and nothing to keep
+    const int cur = c & 1;
+    // ---- the reflector of column c (dlarfg), the same in every block
+    double xn2 = rnrm[0];
+#pragma unroll
+    for (int u = 1; u < W; ++u) xn2 += rnrm[u];
+    const double al = sal;
+    double tau = 0.0, scale = 0.0, beta = al;
+    if (xn2 > 0.0) {
+      const double s2 = fma(al, al, xn2);
+      if (s2 > 1e-280 && s2 < 1e280) {
+        // 1 / sqrt and 1 / x by the hardware's approximations and two Newton steps each (a
+        // few ulps, as rcp_nr's), whose chains are shorter than a square root's and division's
+        double h = __builtin_amdgcn_rsq(s2);
+        h = fma(h, fma(-0.5 * s2 * h, h, 0.5), h);
+        h = fma(h, fma(-0.5 * s2 * h, h, 0.5), h);
+        const double nb = copysign(s2 * h, al);  // -beta
+        beta = -nb;
+        tau = fma(fabs(al), h, 1.0);
+        scale = tri_rcp(al + nb);
+      } else {
+        beta = -copysign(sqrt(s2), al);
+        tau = (beta - al) / beta;
+        scale = 1.0 / (al - beta);
+      }
+    }
+    double vn[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int32_t p = c + 1 - T * k;
+      vn[k] = t == p ? 1.0 : (t > p ? x[k] * scale : 0.0);
+      sv[cur][t + T * k] = vn[k];
+    }
+    // ---- the update by column c - 1 (v, w; zero at first) and the products with vn
+    double z[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int s = 4 * g + u;
+        const double vi = sv[cur ^ 1][r0 + s], wi = sw[r0 + s];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          a[s][k] = fma(-vi, w[k], fma(-wi, v[k], a[s][k]));
+          acc[u] = fma(a[s][k], vn[k], acc[u]);
+        }
+      }
+      z[g] = rows4(acc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // ---- row c + 1 to the others
+    const bool owner = c + 1 >= r0 && c + 1 < r0 + RS;
+    double *const rrow = rb + (int64_t)c * ldb, *const yrow = yb + (int64_t)c * ldb;
+    if (owner) {
+#pragma unroll
+      for (int s = 0; s < RS; ++s)
+        if (c + 1 == r0 + s)
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+            if (t > c - T * k && t < nl - T * k) store_dev(rrow + T * k + t, a[s][k]);
+    }
+    {
+      const double rs = rows_sum<G>(z);
+      if (lane < 16) red[wv][lane] = rs;
+    }
+    __syncthreads();
+    if (t < RS && r0 + t > c && r0 + t < nl) {
+      double y = red[0][t];
+#pragma unroll
+      for (int u = 1; u < W; ++u) y += red[u][t];
+      store_dev(yrow + r0 + t, y);
+    }
+    // ---- everyone's products and row c + 1
+    {
+      double *const y = w, *const r = x;  // their registers
+      int64_t t_end = 0;
+      for (int32_t spin = 0;; ++spin) {
+        bool all = true;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          y[k] = r[k] = 0.0;
+          if (t > c - T * k && t < nl - T * k) {
+            y[k] = load_dev(yrow + T * k + t);
+            r[k] = load_dev(rrow + T * k + t);
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+          all = all && __builtin_bit_cast(uint64_t, y[k]) != kTriNone &&
+                __builtin_bit_cast(uint64_t, r[k]) != kTriNone;
+        if (all) break;
+        if ((spin & 255) == 255) {
+          const int64_t now = (int64_t)wall_clock64();
+          if (t_end == 0) t_end = now + kTriLimit;
+          if (now > t_end ||
+              __hip_atomic_load(ws.sync + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+            dead = 1;
+            break;
+          }
+        }
+      }
+    }
+    double dt = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      dt = fma(w[k], vn[k], dt);
+      if (t == c + 1 - T * k) sy1 = w[k];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) dt += xlane(dt, o);
+    if (lane == 0) rdot[wv] = dt;
+    __syncthreads();
+    if (dead) {
+      if (t == 0) __hip_atomic_store(ws.sync + 1, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    double ydv = rdot[0];
+#pragma unroll
+    for (int u = 1; u < W; ++u) ydv += rdot[u];
+    // w = tau y + alpha v (y and v are zero up to column c), x = row c + 1 - w - w_{c+1} v
+    const double alpha = -0.5 * tau * (tau * ydv);
+    const double w1 = tau * sy1 + alpha;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      v[k] = vn[k];
+      w[k] = tau * w[k] + alpha * vn[k];
+      x[k] = x[k] - w[k] - w1 * vn[k];
+      sw[t + T * k] = w[k];
+    }
+    norm(c + 1);
+    // ---- results of column c, by the owner of row c + 1
+    if (owner) {
+      double *const out = A + (int64_t)c * lda;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        if (t > c - T * k && t < nl - T * k) (out + T * k)[t] = vn[k];
+        if (t == c + 1 - T * k) ws.d[c0 + c + 1] = x[k];
+      }
+      if (t == 0) {
+        ws.e[c0 + c] = beta;
+        ws.e2[c0 + c] = beta * beta;
+        ws.tau[c0 + c] = tau;
+      }
+    }
+    __syncthreads();
+  }
+  // the last update, and the rows back to memory for what follows
+  if (c1 >= n - 1) return;
+  const int last = (cols - 1) & 1;
+#pragma unroll
+  for (int s = 0; s < RS; ++s) {
+    const double vi = sv[last][r0 + s], wi = sw[r0 + s];
+    if (r0 + s < cols || r0 + s >= nl) continue;
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (t >= cols - T * k && t < nl - T * k)
+        (A + (int64_t)(r0 + s) * lda + T * k)[t] = fma(-vi, w[k], fma(-wi, v[k], a[s][k]));
+  }
 }
 
 // ---------------------------------------------------------------- eigenvalues
@@ -1541,40 +1743,14 @@ __global__ __launch_bounds__(256) void k_finish_vec(EigWs ws, int32_t n) {
 }
 
 // ---------------------------------------------------------------- driver
-// wall-clock ticks the w-column blocks of k_column sleep before polling: 80% of the
-// symv part's streaming time at 6.5 TB/s (its measured rate on large trailing
-// matrices), nothing below 2 us
-static int64_t quiet_ticks(int32_t L, int32_t clock_khz) {
-  const double us = 0.8 * (double)L * (double)L * 8.0 / 6.5e12 * 1e6;
-  return us < 2.0 ? 0 : (int64_t)(us * clock_khz / 1000.0);
-}
-
-// Trailing order below which k_column runs (one launch per column); longer columns
-// run k_symv + k_wcol.  Measured on MI355X: merging at every length costs ~10 us per
-// column on 5,000-long columns (the w-column blocks held for the whole stream and the
-// store drain) and saves a few us per column on short ones.  With the 64-row
-// w-column chunks, cuts of 500 to 1,000 were best for n = 3,000 and 5,000 (1 to
-// 3,000 tried; never merging costs 1.1 ms at n = 5,000).
-// EIG_NO_MERGE=1 runs every column as k_symv + k_wcol: counter-collection runs use it,
-// since no launch then waits on other blocks of its own grid.
-constexpr int32_t kMergeBelow = 1000;
-static void launch_tridiag(EigWs ws, int32_t n, int32_t clock_khz, hipStream_t st) {
-  const int32_t merge_below = getenv("EIG_NO_MERGE") != nullptr ? 1 : kMergeBelow;
+static void launch_tridiag(EigWs ws, int32_t n, int32_t stop, hipStream_t st) {
   hipLaunchKernelGGL(k_col0, dim3(1), dim3(256), 0, st, ws, n);
-  int32_t base = 0;  // hand-off tickets taken by the earlier columns
-  for (int32_t c = 0; c + 1 < n; ++c) {
+  for (int32_t c = 0; c + 1 < n && c < stop; ++c) {
     const int32_t j = c % kNB;
     const int32_t L = n - c - 1;
-    const int32_t gsym = (L + kSymvRows - 1) / kSymvRows, gw = (L + kWRows - 1) / kWRows;
-    if (L >= merge_below) {
-      const int32_t g4 = (L + kSymvRowsLong - 1) / kSymvRowsLong;
-      hipLaunchKernelGGL(k_symv<kSymvRowsLong>, dim3((unsigned)g4), dim3(256), 0, st, ws, n, c, j);
-      hipLaunchKernelGGL(k_wcol, dim3((unsigned)gw), dim3(256), 0, st, ws, n, c, j, g4);
-    } else {
-      hipLaunchKernelGGL(k_column, dim3((unsigned)(gw + gsym)), dim3(256), 0, st, ws, n, c, j, base,
-                         quiet_ticks(L, clock_khz));
-      base += gsym;
-    }
+    const int32_t gs = (L + kSymvRows - 1) / kSymvRows, gw = (L + kWRows - 1) / kWRows;
+    hipLaunchKernelGGL(k_symv, dim3((unsigned)gs), dim3(256), 0, st, ws, n, c, j);
+    hipLaunchKernelGGL(k_wcol, dim3((unsigned)gw), dim3(256), 0, st, ws, n, c, j, gs);
     // panel end: update the trailing matrix before the next panel's first symv
     if (j == kNB - 1 && c + 2 < n) {
       const int32_t k1 = c + 1;
@@ -1584,8 +1760,76 @@ static void launch_tridiag(EigWs ws, int32_t n, int32_t clock_khz, hipStream_t s
   }
 }
 
+// ---- the resident part's launch shapes: the order a shape holds, and its kernel.  A stage
+// runs the smallest shape that holds what is left, down to the next smaller one's order:
+// a column costs an exchange (about 1.7 us) and the work between, which grows with the
+// blocks and the columns per thread.  Measured, whole reductions: n = 198 0.46 ms, 512
+// 1.27, 1,000 2.66, 2,048 7.1, where launches per column took 1.5, 4.9, 9.6 and 22.  n =
+// 1,000 in the 1,024 shape alone takes 0.3 ms longer than by stages.  Above 2,048 the rows
+// and the four vectors no longer fit 256 registers a thread: 512 x 6 columns x 12 rows
+// spills and takes 18 to 29 us a column, more than the launches.
+struct TriShape {
+  int32_t cap, T, RS;
+  void (*fn)(EigWs, int32_t, int32_t, int32_t, double *, double *, int64_t);
+};
+static const TriShape kTriShapes[] = {
+    {256, 256, 8, k_tri<256, 1, 8>},   {512, 256, 8, k_tri<256, 2, 8>},
+    {1024, 512, 8, k_tri<512, 2, 8>},  {2048, 512, 8, k_tri<512, 4, 8>},
+};
+constexpr int kTriNum = sizeof(kTriShapes) / sizeof(kTriShapes[0]);
+// one resident launch at a time on a device (see k_tri)
+static std::mutex g_tri_mu[16];
+
+// largest order that a launch of blocks one per CU holds, at most `cap`
+static int32_t tri_cap(const eig_ctx *ctx) {
+  int32_t best = 0;
+  for (const TriShape &h : kTriShapes)
+    if ((h.cap + h.RS - 1) / h.RS <= ctx->num_cu) best = std::max(best, h.cap);
+  return best;
+}
+static int launch_resident(eig_ctx *ctx, const EigWs &ws, int32_t n, int32_t c0, hipStream_t st) {
+  // exchange buffers: products and rows, one word per column and row of a stage
+  auto stage = [&](int32_t c, int32_t &c1) -> const TriShape * {
+    int i = 0;
+    while (kTriShapes[i].cap < n - c) ++i;
+    c1 = i == 0 ? n - 1 : std::min(n - 1, n - kTriShapes[i - 1].cap);
+    return &kTriShapes[i];
+  };
+  int64_t words = 0;
+  for (int32_t c = c0, c1; c < n - 1; c = c1) {
+    stage(c, c1);
+    words = std::max(words, (int64_t)(c1 - c) * (n - c));
+  }
+  EIG_TRY(eig_ensure(ctx, ctx->tribuf, 16 * (size_t)words));
+  double *yb = (double *)ctx->tribuf.p;
+  for (int32_t c = c0, c1; c < n - 1; c = c1) {
+    const TriShape *h = stage(c, c1);
+    const int64_t ld = n - c, cnt = 2 * (int64_t)(c1 - c) * ld;
+    hipLaunchKernelGGL(k_tri_fill, dim3((unsigned)std::min<int64_t>((cnt + 255) / 256, 4096)), dim3(256), 0,
+                       st, (uint64_t *)yb, cnt);
+    hipLaunchKernelGGL(h->fn, dim3((unsigned)((n - c + h->RS - 1) / h->RS)), dim3((unsigned)h->T), 0, st, ws,
+                       n, c, c1, yb, yb + (int64_t)(c1 - c) * ld, ld);
+  }
+  EIG_HIP(ctx, hipGetLastError());
+  return EIG_OK;
+}
+
+static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, double *evals,
+                    double *evecs, bool internal, bool resident, bool *again);
+
 int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, double *evals,
                  double *evecs, bool internal) {
+  bool again = false;
+  EIG_TRY(run_eigh(ctx, d_a, n, nvec, evals, evecs, internal, true, &again));
+  // the resident part gave up waiting for blocks that were not scheduled: start over with
+  // the launches that wait for nothing outside themselves
+  if (again) EIG_TRY(run_eigh(ctx, d_a, n, nvec, evals, evecs, internal, false, &again));
+  return EIG_OK;
+}
+
+static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, double *evals,
+                    double *evecs, bool internal, bool resident, bool *again) {
+  *again = false;
   if (n <= 0) return eig_set_err(ctx, EIG_E_ARG, "eigh: n <= 0");
   if (nvec < 0 || nvec > n) return eig_set_err(ctx, EIG_E_ARG, "eigh: nvec must be in [0, n]");
   if (internal && nvec > kMaxVec)
@@ -1595,7 +1839,7 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
   auto tend = [&](const char *what) { if (!internal) eig_time_end(ctx, what); };
   const int64_t N = n;
   const int32_t lda = (int32_t)(((N + 7) / 8) * 8);
-  const int64_t maxblk = (N + kSymvRowsLong - 1) / kSymvRowsLong + 8;  // symv partials
+  const int64_t maxblk = (N + kSymvRows - 1) / kSymvRows + 8;  // symv partials
   const int64_t maxnv = (int64_t)kNB * kMaxVec;
   const int64_t maxw = (N + kWRows - 1) / kWRows + 2;
   const int64_t npanel = (N + kNB - 1) / kNB + 1;
@@ -1649,14 +1893,31 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
   EIG_HIP(ctx, hipMemsetAsync(ws.xtmp, 0, sizeof(double) * lda, st));
 
   // ---- tridiagonalisation: plain launches.  The host queues a launch in ~3 us, less than
-  // the shortest column takes on the device, so a captured graph of the ~2 N launches
-  // replays no faster (n = 1,000: 9.54 against 9.59 ms, n = 5,000: 97.5 against 96.4) and
-  // capturing it costs every first solve of an order or a context 1.5 and 12.5 ms.
-  int32_t clock_khz = 0;
-  EIG_HIP(ctx, hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, ctx->device));
+  // the shortest column takes on the device, so a captured graph of the launches replays
+  // no faster (n = 5,000: 97.5 against 96.4 ms) and capturing it costs every first solve of
+  // an order or a context 12.5 ms.
   tbeg();
-  launch_tridiag(ws, n, clock_khz, st);
+  // long columns by launches, whole panels, until the resident part holds the rest.
+  // EIG_NO_MERGE=1 runs all columns by launches: counter-collection runs use it, since no
+  // launch then waits on other blocks of its own grid
+  const int32_t cap = resident && getenv("EIG_NO_MERGE") == nullptr ? tri_cap(ctx) : 0;
+  const int32_t stop = cap == 0 ? n : (n > cap ? (n - cap + kNB - 1) / kNB * kNB : 0);
+  if (stop > 0) launch_tridiag(ws, n, stop, st);
   EIG_HIP(ctx, hipGetLastError());
+  if (stop < n - 1) {
+    std::lock_guard<std::mutex> lock(g_tri_mu[ctx->device & 15]);
+    EIG_HIP(ctx, hipMemsetAsync(ws.sync, 0, 8, st));
+    EIG_TRY(launch_resident(ctx, ws, n, stop, st));
+    int32_t gave_up[2] = {0, 0};
+    EIG_HIP(ctx, hipMemcpyAsync(gave_up, ws.sync, sizeof(gave_up), hipMemcpyDeviceToHost, st));
+    EIG_HIP(ctx, hipStreamSynchronize(st));
+    if (gave_up[1] == 2) {
+      *again = true;
+      return EIG_OK;
+    }
+  } else if (n == 1) {
+    hipLaunchKernelGGL(k_col0, dim3(1), dim3(256), 0, st, ws, n);
+  }
   tend("tridiag");
   // ---- eigenvalues
   tbeg();
@@ -1779,8 +2040,6 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
   }
   tend("eigvec");
   std::vector<double> asc(N);
-  int32_t hsync[2] = {0, 0};
-  EIG_HIP(ctx, hipMemcpyAsync(hsync, ws.sync, sizeof(hsync), hipMemcpyDeviceToHost, st));
   EIG_HIP(ctx, hipMemcpyAsync(asc.data(), ws.eval, sizeof(double) * N, hipMemcpyDeviceToHost, st));
   if (nvec > 0 && nvec <= kMaxVec) {
     if (evecs)
@@ -1792,8 +2051,6 @@ int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, doubl
     }
   }
   EIG_HIP(ctx, hipStreamSynchronize(st));
-  if (hsync[1] != 0)
-    return eig_set_err(ctx, EIG_E_CONVERGE, "eigh: tridiagonalisation hand-off timed out");
   for (int64_t i = 0; i < N; ++i) {
     if (std::isnan(asc[i])) return eig_set_err(ctx, EIG_E_CONVERGE, "eigenvalue is NaN");
     if (evals) evals[i] = asc[N - 1 - i];
