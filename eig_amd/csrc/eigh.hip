@@ -1353,30 +1353,30 @@ __global__ __launch_bounds__(256) void k_invit(EigWs ws, int32_t n, int32_t nvec
 }
 
 // ---- more than kMaxVec vectors ----
-// One block per batch of kMaxVec vectors (vector j of the call's list at XT + j n): LU,
-// start vectors and two solves, each followed by a normalisation (a wave per vector).  The
-// batches of a launch do not depend on each other; the vectors are orthogonalised
-// afterwards.
+// One block per batch of kMaxVec vectors (vector j of the call's list at XT + j n): the
+// stages of `flags` and one solve, then a normalisation (a wave per vector).  The batches
+// of a launch do not depend on each other.  The vectors are orthogonalised after each of
+// the two solves: two solves in a row turn the vectors of a repeated eigenvalue towards
+// the one nearest to their shifts, and what is left between them after that is rounding
+// (residuals of 1e-11 of the norm; orthogonalised in between, a few ulps).
 __global__ __launch_bounds__(256) void k_invit_batches(EigWs ws, int32_t n, int32_t nvec,
-                                                       int32_t b0, double *__restrict__ XT,
+                                                       int32_t b0, int32_t flags,
+                                                       double *__restrict__ XT,
                                                        double *__restrict__ lu) {
   const int32_t j0 = (b0 + (int32_t)blockIdx.x) * kMaxVec;
   const int32_t nb = min(kMaxVec, nvec - j0);
   ws.X = XT + (int64_t)j0 * n;
   ws.lu = lu + (int64_t)blockIdx.x * kMaxVec * kLuF * n;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int it = 0; it < 2; ++it) {
-    invit_part(ws, n, nb, j0, (it == 0 ? kInvFactor | kInvStart : 0) | kInvSolve, 1);
-    for (int32_t v = wv; v < nb; v += 4) {
-      double *x = ws.X + (int64_t)v * n;
-      double s = 0.0;
-      for (int32_t i = lane; i < n; i += 64) s += x[i] * x[i];
+  invit_part(ws, n, nb, j0, flags | kInvSolve, 1);
+  for (int32_t v = wv; v < nb; v += 4) {
+    double *x = ws.X + (int64_t)v * n;
+    double s = 0.0;
+    for (int32_t i = lane; i < n; i += 64) s += x[i] * x[i];
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) s += xlane(s, o);
-      const double inv = 1.0 / sqrt(s);
-      for (int32_t i = lane; i < n; i += 64) x[i] *= inv;
-    }
-    __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) s += xlane(s, o);
+    const double inv = 1.0 / sqrt(s);
+    for (int32_t i = lane; i < n; i += 64) x[i] *= inv;
   }
 }
 
@@ -1938,7 +1938,7 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   tend("bisect");
   // ---- eigenvectors: one batch of at most kMaxVec (inverse iteration with Gram-Schmidt,
   // back-transform, sign rule); more vectors run in batches of kMaxVec in eigenvalue
-  // order: every batch's solves, then batch by batch the Gram-Schmidt against the earlier
+  // order: twice every batch's solve and batch by batch the Gram-Schmidt against the earlier
   // vectors and within the batch, then the back-transform of all
   // vectors together as FP64 MFMA products
   const int32_t last = n - 2;  // last reflector row
@@ -1982,24 +1982,28 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
                                                           sq * nblk + sq + lub * group)));
     double *XT = (double *)ctx->evall.p, *Cc = XT + (size_t)N * nvec, *gp = Cc + (size_t)kMaxVec * nvec,
            *Ri = gp + sq * nblk, *lu = Ri + sq;
-    for (int32_t b = 0; b < nbatch; b += group)
-      hipLaunchKernelGGL(k_invit_batches, dim3((unsigned)std::min(group, nbatch - b)), dim3(256), 0, st,
-                         ws, n, nvec, b, XT, lu);
-    EIG_HIP(ctx, hipGetLastError());
     // against every earlier vector, not only those of close eigenvalues: the products are
-    // a small part, and vectors a few 1e-3 ||T|| apart stay orthogonal to the last ulps
-    for (int32_t j0 = 0; j0 < nvec; j0 += kMaxVec) {
-      const int32_t nb = std::min<int32_t>(kMaxVec, nvec - j0), nc = j0;
-      double *X = XT + (size_t)j0 * N;
-      const double *P = XT;
-      for (int rep = 0; rep < 2; ++rep) {
-        if (nc > 0) {
-          EIG_TRY(eig_gemm_f64(ctx, st, true, false, nc, nb, N, 1.0, P, N, 0, X, N, 0, 0.0, Cc, nc, 0, 1));
-          EIG_TRY(eig_gemm_f64(ctx, st, false, false, N, nb, nc, -1.0, P, N, 0, Cc, nc, 0, 1.0, X, N, 0, 1));
+    // a small part, and vectors a few 1e-3 ||T|| apart stay orthogonal to the last ulps.
+    // After the first solve once is enough (the vectors only start the second)
+    for (int it = 0; it < 2; ++it) {
+      const int32_t flags = it == 0 ? kInvFactor | kInvStart : (nbatch > group ? kInvFactor : 0);
+      for (int32_t b = 0; b < nbatch; b += group)
+        hipLaunchKernelGGL(k_invit_batches, dim3((unsigned)std::min(group, nbatch - b)), dim3(256), 0, st,
+                           ws, n, nvec, b, flags, XT, lu);
+      EIG_HIP(ctx, hipGetLastError());
+      for (int32_t j0 = 0; j0 < nvec; j0 += kMaxVec) {
+        const int32_t nb = std::min<int32_t>(kMaxVec, nvec - j0), nc = j0;
+        double *X = XT + (size_t)j0 * N;
+        const double *P = XT;
+        for (int rep = 0; rep <= it; ++rep) {
+          if (nc > 0) {
+            EIG_TRY(eig_gemm_f64(ctx, st, true, false, nc, nb, N, 1.0, P, N, 0, X, N, 0, 0.0, Cc, nc, 0, 1));
+            EIG_TRY(eig_gemm_f64(ctx, st, false, false, N, nb, nc, -1.0, P, N, 0, Cc, nc, 0, 1.0, X, N, 0, 1));
+          }
+          hipLaunchKernelGGL(k_gs_gram, dim3((unsigned)nblk), dim3(256), 0, st, (const double *)X, n, nb, gp);
+          hipLaunchKernelGGL(k_gs_chol, dim3(1), dim3(1024), 0, st, (const double *)gp, nblk, nb, Ri);
+          hipLaunchKernelGGL(k_gs_apply, dim3((unsigned)nblk), dim3(256), 0, st, X, n, nb, (const double *)Ri);
         }
-        hipLaunchKernelGGL(k_gs_gram, dim3((unsigned)nblk), dim3(256), 0, st, (const double *)X, n, nb, gp);
-        hipLaunchKernelGGL(k_gs_chol, dim3(1), dim3(1024), 0, st, (const double *)gp, nblk, nb, Ri);
-        hipLaunchKernelGGL(k_gs_apply, dim3((unsigned)nblk), dim3(256), 0, st, X, n, nb, (const double *)Ri);
       }
     }
     EIG_HIP(ctx, hipGetLastError());
