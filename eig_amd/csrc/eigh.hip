@@ -6,8 +6,8 @@
 //     of the diagonal and every access is a contiguous 16-byte pair.  Each column c
 //     (panel position j) runs in two parts:
 //       symv : the reflector scalars of column c (dlarfg), then y = A_trail v
-//              with v rebuilt on the fly from the unscaled column x; per-block
-//              partial y.v;
+//              from the upper triangle, with v rebuilt on the fly from the
+//              unscaled column x; per-tile shares of y and of y.v;
 //       wcol : w = tau (y - V q - W p) + alpha v, where alpha = -tau/2 w.v is
 //              known up front from w.v = tau (y.v - 2 p.q); in the same pass the
 //              next row x = A[c+1] - (V W^T + W V^T)[c+1] and per-block partials
@@ -52,11 +52,11 @@ struct EigWs {
   double *d, *e, *e2, *tau;
   double *V, *W;  // n x kNB panel vectors (row-major)
   double *xtmp;   // current reflector column, unscaled (length lda, zero padded)
-  double *y;
+  double *yp;     // [tile][lda] shares of y = A v (k_symv)
   double *sc;
   double *part1;          // per-block partial dots of the back-transform
   double *pw;             // [2][maxw][kPW] column hand-off partials (by column parity)
-  double *ps;             // [maxblk] per-block y.v of the symv part
+  double *ps;             // per-block y.v of k_symv
   int32_t *sync;          // [1] set if a resident launch gave up waiting
   int32_t maxw;
   double *eval;           // ascending
@@ -220,138 +220,124 @@ __global__ __launch_bounds__(256) void k_col0(EigWs ws, int32_t n) {
   }
 }
 
-// ---------------------------------------------------------------- symv part
-constexpr int kSymvRows = 4;  // symv rows per block: 106 VGPRs, 4 waves/SIMD; 2 ms less
-                              // than 8 rows at n = 5,000
-__device__ inline void symv_part(const EigWs &ws, int32_t n, int32_t c, int32_t j, int32_t blk) {
-  constexpr int R = kSymvRows;
-  __shared__ double red[4][R];
-  __shared__ double sscale;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int32_t lda = ws.lda;
-  const int32_t r0 = c + 1 + blk * R;
-  // the block's own entries of x, for its rows of v at the end (loaded now, so no
-  // memory round trip follows the stream)
-  const double xown = (threadIdx.x < R && r0 + (int32_t)threadIdx.x < n) ? ws.xtmp[r0 + threadIdx.x] : 0.0;
-  const int32_t a0 = (c + 1) & ~1;
-  const int32_t npair = (((n + 1) & ~1) - a0) >> 1;
-  const double2 *xp = (const double2 *)(ws.xtmp + a0);
-  // rows past n read row r0 instead (in bounds, result discarded), so every load
-  // in the loop is unconditional and all of them are in flight together
-  const double2 *rp[R];
+// one of a pair of values by a lane bit, plus the other lane's other: a step of the
+// butterflies that transpose and sum.  Values, not elements of an array: a select between
+// array elements becomes one of their indices
+__device__ __forceinline__ double xpick(bool b, double x, double y, int o) {
+  return (b ? y : x) + xlane(b ? x : y, o);
+}
+// tile i of the upper triangle of an nt x nt grid, counted from the last row of tiles up:
+// the numbers of the tiles that are left stay the same as leading rows drop out
+__device__ __forceinline__ void upper_tile(int32_t i, int32_t nt, int32_t &I, int32_t &J) {
+  int32_t k = (int32_t)((sqrtf(8.0f * (float)i + 1.0f) - 1.0f) * 0.5f);
+  while ((k + 1) * (k + 2) / 2 <= i) ++k;
+  while (k * (k + 1) / 2 > i) --k;
+  I = nt - 1 - k;
+  J = I + (i - k * (k + 1) / 2);
+}
+
+// ---------------------------------------------------------------- k_symv
+// y = A v from the upper triangle alone, one block per kSyT x kSyT tile of a fixed grid:
+// tile (I, J) gives rows I their share of A v and, off the diagonal, rows J theirs of
+// A^T v.  Row r's shares stand at yp[K][r] for the tiles K = c+1's .. nt-1 that hold it
+// with its own, and k_wcol adds them in that order.  Bound by reading the triangle (from
+// the Infinity Cache: 6.5 TB/s); a pass over whole rows reads twice as much.  A wave takes
+// 32 rows by 128 columns, one 1 KB load per row, eight rows in flight while eight are
+// summed.  A tile keeps its number from column to column, and so its XCD.
+constexpr int kSyT = 128;
+__host__ __device__ inline int32_t symv_tiles(int32_t n, int32_t c) {
+  const int32_t k = (n + kSyT - 1) / kSyT - (c + 1) / kSyT;
+  return k * (k + 1) / 2;
+}
+template <bool kDiag>
+__device__ __forceinline__ double symv_rows8(const double2 (&a)[8], const double *sv, int32_t row,
+                                             int32_t col, double v0, double v1, double &c0,
+                                             double &c1) {
+  double p[8];
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr)
-    rp[rr] = (const double2 *)(ws.a + (int64_t)((r0 + rr) < n ? r0 + rr : r0) * lda + a0);
-  double acc[R];
-#pragma unroll
-  for (int rr = 0; rr < R; ++rr) acc[rr] = 0.0;
-  // the first pairs' loads go out before the reflector scalars are reduced
-  int32_t p = threadIdx.x;
-  double2 x0 = make_double2(0.0, 0.0), x1 = x0, a0v[R], a1v[R];
-  const bool two = p + 256 < npair;
-  if (two) {
-    x0 = xp[p];
-    x1 = xp[p + 256];
-#pragma unroll
-    for (int rr = 0; rr < R; ++rr) {
-      a0v[rr] = rp[rr][p];
-      a1v[rr] = rp[rr][p + 256];
+  for (int u = 0; u < 8; ++u) {
+    const double vr = sv[u];
+    double x = a[u].x, y = a[u].y, xc = x, yc = y;
+    if constexpr (kDiag) {  // the tile's own upper triangle; its diagonal counts once
+      x = col >= row + u ? x : 0.0;
+      y = col + 1 >= row + u ? y : 0.0;
+      xc = col > row + u ? x : 0.0;
+      yc = col + 1 > row + u ? y : 0.0;
     }
+    p[u] = fma(x, v0, y * v1);
+    c0 = fma(xc, vr, c0);
+    c1 = fma(yc, vr, c1);
   }
-  if (wv == 0) {
-    double tau, scale, beta;
-    col_scalars(ws, n, c, tau, scale, beta);
-    if (lane == 0) {
-      sscale = scale;
-      if (blk == 0) {
-        ws.e[c] = beta;
-        ws.e2[c] = beta * beta;
-        ws.tau[c] = tau;
-      }
-    }
-  }
-  __syncthreads();
-  const double scale = sscale;
-  // v: 0 up to column c, 1 at c+1, x*scale beyond (x is zero past n); only the
-  // first pair (p = 0) can hold columns <= c+1
-  auto vpair = [&](const double2 xx, int32_t pp, double &v0, double &v1) {
-    v0 = xx.x * scale;
-    v1 = xx.y * scale;
-    if (pp == 0) {
-      const int32_t s0 = a0;
-      v0 = (s0 <= c) ? 0.0 : ((s0 == c + 1) ? 1.0 : v0);
-      v1 = (s0 + 1 == c + 1) ? 1.0 : v1;
-    }
+  // lane l: row l % 8 over its group of eight lanes
+  const int lane = threadIdx.x & 63;
+  const bool b4 = (lane & 4) != 0, b2 = (lane & 2) != 0, b1 = (lane & 1) != 0;
+  const double q0 = xpick(b4, p[0], p[4], 4), q1 = xpick(b4, p[1], p[5], 4),
+               q2 = xpick(b4, p[2], p[6], 4), q3 = xpick(b4, p[3], p[7], 4);
+  return xpick(b1, xpick(b2, q0, q2, 2), xpick(b2, q1, q3, 2), 1);
+}
+__global__ __launch_bounds__(256, 4) void k_symv(EigWs ws, int32_t n, int32_t c, int32_t j) {
+  __shared__ __align__(16) double sv[2 * kSyT];  // v at the tile's rows, at its columns
+  __shared__ double srow[kSyT], scol[4][kSyT], red[4];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int32_t lda = ws.lda, nt = (n + kSyT - 1) / kSyT;
+  int32_t I, J;
+  upper_tile((int32_t)blockIdx.x, nt, I, J);
+  const bool diag = I == J;
+  // rows up to column c hold reflectors and rows past n nothing: they read a live row, and
+  // meet v = 0 or are not stored; columns past the padding read the row's last pair
+  const int32_t row = I * kSyT + 32 * wv, col = J * kSyT + 2 * lane;
+  const double *ac = ws.a + min(col, lda - 2);
+  double2 a[2][8];
+  auto load = [&](double2 (&d)[8], int32_t r) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      d[u] = *(const double2 *)(ac + (int64_t)min(max(r + u, c + 1), n - 1) * lda);
   };
-  for (bool have = two; have;) {
-    double v0, v1, w0, w1;
-    vpair(x0, p, v0, v1);
-    vpair(x1, p + 256, w0, w1);
-#pragma unroll
-    for (int rr = 0; rr < R; ++rr)
-      acc[rr] += (a0v[rr].x * v0 + a0v[rr].y * v1) + (a1v[rr].x * w0 + a1v[rr].y * w1);
-    p += 512;
-    have = p + 256 < npair;
-    if (have) {
-      x0 = xp[p];
-      x1 = xp[p + 256];
-#pragma unroll
-      for (int rr = 0; rr < R; ++rr) {
-        a0v[rr] = rp[rr][p];
-        a1v[rr] = rp[rr][p + 256];
-      }
-    }
+  load(a[0], row);
+  const int32_t own = t < kSyT ? I * kSyT + t : J * kSyT + (t - kSyT);
+  const double xo = ws.xtmp[min(own, n - 1)];
+  double tau, scale, beta;
+  col_scalars(ws, n, c, tau, scale, beta);
+  if (blockIdx.x == 0 && t == 0) {
+    ws.e[c] = beta;
+    ws.e2[c] = beta * beta;
+    ws.tau[c] = tau;
   }
-  if (p < npair) {
-    const double2 x0 = xp[p];
-    double2 a0v[R];
+  const double vo = own >= n || own <= c ? 0.0 : (own == c + 1 ? 1.0 : xo * scale);
+  sv[t] = vo;
+  __syncthreads();
+  const double2 vc = *(const double2 *)(sv + kSyT + 2 * lane);
+  double c0 = 0.0, c1 = 0.0, z[4];
 #pragma unroll
-    for (int rr = 0; rr < R; ++rr) a0v[rr] = rp[rr][p];
-    double v0, v1;
-    vpair(x0, p, v0, v1);
-#pragma unroll
-    for (int rr = 0; rr < R; ++rr) acc[rr] += a0v[rr].x * v0 + a0v[rr].y * v1;
-  }
-  // butterfly transpose-reduce of the R row sums: after the exchanges at offsets
-  // R/2, ..., 1 lane l holds row (l & (R-1)) summed over its group of R lanes; the
-  // exchanges at R, 2R, ..., 32 sum the groups
-#pragma unroll
-  for (int o = R / 2; o > 0; o >>= 1) {
-    const bool b = (lane & o) != 0;
-#pragma unroll
-    for (int k = 0; k < o; ++k) {
-      // values first: a select between array elements becomes one of their indices
-      const double x = acc[k], y = acc[k + o];
-      acc[k] = (b ? y : x) + xlane(b ? x : y, o);
-    }
+  for (int b = 0; b < 4; ++b) {
+    if (b < 3) load(a[(b + 1) & 1], row + 8 * (b + 1));
+    const double *vr = sv + 32 * wv + 8 * b;
+    z[b] = diag ? symv_rows8<true>(a[b & 1], vr, row + 8 * b, col, vc.x, vc.y, c0, c1)
+                : symv_rows8<false>(a[b & 1], vr, row + 8 * b, col, vc.x, vc.y, c0, c1);
   }
   {
-    double a = acc[0];
-#pragma unroll
-    for (int o = R; o < 64; o <<= 1) a += xlane(a, o);
-    if (lane < R) red[wv][lane] = a;
+    const bool b8 = (lane & 8) != 0, b16 = (lane & 16) != 0;
+    double y = xpick(b16, xpick(b8, z[0], z[1], 8), xpick(b8, z[2], z[3], 8), 16);
+    y += xlane(y, 32);
+    if (lane < 32) srow[32 * wv + lane] = y;
   }
+  scol[wv][2 * lane] = c0;
+  scol[wv][2 * lane + 1] = c1;
   __syncthreads();
-  // per row (lanes 0 .. R-1 of wave 0): y, v into V[j] and A[c], and the row's y.v;
-  // the block's y.v partial is their sum over the wave (a tree of R/2 .. 1 exchanges)
-  if (wv == 0) {
-    double val = 0.0;
-    if (lane < R) {
-      const int rr = lane;
-      const int32_t r = r0 + rr;
-      if (r < n) {
-        const double vr = (r == c + 1) ? 1.0 : xown * scale;
-        const double yr = (red[0][rr] + red[1][rr]) + (red[2][rr] + red[3][rr]);
-        val = yr * vr;
-        ws.y[r] = yr;
-        ws.V[(int64_t)r * kNB + j] = vr;
-        ws.a[(int64_t)c * lda + r] = vr;
-      }
+  const int i = t & (kSyT - 1);
+  const double cs = (scol[0][i] + scol[1][i]) + (scol[2][i] + scol[3][i]);
+  double y = t < kSyT ? srow[i] + (diag ? cs : 0.0) : (diag ? 0.0 : cs);
+  if (own > c && own < n && (t < kSyT || !diag)) {
+    ws.yp[(int64_t)(t < kSyT ? J : I) * lda + own] = y;
+    if (diag) {
+      ws.V[(int64_t)own * kNB + j] = vo;
+      ws.a[(int64_t)c * lda + own] = vo;
     }
-#pragma unroll
-    for (int o = R / 2; o > 0; o >>= 1) val += xlane(val, o);
-    if (lane == 0) ws.ps[blk] = val;
+  } else {
+    y = 0.0;
   }
+  y = block_sum(y * vo, red);
+  if (t == 0) ws.ps[blockIdx.x] = y;
 }
 
 // ---------------------------------------------------------------- wcol part
@@ -405,9 +391,14 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
     const int q = threadIdx.x & (kNB - 1);
     atc = (threadIdx.x < kNB) ? ws.V[(int64_t)c1 * kNB + q] : ws.W[(int64_t)c1 * kNB + q];
   }
-  double yy = ws.y[rs];
-  const double yc1 = ws.y[c1];
-  double yp[8];
+  // the row's shares of y, four threads taking every fourth, and row c+1's, a lane each
+  const int32_t nt = (n + kSyT - 1) / kSyT, i0 = c1 / kSyT;
+  double ly0[8], ly1[8], yp[8];
+  load8(ws.yp + rs, lda, i0 + sub, 4, nt, ly0);
+  load8(ws.yp + rs, lda, i0 + sub + 32, 4, nt, ly1);
+  double yc1 = ws.yp[(int64_t)min(i0 + lane, nt - 1) * lda + c1];
+  yc1 = i0 + lane < nt ? yc1 : 0.0;
+  for (int32_t b = i0 + lane + 64; b < nt; b += 64) yc1 += ws.yp[(int64_t)b * lda + c1];
   load8(ws.ps, 1, threadIdx.x, 256, nps, yp);
   double praw = 0.0;
   {
@@ -431,6 +422,11 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
                      tau, scale, beta);
   }
   double yv = sum_rest(ws.ps, 1, threadIdx.x, 256, nps, yp);
+  double yy = sum8(ly0) + sum_rest(ws.yp + rs, lda, i0 + sub + 32, 4, nt, ly1);
+  yy += xlane(yy, 1);
+  yy += xlane(yy, 2);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) yc1 += xlane(yc1, o);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) yv += xlane(yv, o);
   if (lane == 0) red[wv][0] = yv;
@@ -557,9 +553,6 @@ __device__ inline void wcol_part(const EigWs &ws, int32_t n, int32_t c, int32_t 
   }
 }
 
-__global__ __launch_bounds__(256) void k_symv(EigWs ws, int32_t n, int32_t c, int32_t j) {
-  symv_part(ws, n, c, j, (int32_t)blockIdx.x);
-}
 __global__ __launch_bounds__(256) void k_wcol(EigWs ws, int32_t n, int32_t c, int32_t j, int32_t nps) {
   wcol_part(ws, n, c, j, (int32_t)blockIdx.x, nps);
 }
@@ -602,7 +595,7 @@ __device__ __forceinline__ void s2_store(double (*sm)[kS2Ld], int32_t r0, int32_
   }
 }
 
-// One block per 64x64 tile.  The B operand rows [W_c | V_c] are staged in LDS; each
+// One block per 64x64 tile of the upper triangle (all that is read).  The B operand rows [W_c | V_c] are staged in LDS; each
 // lane's A operand stays in registers: the MFMA sums over k, so lane group g = lane / 16
 // takes k = 16 g + ks at step ks (in A and B alike), and its A entries are 16
 // consecutive doubles of a row of V (g < 2) or W.  33 KB of LDS and ~150 registers
@@ -610,7 +603,8 @@ __device__ __forceinline__ void s2_store(double (*sm)[kS2Ld], int32_t r0, int32_
 __global__ __launch_bounds__(256) void k_syr2k(EigWs ws, int32_t n, int32_t k0, int32_t nb) {
   __shared__ double sb[64][kS2Ld];
   const int32_t nt = (n - k0 + 63) / 64;
-  const int32_t tr = blockIdx.x / nt, tc = blockIdx.x % nt;
+  int32_t tr, tc;
+  upper_tile((int32_t)blockIdx.x, nt, tr, tc);
   const int32_t rb = k0 + tr * 64, cb = k0 + tc * 64;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wr = w >> 1, wc = w & 1, g = lane >> 4;
@@ -721,9 +715,6 @@ __device__ __forceinline__ double load_dev(const double *p) {
 // Sums over the wave of the row values that lanes hold, four rows at a time as they come
 // (few registers live at once), then over the groups: lane l ends with row l % R2's sum
 // (R2 = 8 or 16).  rows4 leaves row l % 4 summed over the lanes' groups of four.
-__device__ __forceinline__ double xpick(bool b, double x, double y, int o) {
-  return (b ? y : x) + xlane(b ? x : y, o);
-}
 __device__ __forceinline__ double rows4(const double (&v)[4]) {
   const int lane = threadIdx.x & 63;
   const bool b2 = (lane & 2) != 0, b1 = (lane & 1) != 0;
@@ -776,8 +767,9 @@ __global__ __launch_bounds__(T) void k_tri(EigWs ws, int32_t n, int32_t c0, int3
   for (int s = 0; s < RS; ++s)
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const double *p = A + (int64_t)min(r0 + s, nl - 1) * lda + T * k;
-      a[s][k] = (r0 + s < nl && t < nl - T * k) ? p[t] : 0.0;
+      const int32_t r = min(r0 + s, nl - 1), q = min(t + T * k, nl - 1);  // upper triangle
+      const double z = A[(int64_t)min(r, q) * lda + max(r, q)];
+      a[s][k] = (r0 + s < nl && t < nl - T * k) ? z : 0.0;
     }
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -1748,14 +1740,15 @@ static void launch_tridiag(EigWs ws, int32_t n, int32_t stop, hipStream_t st) {
   for (int32_t c = 0; c + 1 < n && c < stop; ++c) {
     const int32_t j = c % kNB;
     const int32_t L = n - c - 1;
-    const int32_t gs = (L + kSymvRows - 1) / kSymvRows, gw = (L + kWRows - 1) / kWRows;
+    const int32_t gs = symv_tiles(n, c), gw = (L + kWRows - 1) / kWRows;
     hipLaunchKernelGGL(k_symv, dim3((unsigned)gs), dim3(256), 0, st, ws, n, c, j);
     hipLaunchKernelGGL(k_wcol, dim3((unsigned)gw), dim3(256), 0, st, ws, n, c, j, gs);
     // panel end: update the trailing matrix before the next panel's first symv
     if (j == kNB - 1 && c + 2 < n) {
       const int32_t k1 = c + 1;
       const int32_t nt = (n - k1 + 63) / 64;
-      hipLaunchKernelGGL(k_syr2k, dim3((unsigned)(nt * nt)), dim3(256), 0, st, ws, n, k1, kNB);
+      hipLaunchKernelGGL(k_syr2k, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(256), 0, st, ws, n, k1,
+                         kNB);
     }
   }
 }
@@ -1839,7 +1832,7 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   auto tend = [&](const char *what) { if (!internal) eig_time_end(ctx, what); };
   const int64_t N = n;
   const int32_t lda = (int32_t)(((N + 7) / 8) * 8);
-  const int64_t maxblk = (N + kSymvRows - 1) / kSymvRows + 8;  // symv partials
+  const int64_t maxblk = (N + 3) / 4 + 8, ntile = (N + kSyT - 1) / kSyT;
   const int64_t maxnv = (int64_t)kNB * kMaxVec;
   const int64_t maxw = (N + kWRows - 1) / kWRows + 2;
   const int64_t npanel = (N + kNB - 1) / kNB + 1;
@@ -1850,12 +1843,12 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
     return o;
   };
   size_t o_a = add((size_t)N * lda), o_d = add(N), o_e = add(N), o_e2 = add(N),
-         o_tau = add(N), o_V = add(kNB * N), o_W = add(kNB * N), o_x = add(lda), o_y = add(N),
+         o_tau = add(N), o_V = add(kNB * N), o_W = add(kNB * N), o_x = add(lda), o_y = add((size_t)ntile * lda),
          o_sc = add(S_COUNT), o_p1 = add((size_t)maxblk * maxnv),
          o_ev = add(N),
          o_X = add((size_t)kMaxVec * N), o_lu = add((size_t)kMaxVec * kLuF * N),
          o_Z = add(kNB * kMaxVec), o_T = add((size_t)npanel * kNB * kNB),
-         o_pw = add((size_t)2 * maxw * kPW), o_ps = add((size_t)maxblk), o_sync = add(8);
+         o_pw = add((size_t)2 * maxw * kPW), o_ps = add((size_t)(ntile * (ntile + 1) / 2)), o_sync = add(8);
   EIG_TRY(eig_ensure(ctx, ctx->ework, need));
   char *base = (char *)ctx->ework.p;
   EigWs ws;
@@ -1868,7 +1861,7 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   ws.V = (double *)(base + o_V);
   ws.W = (double *)(base + o_W);
   ws.xtmp = (double *)(base + o_x);
-  ws.y = (double *)(base + o_y);
+  ws.yp = (double *)(base + o_y);
   ws.sc = (double *)(base + o_sc);
   ws.part1 = (double *)(base + o_p1);
   ws.eval = (double *)(base + o_ev);

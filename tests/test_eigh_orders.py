@@ -47,3 +47,10 @@ def test_orders(eng, n, kind):
     assert np.max(np.abs(w - ref)) <= tol * norm
     assert np.max(np.abs(v @ v.T - np.eye(nvec))) <= 8 * tol
     assert np.max(np.abs((v @ a - w[:nvec, None] * v) / norm)) <= tol
+
+
+@pytest.mark.parametrize("n", [2, 3, 31, 34, 127, 128, 129, 130, 161, 257, 385, 700])
+def test_launches_alone(eng, n, monkeypatch):
+    """the launches that longer columns take, at the edges of their 128-wide tiles"""
+    monkeypatch.setenv("EIG_NO_MERGE", "1")
+    test_orders(eng, n, "random")
