@@ -14,9 +14,8 @@
 //
 // The two panel products read X straight from packed codes: in the FP64 form as exact
 // integer products with fixed-point digits of the panel (codes.hip), in the split-BF16
-// form on BF16 MFMA (32x32x16) over hi/lo splits.  The BF16 instances of up to 32 columns
-// load each step's operands while the previous step's MFMAs run (two LDS buffers, one
-// barrier per step).  The tall-skinny Gram and basis products run on the library's FP64
+// form on BF16 MFMA (32x32x16) over hi/lo splits, each stage's operands loaded while the
+// previous stage's MFMAs run (two LDS buffers, one barrier per stage).  The tall-skinny Gram and basis products run on the library's FP64
 // MFMA GEMM (gemm.hip).
 
 #include <algorithm>
@@ -104,8 +103,7 @@ __global__ void k_fpca_reduce(const double *__restrict__ part, int32_t S, int64_
 // and the four products hi*hi, hi*lo, lo*hi, lo*lo run on v_mfma_f32_32x32x16_bf16,
 // in FP32 within a block of the reduction and promoted to FP64 across blocks (as
 // the split-BF16 XTX).  The genotype operand is decoded straight into MFMA operand
-// registers from LDS tables of level pairs; the dense panel is split once per
-// product into transposed bf16 hi / lo arrays.
+// registers; the dense panel is split once per product into hi / lo MFMA operands.
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float fp_f32x16;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 fp_bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t fp_u32x4;
@@ -120,189 +118,77 @@ __global__ void k_fpca_levbf(const double *__restrict__ lf, int64_t M, uint32_t 
   lb[e] = (uint32_t)hi | ((uint32_t)lo << 16);
 }
 
-// th/tl[c][r] = bf16 hi / lo of src[r * lds + c] for r < rows, c < C; zero up to
-// rpad rows and cpad columns (row stride of th/tl: rpad)
-__global__ void k_fpca_split_t(const double *__restrict__ src, int64_t rows, int64_t lds,
-                               int32_t C, int64_t rpad, int32_t cpad, uint16_t *__restrict__ th,
-                               uint16_t *__restrict__ tl) {
+// The dense panel src[k * lds + c] (k < rows, c < C; zero past them) as bf16 hi / lo MFMA
+// operands: column group cg of 32 CT columns, 16-row step s, 32-column tile ct and part hl
+// (0 hi, 1 lo) fill 1 KB at frag + (((cg nstep + s) CT + ct) 2 + hl) * 512, lane l's eight
+// values at 8 l: column l % 32, rows 8 (l / 32) + 0 .. 7.  A stage of the products is one
+// contiguous piece, staged and read without padding or bank conflicts.
+__global__ __launch_bounds__(256) void k_fpca_split(const double *__restrict__ src, int64_t rows,
+                                                    int64_t lds, int32_t C, int64_t nstep,
+                                                    int32_t CT, uint16_t *__restrict__ frag) {
   __shared__ double tile[32][33];
   const int64_t r0 = (int64_t)blockIdx.x * 32;
   const int32_t c0 = blockIdx.y * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 256 threads: 8 rows at a time
+  const int t = threadIdx.x, tx = t & 31, ty = t >> 5;  // 8 rows at a time
   for (int k = ty; k < 32; k += 8) {
     const int64_t r = r0 + k;
     const int32_t c = c0 + tx;
     tile[k][tx] = (r < rows && c < C) ? src[r * lds + c] : 0.0;
   }
   __syncthreads();
-  for (int k = ty; k < 32; k += 8) {
-    const int32_t c = c0 + k;
-    const int64_t r = r0 + tx;
-    if (c >= cpad || r >= rpad) continue;
-    const double v = tile[tx][k];
+  const int s = t >> 7, hl = (t >> 6) & 1, lane = t & 63, h = lane >> 5;
+  const int64_t step = 2 * (int64_t)blockIdx.x + s;
+  if (step >= nstep) return;
+  uint32_t o[4];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const double v = tile[16 * s + 8 * h + j][lane & 31];
     const uint16_t hi = eig_bf16_rne((float)v);
     const uint16_t lo = eig_bf16_rne((float)(v - (double)eig_bf16_to_f32(hi)));
-    th[(int64_t)c * rpad + r] = hi;
-    tl[(int64_t)c * rpad + r] = lo;
+    const uint32_t x = hl ? lo : hi;
+    o[j >> 1] = (j & 1) ? o[j >> 1] | (x << 16) : x;
   }
+  const int32_t cg = blockIdx.y / CT, ct = blockIdx.y % CT;
+  *(uint4 *)(frag + ((((int64_t)cg * nstep + step) * CT + ct) * 2 + hl) * 512 + lane * 8) =
+      make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// Y = X A.  Persistent over SNP tiles of 128 (4 waves x 32 SNPs); a wave's 32 SNPs x
-// 32CT columns accumulate in FP32 over blkt sample tiles, then in FP64.  The table of
-// SNP s (row s, stride 17 against bank conflicts) maps the codes c = code(2p) |
-// code(2p+1) << 2 of two consecutive samples to their two bf16 hi (table 0) or lo
-// (table 1) parts -- one dword of the operand.  Ah/Al: [column][sample], row stride ldt.
+// Y = X A.  Persistent over SNP tiles of 128 (4 waves x 32 SNPs); a wave's 32 SNPs x 32 CT
+// columns accumulate in FP32 over blkt sample tiles, then in FP64.  A lane of the genotype
+// operand is one SNP for the whole sum, so its four levels stay in registers and two codes
+// become an operand word by one v_perm_b32 each for hi and lo, with a selector both share:
+// no table, and LDS (128 bytes a cycle) carries the panel alone.  A table of level pairs in
+// LDS took eight lookups a step, as many LDS cycles as the step has MFMA cycles: at 100,000
+// x 500,000 and 20 columns 12.9 ms, now 11.0 (1.16 PFLOP/s; the matrix units are busy 61 % of
+// the cycles at the 1.8 GHz this load leaves, the decode's 26 VALU instructions a step the
+// rest).  Panel
+// stages of half a sample tile (four steps), global -> registers -> one of two LDS buffers,
+// one barrier per stage.
 template <int CT>
-__global__ __launch_bounds__(256, 2) void k_fpca_xa_bf16(
+__global__ __launch_bounds__(256, CT == 1 ? 4 : 2) void k_fpca_xa_bf16(
     const uint32_t *__restrict__ sel, int64_t M, int32_t nst, const uint32_t *__restrict__ lbf,
-    const uint16_t *__restrict__ Ah, const uint16_t *__restrict__ Al, int64_t ldt,
-    double *__restrict__ Y, int64_t ldy, int32_t C, int32_t blkt) {
-  // two tables 8708 bytes apart: no paired LDS load spans that, so every lookup
-  // lands in its operand register
-  __shared__ uint32_t tt[2][128 * 17 + 1];
-  __shared__ __attribute__((aligned(16))) uint16_t sA[2][32 * CT][128 + 8];
+    const uint16_t *__restrict__ frag, double *__restrict__ Y, int64_t ldy, int32_t C, int32_t blkt) {
+  constexpr int kPan = 512 * CT;  // 16-byte pieces of a stage's panel
+  __shared__ fp_u32x4 sA[2][kPan];
   const int t = threadIdx.x, w = t >> 6, lane = t & 63, h = lane >> 5, r = lane & 31;
   const int64_t ntiles = (M + 127) / 128;
+  const int32_t nstage = 2 * nst;
+  // rotations that bring the lane's eight codes down (codes 0, 2, 4, 6 at bits 0, 4, 8, 12)
+  // and the odd ones to bits 16, 20, 24, 28
+  const uint32_t rot0 = 16u * (uint32_t)h, rot1 = (18u + 16u * (uint32_t)h) & 31u;
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t mb = tile * 128;
-    __syncthreads();  // the previous tile's table reads are done
-    for (int e = t; e < 128 * 16; e += 256) {
-      const int sl = e >> 4, c = e & 15;
-      const int64_t m = mb + sl;
-      uint32_t e0 = 0u, e1 = 0u;
-      if (m < M) {
-        e0 = lbf[4 * m + (c & 3)];
-        e1 = lbf[4 * m + (c >> 2)];
-      }
-      tt[0][sl * 17 + c] = (e0 & 0xFFFFu) | (e1 << 16);
-      tt[1][sl * 17 + c] = (e0 >> 16) | (e1 & 0xFFFF0000u);
-    }
-    const int64_t m = mb + 32 * w + r;  // this lane's SNP
-    const uint32_t rowoff = (uint32_t)((32 * w + r) * 17);
-    fp_f32x16 acc[CT];
-    double dacc[CT][16];
+    const int64_t mb = tile * 128, m = mb + 32 * w + r;  // this lane's SNP
+    const int64_t mr = m < M ? m : M - 1;  // one past M reads SNP M-1's words, its levels are 0
+    fp_u32x4 lv = *(const fp_u32x4 *)(lbf + 4 * mr);
+    if (m >= M) lv = fp_u32x4{0u, 0u, 0u, 0u};
+    const uint32_t h01 = (lv[0] & 0xFFFFu) | (lv[1] << 16), h23 = (lv[2] & 0xFFFFu) | (lv[3] << 16);
+    const uint32_t l01 = (lv[0] >> 16) | (lv[1] & 0xFFFF0000u), l23 = (lv[2] >> 16) | (lv[3] & 0xFFFF0000u);
+    fp_u32x4 pa[2 * CT], wd;
+    auto fetch = [&](int32_t g) {
+      const fp_u32x4 *p = (const fp_u32x4 *)frag + (int64_t)g * kPan + t;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        acc[ct][q] = 0.f;
-        dacc[ct][q] = 0.0;
-      }
-    auto promote = [&]() {
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-          dacc[ct][q] += (double)acc[ct][q];
-          acc[ct][q] = 0.f;
-        }
-    };
-    int32_t left = blkt;
-    for (int32_t st = 0; st < nst; ++st) {
-      __syncthreads();  // the previous sample tile's panel reads are done
-      for (int q = t; q < 2 * 32 * CT * 16; q += 256) {
-        const int hl = q / (32 * CT * 16), rem = q % (32 * CT * 16), c = rem >> 4, ch = rem & 15;
-        const uint16_t *src = (hl ? Al : Ah) + (int64_t)c * ldt + (int64_t)st * kTileS + ch * 8;
-        *(uint4 *)&sA[hl][c][ch * 8] = *(const uint4 *)src;
-      }
-      uint32_t wd[8];
-      if (m < M) {
-        const uint4 a = *(const uint4 *)(sel + ((int64_t)st * M + m) * kTileWords);
-        const uint4 b = *(const uint4 *)(sel + ((int64_t)st * M + m) * kTileWords + 4);
-        wd[0] = a.x; wd[1] = a.y; wd[2] = a.z; wd[3] = a.w;
-        wd[4] = b.x; wd[5] = b.y; wd[6] = b.z; wd[7] = b.w;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) wd[j] = 0xFFFFFFFFu;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {  // 16-sample steps of the tile
-        const uint32_t bits = wd[j] >> (16 * h);
-        fp_u32x4 xh, xl;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t c = (bits >> (4 * q)) & 15u;
-          xh[q] = tt[0][rowoff + c];
-          xl[q] = tt[1][rowoff + c];
-        }
-        const fp_bf16x8 ah = __builtin_bit_cast(fp_bf16x8, xh), al = __builtin_bit_cast(fp_bf16x8, xl);
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          const fp_bf16x8 bh = *(const fp_bf16x8 *)&sA[0][32 * ct + r][16 * j + 8 * h];
-          const fp_bf16x8 bl = *(const fp_bf16x8 *)&sA[1][32 * ct + r][16 * j + 8 * h];
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bl, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc[ct], 0, 0, 0);
-        }
-      }
-      if (--left == 0) {
-        promote();
-        left = blkt;
-      }
-    }
-    promote();
-    // accumulator: lane l, element q -> row 8(q>>2) + 4(l>>5) + (q&3), column l&31
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int64_t row = mb + 32 * w + 8 * (q >> 2) + 4 * h + (q & 3);
-        const int col = 32 * ct + r;
-        if (row < M && col < C) Y[row * ldy + col] = dacc[ct][q];
-      }
-  }
-}
-
-// The same Y = X A with the next sample tile's panel and genotype words loaded
-// before the current tile's MFMAs: the panel goes global -> registers -> one of two
-// LDS buffers, one barrier per tile.  For CT == 1, whose two panel buffers fit
-// beside the tables at two blocks per CU.
-template <int CT>
-__global__ __launch_bounds__(256, 2) void k_fpca_xa_bf16_pf(
-    const uint32_t *__restrict__ sel, int64_t M, int32_t nst, const uint32_t *__restrict__ lbf,
-    const uint16_t *__restrict__ Ah, const uint16_t *__restrict__ Al, int64_t ldt,
-    double *__restrict__ Y, int64_t ldy, int32_t C, int32_t blkt) {
-  constexpr int kPE = 2 * 32 * CT * 16 / 256;  // panel uint4 per thread per tile
-  // tables entry-major (entry c of SNP s at c * 128 + s): the 32 lanes of a half-wave
-  // are 32 SNPs, so their lookups fall in 32 different banks whatever their codes; the
-  // two tables 8196 bytes apart, which no paired LDS load spans
-  __shared__ uint32_t tt[2][16 * 128 + 1];
-  __shared__ __attribute__((aligned(16))) uint16_t sA[2][2][32 * CT][128 + 8];  // [buf][hi/lo]
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63, h = lane >> 5, r = lane & 31;
-  const int64_t ntiles = (M + 127) / 128;
-  fp_u32x4 pa[kPE], wa, wb;
-  int buf = 0;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t mb = tile * 128;
-    __syncthreads();  // the previous tile's table reads are done
-    for (int e = t; e < 128 * 16; e += 256) {
-      const int sl = e & 127, c = e >> 7;
-      const int64_t m = mb + sl;
-      uint32_t e0 = 0u, e1 = 0u;
-      if (m < M) {
-        e0 = lbf[4 * m + (c & 3)];
-        e1 = lbf[4 * m + (c >> 2)];
-      }
-      tt[0][e] = (e0 & 0xFFFFu) | (e1 << 16);
-      tt[1][e] = (e0 >> 16) | (e1 & 0xFFFF0000u);
-    }
-    const int64_t m = mb + 32 * w + r;  // this lane's SNP
-    const uint32_t rowoff = (uint32_t)(32 * w + r);
-    auto fetch = [&](int32_t st) {
-#pragma unroll
-      for (int j = 0; j < kPE; ++j) {
-        const int q = t + 256 * j;
-        const int hl = q / (32 * CT * 16), rem = q % (32 * CT * 16), c = rem >> 4, ch = rem & 15;
-        pa[j] = *(const fp_u32x4 *)((hl ? Al : Ah) + (int64_t)c * ldt + (int64_t)st * kTileS + ch * 8);
-      }
-      // a SNP past M reads SNP M-1's words (in bounds) and takes all-missing codes
-      const uint32_t *ws = sel + ((int64_t)st * M + (m < M ? m : M - 1)) * kTileWords;
-      const fp_u32x4 x0 = *(const fp_u32x4 *)ws, x1 = *(const fp_u32x4 *)(ws + 4);
-      const fp_u32x4 none = {~0u, ~0u, ~0u, ~0u};
-      wa = m < M ? x0 : none;
-      wb = m < M ? x1 : none;
+      for (int j = 0; j < 2 * CT; ++j) pa[j] = p[256 * j];
+      wd = *((const fp_u32x4 *)(sel + ((int64_t)(g >> 1) * M + mr) * kTileWords) + (g & 1));
     };
     fp_f32x16 acc[CT];
     double dacc[CT][16];
@@ -323,34 +209,41 @@ __global__ __launch_bounds__(256, 2) void k_fpca_xa_bf16_pf(
         }
     };
     fetch(0);
-    int32_t left = blkt;
-    for (int32_t st = 0; st < nst; ++st) {
+    __syncthreads();  // the previous tile's panel reads are done
+    int32_t left = 2 * blkt;
+    int buf = 0;
+    for (int32_t g = 0; g < nstage; ++g) {
 #pragma unroll
-      for (int j = 0; j < kPE; ++j) {
-        const int q = t + 256 * j;
-        const int hl = q / (32 * CT * 16), rem = q % (32 * CT * 16), c = rem >> 4, ch = rem & 15;
-        *(fp_u32x4 *)&sA[buf][hl][c][ch * 8] = pa[j];
-      }
-      const fp_u32x4 ca = wa, cb = wb;  // this tile's words; wa, wb take the next tile's
+      for (int j = 0; j < 2 * CT; ++j) sA[buf][t + 256 * j] = pa[j];
+      const fp_u32x4 cw = wd;  // this stage's words; wd takes the next stage's
       // the other buffer was last read before this barrier's previous instance
       __syncthreads();
-      if (st + 1 < nst) fetch(st + 1);
+      if (g + 1 < nstage) fetch(g + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {  // 16-sample steps of the tile
-        const uint32_t bits = (j < 4 ? ca[j & 3] : cb[j & 3]) >> (16 * h);
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t x = cw[j];
+        // bytes: codes 0 | 2 << 4, 4 | 6 << 4, 1 | 3 << 4, 5 | 7 << 4 (and other bits)
+        const uint32_t p = (__builtin_amdgcn_alignbit(x, x, rot0) & 0xFFFFu) |
+                           (__builtin_amdgcn_alignbit(x, x, rot1) & 0xFFFF0000u);
+        // byte selectors 2 c and 2 c + 1 of codes 0, 4, 1, 5, then of 2, 6, 3, 7
+        const uint32_t a0 = (p << 1) & 0x06060606u, a1 = a0 | 0x01010101u;
+        const uint32_t b0 = (p >> 3) & 0x06060606u, b1 = b0 | 0x01010101u;
+        const uint32_t sl[4] = {__builtin_amdgcn_perm(a1, a0, 0x06020400u),
+                                __builtin_amdgcn_perm(b1, b0, 0x06020400u),
+                                __builtin_amdgcn_perm(a1, a0, 0x07030501u),
+                                __builtin_amdgcn_perm(b1, b0, 0x07030501u)};
         fp_u32x4 xh, xl;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const uint32_t c = (bits >> (4 * q)) & 15u;
-          xh[q] = tt[0][c * 128 + rowoff];
-          xl[q] = tt[1][c * 128 + rowoff];
+          xh[q] = __builtin_amdgcn_perm(h23, h01, sl[q]);
+          xl[q] = __builtin_amdgcn_perm(l23, l01, sl[q]);
         }
         const fp_bf16x8 ah = __builtin_bit_cast(fp_bf16x8, xh), al = __builtin_bit_cast(fp_bf16x8, xl);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-          const fp_bf16x8 bh = *(const fp_bf16x8 *)&sA[buf][0][32 * ct + r][16 * j + 8 * h];
-          const fp_bf16x8 bl = *(const fp_bf16x8 *)&sA[buf][1][32 * ct + r][16 * j + 8 * h];
+          const fp_bf16x8 bh = __builtin_bit_cast(fp_bf16x8, sA[buf][(j * CT + ct) * 128 + lane]);
+          const fp_bf16x8 bl = __builtin_bit_cast(fp_bf16x8, sA[buf][(j * CT + ct) * 128 + 64 + lane]);
           acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bl, acc[ct], 0, 0, 0);
           acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc[ct], 0, 0, 0);
           acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc[ct], 0, 0, 0);
@@ -359,7 +252,7 @@ __global__ __launch_bounds__(256, 2) void k_fpca_xa_bf16_pf(
       }
       if (--left == 0) {
         promote();
-        left = blkt;
+        left = 2 * blkt;
       }
       buf ^= 1;
     }
@@ -376,159 +269,142 @@ __global__ __launch_bounds__(256, 2) void k_fpca_xa_bf16_pf(
   }
 }
 
-// Partial X^T B.  Items (sample tile, SNP split, column group of 32 NCT); a block covers
-// one sample tile (4 waves x 32 samples) x 32 NCT columns over SNPs [s*mchunk, ...)
-// (mchunk a multiple of 64).  The genotype operand comes from the grouped layout through
-// per-group tables of level pairs (the split-BF16 XTX's scheme); the panel operand
-// from Bh/Bl [column][SNP] (row stride ldt >= 64 * ceil(M/64)), staged per group.
-// part[s][i][c] with row stride ldp.
+// Level tables of X^T B: per 64-SNP group 512 words of hi pairs, then 512 of lo pairs.  Word
+// ((s4 4 + q) 2 + h) 16 + c holds the levels of SNPs 16 s4 + 2 (4 h + q) + {0, 1} for codes
+// c & 3 and c >> 2, one dword of the operand (the split-BF16 XTX's scheme); zero past M.
 constexpr int kFpTab = 4 * 4 * 2 * 16;
+__global__ __launch_bounds__(256) void k_fpca_tab(const uint32_t *__restrict__ lbf, int64_t M, int64_t G64,
+                                                  uint32_t *__restrict__ tab) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t g = i / kFpTab;
+  if (g >= G64) return;
+  const int e = (int)(i % kFpTab);
+  const int s4 = e >> 7, q = (e >> 5) & 3, hh = (e >> 4) & 1, c = e & 15;
+  const int64_t m = g * kGrp + 16 * s4 + 2 * (4 * hh + q);
+  const uint32_t e0 = m < M ? lbf[4 * m + (c & 3)] : 0u;
+  const uint32_t e1 = m + 1 < M ? lbf[4 * (m + 1) + (c >> 2)] : 0u;
+  tab[2 * kFpTab * g + e] = (e0 & 0xFFFFu) | (e1 << 16);
+  tab[2 * kFpTab * g + kFpTab + e] = (e0 >> 16) | (e1 & 0xFFFF0000u);
+}
+
+// Partial X^T B.  One block per item (sample tile, SNP split, column group of 32 NCT): one
+// sample tile (4 waves x 32 samples) x 32 NCT columns over SNPs [s*mchunk, ...) (mchunk a
+// multiple of 64).  The genotype operand comes from the grouped layout by lookups in the
+// group's level table, the panel operand from frag (k_fpca_split's layout); table and panel
+// stage of a group go global -> registers -> one of two LDS buffers as they lie in memory,
+// one barrier per group: no address arithmetic or packing in the loop, five waves per SIMD
+// (32 columns) and three (64) instead of three and two.  At 100,000 x 500,000 12.3 -> 10.0 ms
+// with 20 columns, 62.7 -> 52.4 with 192 (1.47 PFLOP/s, the matrix units busy 69 % of the
+// cycles at 2 GHz).  part[s][i][c] with row stride ldp.
 template <int NCT>
-__global__ __launch_bounds__(256, 2) void k_fpca_xtb_bf16(
+__global__ __launch_bounds__(256, NCT == 1 ? 4 : 2) void k_fpca_xtb_bf16(
     const uint2 *__restrict__ selg, int64_t G64, int64_t M, int32_t nst,
-    const uint32_t *__restrict__ lbf, const uint16_t *__restrict__ Bh,
-    const uint16_t *__restrict__ Bl, int64_t ldt, int32_t ncg, int32_t S, int64_t mchunk,
+    const uint32_t *__restrict__ tabs, const uint16_t *__restrict__ frag, int32_t S, int64_t mchunk,
     int32_t blkg, double *__restrict__ part, int32_t ldp) {
-  __shared__ uint32_t tab[2][2][kFpTab + 1];  // [buf][hi/lo][entry], as the XTX kernel
-  constexpr int GW = 32 * NCT;  // columns per group
-  __shared__ __attribute__((aligned(16))) uint16_t sB[2][2][GW][64 + 8];  // [buf][hi/lo][col][snp]
+  constexpr int GW = 32 * NCT;          // columns per group
+  constexpr int kPan = 512 * NCT;       // 16-byte pieces of a group's panel
+  constexpr int kLo = kFpTab / 4 + 1;   // the lo table starts 2064 bytes on: no paired LDS load spans it
+  __shared__ fp_u32x4 sT[2][2 * kFpTab / 4 + 1], sB[2][kPan];
   const int t = threadIdx.x, w = t >> 6, lane = t & 63, h = lane >> 5, r = lane & 31;
-  const int64_t items = (int64_t)nst * S * ncg;
   const int64_t npad = (int64_t)nst * kTileS;
-  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
-    const int32_t st = (int32_t)(it % nst);
-    const int64_t rest = it / nst;
-    const int32_t s = (int32_t)(rest % S), cg = (int32_t)(rest / S);
-    const int64_t m_begin = (int64_t)s * mchunk;
-    const int64_t m_end = min(M, m_begin + mchunk);
-    if (m_begin >= m_end) {  // an empty split (M not filling S chunks): zero partial
-      double *out = part + ((int64_t)s * npad + (int64_t)st * kTileS) * ldp;
-      for (int e = t; e < kTileS * GW; e += 256) out[(int64_t)(e / GW) * ldp + GW * cg + e % GW] = 0.0;
-      continue;
-    }
-    const int32_t ng = (int32_t)((m_end - m_begin + kGrp - 1) / kGrp);
-    const int64_t g0 = m_begin / kGrp;
-    const uint2 *src = selg + (((int64_t)st * G64 + g0) * kTileS + 32 * w + r) * 2 + h;
-    auto lev_fetch = [&](int32_t gi, uint32_t (&lv)[4]) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int e = t + 256 * u;
-        const int s4 = e >> 7, q = (e >> 5) & 3, hh = (e >> 4) & 1, c = e & 15;
-        const int64_t m0 = m_begin + (int64_t)gi * kGrp + 16 * s4 + 2 * (4 * hh + q);
-        const uint32_t e0 = lbf[(m0 < m_end ? m0 : m_begin) * 4 + (c & 3)];
-        const uint32_t e1 = lbf[(m0 + 1 < m_end ? m0 + 1 : m_begin) * 4 + (c >> 2)];
-        lv[2 * u] = m0 < m_end ? e0 : 0u;
-        lv[2 * u + 1] = m0 + 1 < m_end ? e1 : 0u;
-      }
-    };
-    auto tab_store = [&](int buf, const uint32_t (&lv)[4]) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int e = t + 256 * u;
-        const uint32_t e0 = lv[2 * u], e1 = lv[2 * u + 1];
-        tab[buf][0][e] = (e0 & 0xFFFFu) | (e1 << 16);
-        tab[buf][1][e] = (e0 >> 16) | (e1 & 0xFFFF0000u);
-      }
-    };
-    // panel chunk of group gi: 2 x GW columns x 64 SNPs, 2 NCT uint4 per thread (hi and
-    // lo rows 32u + (t >> 3), u < NCT)
-    const int pc = t >> 3, pch = t & 7;
-    const uint16_t *ph0 = Bh + (int64_t)(GW * cg + pc) * ldt + m_begin + pch * 8;
-    const uint16_t *pl0 = Bl + (int64_t)(GW * cg + pc) * ldt + m_begin + pch * 8;
-    const int64_t p32 = 32 * ldt;
-    fp_u32x4 pvh[NCT], pvl[NCT];
-    auto pan_fetch = [&](int32_t gi) {
-      const int64_t o = (int64_t)gi * kGrp;
-#pragma unroll
-      for (int u = 0; u < NCT; ++u) {
-        pvh[u] = *(const fp_u32x4 *)(ph0 + u * p32 + o);
-        pvl[u] = *(const fp_u32x4 *)(pl0 + u * p32 + o);
-      }
-    };
-    auto pan_store = [&](int buf) {
-#pragma unroll
-      for (int u = 0; u < NCT; ++u) {
-        *(fp_u32x4 *)&sB[buf][0][32 * u + pc][pch * 8] = pvh[u];
-        *(fp_u32x4 *)&sB[buf][1][32 * u + pc][pch * 8] = pvl[u];
-      }
-    };
-    fp_f32x16 acc[NCT];
-    double dacc[NCT][16];
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        acc[ct][q] = 0.f;
-        dacc[ct][q] = 0.0;
-      }
-    auto promote = [&]() {
-#pragma unroll
-      for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-          dacc[ct][q] += (double)acc[ct][q];
-          acc[ct][q] = 0.f;
-        }
-    };
-    uint32_t lv[4];
-    uint2 cur = src[0], nxt = cur;
-    __syncthreads();  // the previous item's reads of tab and sB are done
-    lev_fetch(0, lv);
-    pan_fetch(0);
-    tab_store(0, lv);
-    pan_store(0);
-    __syncthreads();
-    int32_t left = blkg;
-    for (int32_t gi = 0; gi < ng; ++gi) {
-      const int buf = gi & 1;
-      const int32_t gn = gi + 1 < ng ? gi + 1 : gi;  // the last group loads itself again
-      const uint32_t *th = tab[buf][0], *tl = tab[buf][1];
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        if (s4 == 0) {
-          lev_fetch(gn, lv);
-          pan_fetch(gn);
-          nxt = src[(int64_t)gn * (2 * kTileS)];
-        }
-        const uint32_t word = (s4 < 2) ? cur.x : cur.y;
-        fp_u32x4 xh, xl;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t c = (word >> (16 * (s4 & 1) + 4 * q)) & 15u;
-          const uint32_t idx = (uint32_t)(((s4 * 4 + q) * 2) * 16) + 16u * (uint32_t)h + c;
-          xh[q] = th[idx];
-          xl[q] = tl[idx];
-        }
-        const fp_bf16x8 ah = __builtin_bit_cast(fp_bf16x8, xh), al = __builtin_bit_cast(fp_bf16x8, xl);
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-          const fp_bf16x8 bh = *(const fp_bf16x8 *)&sB[buf][0][32 * ct + r][16 * s4 + 8 * h];
-          const fp_bf16x8 bl = *(const fp_bf16x8 *)&sB[buf][1][32 * ct + r][16 * s4 + 8 * h];
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bl, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc[ct], 0, 0, 0);
-        }
-      }
-      if (--left == 0) {
-        promote();
-        left = blkg;
-      }
-      tab_store(buf ^ 1, lv);
-      pan_store(buf ^ 1);
-      cur = nxt;
-      __syncthreads();
-    }
-    promote();
-    double *out = part + ((int64_t)s * npad + (int64_t)st * kTileS) * ldp;
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int row = 32 * w + 8 * (q >> 2) + 4 * h + (q & 3);
-        out[(int64_t)row * ldp + GW * cg + 32 * ct + r] = dacc[ct][q];
-      }
+  const int64_t it = blockIdx.x;
+  const int32_t st = (int32_t)(it % nst);
+  const int64_t rest = it / nst;
+  const int32_t s = (int32_t)(rest % S), cg = (int32_t)(rest / S);
+  const int64_t m_begin = (int64_t)s * mchunk;
+  const int64_t m_end = min(M, m_begin + mchunk);
+  double *out = part + ((int64_t)s * npad + (int64_t)st * kTileS) * ldp;
+  if (m_begin >= m_end) {  // an empty split (M not filling S chunks): zero partial
+    for (int e = t; e < kTileS * GW; e += 256) out[(int64_t)(e / GW) * ldp + GW * cg + e % GW] = 0.0;
+    return;
   }
+  const int32_t ng = (int32_t)((m_end - m_begin + kGrp - 1) / kGrp);
+  const int64_t g0 = m_begin / kGrp;
+  const uint2 *src = selg + (((int64_t)st * G64 + g0) * kTileS + 32 * w + r) * 2 + h;
+  const fp_u32x4 *tsrc = (const fp_u32x4 *)tabs + g0 * 256 + t;
+  const fp_u32x4 *psrc = (const fp_u32x4 *)frag + ((int64_t)cg * G64 + g0) * kPan + t;
+  const int tdst = t < 128 ? t : t + 1;
+  fp_u32x4 tv, pv[2 * NCT];
+  auto fetch = [&]() {
+    tv = *tsrc;
+#pragma unroll
+    for (int u = 0; u < 2 * NCT; ++u) pv[u] = psrc[256 * u];
+  };
+  auto store = [&](int buf) {
+    sT[buf][tdst] = tv;
+#pragma unroll
+    for (int u = 0; u < 2 * NCT; ++u) sB[buf][t + 256 * u] = pv[u];
+  };
+  fp_f32x16 acc[NCT];
+  double dacc[NCT][16];
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      acc[ct][q] = 0.f;
+      dacc[ct][q] = 0.0;
+    }
+  auto promote = [&]() {
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        dacc[ct][q] += (double)acc[ct][q];
+        acc[ct][q] = 0.f;
+      }
+  };
+  uint2 cur = src[0], nxt;
+  fetch();
+  store(0);
+  __syncthreads();
+  int32_t left = blkg;
+  for (int32_t gi = 0; gi < ng; ++gi) {
+    const int buf = gi & 1;
+    if (gi + 1 < ng) {  // the last group loads itself again
+      src += 2 * kTileS;
+      tsrc += 256;
+      psrc += kPan;
+    }
+    nxt = *src;
+    fetch();
+    const uint32_t *th = (const uint32_t *)&sT[buf][0] + 16 * h, *tl = (const uint32_t *)&sT[buf][kLo] + 16 * h;
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {
+      const uint32_t word = (s4 < 2) ? cur.x : cur.y;
+      fp_u32x4 xh, xl;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t c = (word >> (16 * (s4 & 1) + 4 * q)) & 15u;
+        xh[q] = th[(s4 * 4 + q) * 32 + c];
+        xl[q] = tl[(s4 * 4 + q) * 32 + c];
+      }
+      const fp_bf16x8 ah = __builtin_bit_cast(fp_bf16x8, xh), al = __builtin_bit_cast(fp_bf16x8, xl);
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct) {
+        const fp_bf16x8 bh = __builtin_bit_cast(fp_bf16x8, sB[buf][(s4 * NCT + ct) * 128 + lane]);
+        const fp_bf16x8 bl = __builtin_bit_cast(fp_bf16x8, sB[buf][(s4 * NCT + ct) * 128 + 64 + lane]);
+        acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bl, acc[ct], 0, 0, 0);
+        acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc[ct], 0, 0, 0);
+        acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc[ct], 0, 0, 0);
+        acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc[ct], 0, 0, 0);
+      }
+    }
+    if (--left == 0) {
+      promote();
+      left = blkg;
+    }
+    store(buf ^ 1);
+    cur = nxt;
+    __syncthreads();
+  }
+  promote();
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int row = 32 * w + 8 * (q >> 2) + 4 * h + (q & 3);
+      out[(int64_t)row * ldp + GW * cg + 32 * ct + r] = dacc[ct][q];
+    }
 }
 
 // ---------------------------------------------------------------- Jacobi
@@ -868,37 +744,39 @@ __global__ void k_scale_cols(double *__restrict__ V, int32_t n, int32_t r,
   V[idx] *= s[idx / n];
 }
 
-// X A in the split-BF16 form: A (npad x lda, rows = samples) split into th/tl
-// [cxa][npad], then the persistent product into Y (rows = SNPs, ld ldy)
-static int launch_xa_bf16(eig_ctx *ctx, const Plan &P, const uint32_t *lbf, uint16_t *th,
-                          uint16_t *tl, int32_t cxa, const double *A, int32_t lda, double *Y,
-                          int64_t ldy, int32_t C, int grid, hipStream_t st) {
-  hipLaunchKernelGGL(k_fpca_split_t, dim3((unsigned)(P.npad / 32), (unsigned)(cxa / 32)),
-                     dim3(256), 0, st, A, (int64_t)P.npad, (int64_t)lda, C, (int64_t)P.npad, cxa,
-                     th, tl);
-  if (cxa == 32)
-    hipLaunchKernelGGL(k_fpca_xa_bf16_pf<1>, dim3(grid), dim3(256), 0, st, P.sel, P.M, P.nst, lbf,
-                       (const uint16_t *)th, (const uint16_t *)tl, (int64_t)P.npad, Y, ldy, C, 4);
-  else
-    hipLaunchKernelGGL(k_fpca_xa_bf16<2>, dim3(grid), dim3(256), 0, st, P.sel, P.M, P.nst, lbf,
-                       (const uint16_t *)th, (const uint16_t *)tl, (int64_t)P.npad, Y, ldy, C, 4);
+// X A in the split-BF16 form: A (npad x lda, rows = samples) split into the operands of
+// cxa columns, then the persistent product into Y (rows = SNPs, ld ldy)
+static int launch_xa_bf16(eig_ctx *ctx, const Plan &P, const uint32_t *lbf, uint16_t *frag,
+                          int32_t cxa, const double *A, int32_t lda, double *Y, int64_t ldy, int32_t C,
+                          hipStream_t st) {
+  const int CT = cxa / 32;
+  hipLaunchKernelGGL(k_fpca_split, dim3((unsigned)(P.npad / 32), (unsigned)CT), dim3(256), 0, st, A,
+                     (int64_t)P.npad, (int64_t)lda, C, (int64_t)P.npad / 16, CT, frag);
+  // four blocks a CU with 32 columns, two with 64 (their registers)
+  const int64_t grid =
+      std::min<int64_t>((P.M + 127) / 128, (int64_t)(CT == 1 ? 4 : 2) * std::max(ctx->num_cu, 1));
+  hipLaunchKernelGGL((CT == 1 ? k_fpca_xa_bf16<1> : k_fpca_xa_bf16<2>), dim3((unsigned)grid), dim3(256),
+                     0, st, P.sel, P.M, P.nst, lbf, (const uint16_t *)frag, Y, ldy, C, 4);
   EIG_HIP(ctx, hipGetLastError());
   return EIG_OK;
 }
 
-// scale * X^T B in the split-BF16 form: B (M x ldb, rows = SNPs) split into th/tl
-// [64 ncg][Mpad]; the SNP range is cut into S chunks (multiples of 64) chosen like the
-// XTX's split count; the partials are summed in split order into out (ld ldo)
-static int launch_xtb_bf16(eig_ctx *ctx, const Plan &P, const uint2 *selg, const uint32_t *lbf,
-                           uint16_t *th, uint16_t *tl, int64_t Mpad, const double *B, int64_t ldb,
-                           int32_t C, double *part, size_t part_doubles, double *out, int32_t ldo,
-                           double scale, const int64_t slots[2], hipStream_t st) {
+// scale * X^T B in the split-BF16 form: B (M x ldb, rows = SNPs) split into the operands of
+// its column groups; the SNP range is cut into S chunks (multiples of 64); the partials are
+// summed in split order into out (ld ldo).  The result's rounding depends on the chunks, so
+// they follow a fixed number of blocks per CU (three of 32 columns, two of 64), not the
+// kernels' occupancy.
+static int launch_xtb_bf16(eig_ctx *ctx, const Plan &P, const uint2 *selg, const uint32_t *tabs,
+                           uint16_t *frag, int64_t Mpad, const double *B, int64_t ldb, int32_t C,
+                           double *part, size_t part_doubles, double *out, int32_t ldo, double scale,
+                           hipStream_t st) {
   // 32-column groups for a panel of up to 32 columns (the power iteration's at L <= 32),
   // else 64-column groups, which decode X^T once per 64 columns
   const int nct = C <= 32 ? 1 : 2, gw = 32 * nct;
   const int32_t ncg = (C + gw - 1) / gw, cp = gw * ncg;
-  hipLaunchKernelGGL(k_fpca_split_t, dim3((unsigned)(Mpad / 32), (unsigned)(cp / 32)), dim3(256),
-                     0, st, B, P.M, ldb, C, Mpad, cp, th, tl);
+  const int64_t slots = (int64_t)(nct == 1 ? 3 : 2) * std::max(ctx->num_cu, 1);
+  hipLaunchKernelGGL(k_fpca_split, dim3((unsigned)(Mpad / 32), (unsigned)(cp / 32)), dim3(256), 0, st, B,
+                     P.M, ldb, C, Mpad / 16, nct, frag);
   const int64_t G64 = Mpad / kGrp;
   const int64_t smax = std::max<int64_t>(
       1, std::min<int64_t>({64, G64, (int64_t)(part_doubles / ((size_t)P.npad * cp))}));
@@ -909,7 +787,7 @@ static int launch_xtb_bf16(eig_ctx *ctx, const Plan &P, const uint2 *selg, const
     c = ((c + kGrp - 1) / kGrp) * kGrp;
     const int64_t ns = (P.M + c - 1) / c;
     if (ns != sp) continue;
-    const double rounds = (double)((P.nst * ns * ncg + slots[nct - 1] - 1) / slots[nct - 1]);
+    const double rounds = (double)((P.nst * ns * ncg + slots - 1) / slots);
     const double cost = rounds * (double)c / (double)P.M + 0.001 * (double)ns;
     if (best < 0.0 || cost < best - 1e-12) {
       best = cost;
@@ -918,15 +796,9 @@ static int launch_xtb_bf16(eig_ctx *ctx, const Plan &P, const uint2 *selg, const
     }
   }
   const int64_t items = (int64_t)P.nst * nsplit * ncg;
-  const unsigned grid = (unsigned)std::min<int64_t>(items, slots[nct - 1]);
-  if (nct == 1)
-    hipLaunchKernelGGL(k_fpca_xtb_bf16<1>, dim3(grid), dim3(256), 0, st, selg, G64, P.M, P.nst,
-                       lbf, (const uint16_t *)th, (const uint16_t *)tl, Mpad, ncg, (int32_t)nsplit,
-                       chunk, 8, part, cp);
-  else
-    hipLaunchKernelGGL(k_fpca_xtb_bf16<2>, dim3(grid), dim3(256), 0, st, selg, G64, P.M, P.nst,
-                       lbf, (const uint16_t *)th, (const uint16_t *)tl, Mpad, ncg, (int32_t)nsplit,
-                       chunk, 8, part, cp);
+  hipLaunchKernelGGL((nct == 1 ? k_fpca_xtb_bf16<1> : k_fpca_xtb_bf16<2>), dim3((unsigned)items), dim3(256),
+                     0, st, selg, G64, P.M, P.nst, tabs, (const uint16_t *)frag, (int32_t)nsplit, chunk, 8,
+                     part, cp);
   const int64_t tot = (int64_t)P.npad * cp;
   hipLaunchKernelGGL(k_fpca_reduce, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st,
                      (const double *)part, (int32_t)nsplit, (int64_t)P.npad, cp, scale, out, ldo);
@@ -987,12 +859,14 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   const size_t o_cb = add(sizeof(double) * kJacMax * kJacMax);
   const size_t o_ev = add(sizeof(double) * (size_t)K * npad);
   // split-BF16 form: levels, the X A panel (32 * ceil(L/32) columns) and the X^T B
-  // panel (up to 64 * ceil(C/64) columns, C <= (I+1)L) as transposed bf16 hi / lo
+  // panel (up to 64 * ceil(C/64) columns, C <= (I+1)L) as bf16 hi / lo operands, X^T B's
+  // level tables
   const int64_t Mpad = ((M + kGrp - 1) / kGrp) * kGrp;
   const int32_t cxa = 32 * ((L + 31) / 32), cxb = 64 * ((Ctot + 63) / 64);
   const size_t o_lbf = bf ? add(sizeof(uint32_t) * 4 * M) : 0;
   const size_t o_ta = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxa * npad) : 0;
   const size_t o_tb = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxb * Mpad) : 0;
+  const size_t o_tab = bf ? add(sizeof(uint32_t) * 2 * kFpTab * (size_t)(Mpad / kGrp)) : 0;
   // FP64 form: the code products' digit operands and INT32 sums (codes.hip), one area for
   // the X A, X^T B and finishing X^T U products
   if (!bf) EIG_TRY(eig_ensure_selg(ctx));
@@ -1027,9 +901,8 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   double *Cb = (double *)(base + o_cb);
   const size_t part_doubles = (size_t)Smax * npad * 16 * kMaxCT;
   uint32_t *lbf = bf ? (uint32_t *)(base + o_lbf) : nullptr;
-  uint16_t *tah = bf ? (uint16_t *)(base + o_ta) : nullptr, *tal = tah ? tah + (size_t)cxa * npad : nullptr;
-  uint16_t *tbh = bf ? (uint16_t *)(base + o_tb) : nullptr, *tbl = tbh ? tbh + (size_t)cxb * Mpad : nullptr;
-
+  uint16_t *fa = bf ? (uint16_t *)(base + o_ta) : nullptr, *fb = bf ? (uint16_t *)(base + o_tb) : nullptr;
+  uint32_t *tabs = bf ? (uint32_t *)(base + o_tab) : nullptr;
 
   eig_time_begin(ctx);
   hipLaunchKernelGGL(k_fpca_levels, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, st,
@@ -1048,22 +921,13 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   }
   EIG_HIP(ctx, hipGetLastError());
   Plan P{M, nst, npad, (const uint32_t *)ctx->sel.p, lf};
-  int64_t bslots[2] = {0, 0};  // resident X^T B blocks, 32- and 64-column groups
-  int bxa_grid = 0;
   if (bf) {
     hipLaunchKernelGGL(k_fpca_levbf, dim3((unsigned)((4 * M + 255) / 256)), dim3(256), 0, st,
                        (const double *)lf, M, lbf);
+    hipLaunchKernelGGL(k_fpca_tab, dim3((unsigned)(G64 * (kFpTab / 256))), dim3(256), 0, st,
+                       (const uint32_t *)lbf, M, G64, tabs);
     EIG_HIP(ctx, hipGetLastError());
     EIG_TRY(eig_ensure_selg(ctx));
-    int occ = 0;
-    EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_fpca_xtb_bf16<1>, 256, 0));
-    bslots[0] = (int64_t)std::max(occ, 1) * std::max(ctx->num_cu, 1);
-    occ = 0;
-    EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_fpca_xtb_bf16<2>, 256, 0));
-    bslots[1] = (int64_t)std::max(occ, 1) * std::max(ctx->num_cu, 1);
-    occ = 0;
-    EIG_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_fpca_xa_bf16<2>, 256, 0));
-    bxa_grid = (int)std::min<int64_t>((M + 127) / 128, (int64_t)std::max(occ, 1) * ctx->num_cu);
   }
   // X A and X^T B of the FP64 form: `plan`'s product of the codes with cols, its INT32 sums
   // left in the work area
@@ -1083,15 +947,15 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   };
   auto xa = [&](const double *A_, double *Y_) -> int {
     if (bf)
-      return launch_xa_bf16(ctx, P, lbf, tah, tal, cxa, A_, lda, Y_, ldq, L, bxa_grid, st);
+      return launch_xa_bf16(ctx, P, lbf, fa, cxa, A_, lda, Y_, ldq, L, st);
     EIG_TRY(code_mul(pa, vm, CodeCols{kColPanel, A_, lda, n}));
     return eig_codes_out_pair(ctx, pa, M, cw, cw + pa.head_bytes + up(pa.dig_bytes), lf, nullptr, 1.0,
                               Y_, ldq, 1, st);
   };
   auto xtb = [&](const double *B_, double *out_) -> int {
     if (bf)
-      return launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, lbf, tbh, tbl, Mpad, B_, ldq, L,
-                             part, part_doubles, out_, lda, 1.0 / (double)ncols, bslots, st);
+      return launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, tabs, fb, Mpad, B_, ldq, L,
+                             part, part_doubles, out_, lda, 1.0 / (double)ncols, st);
     return code_xtb(pb, B_, 1.0 / (double)ncols, out_, lda, lda);
   };
   // ---- power iterations
@@ -1186,12 +1050,11 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
     const int32_t rem = r % 64;
     const int32_t r64 = (rem != 0 && rem <= 32 && r - rem + 32 <= ldq) ? r - rem : r;
     if (r64 > 0)
-      EIG_TRY(launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, lbf, tbh, tbl, Mpad, src, ldq,
-                              r64, part, part_doubles, Bm, (int32_t)ldq, 1.0, bslots, st));
+      EIG_TRY(launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, tabs, fb, Mpad, src, ldq,
+                              r64, part, part_doubles, Bm, (int32_t)ldq, 1.0, st));
     if (r64 < r)
-      EIG_TRY(launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, lbf, tbh, tbl, Mpad, src + r64,
-                              ldq, r - r64, part, part_doubles, Bm + r64, (int32_t)ldq, 1.0, bslots,
-                              st));
+      EIG_TRY(launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, tabs, fb, Mpad, src + r64,
+                              ldq, r - r64, part, part_doubles, Bm + r64, (int32_t)ldq, 1.0, st));
   } else {
     // the plan made for every column serves a basis of fewer (r <= Ctot): the missing
     // ones have no digits
