@@ -144,6 +144,12 @@ int eig_gemm_f64(eig_ctx *ctx, hipStream_t st, bool ta, bool tb, int64_t m, int6
                  double alpha, const double *A, int64_t lda, int64_t sA, const double *B,
                  int64_t ldb, int64_t sB, double beta, double *C, int64_t ldc, int64_t sC,
                  int32_t batch, bool lower = false);
+// the same product with k cut into parts where its tiles are few; part: room for the parts'
+// m x n results (part_doubles of them; parts that do not fit are not made)
+int eig_gemm_f64_long(eig_ctx *ctx, hipStream_t st, bool ta, bool tb, int64_t m, int64_t n, int64_t k,
+                      double alpha, const double *A, int64_t lda, const double *B, int64_t ldb,
+                      double beta, double *C, int64_t ldc, bool lower, double *part,
+                      size_t part_doubles);
 
 // lsqproject's population fill table (usepopsformissing) from the loaded genotypes and
 // the current ignore mask: types itype[q] (nind host entries, < 0 = none), npop types,

@@ -1388,48 +1388,63 @@ __global__ __launch_bounds__(256) void k_gs_gram(const double *__restrict__ X, i
     sx[v][i] = (v < nb && r0 + i < n) ? X[(int64_t)v * n + r0 + i] : 0.0;
   }
   __syncthreads();
-  const int v0 = (t >> 4) * 4, u0 = (t & 15) * 4;
+  // 16 apart, so that the 16 lanes of a row of products read different banks
+  const int v0 = t >> 4, u0 = t & 15;
   double g[4][4] = {};
+#pragma unroll 4
   for (int i = 0; i < kGsRows; ++i)
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) g[a][b] += sx[v0 + a][i] * sx[u0 + b][i];
+      for (int b = 0; b < 4; ++b) g[a][b] += sx[v0 + 16 * a][i] * sx[u0 + 16 * b][i];
   double *out = part + (int64_t)blockIdx.x * kMaxVec * kMaxVec;
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) out[(v0 + a) * kMaxVec + u0 + b] = g[a][b];
+    for (int b = 0; b < 4; ++b) out[(v0 + 16 * a) * kMaxVec + u0 + 16 * b] = g[a][b];
 }
 // Rinv (upper triangular, [u][v]) from the nblk partial Gram matrices, summed in order.
 // A vector that depends on the earlier ones to rounding gets a pivot of at least 1e-30 of
 // its square norm, so that the factor stays finite.
 __global__ __launch_bounds__(1024) void k_gs_chol(const double *__restrict__ part, int32_t nblk,
                                                   int32_t nb, double *__restrict__ Rinv) {
-  __shared__ double G[kMaxVec][kMaxVec + 1], E[kMaxVec][kMaxVec + 1], d0[kMaxVec], d[kMaxVec];
-  const int t = threadIdx.x, c = t & 63, q = t >> 6;
+  __shared__ double row[2][kMaxVec], mul[2][kMaxVec], d0[kMaxVec], d[kMaxVec];
+  const int c = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // rows q, q + 16, .. of column c: of G right of the column being eliminated, of the
+  // inverse up to it
+  double x[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+  for (int32_t b = 0; b < nblk; ++b)
 #pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    const int r = q + 16 * h;
-    G[r][c] = sum_strided(part + r * kMaxVec + c, kMaxVec * kMaxVec, 0, 1, nblk);
-    E[r][c] = r == c ? 1.0 : 0.0;
-    if (r == c) d0[r] = G[r][c];
-  }
+    for (int h = 0; h < 4; ++h) x[h] += part[((int64_t)b * kMaxVec + q + 16 * h) * kMaxVec + c];
+#pragma unroll
+  for (int h = 0; h < 4; ++h)
+    if (c == q + 16 * h) d0[c] = x[h];
+  // the owners (a wave) of row k leave it in LDS, and its multipliers: G stays symmetric, so
+  // the row over the pivot is the column of multipliers too
+  auto emit = [&](int k, double v) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), k);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), k);
+    const double dk = fmax(__hiloint2double(hi, lo), 1e-30 * d0[k]);
+    row[k & 1][c] = v;
+    mul[k & 1][c] = v * rcp_nr(dk);
+    if (c == 0) d[k] = dk;
+  };
   __syncthreads();
-  // elimination of [G | I] without square roots: step k changes the rows below k only,
-  // right of column k in G and up to column k in the inverse, so one barrier a step
-  // separates it from the next (54 us; a Cholesky factor and a back substitution took 103)
+  if (q == 0) emit(0, x[0]);
+  __syncthreads();
+  // elimination of [G | I] without square roots: step k changes the rows below k only, by
+  // row k: one barrier a step (30 us at 19 parts; G and the inverse in LDS took 54, a
+  // Cholesky factor and a back substitution 103)
   for (int k = 0; k < nb; ++k) {
-    const double dk = fmax(G[k][k], 1e-30 * d0[k]);
-    if (t == 0) d[k] = dk;
-    const double gk = G[k][c], ek = E[k][c], rk = 1.0 / dk;
+    const double gc = row[k & 1][c];
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
       const int r = q + 16 * h;
       if (r > k) {
-        const double m = G[r][k] * rk;
-        if (c > k) G[r][c] -= m * gk;
-        else E[r][c] -= m * ek;
+        const double m = mul[k & 1][r];
+        x[h] = c == k ? -m : x[h] - m * gc;
+        if (r == k + 1) emit(r, x[h]);
       }
     }
     __syncthreads();
@@ -1438,7 +1453,7 @@ __global__ __launch_bounds__(1024) void k_gs_chol(const double *__restrict__ par
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
     const int v = q + 16 * h;
-    Rinv[c * kMaxVec + v] = (v < nb && c <= v) ? E[v][c] / sqrt(d[v]) : 0.0;
+    Rinv[c * kMaxVec + v] = (v < nb && c <= v) ? (c == v ? 1.0 : x[h]) / sqrt(d[v]) : 0.0;
   }
 }
 __global__ __launch_bounds__(256) void k_gs_apply(double *__restrict__ X, int32_t n, int32_t nb,
@@ -1451,12 +1466,22 @@ __global__ __launch_bounds__(256) void k_gs_apply(double *__restrict__ X, int32_
     sr[e / kMaxVec][e % kMaxVec] = Rinv[e];
   }
   __syncthreads();
-  const int i = t & 63;
-  for (int v = t >> 6; v < nb; v += 4) {
-    double s = 0.0;
-    for (int u = 0; u <= v; ++u) s += sx[u][i] * sr[u][v];
-    if (r0 + i < n) X[(int64_t)v * n + r0 + i] = s;
-  }
+  // 4 rows x 4 vectors a thread, rows 16 apart (different banks), vectors 16 apart
+  const int i0 = t & 15, v0 = t >> 4;
+  double y[4][4] = {};
+#pragma unroll 4
+  for (int u = 0; u < nb; ++u)
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) y[a][b] += sx[u][i0 + 16 * a] * sr[u][v0 + 16 * b];
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const int i = i0 + 16 * a, v = v0 + 16 * b;
+      if (v < nb && r0 + i < n) X[(int64_t)v * n + r0 + i] = y[a][b];
+    }
 }
 
 // zeros in place of what the matrix held left of each reflector's first entry within its
@@ -1971,10 +1996,11 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
     const size_t lub = (size_t)kMaxVec * kLuF * N;
     const int32_t group = (int32_t)std::max<size_t>(1, std::min<size_t>(nbatch, ((size_t)1 << 28) / lub));
     const size_t sq = (size_t)kMaxVec * kMaxVec;
+    const size_t kpart = (size_t)8 * kMaxVec * N;  // the parts of products over a long k
     EIG_TRY(eig_ensure(ctx, ctx->evall, sizeof(double) * ((size_t)N * nvec + (size_t)kMaxVec * nvec +
-                                                          sq * nblk + sq + lub * group)));
+                                                          sq * nblk + sq + lub * group + kpart)));
     double *XT = (double *)ctx->evall.p, *Cc = XT + (size_t)N * nvec, *gp = Cc + (size_t)kMaxVec * nvec,
-           *Ri = gp + sq * nblk, *lu = Ri + sq;
+           *Ri = gp + sq * nblk, *lu = Ri + sq, *kp = lu + lub * group;
     // against every earlier vector, not only those of close eigenvalues: the products are
     // a small part, and vectors a few 1e-3 ||T|| apart stay orthogonal to the last ulps.
     // After the first solve once is enough (the vectors only start the second)
@@ -1990,8 +2016,10 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
         const double *P = XT;
         for (int rep = 0; rep <= it; ++rep) {
           if (nc > 0) {
-            EIG_TRY(eig_gemm_f64(ctx, st, true, false, nc, nb, N, 1.0, P, N, 0, X, N, 0, 0.0, Cc, nc, 0, 1));
-            EIG_TRY(eig_gemm_f64(ctx, st, false, false, N, nb, nc, -1.0, P, N, 0, Cc, nc, 0, 1.0, X, N, 0, 1));
+            EIG_TRY(eig_gemm_f64_long(ctx, st, true, false, nc, nb, N, 1.0, P, N, X, N, 0.0, Cc, nc, false,
+                                      kp, kpart));
+            EIG_TRY(eig_gemm_f64_long(ctx, st, false, false, N, nb, nc, -1.0, P, N, Cc, nc, 1.0, X, N,
+                                      false, kp, kpart));
           }
           hipLaunchKernelGGL(k_gs_gram, dim3((unsigned)nblk), dim3(256), 0, st, (const double *)X, n, nb, gp);
           hipLaunchKernelGGL(k_gs_chol, dim3(1), dim3(1024), 0, st, (const double *)gp, nblk, nb, Ri);
@@ -2012,8 +2040,8 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
         const int32_t c0 = p * kNB, np = std::min(kNB, last - c0 + 1);
         const int64_t rows = N - c0 - 1;
         const double *Vp = ws.a + (size_t)c0 * lda + c0 + 1;
-        EIG_TRY(eig_gemm_f64(ctx, st, true, false, np, nvec, rows, 1.0, Vp, lda, 0, XT + c0 + 1, N, 0,
-                             0.0, Cc, kNB, 0, 1));
+        EIG_TRY(eig_gemm_f64_long(ctx, st, true, false, np, nvec, rows, 1.0, Vp, lda, XT + c0 + 1, N,
+                                  0.0, Cc, kNB, false, kp, kpart));
         EIG_TRY(eig_gemm_f64(ctx, st, true, false, np, nvec, np, 1.0, ws.Tall + (size_t)p * kNB * kNB,
                              kNB, 0, Cc, kNB, 0, 0.0, Z, kNB, 0, 1));
         EIG_TRY(eig_gemm_f64(ctx, st, false, false, rows, nvec, np, -1.0, Vp, lda, 0, Z, kNB, 0, 1.0,

@@ -327,12 +327,15 @@ __global__ __launch_bounds__(256) void k_colnorm2(const double *__restrict__ R, 
   if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
-// trace of the n x n matrix X (column-major, lower tiles formed), in diagonal order
-__global__ void k_dense_trace(const double *__restrict__ X, int32_t n, double *__restrict__ tr) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// trace of the n x n matrix X (column-major, lower tiles formed): one block, each thread
+// every 256th entry (a single thread took 189 us at n = 1,003, a load's latency each)
+__global__ __launch_bounds__(256) void k_dense_trace(const double *__restrict__ X, int32_t n,
+                                                     double *__restrict__ tr) {
+  __shared__ double red[256];
   double s = 0.0;
-  for (int32_t i = 0; i < n; ++i) s += X[(int64_t)i * n + i];
-  *tr = s;
+  for (int32_t i = threadIdx.x; i < n; i += 256) s += X[(int64_t)i * n + i];
+  s = block_sum(s, red);
+  if (threadIdx.x == 0) *tr = s;
 }
 
 // X[i][j] = X[j][i] = X_lower[max][min] / y for the whole matrix (symmetric result)
@@ -551,7 +554,9 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
   }
 
   // ---- chunks of kept SNPs
-  const int64_t B = W > 0 ? 256 : 1024;
+  // (without a window the chunk only bounds the columns' memory: at 1,003 x 30,011 the
+  // products take 2.25 ms unsplit in chunks of 1,024, 1.4 split in chunks of 4,096)
+  const int64_t B = W > 0 ? 256 : std::max<int64_t>(1, std::min<int64_t>(nk, 4096));
   if (W > 0 && B + W > kMaxLdNc)
     return eig_set_err(ctx, EIG_E_ARG, "eig_xtx_normal: ldregress <= %d", kMaxLdNc - 256);
   const int64_t ldz = n;
@@ -570,6 +575,8 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
                o_ws = add(W > 0 ? 8 * (size_t)(nk + 1) : 0), o_drop = add(W > 0 ? (size_t)nk + 1 : 0),
                o_ns = add(4 * (size_t)B), o_src = add(W > 0 ? 4 * (size_t)B * W : 0),
                o_nrm = add(8 * (size_t)B);
+  const size_t part_doubles = (size_t)8 << 20;  // XTX's parts
+  const size_t o_part = add(8 * part_doubles);
   EIG_TRY(eig_ensure(ctx, ctx->scratch2, need));
   EIG_TRY(eig_ensure(ctx, ctx->xtx, 8 * (size_t)n * n));
   char *base = (char *)ctx->scratch2.p;
@@ -579,7 +586,7 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
   int64_t *d_ws = (int64_t *)(base + o_ws);
   uint8_t *d_drop = (uint8_t *)(base + o_drop);
   int32_t *d_ns = (int32_t *)(base + o_ns), *d_src = (int32_t *)(base + o_src);
-  double *d_nrm = (double *)(base + o_nrm);
+  double *d_nrm = (double *)(base + o_nrm), *d_part = (double *)(base + o_part);
   double *X = (double *)ctx->xtx.p;
   if (W > 0) {
     EIG_HIP(ctx, hipMemcpyAsync(d_ws, ws.data(), 8 * (size_t)nk, hipMemcpyHostToDevice, st));
@@ -622,8 +629,8 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
       EIG_HIP(ctx, hipMemcpy2DAsync(zn.data(), 8, d_G + (k0 - h0) * (nc + 1), 8 * (nc + 1), 8, nb,
                                     hipMemcpyDeviceToHost, st));
     }
-    EIG_TRY(eig_gemm_f64(ctx, st, false, true, n, n, nb, 1.0, R, ldz, 0, R, ldz, 0,
-                         first ? 0.0 : 1.0, X, n, 0, 1, true));
+    EIG_TRY(eig_gemm_f64_long(ctx, st, false, true, n, n, nb, 1.0, R, ldz, R, ldz, first ? 0.0 : 1.0, X, n,
+                              true, d_part, part_doubles));
     first = false;
     if (W > 0) {
       EIG_HIP(ctx, hipStreamSynchronize(st));
@@ -636,7 +643,7 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
   if (first) EIG_HIP(ctx, hipMemsetAsync(X, 0, 8 * (size_t)n * n, st));
   eig_time_end(ctx, "xtx_normal");
   double *d_tr = d_nrm;
-  hipLaunchKernelGGL(k_dense_trace, dim3(1), dim3(64), 0, st, (const double *)X, n, d_tr);
+  hipLaunchKernelGGL(k_dense_trace, dim3(1), dim3(256), 0, st, (const double *)X, n, d_tr);
   double tr = 0.0;
   EIG_HIP(ctx, hipMemcpyAsync(&tr, d_tr, 8, hipMemcpyDeviceToHost, st));
   EIG_HIP(ctx, hipStreamSynchronize(st));
