@@ -23,7 +23,7 @@
 //     Gershgorin interval, then 9-way multisection (8 lanes per eigenvalue, one
 //     count each).
 //  3. The top nvec eigenvectors of T by inverse iteration (LU with partial
-//     pivoting), Gram-Schmidt inside clusters of close eigenvalues.
+//     pivoting, a block per vector), Gram-Schmidt inside clusters of close eigenvalues.
 //  4. Back-transform X = Q Y in compact-WY form Q_p = I - V_p T_p V_p^T, last
 //     panel first; all T_p are formed up front (the Gram matrices V_p^T V_p over
 //     row ranges, then T_p per panel), then per panel one kernel applies the
@@ -1135,242 +1135,266 @@ __device__ inline double rcp_nr(double a) {
   return fma(r, fma(-a, r, 1.0), r);
 }
 
-constexpr int kInvB = 16;  // recurrence steps per batch of loads
-// Inverse iteration for the eigenvalues j0 .. j0+nvec-1 (descending order) of the
-// tridiagonal, one lane per vector.  flags select the stages of this launch: kInvFactor
-// (the pivoted LU of T - lambda I), kInvStart (start vectors), kInvSolve and kInvGs (per
-// iteration: the two triangular solves, then Gram-Schmidt against the batch's earlier
-// vectors of the same cluster and normalisation), for `iters` iterations.  A single
-// batch of at most kMaxVec vectors runs all stages in one launch (k_invit); more vectors
-// run the first three per batch (k_invit_batches).
-enum { kInvFactor = 1, kInvStart = 2, kInvSolve = 4, kInvGs = 8, kInvAll = 15 };
-// The LU factors are interleaved over the vectors, so that one recurrence step's
-// accesses of all lanes share a cache line: field f of step i of vector kv sits at
-// lu[(i * kLuF + f) * kMaxVec + kv] (f: 0 pivot reciprocal, 1 and 2 the U
-// superdiagonals, 3 multiplier, 4 pivot flag).
+// One inverse iteration for the eigenvalues j0 + blockIdx.x (descending order) of the
+// tridiagonal, one block per vector: with `first` from a fixed start vector, else from
+// X[j]; the pivoted LU of T - lambda I is formed with `factor`, else read back; the result is
+// normalised.  The three recurrences (LU, forward, backward) are serial, about 130, 40 and 40
+// cycles a step by their chains, and the rest has to stay off them: kInvC steps at a time are
+// brought to LDS by the whole block, one lane runs them there, kInvB steps of operands read
+// ahead, and the block writes the results back in whole lines.  The forward solve of a
+// factoring pass runs in the LU's loop, behind its longer chain.  A lane per vector with its
+// loads and stores in global memory, sixteen steps ahead, spent 0.65 us a row on two
+// iterations of ten vectors (every store had to end before a later load counted).
+//
+// The LU factors: field f of step i of block b at lu[(b kLuF + f) n + i] (f: 0 pivot
+// reciprocal, 1 and 2 the U superdiagonals, 3 multiplier, 4 pivot flag).
 constexpr int kLuF = 5;
-struct LuCol {
-  double *p;  // lu + f * kMaxVec + kv
-  __device__ double &operator[](int32_t i) const { return p[(int64_t)i * (kLuF * kMaxVec)]; }
-};
-__device__ __forceinline__ void invit_part(const EigWs &ws, int32_t n, int32_t nvec, int32_t j0,
-                                           int32_t flags, int32_t iters) {
-  __shared__ double red[4];
-  __shared__ double dots[2];
-  const double tnorm = ws.sc[S_TNORM];
-  const double eps = 2.220446049250313e-16;
-  const double tiny = eps * tnorm;
+constexpr int kInvB = 8;
+constexpr int kInvC = 512;
+__global__ __launch_bounds__(256) void k_invit_solve(EigWs ws, int32_t n, int32_t j0, int32_t first,
+                                                     int32_t factor, double *__restrict__ X,
+                                                     double *__restrict__ lu) {
+  // fields 0-4 as above (d and e come in as 0 and 1), 5 x; entry kInvC of field 1 is the e
+  // after the chunk
+  __shared__ __align__(16) double f[kLuF + 1][kInvC + 2];
+  __shared__ double red[4], sinv;
   const int tid = threadIdx.x;
-  if ((flags & kInvFactor) && tid < nvec) {
-    const int kv = tid;
-    const double lam = ws.eval[n - 1 - (j0 + kv)];
-    const LuCol u0{ws.lu + kv}, u1{ws.lu + kMaxVec + kv}, u2{ws.lu + 2 * kMaxVec + kv},
-        ml{ws.lu + 3 * kMaxVec + kv}, pv{ws.lu + 4 * kMaxVec + kv};  // u0: pivot reciprocals
-    double acur = ws.d[0] - lam, bcur = (n > 1) ? ws.e[0] : 0.0;
-    // the recurrence is serial; its operands are loaded kInvB steps at a time, one
-    // batch ahead of the batch being computed, so memory latency stays hidden
-    auto ldf = [&](int32_t i0, double (&eb)[kInvB + 1], double (&db)[kInvB]) {
-#pragma unroll
-      for (int k = 0; k <= kInvB; ++k) eb[k] = (i0 + k < n - 1) ? ws.e[i0 + k] : 0.0;
-#pragma unroll
-      for (int k = 0; k < kInvB; ++k) db[k] = (i0 + k + 1 < n) ? ws.d[i0 + k + 1] : 0.0;
-    };
-    // full: the whole batch is inside the recurrence (no per-step bound check).  The
-    // pivot choice is a select, not a branch: lanes (vectors) pivot differently, and
-    // both reciprocals are formed, that of l off the serial chain.
-    auto runf = [&](bool full, int32_t i0, const double (&eb)[kInvB + 1],
-                    const double (&db)[kInvB]) {
-#pragma unroll
-      for (int k = 0; k < kInvB; ++k) {
-        const int32_t i = i0 + k;
-        if (full || i < n - 1) {
-          const double l = eb[k];
-          const double an = db[k] - lam, bn = eb[k + 1];
-          const bool sw = fabs(acur) < fabs(l);  // row interchange
-          double a0 = acur;
-          if (fabs(a0) < tiny) a0 = copysign(tiny, a0 == 0.0 ? 1.0 : a0);
-          const double rl = rcp_nr(l), ra = rcp_nr(a0);
-          const double r = sw ? rl : ra;
-          const double m = (sw ? acur : l) * r;
-          u0[i] = r; u1[i] = sw ? an : bcur; u2[i] = sw ? bn : 0.0; ml[i] = m; pv[i] = sw ? 1.0 : 0.0;
-          const double na = sw ? bcur - m * an : an - m * bcur;
-          bcur = sw ? -m * bn : bn;
-          acur = na;
-        }
+  const int32_t j = j0 + (int32_t)blockIdx.x;
+  const double lam = ws.eval[n - 1 - j];
+  const double tiny = 2.220446049250313e-16 * ws.sc[S_TNORM];
+  double *x = X + (int64_t)j * n, *L = lu + (int64_t)blockIdx.x * kLuF * n;
+  // start vectors: a fixed hash of index and vector
+  auto start = [&](int32_t i) {
+    uint32_t h = (uint32_t)(i + 1) * 2654435761u ^ (uint32_t)(j + 7) * 40503u;
+    h ^= h >> 15; h *= 2246822519u; h ^= h >> 13;
+    return 0.5 + (double)(h & 0xFFFFFF) / 16777216.0;
+  };
+  // ---- LU and forward solve P L: step i works on rows i and i + 1.  Lane 0 carries the
+  // current row (acur, bcur) and x from chunk to chunk
+  double acur = ws.d[0] - lam, bcur = n > 1 ? ws.e[0] : 0.0;
+  double carry = first ? start(0) : x[0];
+  for (int32_t c0 = 0; c0 < n - 1; c0 += kInvC) {
+    const int32_t m = min(kInvC, n - 1 - c0);  // steps of this chunk
+    for (int32_t i = tid; i < kInvC; i += 256) {
+      const bool in = i < m;
+      const int32_t g = in ? c0 + i : n - 2;
+      if (factor) {
+        f[0][i] = ws.d[g + 1];
+        f[1][i] = ws.e[g];
+      } else {
+        f[3][i] = L[3 * (int64_t)n + g];
+        f[4][i] = L[4 * (int64_t)n + g];
       }
-    };
-    {
-      double eA[kInvB + 1], dA[kInvB], eB[kInvB + 1], dB[kInvB];
-      ldf(0, eA, dA);
-      for (int32_t i0 = 0; i0 < n - 1; i0 += 2 * kInvB) {
-        ldf(i0 + kInvB, eB, dB);
-        if (i0 + kInvB <= n - 1) runf(true, i0, eA, dA); else runf(false, i0, eA, dA);
-        ldf(i0 + 2 * kInvB, eA, dA);
-        if (i0 + 2 * kInvB <= n - 1) runf(true, i0 + kInvB, eB, dB); else runf(false, i0 + kInvB, eB, dB);
-      }
+      f[5][i] = first ? start(g + 1) : x[g + 1];
     }
-    if (fabs(acur) < tiny) acur = copysign(tiny, acur == 0.0 ? 1.0 : acur);
-    u0[n - 1] = rcp_nr(acur);
-    u1[n - 1] = 0.0; u2[n - 1] = 0.0; ml[n - 1] = 0.0; pv[n - 1] = 0.0;
-  }
-  // start vectors (a fixed hash of index and vector), filled by the whole block
-  if (flags & kInvStart)
-    for (int kv = 0; kv < nvec; ++kv) {
-      double *x = ws.X + (int64_t)kv * n;
-      const int kg = j0 + kv;
-      for (int32_t i = tid; i < n; i += 256) {
-        uint32_t h = (uint32_t)(i + 1) * 2654435761u ^ (uint32_t)(kg + 7) * 40503u;
-        h ^= h >> 15; h *= 2246822519u; h ^= h >> 13;
-        x[i] = 0.5 + (double)(h & 0xFFFFFF) / 16777216.0;
-      }
-    }
-  __syncthreads();
-  for (int it = 0; it < iters; ++it) {
-    if ((flags & kInvSolve) && tid < nvec) {
-      const int kv = tid;
-      const LuCol u0{ws.lu + kv}, u1{ws.lu + kMaxVec + kv}, u2{ws.lu + 2 * kMaxVec + kv},
-          ml{ws.lu + 3 * kMaxVec + kv}, pv{ws.lu + 4 * kMaxVec + kv};
-      double *x = ws.X + (int64_t)kv * n;
-      double carry = x[0];
-      // forward: P L; batch i0 reads x[i0+1 .. i0+kInvB] and writes x[i0 .. i0+kInvB-1],
-      // so the next batch's loads (issued before this batch runs) read values no
-      // earlier batch writes
-      auto ldx = [&](int32_t i0, double (&xb)[kInvB], double (&pb)[kInvB], double (&mb)[kInvB]) {
+    if (tid == 0) f[1][kInvC] = c0 + kInvC < n - 1 ? ws.e[c0 + kInvC] : 0.0;
+    __syncthreads();
+    if (tid == 0) {
+      if (factor) {
+        // the e after the last step is outside the recurrence
+        if (m < kInvC) f[1][m] = 0.0;
+        double db[kInvB], eb[kInvB], xb[kInvB], dn[kInvB], en[kInvB], xn[kInvB];
+        auto ld = [&](int32_t i, double (&d)[kInvB], double (&e)[kInvB], double (&y)[kInvB]) {
+          i = min(i, kInvC - kInvB);
 #pragma unroll
-        for (int k = 0; k < kInvB; ++k) {
-          const bool in = i0 + k < n - 1;
-          xb[k] = in ? x[i0 + k + 1] : 0.0;
-          pb[k] = in ? pv[i0 + k] : 0.0;
-          mb[k] = in ? ml[i0 + k] : 0.0;
-        }
-      };
-      auto runx = [&](bool full, int32_t i0, const double (&xb)[kInvB], const double (&pb)[kInvB],
-                      const double (&mb)[kInvB]) {
-#pragma unroll
-        for (int k = 0; k < kInvB; ++k) {
-          const int32_t i = i0 + k;
-          if (full || i < n - 1) {
-            const bool sw = pb[k] != 0.0;
-            const double lo = sw ? xb[k] : carry, nx = sw ? carry : xb[k];
-            x[i] = lo;
-            carry = nx - mb[k] * lo;
+          for (int k = 0; k < kInvB; ++k) {
+            d[k] = f[0][i + k];
+            e[k] = f[1][i + k + 1];
+            y[k] = f[5][i + k];
           }
-        }
-      };
-      {
-        double xA[kInvB], pA[kInvB], mA[kInvB], xB[kInvB], pB[kInvB], mB[kInvB];
-        ldx(0, xA, pA, mA);
-        for (int32_t i0 = 0; i0 < n - 1; i0 += 2 * kInvB) {
-          ldx(i0 + kInvB, xB, pB, mB);
-          if (i0 + kInvB <= n - 1) runx(true, i0, xA, pA, mA); else runx(false, i0, xA, pA, mA);
-          ldx(i0 + 2 * kInvB, xA, pA, mA);
-          if (i0 + 2 * kInvB <= n - 1) runx(true, i0 + kInvB, xB, pB, mB);
-          else runx(false, i0 + kInvB, xB, pB, mB);
-        }
-      }
-      x[n - 1] = carry;
-      // backward: U; batch i0 reads and writes x[i0 - kInvB + 1 .. i0] only
-      double x2 = 0.0, x1 = x[n - 1] * u0[n - 1];
-      x[n - 1] = x1;
-      auto ldb = [&](int32_t i0, double (&xb)[kInvB], double (&ab)[kInvB], double (&bb)[kInvB],
-                     double (&cb)[kInvB]) {
+        };
+        double l = f[1][0];
+        auto run = [&](bool full, int32_t i0, const double (&d)[kInvB], const double (&e)[kInvB],
+                       const double (&y)[kInvB]) {
 #pragma unroll
-        for (int k = 0; k < kInvB; ++k) {
-          const int32_t i = i0 - k;
-          const bool in = i >= 0;
-          xb[k] = in ? x[i] : 0.0;
-          ab[k] = in ? u0[i] : 1.0;
-          bb[k] = in ? u1[i] : 0.0;
-          cb[k] = in ? u2[i] : 0.0;
-        }
-      };
-      auto runb = [&](bool full, int32_t i0, const double (&xb)[kInvB], const double (&ab)[kInvB],
-                      const double (&bb)[kInvB], const double (&cb)[kInvB]) {
-#pragma unroll
-        for (int k = 0; k < kInvB; ++k) {
-          const int32_t i = i0 - k;
-          if (full || i >= 0) {
-            const double xi = (xb[k] - bb[k] * x1 - cb[k] * x2) * ab[k];
-            x[i] = xi;
-            x2 = x1;
-            x1 = xi;
+          for (int k = 0; k < kInvB; ++k) {
+            const int32_t i = i0 + k;
+            if (full || i < m) {
+              const double an = d[k] - lam, bn = e[k];
+              const bool sw = fabs(acur) < fabs(l);  // row interchange
+              const double a0 = fabs(acur) < tiny ? copysign(tiny, acur == 0.0 ? 1.0 : acur) : acur;
+              const double r = rcp_nr(sw ? l : a0);
+              const double mu = (sw ? acur : l) * r;
+              f[0][i] = r;
+              f[1][i] = sw ? an : bcur;
+              f[2][i] = sw ? bn : 0.0;
+              f[3][i] = mu;
+              f[4][i] = sw ? 1.0 : 0.0;
+              const double na = sw ? bcur - mu * an : an - mu * bcur;
+              bcur = sw ? -mu * bn : bn;
+              acur = na;
+              l = bn;
+              const double lo = sw ? y[k] : carry, nx = sw ? carry : y[k];
+              f[5][i] = lo;
+              carry = nx - mu * lo;
+            }
           }
+        };
+        // a batch is read before the one ahead of it is written: no step reads what an
+        // earlier one wrote
+        ld(0, db, eb, xb);
+        for (int32_t i0 = 0; i0 < m; i0 += 2 * kInvB) {
+          ld(i0 + kInvB, dn, en, xn);
+          if (i0 + kInvB <= m) run(true, i0, db, eb, xb); else run(false, i0, db, eb, xb);
+          ld(i0 + 2 * kInvB, db, eb, xb);
+          if (i0 + 2 * kInvB <= m) run(true, i0 + kInvB, dn, en, xn); else run(false, i0 + kInvB, dn, en, xn);
         }
-      };
-      {
-        double xA[kInvB], aA[kInvB], bA[kInvB], cA[kInvB];
-        double xB[kInvB], aB[kInvB], bB[kInvB], cB[kInvB];
-        ldb(n - 2, xA, aA, bA, cA);
-        for (int32_t i0 = n - 2; i0 >= 0; i0 -= 2 * kInvB) {
-          ldb(i0 - kInvB, xB, aB, bB, cB);
-          if (i0 - kInvB + 1 >= 0) runb(true, i0, xA, aA, bA, cA); else runb(false, i0, xA, aA, bA, cA);
-          ldb(i0 - 2 * kInvB, xA, aA, bA, cA);
-          if (i0 - 2 * kInvB + 1 >= 0) runb(true, i0 - kInvB, xB, aB, bB, cB);
-          else runb(false, i0 - kInvB, xB, aB, bB, cB);
+      } else {
+        double mb[kInvB], pb[kInvB], xb[kInvB], mn[kInvB], pn[kInvB], xn[kInvB];
+        auto ld = [&](int32_t i, double (&u)[kInvB], double (&p)[kInvB], double (&y)[kInvB]) {
+          i = min(i, kInvC - kInvB);
+#pragma unroll
+          for (int k = 0; k < kInvB; ++k) {
+            u[k] = f[3][i + k];
+            p[k] = f[4][i + k];
+            y[k] = f[5][i + k];
+          }
+        };
+        auto run = [&](bool full, int32_t i0, const double (&u)[kInvB], const double (&p)[kInvB],
+                       const double (&y)[kInvB]) {
+#pragma unroll
+          for (int k = 0; k < kInvB; ++k) {
+            const int32_t i = i0 + k;
+            if (full || i < m) {
+              const bool sw = p[k] != 0.0;
+              const double lo = sw ? y[k] : carry, nx = sw ? carry : y[k];
+              f[5][i] = lo;
+              carry = nx - u[k] * lo;
+            }
+          }
+        };
+        ld(0, mb, pb, xb);
+        for (int32_t i0 = 0; i0 < m; i0 += 2 * kInvB) {
+          ld(i0 + kInvB, mn, pn, xn);
+          if (i0 + kInvB <= m) run(true, i0, mb, pb, xb); else run(false, i0, mb, pb, xb);
+          ld(i0 + 2 * kInvB, mb, pb, xb);
+          if (i0 + 2 * kInvB <= m) run(true, i0 + kInvB, mn, pn, xn); else run(false, i0 + kInvB, mn, pn, xn);
         }
       }
     }
     __syncthreads();
-    if (!(flags & kInvGs)) continue;
-    for (int kv = 0; kv < nvec; ++kv) {
-      double *x = ws.X + (int64_t)kv * n;
-      const double lam = ws.eval[n - 1 - (j0 + kv)];
-      for (int pv2 = 0; pv2 < kv; ++pv2) {
-        const double lp = ws.eval[n - 1 - (j0 + pv2)];
-        if (fabs(lam - lp) > 1e-3 * tnorm) continue;
-        const double *p = ws.X + (int64_t)pv2 * n;
-        double s = 0.0;
-        for (int32_t i = tid; i < n; i += 256) s += x[i] * p[i];
-        s = block_sum(s, red);
-        for (int32_t i = tid; i < n; i += 256) x[i] -= s * p[i];
-        __syncthreads();
-      }
-      double s = 0.0;
-      for (int32_t i = tid; i < n; i += 256) s += x[i] * x[i];
-      s = block_sum(s, red);
-      if (tid == 0) dots[0] = 1.0 / sqrt(s);
-      __syncthreads();
-      const double inv = dots[0];
-      for (int32_t i = tid; i < n; i += 256) x[i] *= inv;
-      __syncthreads();
+    for (int32_t i = tid; i < m; i += 256) {
+      if (factor)
+#pragma unroll
+        for (int k = 0; k < kLuF; ++k) L[k * (int64_t)n + c0 + i] = f[k][i];
+      x[c0 + i] = f[5][i];
     }
+    __syncthreads();
   }
+  if (tid == 0) {
+    if (factor) {
+      if (fabs(acur) < tiny) acur = copysign(tiny, acur == 0.0 ? 1.0 : acur);
+      L[n - 1] = rcp_nr(acur);
+      L[2 * (int64_t)n - 1] = L[3 * (int64_t)n - 1] = 0.0;
+    }
+    x[n - 1] = carry;
+  }
+  __syncthreads();
+  // ---- backward solve U, chunks from the end
+  double x1 = 0.0, x2 = 0.0, ss = 0.0;
+  for (int32_t e0 = n; e0 > 0; e0 -= kInvC) {
+    const int32_t c0 = max(0, e0 - kInvC), m = e0 - c0;
+    for (int32_t i = tid; i < m; i += 256) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) f[k][i] = L[k * (int64_t)n + c0 + i];
+      f[5][i] = x[c0 + i];
+    }
+    __syncthreads();
+    if (tid == 0) {
+      double yb[kInvB], ab[kInvB], bb[kInvB], cb[kInvB], yn[kInvB], an[kInvB], bn[kInvB], cn[kInvB];
+      // rows i0, i0 - 1, .. (those below 0 are not used)
+      auto ld = [&](int32_t i0, double (&y)[kInvB], double (&u)[kInvB], double (&v)[kInvB],
+                    double (&w)[kInvB]) {
+        i0 = max(i0, kInvB - 1);
+#pragma unroll
+        for (int k = 0; k < kInvB; ++k) {
+          y[k] = f[5][i0 - k];
+          u[k] = f[0][i0 - k];
+          v[k] = f[1][i0 - k];
+          w[k] = f[2][i0 - k];
+        }
+      };
+      auto run = [&](int32_t i0, const double (&y)[kInvB], const double (&u)[kInvB],
+                     const double (&v)[kInvB], const double (&w)[kInvB]) {
+#pragma unroll
+        for (int k = 0; k < kInvB; ++k) {
+          const double xi = (y[k] - v[k] * x1 - w[k] * x2) * u[k];
+          f[5][i0 - k] = xi;
+          x2 = x1;
+          x1 = xi;
+        }
+      };
+      // whole batches from the end, then the first rows one by one
+      int32_t i0 = m - 1;
+      if (i0 >= kInvB - 1) ld(i0, yb, ab, bb, cb);
+      for (; i0 >= 2 * kInvB - 1; i0 -= 2 * kInvB) {
+        ld(i0 - kInvB, yn, an, bn, cn);
+        run(i0, yb, ab, bb, cb);
+        ld(i0 - 2 * kInvB, yb, ab, bb, cb);
+        run(i0 - kInvB, yn, an, bn, cn);
+      }
+      if (i0 >= kInvB - 1) {
+        run(i0, yb, ab, bb, cb);
+        i0 -= kInvB;
+      }
+      for (; i0 >= 0; --i0) {
+        const double xi = (f[5][i0] - f[1][i0] * x1 - f[2][i0] * x2) * f[0][i0];
+        f[5][i0] = xi;
+        x2 = x1;
+        x1 = xi;
+      }
+    }
+    __syncthreads();
+    for (int32_t i = tid; i < m; i += 256) {
+      const double v = f[5][i];
+      ss += v * v;
+      x[c0 + i] = v;
+    }
+    __syncthreads();
+  }
+  ss = block_sum(ss, red);
+  if (tid == 0) sinv = 1.0 / sqrt(ss);
+  __syncthreads();
+  for (int32_t i = tid; i < n; i += 256) x[i] *= sinv;
 }
 
-__global__ __launch_bounds__(256) void k_invit(EigWs ws, int32_t n, int32_t nvec) {
-  // two iterations: the eigenvalues are accurate to a few ulps, so one solve already
-  // leaves contamination of order eps ||T|| / gap from outside a cluster, and the
-  // second squares it (the parity tests pass with one; two keep a margin)
-  invit_part(ws, n, nvec, 0, kInvAll, 2);
+// Gram-Schmidt of at most kMaxVec normalised vectors against the earlier ones of the same
+// cluster, in order, and normalisation; a vector without close ones stays as it is.
+__global__ __launch_bounds__(256) void k_invit_gs(EigWs ws, int32_t n, int32_t nvec) {
+  __shared__ double red[4];
+  __shared__ double sinv;
+  const double tnorm = ws.sc[S_TNORM];
+  const int tid = threadIdx.x;
+  for (int kv = 1; kv < nvec; ++kv) {
+    double *x = ws.X + (int64_t)kv * n;
+    const double lam = ws.eval[n - 1 - kv];
+    bool any = false;
+    for (int pv = 0; pv < kv; ++pv) {
+      if (fabs(lam - ws.eval[n - 1 - pv]) > 1e-3 * tnorm) continue;
+      any = true;
+      const double *p = ws.X + (int64_t)pv * n;
+      double s = 0.0;
+      for (int32_t i = tid; i < n; i += 256) s += x[i] * p[i];
+      s = block_sum(s, red);
+      for (int32_t i = tid; i < n; i += 256) x[i] -= s * p[i];
+      __syncthreads();
+    }
+    if (!any) continue;
+    double s = 0.0;
+    for (int32_t i = tid; i < n; i += 256) s += x[i] * x[i];
+    s = block_sum(s, red);
+    if (tid == 0) sinv = 1.0 / sqrt(s);
+    __syncthreads();
+    for (int32_t i = tid; i < n; i += 256) x[i] *= sinv;
+    __syncthreads();
+  }
 }
 
 // ---- more than kMaxVec vectors ----
-// One block per batch of kMaxVec vectors (vector j of the call's list at XT + j n): the
-// stages of `flags` and one solve, then a normalisation (a wave per vector).  The batches
-// of a launch do not depend on each other.  The vectors are orthogonalised after each of
-// the two solves: two solves in a row turn the vectors of a repeated eigenvalue towards
+// The vectors are orthogonalised after each of the two solves, batch by batch of kMaxVec:
+// two solves in a row turn the vectors of a repeated eigenvalue towards
 // the one nearest to their shifts, and what is left between them after that is rounding
 // (residuals of 1e-11 of the norm; orthogonalised in between, a few ulps).
-__global__ __launch_bounds__(256) void k_invit_batches(EigWs ws, int32_t n, int32_t nvec,
-                                                       int32_t b0, int32_t flags,
-                                                       double *__restrict__ XT,
-                                                       double *__restrict__ lu) {
-  const int32_t j0 = (b0 + (int32_t)blockIdx.x) * kMaxVec;
-  const int32_t nb = min(kMaxVec, nvec - j0);
-  ws.X = XT + (int64_t)j0 * n;
-  ws.lu = lu + (int64_t)blockIdx.x * kMaxVec * kLuF * n;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  invit_part(ws, n, nb, j0, flags | kInvSolve, 1);
-  for (int32_t v = wv; v < nb; v += 4) {
-    double *x = ws.X + (int64_t)v * n;
-    double s = 0.0;
-    for (int32_t i = lane; i < n; i += 64) s += x[i] * x[i];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += xlane(s, o);
-    const double inv = 1.0 / sqrt(s);
-    for (int32_t i = lane; i < n; i += 64) x[i] *= inv;
-  }
-}
 
 // Orthonormalisation of a batch of nb <= 64 vectors (X, vector v at X + v n) among
 // themselves by its Gram matrix: X <- X R^-1 with G = R^T R (Cholesky), the same vectors
@@ -1980,7 +2004,14 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   };
   tbeg();
   if (nvec > 0 && nvec <= kMaxVec) {
-    hipLaunchKernelGGL(k_invit, dim3(1), dim3(256), 0, st, ws, n, nvec);
+    // two iterations: the eigenvalues are accurate to a few ulps, so one solve already
+    // leaves contamination of order eps ||T|| / gap from outside a cluster, and the
+    // second squares it (the parity tests pass with one; two keep a margin)
+    for (int it = 0; it < 2; ++it) {
+      hipLaunchKernelGGL(k_invit_solve, dim3((unsigned)nvec), dim3(256), 0, st, ws, n, 0, (int32_t)(it == 0),
+                         (int32_t)(it == 0), ws.X, ws.lu);
+      hipLaunchKernelGGL(k_invit_gs, dim3(1), dim3(256), 0, st, ws, n, nvec);
+    }
     tend("invit");
     tbeg();
     if (last >= 0) {
@@ -1991,10 +2022,10 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
     EIG_TRY(back_transform(nvec));
   } else if (nvec > kMaxVec) {
     // all vectors (vector j at j N), the Gram-Schmidt and back-transform coefficients, the
-    // partial Gram matrices, R^-1, and the LU factors of as many batches as 2 GiB hold
-    const int32_t nbatch = (nvec + kMaxVec - 1) / kMaxVec, nblk = (n + kGsRows - 1) / kGsRows;
-    const size_t lub = (size_t)kMaxVec * kLuF * N;
-    const int32_t group = (int32_t)std::max<size_t>(1, std::min<size_t>(nbatch, ((size_t)1 << 28) / lub));
+    // partial Gram matrices, R^-1, and the LU factors of as many vectors as 2 GiB hold
+    const int32_t nblk = (n + kGsRows - 1) / kGsRows;
+    const size_t lub = (size_t)kLuF * N;
+    const int32_t group = (int32_t)std::max<size_t>(1, std::min<size_t>(nvec, ((size_t)1 << 28) / lub));
     const size_t sq = (size_t)kMaxVec * kMaxVec;
     const size_t kpart = (size_t)8 * kMaxVec * N;  // the parts of products over a long k
     EIG_TRY(eig_ensure(ctx, ctx->evall, sizeof(double) * ((size_t)N * nvec + (size_t)kMaxVec * nvec +
@@ -2005,10 +2036,9 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
     // a small part, and vectors a few 1e-3 ||T|| apart stay orthogonal to the last ulps.
     // After the first solve once is enough (the vectors only start the second)
     for (int it = 0; it < 2; ++it) {
-      const int32_t flags = it == 0 ? kInvFactor | kInvStart : (nbatch > group ? kInvFactor : 0);
-      for (int32_t b = 0; b < nbatch; b += group)
-        hipLaunchKernelGGL(k_invit_batches, dim3((unsigned)std::min(group, nbatch - b)), dim3(256), 0, st,
-                           ws, n, nvec, b, flags, XT, lu);
+      for (int32_t b = 0; b < nvec; b += group)
+        hipLaunchKernelGGL(k_invit_solve, dim3((unsigned)std::min(group, nvec - b)), dim3(256), 0, st, ws, n,
+                           b, (int32_t)(it == 0), (int32_t)(it == 0 || nvec > group), XT, lu);
       EIG_HIP(ctx, hipGetLastError());
       for (int32_t j0 = 0; j0 < nvec; j0 += kMaxVec) {
         const int32_t nb = std::min<int32_t>(kMaxVec, nvec - j0), nc = j0;
