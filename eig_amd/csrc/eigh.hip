@@ -20,7 +20,7 @@
 //     k_syr2k applies A -= V W^T + W V^T to the trailing matrix.  The reflector of
 //     row c is left in A[c][c+1:], with tau[c].
 //  2. All eigenvalues of the tridiagonal T: Sturm counts on a shared grid of the
-//     Gershgorin interval, then 9-way multisection (8 lanes per eigenvalue, one
+//     Gershgorin interval, then multisection (8 to 64 lanes per eigenvalue, one
 //     count each).
 //  3. The top nvec eigenvectors of T by inverse iteration (LU with partial
 //     pivoting, a block per vector), Gram-Schmidt inside clusters of close eigenvalues.
@@ -42,7 +42,7 @@ constexpr int kNB = 32;      // panel width
 constexpr int kMaxVec = 64;  // max eigenvectors computed
 
 enum {
-  S_GL = 0, S_GU, S_PIVMIN, S_TNORM,
+  S_GL = 0, S_GU, S_PIVMIN, S_TNORM, S_SCALE,
   S_COUNT
 };
 
@@ -60,6 +60,7 @@ struct EigWs {
   int32_t *sync;          // [1] set if a resident launch gave up waiting
   int32_t maxw;
   double *eval;           // ascending
+  double2 *st;            // (d, e^2) of T scaled to a norm of 1/2 .. 1, for the Sturm counts
   double *X;              // nvec x n eigenvectors
   double *lu;             // n x 5 x kMaxVec LU factors of inverse iteration
   double *Z;              // kNB x kMaxVec
@@ -993,74 +994,89 @@ __global__ void k_gersh(EigWs ws, int32_t n) {
     ws.sc[S_GU] = hi[0] + 2.0 * eps * tnorm * n + 2.0 * pivmin;
     ws.sc[S_PIVMIN] = pivmin;
     ws.sc[S_TNORM] = fmax(tnr[0], 1e-300);
+    ws.sc[S_SCALE] = ldexp(1.0, -ilogb(ws.sc[S_TNORM]) - 1);
   }
 }
 
-// Two Sturm counts (eigenvalues of T below x and below x2), interleaved.  The
-// reciprocal is v_rcp_f64 refined by two Newton steps (relative error ~1e-16),
-// which perturbs each pivot far below the bisection tolerance.  d and e2 are read
-// a batch of four entries ahead of use.
-// number of eigenvalues of T below x (Sturm count of T - x I), with q clamped away
-// from zero by pivmin as in LAPACK's dstebz
-__device__ inline int32_t sturm1(const double *__restrict__ d, const double *__restrict__ e2,
-                                 int32_t n, double x, double pivmin) {
-  int32_t cnt = 0;
-  double q = d[0] - x;
-  if (q <= pivmin) { ++cnt; q = fmin(q, -pivmin); }
-  auto step = [&](double di, double ei) {
-    double r = __builtin_amdgcn_rcp(q);
-    r = fma(r, fma(-q, r, 1.0), r);
-    q = (di - x) - ei * r;
-    if (q <= pivmin) { ++cnt; q = fmin(q, -pivmin); }
-  };
-  // batches of four steps in two alternating register sets: the next batch's
-  // (wave-uniform, scalar) loads are issued before the current batch's steps, so their
-  // latency hides behind the recurrence
-  int32_t i = 1;
-  double ad[4], af[4], bd[4], bf[4];
-  auto ld = [&](int32_t j0, double (&xd)[4], double (&xf)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      xd[u] = d[j0 + u];
-      xf[u] = e2[j0 - 1 + u];
-    }
-  };
-  auto run = [&](const double (&xd)[4], const double (&xf)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) step(xd[u], xf[u]);
-  };
-  if (i + 3 < n) {
-    ld(i, ad, af);
-    for (;;) {
-      // set a holds steps i .. i+3 (all < n)
-      if (i + 7 >= n) {
-        run(ad, af);
-        i += 4;
-        break;
-      }
-      ld(i + 4, bd, bf);
-      run(ad, af);
-      i += 4;
-      // set b holds steps i .. i+3
-      if (i + 7 >= n) {
-        run(bd, bf);
-        i += 4;
-        break;
-      }
-      ld(i + 4, ad, af);
-      run(bd, bf);
-      i += 4;
-    }
+// T over a power of two of its norm, as the Sturm counts read it: (d_i, e_{i-1}^2) in steps
+// of 2 kStB, the last ones filled with rows that change no sign, and one batch more that is
+// read ahead.  e^2 is kept at 2^-160 at least (2^-80 of the norm, far below an eigenvalue's
+// rounding), so that a zero minor is followed by one that is not.
+constexpr int kStB = 8;
+__host__ __device__ inline int32_t sturm_rows(int32_t n) { return (n + 2 * kStB - 1) / (2 * kStB) * (2 * kStB); }
+__global__ __launch_bounds__(256) void k_sturm_prep(EigWs ws, int32_t n) {
+  const int32_t i = (int32_t)(blockIdx.x * 256 + threadIdx.x);
+  if (i >= sturm_rows(n) + kStB) return;
+  const double s = ws.sc[S_SCALE];
+  double2 v = make_double2(8.0, 0x1p-160);
+  if (i < n) {
+    v.x = ws.d[i] * s;
+    const double e = i > 0 ? ws.e[i - 1] * s : 0.0;
+    v.y = fmax(e * e, 0x1p-160);
   }
-  for (; i < n; ++i) step(d[i], e2[i - 1]);
+  ws.st[i] = v;
+}
+
+// the block pulls T into its L2 together: scalar loads that miss there one batch after the
+// other took 47 ns a step of a launch's first count
+__device__ __forceinline__ void sturm_warm(const double2 *__restrict__ T, int32_t n) {
+  for (int32_t i = kStB * (int32_t)threadIdx.x; i < n; i += kStB * 256) {
+    const double v = T[i].x;
+    asm volatile("" ::"v"(v));
+  }
+}
+
+// Number of eigenvalues of T below x: the sign changes in the sequence of leading minors
+// p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2} of the scaled T - x I.  Only its one fused
+// multiply-add is on the chain from step to step (the recurrence of quotients has a
+// reciprocal there: 78 cycles a step, now 35); each step's rounding amounts to a relative
+// change of d_i - x and of e_{i-1}^2.  A batch grows by at most 2^16 and shrinks by 2^-640 or
+// so where minors vanish, and is followed by a common scaling of the last two.  Signs are
+// shifted into a word and their changes counted per batch.  d and e^2 are wave-uniform
+// (scalar) loads, one batch ahead of use.
+__device__ inline int32_t sturm1(const double2 *T2, int32_t n, double x) {
+  // constant address space: uniform reads of it are scalar loads
+  typedef const __attribute__((address_space(4))) double *Scalars;
+  const Scalars T = (Scalars)(uintptr_t)T2;
+  int32_t cnt = 0;
+  uint32_t bits = 0;
+  double p1 = 1.0, p2 = 0.0;
+  auto run = [&](const double (&v)[2 * kStB]) {
+#pragma unroll
+    for (int u = 0; u < kStB; ++u) {
+      const double p = fma(v[2 * u] - x, p1, -(v[2 * u + 1] * p2));
+      p2 = p1;
+      p1 = p;
+      bits = __builtin_amdgcn_alignbit(bits, (uint32_t)__double2hiint(p), 31);
+    }
+    cnt += __popc((bits ^ (bits >> 1)) & ((1u << kStB) - 1u));
+    const double m = fmax(fabs(p1), fabs(p2));
+    const int ex = __builtin_amdgcn_frexp_exp(m);
+    p1 = m > 0.0 ? __builtin_amdgcn_ldexp(p1, -ex) : 1.0;
+    p2 = __builtin_amdgcn_ldexp(p2, -ex);
+  };
+  // the loads of v, once those of w have arrived (scalar loads end in any order, so a wait is
+  // for all that are out)
+  auto ld = [&](int32_t i, double (&v)[2 * kStB], const double (&w)[2 * kStB]) {
+    asm volatile("" ::"s"(w[0]), "s"(w[2 * kStB - 1]));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2 * kStB; ++u) v[u] = T[2 * i + u];
+    __builtin_amdgcn_sched_barrier(0);  // not moved down to their use
+  };
+  double a[2 * kStB], b[2 * kStB];
+#pragma unroll
+  for (int u = 0; u < 2 * kStB; ++u) a[u] = T[u];
+  const int32_t rows = sturm_rows(n);
+  for (int32_t i = 0; i < rows; i += 2 * kStB) {
+    ld(i + kStB, b, a);
+    run(a);
+    ld(i + 2 * kStB, a, b);
+    run(b);
+  }
   return cnt;
 }
 
-// kMS lanes per eigenvalue (k-th smallest): each round the lanes evaluate kMS interior
-// points of [lo, hi] and keep the sub-interval holding eigenvalue k.  One count per
-// lane; at N=5,000 (after the grid) 8 lanes took 2.52 ms, 4 lanes 3.16, 16 lanes 2.94
-// and 32 lanes 3.70: more lanes cut the rounds but add each round's work.
-constexpr int kMS = 8;
 // Shared first level: Sturm counts at kMsGrid evenly spaced interior points of the
 // Gershgorin interval, one per thread (each a count over the whole tridiagonal, like
 // one round of the multisection for kMsGrid / 16 eigenvalues).  Every eigenvalue then
@@ -1072,9 +1088,17 @@ __device__ __forceinline__ double msgrid_x(double glo, double ghi, int32_t j) {
 }
 __global__ __launch_bounds__(256) void k_msgrid(EigWs ws, int32_t n, int32_t *__restrict__ gcnt) {
   const int32_t j = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);  // kMsGrid threads
-  gcnt[j] = sturm1(ws.d, ws.e2, n, msgrid_x(ws.sc[S_GL], ws.sc[S_GU], j), ws.sc[S_PIVMIN]);
+  sturm_warm(ws.st, n);
+  gcnt[j] = sturm1(ws.st, n, msgrid_x(ws.sc[S_GL], ws.sc[S_GU], j) * ws.sc[S_SCALE]);
 }
+// kMS lanes per eigenvalue (k-th smallest): each round the lanes evaluate kMS interior
+// points of [lo, hi] and keep the sub-interval holding eigenvalue k.  One count per lane.  A
+// round takes the same time while the waves fit one per SIMD and more lanes save rounds, so
+// the launch takes 64 lanes up to order 1,024 and halves them for every doubling, down to 8;
+// with more waves than SIMDs a round's work counts.  With the counts' grid: order 198 108 ->
+// 33 us, 1,000 490 -> 125, 1,203 590 -> 180, 5,000 2.46 -> 1.05 ms.
 // gcnt: k_msgrid's counts, or null to start from the Gershgorin interval
+template <int kMS>
 __global__ __launch_bounds__(256) void k_multisect(EigWs ws, int32_t n,
                                                    const int32_t *__restrict__ gcnt) {
   const int32_t k = (int32_t)((blockIdx.x * blockDim.x + threadIdx.x) / kMS);
@@ -1100,6 +1124,7 @@ __global__ __launch_bounds__(256) void k_multisect(EigWs ws, int32_t n,
   // eigenvalue at zero (the centred matrix has one) converges in ~13 rounds instead
   // of running to the round cap with a relative tolerance alone
   const double atol = eps * ws.sc[S_TNORM];
+  sturm_warm(ws.st, n);
   for (int it = 0; it < 96; ++it) {
     const double tol = 2.0 * eps * fmax(fabs(lo), fabs(hi)) + 4.0 * pivmin + atol;
     const bool done = (hi - lo <= tol);
@@ -1108,7 +1133,7 @@ __global__ __launch_bounds__(256) void k_multisect(EigWs ws, int32_t n,
     const double w = (hi - lo) / (double)(kMS + 1);
     const double x = lo + w * (double)(sub + 1);
     int32_t cnt = 0;
-    if (active && !done) cnt = sturm1(ws.d, ws.e2, n, x, pivmin);
+    if (active && !done) cnt = sturm1(ws.st, n, x * ws.sc[S_SCALE]);
     // new lo = largest point with count <= k ; new hi = smallest point with count > k
     double cand_lo = (cnt <= k) ? x : -1e300;
     double cand_hi = (cnt > k) ? x : 1e300;
@@ -1894,7 +1919,7 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   size_t o_a = add((size_t)N * lda), o_d = add(N), o_e = add(N), o_e2 = add(N),
          o_tau = add(N), o_V = add(kNB * N), o_W = add(kNB * N), o_x = add(lda), o_y = add((size_t)ntile * lda),
          o_sc = add(S_COUNT), o_p1 = add((size_t)maxblk * maxnv),
-         o_ev = add(N),
+         o_ev = add(N), o_st = add(2 * (size_t)(sturm_rows(n) + kStB)),
          o_X = add((size_t)kMaxVec * N), o_lu = add((size_t)kMaxVec * kLuF * N),
          o_Z = add(kNB * kMaxVec), o_T = add((size_t)npanel * kNB * kNB),
          o_pw = add((size_t)2 * maxw * kPW), o_ps = add((size_t)(ntile * (ntile + 1) / 2)), o_sync = add(8);
@@ -1914,6 +1939,7 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   ws.sc = (double *)(base + o_sc);
   ws.part1 = (double *)(base + o_p1);
   ws.eval = (double *)(base + o_ev);
+  ws.st = (double2 *)(base + o_st);
   ws.X = (double *)(base + o_X);
   ws.lu = (double *)(base + o_lu);
   ws.Z = (double *)(base + o_Z);
@@ -1964,8 +1990,8 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   // ---- eigenvalues
   tbeg();
   hipLaunchKernelGGL(k_gersh, dim3(1), dim3(256), 0, st, ws, n);
+  hipLaunchKernelGGL(k_sturm_prep, dim3((unsigned)((sturm_rows(n) + kStB + 255) / 256)), dim3(256), 0, st, ws, n);
   {
-    int64_t threads = (int64_t)n * kMS;
     // the grid's counts go to the inverse iteration's LU area, unused until then
     // (kMaxVec * 5 * N doubles hold the kMsGrid counts from N = 103 on)
     int32_t *gcnt = nullptr;
@@ -1973,7 +1999,13 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
       gcnt = (int32_t *)ws.lu;
       hipLaunchKernelGGL(k_msgrid, dim3(kMsGrid / 256), dim3(256), 0, st, ws, n, gcnt);
     }
-    hipLaunchKernelGGL(k_multisect, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, ws, n,
+    int32_t lanes = 64;
+    while (lanes > 8 && (int64_t)n * lanes > (int64_t)ctx->num_cu * 256) lanes /= 2;
+    auto kern = lanes == 64   ? k_multisect<64>
+                : lanes == 32 ? k_multisect<32>
+                : lanes == 16 ? k_multisect<16>
+                              : k_multisect<8>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(((int64_t)n * lanes + 255) / 256)), dim3(256), 0, st, ws, n,
                        (const int32_t *)gcnt);
   }
   EIG_HIP(ctx, hipGetLastError());
