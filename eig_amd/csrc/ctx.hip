@@ -1,8 +1,12 @@
 // Context, device memory, genotype upload, synthetic generator, sample selection
 // and per-SNP column statistics.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
+#include <exception>
+#include <thread>
+#include <utility>
 #include <vector>
 
 #include "eig_internal.h"
@@ -38,11 +42,114 @@ int eig_ensure(eig_ctx *ctx, DevBuf &b, size_t bytes) {
 void eig_time_begin(eig_ctx *ctx) { hipEventRecord(ctx->ev0, ctx->stream); }
 
 void eig_time_end(eig_ctx *ctx, const char *what) {
-  hipEventRecord(ctx->ev1, ctx->stream);
-  hipEventSynchronize(ctx->ev1);
-  float ms = -1.f;
-  hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
-  ctx->ms[what] = ms;
+  eig_ctx::Stage &s = ctx->stages[what];
+  if (!s.begin && hipEventCreate(&s.begin) != hipSuccess) s.begin = nullptr;
+  if (!s.end && hipEventCreate(&s.end) != hipSuccess) s.end = nullptr;
+  if (!s.begin || !s.end) return;
+  std::swap(s.begin, ctx->ev0);
+  hipEventRecord(s.end, ctx->stream);
+}
+
+// ---- results to pageable host memory
+namespace {
+constexpr size_t kPinSmall = (size_t)1 << 20;   // pinned room for small results
+constexpr size_t kFetchSmall = (size_t)1 << 18;  // a result that goes there
+constexpr size_t kFetchBig = (size_t)2 << 20;    // one that several threads copy
+constexpr size_t kPiece = (size_t)1 << 20;
+constexpr int kFetchThreads = 4;
+}  // namespace
+
+static int ensure_pinned(eig_ctx *ctx, size_t bytes) {
+  DevBuf &b = ctx->hostpin;
+  if (b.bytes >= bytes) return EIG_OK;
+  if (b.p) {
+    EIG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    hipHostFree(b.p);
+    b = DevBuf();
+  }
+  if (hipHostMalloc(&b.p, bytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();  // the caller copies without it
+    b.p = nullptr;
+    return EIG_E_NOMEM;
+  }
+  b.bytes = bytes;
+  return EIG_OK;
+}
+
+int EigFetch::get(void *dst, const void *src, size_t bytes) {
+  if (!dst || bytes == 0) return EIG_OK;
+  if (bytes >= kFetchBig) return big((char *)dst, (const char *)src, bytes);
+  if (bytes > kFetchSmall || used_ + bytes > kPinSmall || ensure_pinned(ctx_, kPinSmall) != EIG_OK) {
+    EIG_HIP(ctx_, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx_->stream));
+    return EIG_OK;
+  }
+  EIG_HIP(ctx_, hipMemcpyAsync((char *)ctx_->hostpin.p + used_, src, bytes, hipMemcpyDeviceToHost,
+                               ctx_->stream));
+  small_.push_back({dst, used_, bytes});
+  used_ += (bytes + 63) & ~(size_t)63;
+  return EIG_OK;
+}
+
+int EigFetch::wait() {
+  EIG_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
+  for (const Piece &q : small_) std::memcpy(q.dst, (const char *)ctx_->hostpin.p + q.at, q.bytes);
+  small_.clear();
+  used_ = 0;
+  return EIG_OK;
+}
+
+// Thread w takes pieces w, w + kFetchThreads, ..: the copy of its next piece is queued before
+// it waits for the one under way.  Loadings and projections of 5,000 x 600,000 with ten
+// columns of results (48 MB) took 8.4 ms, 4.1 of them one hipMemcpyAsync; now 5.6.
+int EigFetch::big(char *dst, const char *src, size_t bytes) {
+  // the pinned area may move while it grows: the small ones in it first
+  if (!small_.empty() || used_) EIG_TRY(wait());
+  if (ensure_pinned(ctx_, kPinSmall + 2 * kFetchThreads * kPiece) != EIG_OK) {
+    EIG_HIP(ctx_, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx_->stream));
+    return EIG_OK;
+  }
+  const size_t np = (bytes + kPiece - 1) / kPiece;
+  char *ring = (char *)ctx_->hostpin.p + kPinSmall;
+  hipError_t err[kFetchThreads] = {};
+  auto work = [&](int w) {
+    hipError_t &e = err[w];
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    e = hipSetDevice(ctx_->device);
+    for (hipEvent_t &v : ev)
+      if (e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+    auto room = [&](int k) { return ring + (2 * (size_t)w + k) * kPiece; };
+    auto len = [&](size_t i) { return std::min(kPiece, bytes - i * kPiece); };
+    auto queue = [&](size_t i, int k) {
+      e = hipMemcpyAsync(room(k), src + i * kPiece, len(i), hipMemcpyDeviceToHost, ctx_->stream);
+      if (e == hipSuccess) e = hipEventRecord(ev[k], ctx_->stream);
+    };
+    int k = 0;
+    if (e == hipSuccess && (size_t)w < np) queue(w, k);
+    for (size_t i = w; e == hipSuccess && i < np; i += kFetchThreads, k ^= 1) {
+      if (i + kFetchThreads < np) queue(i + kFetchThreads, k ^ 1);
+      if (e == hipSuccess) e = hipEventSynchronize(ev[k]);
+      if (e == hipSuccess) std::memcpy(dst + i * kPiece, room(k), len(i));
+    }
+    for (hipEvent_t v : ev)
+      if (v) hipEventDestroy(v);
+  };
+  std::thread th[kFetchThreads];
+  bool ran[kFetchThreads] = {};
+  for (int w = 1; w < kFetchThreads; ++w) try {
+      th[w] = std::thread(work, w);
+      ran[w] = true;
+    } catch (const std::exception &) {
+    }
+  work(0);
+  for (int w = 1; w < kFetchThreads; ++w)
+    if (ran[w]) th[w].join();
+    else work(w);  // no thread to be had
+  for (hipError_t e : err)
+    if (e != hipSuccess) {
+      hipStreamSynchronize(ctx_->stream);
+      return eig_set_err(ctx_, EIG_E_HIP, "copy of results: %s", hipGetErrorString(e));
+    }
+  return EIG_OK;
 }
 
 static void free_buf(DevBuf &b) {
@@ -81,7 +188,7 @@ extern "C" int eig_open(int device, eig_ctx **out) {
   c->noalloc = ws;
   c->noalloc_bytes = kNoAllocBytes;
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
+      hipEventCreate(&c->ev0) != hipSuccess) {
     delete c;
     return EIG_E_HIP;
   }
@@ -103,7 +210,10 @@ extern "C" void eig_close(eig_ctx *ctx) {
   for (DevBuf *b : bufs) free_buf(*b);
   if (ctx->hostpin.p) hipHostFree(ctx->hostpin.p);
   hipEventDestroy(ctx->ev0);
-  hipEventDestroy(ctx->ev1);
+  for (auto &s : ctx->stages) {
+    if (s.second.begin) hipEventDestroy(s.second.begin);
+    if (s.second.end) hipEventDestroy(s.second.end);
+  }
   hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -114,6 +224,14 @@ extern "C" const char *eig_last_error(const eig_ctx *ctx) {
 
 extern "C" double eig_last_ms(const eig_ctx *ctx, const char *what) {
   if (!ctx || !what) return -1.0;
+  auto st = ctx->stages.find(what);
+  if (st != ctx->stages.end()) {
+    float t = -1.f;
+    if (!st->second.begin || !st->second.end || hipEventSynchronize(st->second.end) != hipSuccess ||
+        hipEventElapsedTime(&t, st->second.begin, st->second.end) != hipSuccess)
+      return -1.0;
+    return t;
+  }
   auto it = ctx->ms.find(what);
   return it == ctx->ms.end() ? -1.0 : it->second;
 }
@@ -355,6 +473,7 @@ extern "C" int eig_select(eig_ctx *ctx, const int32_t *xindex, int32_t nrows) {
                      ident, (uint32_t *)ctx->sel.p);
   EIG_HIP(ctx, hipGetLastError());
   eig_time_end(ctx, "select");
+  EIG_HIP(ctx, hipStreamSynchronize(ctx->stream));  // xindex is the caller's
   ctx->nrows = nrows;
   ctx->nst = nst;
   ctx->have_sel = true;
@@ -487,9 +606,9 @@ extern "C" int eig_snpstats(eig_ctx *ctx, const uint8_t *live, int32_t altnorm,
     size_t b;
   } outs[] = {{c0, &ctx->c0, 4 * M},     {c1, &ctx->c1, 4 * M},     {nmiss, &ctx->nmiss, 4 * M},
               {mean, &ctx->mean, 8 * M}, {fancy, &ctx->fancy, 8 * M}, {status, &ctx->status, 4 * M}};
-  for (auto &o : outs)
-    if (o.h) EIG_HIP(ctx, hipMemcpyAsync(o.h, o.d->p, o.b, hipMemcpyDeviceToHost, ctx->stream));
-  EIG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  EigFetch f(ctx);
+  for (auto &o : outs) EIG_TRY(f.get(o.h, o.d->p, o.b));
+  EIG_TRY(f.wait());
   ctx->have_stats = true;
   ctx->have_xtx = ctx->have_load = false;
   return EIG_OK;

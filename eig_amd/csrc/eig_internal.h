@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <map>
 #include <string>
+#include <vector>
 
 #include "../../include/eig_abi.h"
 
@@ -27,9 +28,14 @@ struct DevBuf {
 struct eig_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  hipEvent_t ev0 = nullptr;  // begin of the stage under way
   std::string err;
   std::map<std::string, double> ms;
+  // stage times: the events around each stage's last run, read when they are asked for
+  struct Stage {
+    hipEvent_t begin = nullptr, end = nullptr;
+  };
+  std::map<std::string, Stage> stages;
   int num_cu = 0;
 
   // genotypes as loaded (GENO row layout)
@@ -90,6 +96,27 @@ struct eig_ctx {
 
 int eig_set_err(eig_ctx *ctx, int code, const char *fmt, ...);
 int eig_ensure(eig_ctx *ctx, DevBuf &b, size_t bytes);
+// Results to the caller's (pageable) memory.  The runtime's own copies wait for each one,
+// and move 12 GB/s.  get() queues a small copy into pinned memory, and the caller's memory
+// is filled in wait(); a large one is done at once by several threads, each with two pinned
+// pieces, one arriving while the other is copied on.  One at a time per context.
+class EigFetch {
+ public:
+  explicit EigFetch(eig_ctx *ctx) : ctx_(ctx) {}
+  int get(void *dst, const void *src, size_t bytes);
+  int wait();  // the stream is idle and everything is in place
+
+ private:
+  struct Piece {
+    void *dst;
+    size_t at, bytes;
+  };
+  int big(char *dst, const char *src, size_t bytes);
+  eig_ctx *ctx_;
+  std::vector<Piece> small_;
+  size_t used_ = 0;
+};
+// a stage's events; its time is read by eig_last_ms, and nothing waits here
 void eig_time_begin(eig_ctx *ctx);
 void eig_time_end(eig_ctx *ctx, const char *what);
 

@@ -2114,8 +2114,6 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
     wx.X = XT;
     hipLaunchKernelGGL(k_finish_vec, dim3((unsigned)nvec), dim3(256), 0, st, wx, n);
     EIG_HIP(ctx, hipGetLastError());
-    if (evecs)
-      EIG_HIP(ctx, hipMemcpyAsync(evecs, XT, sizeof(double) * N * nvec, hipMemcpyDeviceToHost, st));
     if (!internal) {
       EIG_TRY(eig_ensure(ctx, ctx->evecs_dev, sizeof(double) * N * kMaxVec));
       EIG_HIP(ctx, hipMemcpyAsync(ctx->evecs_dev.p, XT, sizeof(double) * N * kMaxVec,
@@ -2127,17 +2125,16 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   }
   tend("eigvec");
   std::vector<double> asc(N);
-  EIG_HIP(ctx, hipMemcpyAsync(asc.data(), ws.eval, sizeof(double) * N, hipMemcpyDeviceToHost, st));
-  if (nvec > 0 && nvec <= kMaxVec) {
-    if (evecs)
-      EIG_HIP(ctx, hipMemcpyAsync(evecs, ws.X, sizeof(double) * N * nvec, hipMemcpyDeviceToHost, st));
-    if (!internal) {
-      EIG_TRY(eig_ensure(ctx, ctx->evecs_dev, sizeof(double) * N * std::max(nvec, 1)));
-      EIG_HIP(ctx, hipMemcpyAsync(ctx->evecs_dev.p, ws.X, sizeof(double) * N * nvec,
-                                  hipMemcpyDeviceToDevice, st));
-    }
+  EigFetch f(ctx);
+  EIG_TRY(f.get(asc.data(), ws.eval, sizeof(double) * N));
+  if (nvec > 0 && evecs)
+    EIG_TRY(f.get(evecs, nvec <= kMaxVec ? ws.X : (double *)ctx->evall.p, sizeof(double) * N * nvec));
+  if (nvec > 0 && nvec <= kMaxVec && !internal) {
+    EIG_TRY(eig_ensure(ctx, ctx->evecs_dev, sizeof(double) * N * nvec));
+    EIG_HIP(ctx, hipMemcpyAsync(ctx->evecs_dev.p, ws.X, sizeof(double) * N * nvec,
+                                hipMemcpyDeviceToDevice, st));
   }
-  EIG_HIP(ctx, hipStreamSynchronize(st));
+  EIG_TRY(f.wait());
   for (int64_t i = 0; i < N; ++i) {
     if (std::isnan(asc[i])) return eig_set_err(ctx, EIG_E_CONVERGE, "eigenvalue is NaN");
     if (evals) evals[i] = asc[N - 1 - i];

@@ -867,9 +867,9 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   const size_t o_ta = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxa * npad) : 0;
   const size_t o_tb = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxb * Mpad) : 0;
   const size_t o_tab = bf ? add(sizeof(uint32_t) * 2 * kFpTab * (size_t)(Mpad / kGrp)) : 0;
+  EIG_TRY(eig_ensure_selg(ctx));
   // FP64 form: the code products' digit operands and INT32 sums (codes.hip), one area for
   // the X A, X^T B and finishing X^T U products
-  if (!bf) EIG_TRY(eig_ensure_selg(ctx));
   const int64_t G64 = Mpad / kGrp;
   const CodeView vm{(const uint8_t *)ctx->sel.p, nullptr, 128 * 32, 32, M * 32, 16, M, (int64_t)nst * 8,
                     kCodeLinear};
@@ -927,7 +927,6 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
     hipLaunchKernelGGL(k_fpca_tab, dim3((unsigned)(G64 * (kFpTab / 256))), dim3(256), 0, st,
                        (const uint32_t *)lbf, M, G64, tabs);
     EIG_HIP(ctx, hipGetLastError());
-    EIG_TRY(eig_ensure_selg(ctx));
   }
   // X A and X^T B of the FP64 form: `plan`'s product of the codes with cols, its INT32 sums
   // left in the work area

@@ -511,14 +511,15 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
                      (double *)ctx->fancy.p, (double *)ctx->lev.p);
   EIG_HIP(ctx, hipGetLastError());
   std::vector<int32_t> hst(M);
-  EIG_HIP(ctx, hipMemcpyAsync(hst.data(), ctx->status.p, 4 * (size_t)M, hipMemcpyDeviceToHost, st));
+  EigFetch f(ctx);
+  EIG_TRY(f.get(hst.data(), ctx->status.p, 4 * (size_t)M));
   struct {
     int32_t *h;
     DevBuf *d;
   } outs[] = {{c0, &ctx->c0}, {c1, &ctx->c1}, {nmiss, &ctx->nmiss}};
   for (auto &o : outs)
-    if (o.h) EIG_HIP(ctx, hipMemcpyAsync(o.h, o.d->p, 4 * (size_t)M, hipMemcpyDeviceToHost, st));
-  EIG_HIP(ctx, hipStreamSynchronize(st));
+    EIG_TRY(f.get(o.h, o.d->p, 4 * (size_t)M));
+  EIG_TRY(f.wait());
   if (status) std::memcpy(status, hst.data(), 4 * (size_t)M);
   std::vector<int32_t> kl;  // kept SNPs in order
   for (int64_t m = 0; m < M; ++m)

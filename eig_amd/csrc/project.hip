@@ -281,10 +281,10 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
   hipLaunchKernelGGL(k_fxscal, dim3((unsigned)K), dim3(256), 0, st, (const double *)d_fxv, n, d_fx);
   EIG_HIP(ctx, hipGetLastError());
   eig_time_end(ctx, "loadings");
-  if (ffvecs)
-    EIG_HIP(ctx, hipMemcpyAsync(ffvecs, ctx->ffvecs.p, 8 * (size_t)K * M, hipMemcpyDeviceToHost, st));
-  if (fxscal) EIG_HIP(ctx, hipMemcpyAsync(fxscal, d_fx, 8 * (size_t)K, hipMemcpyDeviceToHost, st));
-  EIG_HIP(ctx, hipStreamSynchronize(st));
+  EigFetch f(ctx);
+  EIG_TRY(f.get(ffvecs, ctx->ffvecs.p, 8 * (size_t)K * M));
+  EIG_TRY(f.get(fxscal, d_fx, 8 * (size_t)K));
+  EIG_TRY(f.wait());
   ctx->last_K = K;
   ctx->have_load = true;
   return EIG_OK;
@@ -475,10 +475,11 @@ static int lsqproject(eig_ctx *ctx, const int32_t *use, const int32_t *itype, in
   eig_time_end(ctx, "lsqproject");
   std::vector<double> ans((size_t)K * nind), rhs((size_t)K * nind);
   std::vector<int32_t> sv(nind);
-  EIG_HIP(ctx, hipMemcpyAsync(ans.data(), d_ans, 8 * (size_t)K * nind, hipMemcpyDeviceToHost, st));
-  EIG_HIP(ctx, hipMemcpyAsync(rhs.data(), d_rhs, 8 * (size_t)K * nind, hipMemcpyDeviceToHost, st));
-  EIG_HIP(ctx, hipMemcpyAsync(sv.data(), d_st, 4 * (size_t)nind, hipMemcpyDeviceToHost, st));
-  EIG_HIP(ctx, hipStreamSynchronize(st));
+  EigFetch f(ctx);
+  EIG_TRY(f.get(ans.data(), d_ans, 8 * (size_t)K * nind));
+  EIG_TRY(f.get(rhs.data(), d_rhs, 8 * (size_t)K * nind));
+  EIG_TRY(f.get(sv.data(), d_st, 4 * (size_t)nind));
+  EIG_TRY(f.wait());
   // regans persists across individuals in the reference (smartpca.c:4656,
   // regsubs.c:51-53): a failed solve keeps the previous individual's answer.
   double last[kMaxK];

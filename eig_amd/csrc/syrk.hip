@@ -621,8 +621,12 @@ int eig_run_syrk(eig_ctx *ctx, int form, int bf16_block, double *trace_scale) {
                      (const double *)ctx->part.p, P, nsplit, n, d_tr, (double *)ctx->xtx.p);
   EIG_HIP(ctx, hipGetLastError());
   double tr = 0.0;
-  EIG_HIP(ctx, hipMemcpyAsync(&tr, d_tr, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   eig_time_end(ctx, "xtx_finalize");
+  {
+    EigFetch f(ctx);
+    EIG_TRY(f.get(&tr, d_tr, sizeof(double)));
+    EIG_TRY(f.wait());
+  }
   double y = tr / (double)(n - 1);
   if (trace_scale) *trace_scale = y;
   if (std::isnan(y)) return eig_set_err(ctx, EIG_E_NUMERIC, "bad XTX matrix");
@@ -645,9 +649,9 @@ extern "C" int eig_xtx(eig_ctx *ctx, int32_t form, int32_t bf16_block, double *t
   ctx->have_xtx = false;
   EIG_TRY(eig_run_syrk(ctx, form, bf16_block, trace_scale));
   if (xtx_out) {
-    EIG_HIP(ctx, hipMemcpyAsync(xtx_out, ctx->xtx.p, sizeof(double) * (size_t)ctx->nrows * ctx->nrows,
-                                hipMemcpyDeviceToHost, ctx->stream));
-    EIG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    EigFetch f(ctx);
+    EIG_TRY(f.get(xtx_out, ctx->xtx.p, sizeof(double) * (size_t)ctx->nrows * ctx->nrows));
+    EIG_TRY(f.wait());
   }
   ctx->have_xtx = true;
   return EIG_OK;
