@@ -1605,7 +1605,7 @@ __global__ __launch_bounds__(256) void k_bt_gram(EigWs ws, int32_t n, int32_t la
   for (int k = 0; k < 4; ++k) out[threadIdx.x + 256 * k] = g[k];
 }
 __global__ __launch_bounds__(256) void k_bt_prep(EigWs ws, int32_t n, int32_t last) {
-  __shared__ double G[kNB][kNB + 1], T[kNB][kNB + 1];
+  __shared__ double G[kNB][kNB + 1], tau[kNB];
   const int32_t p = blockIdx.x;
   const int32_t c0 = p * kNB;
   const int32_t nb = min(kNB, last - c0 + 1);
@@ -1621,22 +1621,98 @@ __global__ __launch_bounds__(256) void k_bt_prep(EigWs ws, int32_t n, int32_t la
     const int idx = threadIdx.x + 256 * k;
     G[idx / kNB][idx % kNB] = g[k];
   }
-  for (int idx = threadIdx.x; idx < kNB * kNB; idx += 256) T[idx / kNB][idx % kNB] = 0.0;
+  if (threadIdx.x < kNB) tau[threadIdx.x] = (int)threadIdx.x < nb ? ws.tau[c0 + threadIdx.x] : 0.0;
   __syncthreads();
-  for (int jj = 0; jj < nb; ++jj) {
-    const double tj = ws.tau[c0 + jj];
-    // T[i][jj] for i < jj in parallel; T is upper triangular
+  if (threadIdx.x >= kNB) return;
+  // a row of T needs only itself and G: a lane per row, no barriers (column by column with
+  // the rows in LDS took 29 us, now 10)
+  const int i = threadIdx.x;
+  double row[kNB];
+#pragma unroll
+  for (int jj = 0; jj < kNB; ++jj) {
     double s = 0.0;
-    const int i = threadIdx.x;
-    if (i < jj)
-      for (int k = i; k < jj; ++k) s += T[i][k] * G[k][jj];
+#pragma unroll
+    for (int k = 0; k < jj; ++k) s += row[k] * G[k][jj];
+    row[jj] = i < jj ? -tau[jj] * s : (i == jj ? tau[jj] : 0.0);
+  }
+  double *T = ws.Tall + ((int64_t)p * kNB + i) * kNB;
+#pragma unroll
+  for (int jj = 0; jj < kNB; ++jj) T[jj] = row[jj];
+}
+
+// All panels for one vector (a block): no launch per panel and no sums between blocks.  A
+// wave forms the dots of four reflectors, a thread two products of T, then the threads update
+// a row each, whose reflector entries are loaded before the dots are known.  Bound by those
+// two trips to L2 a panel and by what one block can read: with T, ten vectors of order 300
+// take 0.086 ms (0.161 by k_bt_step and k_bt_reduce), 1,000 0.28 (0.39), 1,600 0.53 (0.60),
+// 2,000 0.76 (0.75), where the line lies.
+constexpr int kBtVecN = 1600;
+__global__ __launch_bounds__(512) void k_bt_vec(EigWs ws, int32_t n, int32_t last) {
+  constexpr int R = kNB / 8;  // reflectors per wave
+  __shared__ double sx[kBtVecN], ss[kNB], sz[kNB];
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int32_t lda = ws.lda;
+  double *x = ws.X + (int64_t)blockIdx.x * n;
+  for (int32_t i = t; i < n; i += 512) sx[i] = x[i];
+  __syncthreads();
+  for (int32_t p = last / kNB; p >= 0; --p) {
+    const int32_t c0 = p * kNB, nb = min(kNB, last - c0 + 1);
+    const double *T = ws.Tall + (int64_t)p * kNB * kNB + t;  // T_p[t / 32][t % 32] and 16 rows on
+    const double t0 = T[0], t1 = T[512];
+    const double *vq[R];
+    double s[R];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      vq[u] = ws.a + (int64_t)(c0 + min(R * w + u, nb - 1)) * lda;
+      s[u] = 0.0;
+    }
+#pragma unroll 4
+    for (int32_t r = c0 + 1 + lane; r < n; r += 64) {
+      const double xr = sx[r];
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const double a = vq[u][r];
+        s[u] += (r > c0 + R * w + u ? a : 0.0) * xr;
+      }
+    }
+    auto entries = [&](int32_t r, double (&v)[kNB]) {
+      const int32_t at = min(r, n - 1);  // rows past the end read the last one
+#pragma unroll
+      for (int q = 0; q < kNB; ++q) v[q] = (ws.a + (int64_t)(c0 + min(q, nb - 1)) * lda)[at];
+    };
+    double v[kNB];
+    int32_t r = c0 + 1 + t;
+    entries(r, v);
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) s[u] += xlane(s[u], o);
+      if (lane == 0) ss[R * w + u] = R * w + u < nb ? s[u] : 0.0;
+    }
     __syncthreads();
-    if (i < jj) T[i][jj] = -tj * s;
-    if (i == jj) T[jj][jj] = tj;
+    double z0 = t0 * ss[t & (kNB - 1)], z1 = t1 * ss[t & (kNB - 1)];
+#pragma unroll
+    for (int o = kNB / 2; o > 0; o >>= 1) {
+      z0 += xlane(z0, o);
+      z1 += xlane(z1, o);
+    }
+    if ((t & (kNB - 1)) == 0) {
+      sz[t / kNB] = t / kNB < nb ? z0 : 0.0;
+      sz[t / kNB + 16] = t / kNB + 16 < nb ? z1 : 0.0;
+    }
+    __syncthreads();
+    for (;;) {
+      double y = 0.0;
+#pragma unroll
+      for (int q = 0; q < kNB; ++q) y += (r > c0 + q ? v[q] : 0.0) * sz[q];
+      if (r < n) sx[r] -= y;
+      r += 512;
+      if (r >= n) break;
+      entries(r, v);
+    }
     __syncthreads();
   }
-  for (int idx = threadIdx.x; idx < kNB * kNB; idx += 256)
-    ws.Tall[(int64_t)p * kNB * kNB + idx] = T[idx / kNB][idx % kNB];
+  for (int32_t i = t; i < n; i += 512) x[i] = sx[i];
 }
 
 // Fused step for panel p: X[r] -= sum_q v_{p+1,q}[r] Z[q] (previous panel, if any),
@@ -2018,7 +2094,9 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   const int32_t last = n - 2;  // last reflector row
   const int32_t p_last = last >= 0 ? last / kNB : -1;
   auto back_transform = [&](int32_t nb) -> int {
-    if (last >= 0) {
+    if (last >= 0 && n <= kBtVecN) {
+      hipLaunchKernelGGL(k_bt_vec, dim3((unsigned)nb), dim3(512), 0, st, ws, n, last);
+    } else if (last >= 0) {
       for (int32_t p = p_last; p >= 0; --p) {
         const int32_t c0 = p * kNB;
         const unsigned g = (unsigned)((n - c0 - 1 + kBtRows - 1) / kBtRows);

@@ -54,3 +54,9 @@ def _check(eng, kind, n):
     assert np.max(np.abs(w - ref)) <= tol * norm
     assert np.max(np.abs(v @ v.T - np.eye(nvec))) <= 8 * tol
     assert np.max(np.abs((v @ a - w[:nvec, None] * v) / norm)) <= tol
+
+
+@pytest.mark.parametrize("n", [2, 33, 34, 65, 512, 513, 545, 1025, 1599, 1600, 1601])
+def test_back_transform(eng, n):
+    """Panels of 32 reflectors, a thread's 512 rows, and the line between the two kernels."""
+    _check(eng, "random", n)
