@@ -445,7 +445,10 @@ def main():
     alg_flops = 3.0 * N * (N + 1) * M    # the compensated SYRK's three products
     useful_flops = 1.0 * N * (N + 1) * M  # the XTX itself (lower triangle, 2 flop/MAC)
     syrk_s = b["syrk_ms"] * 1e-3
-    tri_bytes = 8 * (N - 1) * N * (2 * N - 1) // 6  # sum over L = 1 .. N-1 of L^2 doubles
+    # the upper triangle of the trailing matrix per column of more than 2,048 rows (the rest
+    # stays in registers): sum over L = 2049 .. N-1 of L (L + 1) / 2 doubles
+    tri_sum = lambda L: L * (L + 1) * (L + 2) // 6
+    tri_bytes = 8 * max(0, tri_sum(N - 1) - tri_sum(2048))
     tri_ach = tri_bytes / (b["parts"]["tridiag"] * 1e-3) / 1e9
     # decode + normalise: GENO rows read (rlen each) and 28 B of per-SNP statistics written
     rlen = max(48, (2 * N + 7) // 8)
@@ -482,14 +485,14 @@ def main():
                                  "syrk": b["syrk_ms"], **b["parts"]},
                       "bf16x3": {"syrk": b3["syrk_ms"], **b3["parts"]},
                       "fp64": {"syrk": f["syrk_ms"], **f["parts"]}},
-        # the dominant stage of the headline pass: the tridiagonalisation, one graph
-        # launch per pass (k_symv / k_wcol / k_column / k_syr2k); its symv streams each
-        # column's L x L trailing square once (L = N-1 .. 1); HIP-event time of the
-        # launch on the context stream, per-column latency included
+        # the dominant stage of the headline pass: the tridiagonalisation (k_symv / k_wcol /
+        # k_syr2k down to order 2,048, then k_tri); its symv streams the upper triangle of
+        # each column's trailing matrix once; HIP-event time of the stage on the context
+        # stream, per-column latency and the resident columns included
         "roofline": {"bound": "hbm", "achieved": round(tri_ach, 1), "peak": PEAK_HBM,
                      "unit": "GB/s", "frac": round(tri_ach / PEAK_HBM, 4), "traffic": traffic,
                      "traffic_source": tsrc,
-                     "kernel": "tridiagonalisation graph (k_symv<4>, k_wcol, k_column, k_syr2k)",
+                     "kernel": "tridiagonalisation (k_symv, k_wcol, k_syr2k, k_tri)",
                      "algorithmic_bytes": tri_bytes, "ms": round(b["parts"]["tridiag"], 3)},
         "syrk_roofline": {"kernel": "k_syrk_bf16<true, true>", "bound": "mfma", "ms": round(b["syrk_ms"], 3),
                           "peak": PEAK_BF16, "unit": "TFLOP/s",
@@ -499,10 +502,12 @@ def main():
                           "alg_3product_frac": round(alg_flops / syrk_s / 1e12 / PEAK_BF16, 4),
                           "useful_rate": round(useful_flops / syrk_s / 1e12, 1),
                           "mfma_flops": mfma_flops, "alg_flops": alg_flops},
-        "fp64_syrk_roofline": {"kernel": "k_syrk_f64",
+        # the FP64 form's products run on the INT8 matrix cores (digit planes): the XTX's own
+        # operations over the stage's time, against what the FP64 matrix cores could do
+        "fp64_syrk_roofline": {"kernel": "k_xd_gemm", "bound": "int8 mfma",
                                "achieved": round(useful_flops / (f["syrk_ms"] * 1e-3) / 1e12, 2),
-                               "peak": PEAK_FP64, "unit": "TFLOP/s",
-                               "frac": round(useful_flops / (f["syrk_ms"] * 1e-3) / 1e12 / PEAK_FP64, 4)},
+                               "unit": "TFLOP/s", "fp64_mfma_peak": PEAK_FP64,
+                               "ms": round(f["syrk_ms"], 3)},
         "decode_normalise": {"kernels": "k_select + k_snpstats", "bytes": dec_bytes,
                              "ms": round(dec_ms, 4),
                              "achieved_GBps": round(dec_bytes / (dec_ms * 1e-3) / 1e9, 1),

@@ -52,8 +52,8 @@ void eig_time_end(eig_ctx *ctx, const char *what) {
 
 // ---- results to pageable host memory
 namespace {
-constexpr size_t kPinSmall = (size_t)1 << 20;   // pinned room for small results
-constexpr size_t kFetchSmall = (size_t)1 << 18;  // a result that goes there
+constexpr size_t kPinSmall = (size_t)1 << 19;    // pinned room for small results
+constexpr size_t kFetchSmall = (size_t)1 << 17;  // a result that goes there
 constexpr size_t kFetchBig = (size_t)2 << 20;    // one that several threads copy
 constexpr size_t kPiece = (size_t)1 << 20;
 constexpr int kFetchThreads = 4;
@@ -100,7 +100,8 @@ int EigFetch::wait() {
 
 // Thread w takes pieces w, w + kFetchThreads, ..: the copy of its next piece is queued before
 // it waits for the one under way.  Loadings and projections of 5,000 x 600,000 with ten
-// columns of results (48 MB) took 8.4 ms, 4.1 of them one hipMemcpyAsync; now 5.6.
+// columns of results (48 MB) took 8.4 ms, 4.1 of them one hipMemcpyAsync; now 5.6
+// (pieces of 256 KB: 7.6).
 int EigFetch::big(char *dst, const char *src, size_t bytes) {
   // the pinned area may move while it grows: the small ones in it first
   if (!small_.empty() || used_) EIG_TRY(wait());

@@ -230,9 +230,9 @@ typedef struct eig_server eig_server;
  * eig_loadings with K eigenvectors).  eigscale: K factors (NULL = 1).  nlanes:
  * batches in flight at once (0 = 4, at most 8); max_batch: samples per batch
  * (0 = 1024, at most 1024) -- together they bound the device memory admitted
- * requests may use.  chunk: SNPs per partial sum (multiple of 64; 0 = chosen by
- * the built-in launch-shape tuner at start-up).  The context may be used or
- * closed afterwards; the server owns its copies. */
+ * requests may use.  chunk: SNPs at least per partial sum (multiple of 64; 0 =
+ * 4,096); results do not depend on it.  The context may be used or closed
+ * afterwards; the server owns its copies. */
 int eig_server_start(eig_ctx *ctx, const double *eigscale, int32_t nlanes, int32_t max_batch,
                      int32_t chunk, eig_server **out);
 /* Queue nq (1..max_batch) query rows of `stride` bytes.  on_device != 0: rows is
@@ -248,7 +248,7 @@ int eig_server_submit(eig_server *s, const uint8_t *rows, int64_t stride, int32_
  * != 0 blocks).  A finished ticket is released by the poll that returns it. */
 int eig_server_poll(eig_server *s, int64_t ticket, int32_t wait, double *coords,
                     int32_t *status, double *latency_ms);
-/* Shape and counters: K, nsnp, padded device row bytes, the chunk and persistent
+/* Shape and counters: K, nsnp, padded device row bytes, the chunk and the largest
  * grid in use, batches launched and samples admitted so far.  Any may be NULL. */
 int eig_server_info(eig_server *s, int32_t *K, int64_t *nsnp, int64_t *rowpad, int32_t *chunk,
                     int32_t *grid, int64_t *batches, int64_t *samples);

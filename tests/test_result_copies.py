@@ -1,4 +1,4 @@
-"""Results of every size that reaches the host by its own route: up to 256 KB together, up
+"""Results of every size that reaches the host by its own route: up to 128 KB together, up
 to 2 MB alone, and beyond in 1 MB pieces by several threads.  Statistics are whole numbers
 and single roundings; a loading is a sum of N products, off by at most (N + 4) 2^-53 of the
 sum of their magnitudes."""
