@@ -13,7 +13,7 @@
 // Device work per chunk of kept SNPs: the columns are materialised from the tile
 // layout (k_normcols), their Gram matrix and the residual columns are FP64 MFMA
 // products (eig_gemm_f64), the drop decisions run in SNP order in one block
-// (k_ld_scan), each SNP's normal equations are solved by one block (k_ld_solve,
+// (k_ld_scan) or wave (k_ld_scan_wave), each SNP's normal equations are solved by one block (k_ld_solve,
 // choldc/cholsl order), and the XTX update is a lower-tile FP64 MFMA product.
 // Built without FMA contraction: the column statistics round as the reference's C.
 #include <algorithm>
@@ -251,6 +251,61 @@ __global__ __launch_bounds__(256) void k_ld_scan(const double *__restrict__ G, i
       nsrc[k - k0] = kill ? -1 : total;
     }
     __syncthreads();
+  }
+}
+
+// The same for windows of at most 64 SNPs.  The correlations do not depend on the decisions:
+// k_ld_bits, a wave per SNP, leaves two words of bits, bit j for position k - 1 - j above
+// r2hi (of[2 i]) and between the limits (of[2 i + 1]).  k_ld_scan_wave then decides in order,
+// the dropped ones of the last 64 positions as a word: a few scalar instructions a SNP.  A
+// chunk of 256 with a window of two took 416 us by the block, now 30.
+constexpr int kLdWave = 64;
+__global__ __launch_bounds__(256) void k_ld_bits(const double *__restrict__ G, int64_t nc, int64_t h0,
+                                                 int64_t k0, int64_t k1, const int64_t *__restrict__ ws,
+                                                 double scale, double r2lo, double r2hi,
+                                                 uint64_t *__restrict__ of) {
+  const int lane = threadIdx.x & 63;
+  const int64_t k = k0 + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (k >= k1) return;
+  const bool in = lane < k - ws[k];
+  const double c = in ? G[(k - h0) * nc + (k - 1 - lane - h0)] * scale : 0.0, r2 = c * c;
+  const uint64_t hi = __ballot(in && r2 > r2hi), sel = __ballot(in && !(r2 > r2hi) && r2 > r2lo);
+  if (lane == 0) {
+    of[2 * (k - k0)] = hi;
+    of[2 * (k - k0) + 1] = sel;
+  }
+}
+__device__ inline uint64_t lane_word(uint64_t v, int l) {
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32 |
+         (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__global__ __launch_bounds__(64) void k_ld_scan_wave(const uint64_t *__restrict__ of, int64_t k0, int64_t k1,
+                                                     uint8_t *__restrict__ dropped,
+                                                     int32_t *__restrict__ nsrc,
+                                                     int32_t *__restrict__ src, int32_t W) {
+  const int lane = threadIdx.x;
+  uint64_t hist = __ballot(k0 - 1 - lane >= 0 && dropped[max(k0 - 1 - lane, (int64_t)0)] != 0);
+  for (int64_t kb = k0; kb < k1; kb += 64) {
+    const int m = (int)min((int64_t)64, k1 - kb);
+    uint64_t hi = 0, sel = 0;
+    if (lane < m) {
+      hi = of[2 * (kb - k0 + lane)];
+      sel = of[2 * (kb - k0 + lane) + 1];
+    }
+    int32_t mine = 0;  // lane u's result: SNP kb + u
+    for (int u = 0; u < m; ++u) {
+      const bool kill = (lane_word(hi, u) & ~hist) != 0;
+      const uint64_t s = lane_word(sel, u) & ~hist;
+      // sources in position order: the later lanes' come first
+      if ((s >> lane) & 1)
+        src[(kb + u - k0) * (int64_t)W + __popcll((s >> lane) >> 1)] = (int32_t)(kb + u - 1 - lane);
+      if (lane == u) mine = kill ? -1 : __popcll(s);
+      hist = hist << 1 | (kill ? 1u : 0u);
+    }
+    if (lane < m) {
+      dropped[kb + lane] = mine < 0;
+      nsrc[kb - k0 + lane] = mine;
+    }
   }
 }
 
@@ -568,14 +623,14 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
     need += (bytes + 255) & ~(size_t)255;
     return o;
   };
-  const size_t o_idx = add(4 * (size_t)ncmax), o_Z = add(8 * (size_t)ldz * ncmax),
+  const size_t o_idx = add(4 * (size_t)std::max<int64_t>(nk, 1)), o_Z = add(8 * (size_t)ldz * ncmax),
                o_R = add(W > 0 ? 8 * (size_t)ldz * B : 0),
                o_G = add(W > 0 ? 8 * (size_t)ncmax * ncmax : 0),
                o_Bc = add(W > 0 ? 8 * (size_t)ncmax * B : 0),
                o_work = add(W > 0 ? 8 * (size_t)B * ((size_t)W * W + 2 * W) : 0),
                o_ws = add(W > 0 ? 8 * (size_t)(nk + 1) : 0), o_drop = add(W > 0 ? (size_t)nk + 1 : 0),
-               o_ns = add(4 * (size_t)B), o_src = add(W > 0 ? 4 * (size_t)B * W : 0),
-               o_nrm = add(8 * (size_t)B);
+               o_ns = add(4 * (size_t)(nk + 1)), o_zn = add(8 * (size_t)(nk + 1)), o_src = add(W > 0 ? 4 * (size_t)B * W : 0),
+               o_bits = add(16 * (size_t)B), o_nrm = add(8 * (size_t)(nk + 1));
   const size_t part_doubles = (size_t)8 << 20;  // XTX's parts
   const size_t o_part = add(8 * part_doubles);
   EIG_TRY(eig_ensure(ctx, ctx->scratch2, need));
@@ -588,6 +643,8 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
   uint8_t *d_drop = (uint8_t *)(base + o_drop);
   int32_t *d_ns = (int32_t *)(base + o_ns), *d_src = (int32_t *)(base + o_src);
   double *d_nrm = (double *)(base + o_nrm), *d_part = (double *)(base + o_part);
+  double *d_zn = (double *)(base + o_zn);
+  uint64_t *d_bits = (uint64_t *)(base + o_bits);
   double *X = (double *)ctx->xtx.p;
   if (W > 0) {
     EIG_HIP(ctx, hipMemcpyAsync(d_ws, ws.data(), 8 * (size_t)nk, hipMemcpyHostToDevice, st));
@@ -595,51 +652,59 @@ extern "C" int eig_xtx_normal(eig_ctx *ctx, const int32_t *xtypes, int32_t npop,
   }
   double ysnps = 0.0;
   bool first = true;
-  std::vector<double> rn(B), zn(B);
-  std::vector<int32_t> hns(B);
+  if (nk > 0) EIG_HIP(ctx, hipMemcpyAsync(d_idx, kl.data(), 4 * (size_t)nk, hipMemcpyHostToDevice, st));
   const double scale = 1.0 / (2.0 * (double)(n - 1));  // ldregx: cor = dot / (2 (n-1))
   for (int64_t k0 = 0; k0 < nk; k0 += B) {
     const int64_t k1 = std::min(nk, k0 + B), nb = k1 - k0;
     int64_t h0 = k0;
     for (int64_t k = k0; k < k1; ++k) h0 = std::min(h0, ws[k]);
     const int64_t nc = k1 - h0;
-    EIG_HIP(ctx, hipMemcpyAsync(d_idx, kl.data() + h0, 4 * (size_t)nc, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_normcols, dim3((unsigned)nc), dim3(256), 0, st,
                        (const uint32_t *)ctx->sel.p, M, n, (const int32_t *)d_xt, npop,
                        (const double *)ctx->mean.p, (const double *)ctx->fancy.p,
-                       (const double *)d_w, (const int32_t *)d_idx, ldz, d_Z);
+                       (const double *)d_w, (const int32_t *)d_idx + h0, ldz, d_Z);
     EIG_HIP(ctx, hipGetLastError());
     const double *R = d_Z + (k0 - h0) * ldz;  // no regression: the columns themselves
     if (W > 0) {
-      EIG_TRY(eig_gemm_f64(ctx, st, true, false, nc, nc, n, 1.0, d_Z, ldz, 0, d_Z, ldz, 0, 0.0, d_G,
-                           nc, 0, 1));
-      hipLaunchKernelGGL(k_ld_scan, dim3(1), dim3(256), 0, st, (const double *)d_G, nc, h0, k0, k1,
-                         (const int64_t *)d_ws, scale, ldr2lo, ldr2hi, d_drop, d_ns, d_src, W);
+      EIG_TRY(eig_gemm_f64_long(ctx, st, true, false, nc, nc, n, 1.0, d_Z, ldz, d_Z, ldz, 0.0, d_G, nc,
+                                false, d_part, part_doubles));
+      if (W <= kLdWave) {
+        hipLaunchKernelGGL(k_ld_bits, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, st, (const double *)d_G,
+                           nc, h0, k0, k1, (const int64_t *)d_ws, scale, ldr2lo, ldr2hi, d_bits);
+        hipLaunchKernelGGL(k_ld_scan_wave, dim3(1), dim3(64), 0, st, (const uint64_t *)d_bits, k0, k1, d_drop,
+                           d_ns + k0, d_src, W);
+      } else {
+        hipLaunchKernelGGL(k_ld_scan, dim3(1), dim3(256), 0, st, (const double *)d_G, nc, h0, k0, k1,
+                           (const int64_t *)d_ws, scale, ldr2lo, ldr2hi, d_drop, d_ns + k0, d_src, W);
+      }
       hipLaunchKernelGGL(k_ld_solve, dim3((unsigned)nb), dim3(256), 0, st, (const double *)d_G, nc,
-                         h0, k0, (const int32_t *)d_ns, (const int32_t *)d_src, W, d_work, d_Bc);
+                         h0, k0, (const int32_t *)d_ns + k0, (const int32_t *)d_src, W, d_work, d_Bc);
       EIG_HIP(ctx, hipGetLastError());
       EIG_TRY(eig_gemm_f64(ctx, st, false, false, n, nb, nc, 1.0, d_Z, ldz, 0, d_Bc, nc, 0, 0.0,
                            d_R, ldz, 0, 1));
       hipLaunchKernelGGL(k_colnorm2, dim3((unsigned)nb), dim3(256), 0, st, (const double *)d_R, ldz,
-                         n, d_nrm);
+                         n, d_nrm + k0);
       EIG_HIP(ctx, hipGetLastError());
       R = d_R;
-      // ynumsnps += |r|^2 / |z|^2 for each SNP not dropped (smartpca.c:1157-1162)
-      EIG_HIP(ctx, hipMemcpyAsync(rn.data(), d_nrm, 8 * (size_t)nb, hipMemcpyDeviceToHost, st));
-      EIG_HIP(ctx, hipMemcpyAsync(hns.data(), d_ns, 4 * (size_t)nb, hipMemcpyDeviceToHost, st));
-      EIG_HIP(ctx, hipMemcpy2DAsync(zn.data(), 8, d_G + (k0 - h0) * (nc + 1), 8 * (nc + 1), 8, nb,
-                                    hipMemcpyDeviceToHost, st));
+      EIG_HIP(ctx, hipMemcpy2DAsync(d_zn + k0, 8, d_G + (k0 - h0) * (nc + 1), 8 * (nc + 1), 8, nb,
+                                    hipMemcpyDeviceToDevice, st));
     }
     EIG_TRY(eig_gemm_f64_long(ctx, st, false, true, n, n, nb, 1.0, R, ldz, R, ldz, first ? 0.0 : 1.0, X, n,
                               true, d_part, part_doubles));
     first = false;
-    if (W > 0) {
-      EIG_HIP(ctx, hipStreamSynchronize(st));
-      for (int64_t c = 0; c < nb; ++c)
-        if (hns[c] >= 0) ysnps += rn[c] / zn[c];
-    } else {
-      ysnps += (double)nb;
-    }
+    if (W <= 0) ysnps += (double)nb;
+  }
+  if (W > 0 && nk > 0) {
+    // ynumsnps += |r|^2 / |z|^2 for each SNP not dropped (smartpca.c:1157-1162)
+    std::vector<double> rn(nk), zn(nk);
+    std::vector<int32_t> hns(nk);
+    EigFetch y(ctx);
+    EIG_TRY(y.get(rn.data(), d_nrm, 8 * (size_t)nk));
+    EIG_TRY(y.get(zn.data(), d_zn, 8 * (size_t)nk));
+    EIG_TRY(y.get(hns.data(), d_ns, 4 * (size_t)nk));
+    EIG_TRY(y.wait());
+    for (int64_t k = 0; k < nk; ++k)
+      if (hns[k] >= 0) ysnps += rn[k] / zn[k];
   }
   if (first) EIG_HIP(ctx, hipMemsetAsync(X, 0, 8 * (size_t)n * n, st));
   eig_time_end(ctx, "xtx_normal");
