@@ -667,6 +667,64 @@ __global__ __launch_bounds__(256) void k_sum_parts(const double *__restrict__ pa
   }
 }
 
+// C_z (m x n, column-major, ld ldc, at C + z sC) = A_z B_z^T over chunk z's k (A and B
+// column-major, sA and sB from chunk to chunk): k_gemm_f64's MFMAs in its order, element by
+// element the same bits, but a wave per 16 x 16 tile instead of four per 64 x 64.  The sum
+// over k is a serial chain of MFMAs (64 cycles each) that must not be cut, so skinny products
+// take as many waves as they have tiles, each with its own loads, eight steps ahead.  All of
+// them at 100,000 x 500,000 took 27 ms a call by k_gemm_f64, 12 now.
+typedef __attribute__((__vector_size__(4 * sizeof(double)))) double fp_f64x4;
+__global__ __launch_bounds__(256) void k_gemm_nt_waves(int32_t m, int32_t n, int64_t k,
+                                                       const double *__restrict__ A, int64_t lda, int64_t sA,
+                                                       const double *__restrict__ B, int64_t ldb, int64_t sB,
+                                                       double *__restrict__ C, int64_t ldc, int64_t sC) {
+  constexpr int U = 8;
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int32_t mt = (m + 15) / 16, nt = (n + 15) / 16;
+  const int32_t tile = (int32_t)blockIdx.x * 4 + (int32_t)(threadIdx.x >> 6);
+  if (tile >= mt * nt) return;
+  const int32_t i0 = (tile % mt) * 16, j0 = (tile / mt) * 16;
+  // rows past the end read the last one and are not stored
+  const double *pa = A + (int64_t)blockIdx.y * sA + min(i0 + r, m - 1) + q * lda;
+  const double *pb = B + (int64_t)blockIdx.y * sB + min(j0 + r, n - 1) + q * ldb;
+  auto ld = [&](int64_t s0, double (&a)[U], double (&b)[U]) {
+    if (4 * (s0 + U) <= k) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        a[u] = pa[4 * (s0 + u) * lda];
+        b[u] = pb[4 * (s0 + u) * ldb];
+      }
+    } else {  // zeros past k, which leave the sums as they are
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool in = 4 * (s0 + u) + q < k;
+        a[u] = in ? pa[4 * (s0 + u) * lda] : 0.0;
+        b[u] = in ? pb[4 * (s0 + u) * ldb] : 0.0;
+      }
+    }
+  };
+  fp_f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+  auto mma = [&](const double (&a)[U], const double (&b)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b[u], a[u], acc, 0, 0, 0);
+  };
+  const int64_t steps = (k + 3) / 4;
+  double a0[U], b0[U], a1[U], b1[U];
+  ld(0, a0, b0);
+  for (int64_t s = 0; s < steps; s += 2 * U) {
+    ld(s + U, a1, b1);
+    mma(a0, b0);
+    ld(s + 2 * U, a0, b0);
+    mma(a1, b1);
+  }
+  C += (int64_t)blockIdx.y * sC;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int32_t row = i0 + r, col = j0 + q + 4 * e;
+    if (row < m && col < n) C[row + col * ldc] = acc[e];
+  }
+}
+
 // C (m x n, column-major, ld ldc) = A B^T, A m x k (ld lda) and B n x k (ld ldb) column-major,
 // for a long k: k is cut into S equal chunks (one batched product) and a remainder,
 // whose partial products are summed.  A single product of these shapes has only a few
@@ -684,15 +742,23 @@ static int gemm_nt_long(eig_ctx *ctx, bool fine, int32_t m, int32_t n, int64_t k
   int64_t S = fine ? std::min<int64_t>(std::max<int64_t>(1, 1024 / tiles), k / 256)
                    : std::min<int64_t>(64, k / 4096);
   S = std::min<int64_t>(S, (int64_t)(part_doubles / std::max<int64_t>(mn, 1)) - 1);
-  if (S < 2)
-    return eig_gemm_f64(ctx, st, false, true, m, n, k, 1.0, A, lda, 0, B, ldb, 0, 0.0, C, ldc, 0, 1);
+  // skinny products of the coarse chunks: a wave per tile, the same bits
+  auto mul = [&](int64_t kk, const double *a, int64_t sA, const double *b, int64_t sB, double *c, int64_t ldr,
+                 int32_t batch) -> int {
+    if (fine || n > 32)
+      return eig_gemm_f64(ctx, st, false, true, m, n, kk, 1.0, a, lda, sA, b, ldb, sB, 0.0, c, ldr, mn, batch);
+    const int32_t wv = ((m + 15) / 16) * ((n + 15) / 16);
+    hipLaunchKernelGGL(k_gemm_nt_waves, dim3((unsigned)((wv + 3) / 4), (unsigned)batch), dim3(256), 0, st, m, n,
+                       kk, a, lda, sA, b, ldb, sB, c, ldr, mn);
+    EIG_HIP(ctx, hipGetLastError());
+    return EIG_OK;
+  };
+  if (S < 2) return mul(k, A, 0, B, 0, C, ldc, 1);
   const int64_t kc = k / S, rem = k - S * kc;
-  EIG_TRY(eig_gemm_f64(ctx, st, false, true, m, n, kc, 1.0, A, lda, kc * lda, B, ldb, kc * ldb, 0.0,
-                       part, m, mn, (int32_t)S));
+  EIG_TRY(mul(kc, A, kc * lda, B, kc * ldb, part, m, (int32_t)S));
   int32_t nparts = (int32_t)S;
   if (rem > 0) {
-    EIG_TRY(eig_gemm_f64(ctx, st, false, true, m, n, rem, 1.0, A + S * kc * lda, lda, 0,
-                         B + S * kc * ldb, ldb, 0, 0.0, part + S * mn, m, 0, 1));
+    EIG_TRY(mul(rem, A + S * kc * lda, 0, B + S * kc * ldb, 0, part + S * mn, m, 1));
     ++nparts;
   }
   if (fine)

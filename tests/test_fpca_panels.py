@@ -1,6 +1,6 @@
 """Split-BF16 fastmode products at the edges of their tiles: SNP counts around the 64-SNP
 groups and 128-SNP tiles, sample counts around the 128-sample tiles, panels of 32 and 64
-columns, against the FP64 form with the same start panel.
+columns, basis products in two chunks and a remainder of one SNP, against the FP64 form with the same start panel.
 
 A value's bf16 hi + lo parts leave at most 2^-17 of it, so a product of two split operands
 is off by at most 2^-16 of its terms.  The three population axes stand well apart (their
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("L,I", [(6, 5), (33, 4)])
-@pytest.mark.parametrize("N,M", [(127, 700), (128, 1024), (129, 1025), (257, 639), (384, 1153)])
+@pytest.mark.parametrize("N,M", [(127, 700), (128, 1024), (129, 1025), (257, 639), (384, 1153), (130, 9001)])
 def test_split_bf16_panel_edges(N, M, L, I):
     import eig_amd
     rng = np.random.default_rng(N * 31 + M)
