@@ -1992,13 +1992,15 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
     need += ((cnt * 8 + 255) / 256) * 256;
     return o;
   };
-  size_t o_a = add((size_t)N * lda), o_d = add(N), o_e = add(N), o_e2 = add(N),
-         o_tau = add(N), o_V = add(kNB * N), o_W = add(kNB * N), o_x = add(lda), o_y = add((size_t)ntile * lda),
-         o_sc = add(S_COUNT), o_p1 = add((size_t)maxblk * maxnv),
+  size_t o_a = add((size_t)N * lda);
+  // cleared before a solve, one range
+  size_t o_sc = add(S_COUNT), o_e = add(N), o_e2 = add(N), o_tau = add(N), o_V = add(kNB * N),
+         o_W = add(kNB * N), o_x = add(lda), o_sync = add(8);
+  size_t o_d = add(N), o_y = add((size_t)ntile * lda), o_p1 = add((size_t)maxblk * maxnv),
          o_ev = add(N), o_st = add(2 * (size_t)(sturm_rows(n) + kStB)),
          o_X = add((size_t)kMaxVec * N), o_lu = add((size_t)kMaxVec * kLuF * N),
          o_Z = add(kNB * kMaxVec), o_T = add((size_t)npanel * kNB * kNB),
-         o_pw = add((size_t)2 * maxw * kPW), o_ps = add((size_t)(ntile * (ntile + 1) / 2)), o_sync = add(8);
+         o_pw = add((size_t)2 * maxw * kPW), o_ps = add((size_t)(ntile * (ntile + 1) / 2));
   EIG_TRY(eig_ensure(ctx, ctx->ework, need));
   char *base = (char *)ctx->ework.p;
   EigWs ws;
@@ -2028,13 +2030,7 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   if (lda != n) EIG_HIP(ctx, hipMemsetAsync(ws.a, 0, sizeof(double) * N * lda, st));
   EIG_HIP(ctx, hipMemcpy2DAsync(ws.a, sizeof(double) * lda, d_a, sizeof(double) * N,
                                 sizeof(double) * N, N, hipMemcpyDeviceToDevice, st));
-  EIG_HIP(ctx, hipMemsetAsync(ws.sc, 0, sizeof(double) * S_COUNT, st));
-  EIG_HIP(ctx, hipMemsetAsync(ws.e, 0, sizeof(double) * N, st));
-  EIG_HIP(ctx, hipMemsetAsync(ws.e2, 0, sizeof(double) * N, st));
-  EIG_HIP(ctx, hipMemsetAsync(ws.tau, 0, sizeof(double) * N, st));
-  EIG_HIP(ctx, hipMemsetAsync(ws.V, 0, sizeof(double) * kNB * N, st));
-  EIG_HIP(ctx, hipMemsetAsync(ws.W, 0, sizeof(double) * kNB * N, st));
-  EIG_HIP(ctx, hipMemsetAsync(ws.xtmp, 0, sizeof(double) * lda, st));
+  EIG_HIP(ctx, hipMemsetAsync(base + o_sc, 0, o_d - o_sc, st));
 
   // ---- tridiagonalisation: plain launches.  The host queues a launch in ~3 us, less than
   // the shortest column takes on the device, so a captured graph of the launches replays
@@ -2050,7 +2046,6 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
   EIG_HIP(ctx, hipGetLastError());
   if (stop < n - 1) {
     std::lock_guard<std::mutex> lock(g_tri_mu[ctx->device & 15]);
-    EIG_HIP(ctx, hipMemsetAsync(ws.sync, 0, 8, st));
     EIG_TRY(launch_resident(ctx, ws, n, stop, st));
     int32_t gave_up[2] = {0, 0};
     EIG_HIP(ctx, hipMemcpyAsync(gave_up, ws.sync, sizeof(gave_up), hipMemcpyDeviceToHost, st));
