@@ -25,12 +25,6 @@ typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4;
 typedef unsigned long long u64;
 
 namespace {
-constexpr int kDig = 7;      // digits per column
-constexpr int kSt = 128;     // k per stage
-constexpr int kFragB = 1024;  // bytes of a digit operand: 16 digit columns x 64 k
-constexpr int kMaxCols = 20;  // columns of a group of nine tiles (140 of 144 digit columns)
-constexpr int kMaxNT = 9;
-
 // ------------------------------------------------------------------ columns
 // The three FP64 values of column c at index k: v1 multiplies the code, v2 the missing
 // bit, v3 is summed alone.
@@ -177,14 +171,14 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
                                                   uint8_t *__restrict__ dst, u64 *__restrict__ sums) {
   constexpr int planes = MODE == kCdSum ? 2 : 1;
   constexpr bool rowmajor = KIND == kColPanel || KIND == kColLevB;
-  __shared__ __align__(16) uint8_t img[2 * kMaxNT * 2 * kFragB];
-  __shared__ u64 ssum[2 * kMaxCols];
+  __shared__ __align__(16) uint8_t img[2 * kCdMaxNT * 2 * kCdFrag];
+  __shared__ u64 ssum[2 * kCdMaxCols];
   const int t = threadIdx.x;
   const int32_t c0 = blockIdx.y * Cg, nc = min(Cg, C - c0);
   const int64_t blk = blockIdx.x;
-  const int32_t bytes = planes * NT * 2 * kFragB;
+  const int32_t bytes = planes * NT * 2 * kCdFrag;
   for (int e = t * 16; e < bytes; e += 256 * 16) *(uint4 *)&img[e] = make_uint4(0, 0, 0, 0);
-  if (t < 2 * kMaxCols) ssum[t] = 0;
+  if (t < 2 * kCdMaxCols) ssum[t] = 0;
   __syncthreads();
   // an item is one dword of an operand: the code slots u, u + 4, u + 8, u + 12 of a word
   for (int e = t; e < 32 * nc; e += 256) {
@@ -202,7 +196,7 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
       int64_t q[4] = {llrint(scalbn(x0, sh)), llrint(scalbn(x1, sh)), llrint(scalbn(x2, sh)),
                       llrint(scalbn(x3, sh))};
 #pragma unroll
-      for (int s = kDig - 1; s >= 0; --s) {
+      for (int s = kCdDig - 1; s >= 0; --s) {
         uint32_t w = 0;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
@@ -211,7 +205,7 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
           w |= ((uint32_t)d & 0xFFu) << (8 * b);
         }
         const int dc = s * Cg + c;
-        *(uint32_t *)&img[((jl & 1) * planes * NT + plane * NT + (dc >> 4)) * kFragB + (dc & 15) * 16 + at] = w;
+        *(uint32_t *)&img[((jl & 1) * planes * NT + plane * NT + (dc >> 4)) * kCdFrag + (dc & 15) * 16 + at] = w;
       }
     };
     if (MODE == kCdMiss) {
@@ -237,10 +231,6 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
 }
 
 // ------------------------------------------------------------------ the product
-// row tiles of 16 per wave at most (a block is four waves)
-constexpr int cd_tiles(int mode, int NT) {
-  return mode == kCdPair ? 2 : mode == kCdSum && NT == kMaxNT ? 3 : 4;
-}
 struct MulArgs {
   CodeView v;
   const uint8_t *dig;
@@ -263,7 +253,7 @@ struct MulArgs {
 template <int NT, int MODE, int R>
 __global__ __launch_bounds__(256, 2) void k_cd_mul(MulArgs A) {
   constexpr int planes = MODE == kCdSum ? 2 : 1, nacc = MODE == kCdPair ? 2 : 1;
-  constexpr int bytes = planes * NT * kFragB, nld = bytes / 4096;  // of a half stage
+  constexpr int bytes = planes * NT * kCdFrag, nld = bytes / 4096;  // of a half stage
   constexpr int tail = bytes % 4096 / 16;  // threads with one more piece
   __shared__ __align__(16) uint8_t lds[2][bytes];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane >> 4;
@@ -335,7 +325,7 @@ __global__ __launch_bounds__(256, 2) void k_cd_mul(MulArgs A) {
           for (int u = 0; u < 4; ++u) f[r][u] = (int)((ms >> (2 * u)) & 0x01010101u);
         }
       };
-      auto dig_op = [&](int n) { return *(const i32x4 *)&lds[a][n * kFragB + lane * 16]; };
+      auto dig_op = [&](int n) { return *(const i32x4 *)&lds[a][n * kCdFrag + lane * 16]; };
       auto mul = [&](const i32x4 (&f)[R], const i32x4 &d, i32x4 (&c)[R]) {
 #pragma unroll
         for (int r = 0; r < R; ++r) c[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[r], d, c[r], 0, 0, 0);
@@ -391,7 +381,7 @@ template <int NT, int MODE>
 __global__ __launch_bounds__(256) void k_cd_stream(const uint8_t *__restrict__ dig_, int32_t *__restrict__ part,
                                                    CodeRows rows, int64_t nword, int64_t nblk, int64_t per,
                                                    int32_t ngroup, int32_t nsplit) {
-  constexpr int planes = MODE == kCdSum ? 2 : 1, F = planes * NT, bytes = F * kFragB;
+  constexpr int planes = MODE == kCdSum ? 2 : 1, F = planes * NT, bytes = F * kCdFrag;
   const int lane = threadIdx.x & 63, q = lane >> 4;
   const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (item >= (int64_t)ngroup * nsplit) return;
@@ -405,7 +395,7 @@ __global__ __launch_bounds__(256) void k_cd_stream(const uint8_t *__restrict__ d
   auto load = [&](int64_t h, i32x4 (&d)[F]) {
     const uint8_t *s = dig + min(h, 2 * k1 - 1) * bytes;
 #pragma unroll
-    for (int n = 0; n < F; ++n) d[n] = *(const i32x4 *)(s + n * kFragB);
+    for (int n = 0; n < F; ++n) d[n] = *(const i32x4 *)(s + n * kCdFrag);
   };
   auto codes = [&](int64_t k) {
     uint2 c = make_uint2(~0u, ~0u);
@@ -474,7 +464,7 @@ __device__ __forceinline__ void out_rows(const int32_t *__restrict__ part, int32
 __device__ __forceinline__ void digit_sum(const int64_t *p, int32_t Cg, int64_t &hi, int64_t &lo) {
   hi = lo = 0;
 #pragma unroll
-  for (int s = 0; s < kDig; ++s) {
+  for (int s = 0; s < kCdDig; ++s) {
     if (s < 4) hi = hi * 256 + p[s * Cg];
     else lo = lo * 256 + p[s * Cg];
   }
@@ -492,7 +482,7 @@ __global__ __launch_bounds__(256) void k_cd_out_sum(const int32_t *__restrict__ 
                                                     const u64 *__restrict__ sums, double scale,
                                                     double *__restrict__ out, int64_t ldr, int64_t ldc,
                                                     int32_t add) {
-  __shared__ int64_t sm[kOutRows * kMaxNT * 16];
+  __shared__ int64_t sm[kOutRows * kCdMaxNT * 16];
   const int64_t row0 = (int64_t)blockIdx.x * kOutRows;
   const int32_t g = blockIdx.y, c0 = g * Cg, c1 = g + 1 == (int32_t)gridDim.y ? Cpad : c0 + Cg;
   out_rows<1>(part + (int64_t)g * nsplit * rowpad * NTc, NTc, rowpad, nsplit, row0, sm);
@@ -523,7 +513,7 @@ __global__ __launch_bounds__(1024) void k_cd_out_small(const int32_t *__restrict
                                                        const u64 *__restrict__ mx,
                                                        const u64 *__restrict__ sums,
                                                        double *__restrict__ out, int64_t ldr) {
-  __shared__ int64_t sl[7][kMaxNT * 16], sm[kMaxNT * 16];
+  __shared__ int64_t sl[7][kCdMaxNT * 16], sm[kCdMaxNT * 16];
   const int32_t row = blockIdx.x, g = blockIdx.y;
   const int t = threadIdx.x, j = t % NTc, s = t / NTc;
   if (s < 7) {
@@ -560,7 +550,7 @@ __global__ __launch_bounds__(256) void k_cd_out_pair(const int32_t *__restrict__
                                                      const double *__restrict__ lev,
                                                      const uint8_t *__restrict__ ignore, double scale,
                                                      double *__restrict__ out, int64_t ldr, int64_t ldc) {
-  __shared__ int64_t sm[2 * kOutRows * kMaxNT * 16];
+  __shared__ int64_t sm[2 * kOutRows * kCdMaxNT * 16];
   const int64_t row0 = (int64_t)blockIdx.x * kOutRows;
   const int32_t g = blockIdx.y, c0 = g * Cg, w = min(Cg, C - c0);
   out_rows<2>(part + (int64_t)g * nsplit * 2 * rowpad * NTc, NTc, rowpad, nsplit, row0, sm);
@@ -592,50 +582,6 @@ void launch_mul(const MulArgs &A, int R, hipStream_t st) {
   else hipLaunchKernelGGL((k_cd_mul<NT, MODE, RX>), grid, dim3(256), 0, st, A);
 }
 }  // namespace
-
-// column groups: at most 20 columns (nine tiles), or 11 (five) when that is all
-static void cd_groups(int32_t C, int32_t &ngroup, int32_t &Cg, int32_t &NT) {
-  ngroup = (C + kMaxCols - 1) / kMaxCols;
-  Cg = (C + ngroup - 1) / ngroup;
-  NT = Cg * kDig <= 80 ? 5 : 9;
-}
-
-CodesPlan eig_codes_plan(int num_cu, int mode, int32_t C, int64_t nrow, int64_t nblk, int32_t smax) {
-  CodesPlan P;
-  P.mode = mode;
-  P.C = C;
-  P.nblk = nblk;
-  cd_groups(C, P.ngroup, P.Cg, P.NT);
-  // fewer row tiles a wave where the rows fill no more (three run as the most)
-  P.R = (int32_t)std::min<int64_t>(cd_tiles(mode, P.NT), (nrow + 63) / 64);
-  if (P.R > 2) P.R = cd_tiles(mode, P.NT);
-  const int32_t rows = 64 * P.R;
-  P.nrowblk = (int32_t)((nrow + rows - 1) / rows);
-  P.rowpad = (int64_t)P.nrowblk * rows;
-  // splits: rounds of the blocks the chip holds (two per CU) times stages each, plus the
-  // sums' way to memory and back, worth about two stages a block
-  const int64_t slots = 2 * (int64_t)std::max(num_cu, 1);
-  double best = 0.0;
-  P.nsplit = 1;
-  P.per = nblk;
-  for (int32_t s = 1; s <= (int32_t)std::min<int64_t>(nblk, std::max<int64_t>(smax, nblk * kSt / kCodesMaxK + 2)); ++s) {
-    const int64_t pe = (nblk + s - 1) / s;
-    if ((nblk + pe - 1) / pe != s) continue;
-    if (pe * kSt > kCodesMaxK) continue;  // INT32 sums
-    const double rounds = (double)(((int64_t)P.nrowblk * P.ngroup * s + slots - 1) / slots);
-    const double cost = rounds * ((double)pe + 2.0) + 1.0 * (double)P.nrowblk * P.ngroup * s / slots;
-    if (best == 0.0 || cost < best) {
-      best = cost;
-      P.nsplit = s;
-      P.per = pe;
-    }
-  }
-  const int32_t planes = mode == kCdSum ? 2 : 1, nacc = mode == kCdPair ? 2 : 1;
-  P.head_bytes = ((size_t)C * 24 + 255) / 256 * 256;
-  P.dig_bytes = (size_t)P.ngroup * nblk * planes * P.NT * 2 * kFragB;
-  P.part_bytes = (size_t)P.ngroup * P.nsplit * nacc * P.rowpad * P.NT * 16 * 4;
-  return P;
-}
 
 #define CD_KIND(K, ...)              \
   case K: {                          \

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/eig_abi.h"
+#include "plans.h"
 
 // Sample tile of the selected-genotype layout: 128 samples = 8 x 32-bit words of
 // 2-bit codes (sample 16w+i of the tile at bits 2i..2i+1 of word w).
@@ -208,16 +209,6 @@ struct CodeCols {
   const double *fxscal = nullptr;
   int32_t K = 0;
 };
-enum { kCdPair, kCdSum, kCdMiss };
-struct CodesPlan {
-  int mode;
-  int32_t C, ngroup, Cg, NT, R, nrowblk, nsplit;
-  int64_t nblk, per, rowpad;
-  size_t head_bytes, dig_bytes, part_bytes;
-};
-// one INT32 sum holds this many terms (digit 128, code 3)
-constexpr int64_t kCodesMaxK = (int64_t)5 << 20;
-CodesPlan eig_codes_plan(int num_cu, int mode, int32_t C, int64_t nrow, int64_t nblk, int32_t smax);
 int eig_codes_scales(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, void *head, hipStream_t st);
 int eig_codes_restart(eig_ctx *ctx, const CodesPlan &P, void *head, hipStream_t st);
 int eig_codes_build(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, int32_t layout, int64_t b0,

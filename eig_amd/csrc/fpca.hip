@@ -978,22 +978,13 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
                     kCodeLinear};
   const CodeView vs{(const uint8_t *)ctx->selg.p, nullptr, G64 * 2048, 16, 4096, 2048, npad, G64 * 4,
                     kCodeGrouped};
-  CodesPlan pa{}, pb{}, pu{};
+  FpcaPlans F{};
   size_t o_cw = 0;
   if (!bf) {
-    // splits whose sums stay within 2 GiB
-    auto smax = [](size_t one) { return (int32_t)std::max<size_t>(1, std::min<size_t>(32, ((size_t)2 << 30) / one)); };
-    pa = eig_codes_plan(ctx->num_cu, kCdPair, L, M, nst, 1);
-    pa = eig_codes_plan(ctx->num_cu, kCdPair, L, M, nst, smax(pa.part_bytes));
-    pb = eig_codes_plan(ctx->num_cu, kCdSum, L, npad, (G64 + 1) / 2, 1);
-    pb = eig_codes_plan(ctx->num_cu, kCdSum, L, npad, (G64 + 1) / 2, smax(pb.part_bytes / pb.nsplit));
-    pu = eig_codes_plan(ctx->num_cu, kCdSum, Ctot, npad, (G64 + 1) / 2, 1);
-    pu = eig_codes_plan(ctx->num_cu, kCdSum, Ctot, npad, (G64 + 1) / 2, smax(pu.part_bytes / pu.nsplit));
-    size_t cw = 0;
-    for (const CodesPlan *q : {&pa, &pb, &pu})
-      cw = std::max(cw, q->head_bytes + up(q->dig_bytes) + q->part_bytes);
-    o_cw = add(cw);
+    F = eig_fpca_plans(ctx->num_cu, M, nst, K, L, Ctot);
+    o_cw = add(F.area);
   }
+  const CodesPlan &pa = F.pa, &pb = F.pb;
   EIG_TRY(eig_ensure(ctx, ctx->scratch2, off));
   char *base = (char *)ctx->scratch2.p;
   double *lf = (double *)(base + o_lf), *A0 = (double *)(base + o_a0), *A1 = (double *)(base + o_a1);
@@ -1035,23 +1026,24 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   // left in the work area
   char *cw = base + o_cw;
   auto code_mul = [&](const CodesPlan &plan, const CodeView &v, const CodeCols &cols) -> int {
+    if (eig_codes_area(plan) > F.area) return eig_set_err(ctx, EIG_E_STATE, "eig_fpca: work area");
     EIG_TRY(eig_codes_scales(ctx, plan, cols, cw, st));
     return eig_codes_mul(ctx, plan, v, cols, 0, cw, cw + plan.head_bytes,
-                         cw + plan.head_bytes + up(plan.dig_bytes), false, st);
+                         cw + plan.head_bytes + plan.dig_bytes, false, st);
   };
   auto code_xtb = [&](const CodesPlan &plan, const double *B_, double scale, double *out, int64_t ldo,
                       int32_t Cpad) -> int {
     CodeCols c{kColLevB, B_, ldq, M};
     c.lev = lf;
     EIG_TRY(code_mul(plan, vs, c));
-    return eig_codes_out_sum(ctx, plan, npad, cw, cw + plan.head_bytes + up(plan.dig_bytes), scale, out,
+    return eig_codes_out_sum(ctx, plan, npad, cw, cw + plan.head_bytes + plan.dig_bytes, scale, out,
                              ldo, 1, Cpad, false, st);
   };
   auto xa = [&](const double *A_, double *Y_) -> int {
     if (bf)
       return launch_xa_bf16(ctx, P, lbf, fa, cxa, A_, lda, Y_, ldq, L, st);
     EIG_TRY(code_mul(pa, vm, CodeCols{kColPanel, A_, lda, n}));
-    return eig_codes_out_pair(ctx, pa, M, cw, cw + pa.head_bytes + up(pa.dig_bytes), lf, nullptr, 1.0,
+    return eig_codes_out_pair(ctx, pa, M, cw, cw + pa.head_bytes + pa.dig_bytes, lf, nullptr, 1.0,
                               Y_, ldq, 1, st);
   };
   auto xtb = [&](const double *B_, double *out_) -> int {
@@ -1158,10 +1150,8 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
       EIG_TRY(launch_xtb_bf16(ctx, P, (const uint2 *)ctx->selg.p, tabs, fb, Mpad, src + r64,
                               ldq, r - r64, part, part_doubles, Bm + r64, (int32_t)ldq, 1.0, st));
   } else {
-    // the plan made for every column serves a basis of fewer (r <= Ctot): the missing
-    // ones have no digits
-    CodesPlan pr = eig_codes_plan(ctx->num_cu, kCdSum, r, npad, (G64 + 1) / 2, pu.nsplit);
-    EIG_TRY(code_xtb(pr, src, 1.0, Bm, ldq, r));
+    // planned for the rank that the basis has; the area holds the plan of every rank
+    EIG_TRY(code_xtb(eig_fpca_basis_plan(ctx->num_cu, M, nst, r), src, 1.0, Bm, ldq, r));
   }
   EIG_TRY(gemm_nt_long(ctx, !bf, r, r, npad, Bm, ldq, Bm, ldq, G, r, part, part_doubles, st));
   // top-K eigenpairs of B^T B (order r up to 256) by the FP64 eigensolver: all

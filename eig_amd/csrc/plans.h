@@ -1,0 +1,106 @@
+// Launch plans and the sizes of the work areas they need: host arithmetic alone (no HIP), so
+// that what a kernel will write can be checked against what is allocated without a GPU.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+
+// ---- products of packed codes with FP64 columns (codes.hip)
+constexpr int kCdDig = 7;        // digits per column
+constexpr int kCdStage = 128;    // k per stage
+constexpr int kCdFrag = 1024;    // bytes of a digit operand: 16 digit columns x 64 k
+constexpr int kCdMaxCols = 20;   // columns of a group of nine tiles (140 of 144 digit columns)
+constexpr int kCdMaxNT = 9;
+// one INT32 sum holds this many terms (digit 128, code 3)
+constexpr int64_t kCodesMaxK = (int64_t)5 << 20;
+
+enum { kCdPair, kCdSum, kCdMiss };
+struct CodesPlan {
+  int mode;
+  int32_t C, ngroup, Cg, NT, R, nrowblk, nsplit;
+  int64_t nblk, per, rowpad;
+  size_t head_bytes, dig_bytes, part_bytes;
+};
+
+// row tiles of 16 per wave at most (a block is four waves)
+constexpr int cd_tiles(int mode, int NT) {
+  return mode == kCdPair ? 2 : mode == kCdSum && NT == kCdMaxNT ? 3 : 4;
+}
+
+// column groups: at most 20 columns (nine tiles), or 11 (five) when that is all
+inline void cd_groups(int32_t C, int32_t &ngroup, int32_t &Cg, int32_t &NT) {
+  ngroup = (C + kCdMaxCols - 1) / kCdMaxCols;
+  Cg = (C + ngroup - 1) / ngroup;
+  NT = Cg * kCdDig <= 80 ? 5 : 9;
+}
+
+// The product of nrow rows of codes with C columns over nblk stages, in at most smax splits
+// (more only where an INT32 sum would not hold a split).
+inline CodesPlan eig_codes_plan(int num_cu, int mode, int32_t C, int64_t nrow, int64_t nblk, int32_t smax) {
+  CodesPlan P;
+  P.mode = mode;
+  P.C = C;
+  P.nblk = nblk;
+  cd_groups(C, P.ngroup, P.Cg, P.NT);
+  // fewer row tiles a wave where the rows fill no more (three run as the most)
+  P.R = (int32_t)std::min<int64_t>(cd_tiles(mode, P.NT), (nrow + 63) / 64);
+  if (P.R > 2) P.R = cd_tiles(mode, P.NT);
+  const int32_t rows = 64 * P.R;
+  P.nrowblk = (int32_t)((nrow + rows - 1) / rows);
+  P.rowpad = (int64_t)P.nrowblk * rows;
+  // splits: rounds of the blocks the chip holds (two per CU) times stages each, plus the
+  // sums' way to memory and back, worth about two stages a block
+  const int64_t slots = 2 * (int64_t)std::max(num_cu, 1);
+  const int64_t pmax = kCodesMaxK / kCdStage;  // stages of one INT32 sum
+  const int64_t smin = (nblk + pmax - 1) / pmax;
+  double best = 0.0;
+  P.nsplit = 1;
+  P.per = nblk;
+  for (int64_t s = smin; s <= std::min<int64_t>(nblk, std::max<int64_t>(smax, smin)); ++s) {
+    const int64_t pe = (nblk + s - 1) / s;
+    if ((nblk + pe - 1) / pe != s) continue;
+    const double rounds = (double)(((int64_t)P.nrowblk * P.ngroup * s + slots - 1) / slots);
+    const double cost = rounds * ((double)pe + 2.0) + 1.0 * (double)P.nrowblk * P.ngroup * (double)s / (double)slots;
+    if (best == 0.0 || cost < best) {
+      best = cost;
+      P.nsplit = (int32_t)s;
+      P.per = pe;
+    }
+  }
+  const int32_t planes = mode == kCdSum ? 2 : 1, nacc = mode == kCdPair ? 2 : 1;
+  P.head_bytes = ((size_t)C * 24 + 255) / 256 * 256;
+  P.dig_bytes = (size_t)P.ngroup * nblk * planes * P.NT * 2 * kCdFrag;
+  P.part_bytes = (size_t)P.ngroup * P.nsplit * nacc * P.rowpad * P.NT * 16 * 4;
+  return P;
+}
+// a plan's scales, digit operands (a multiple of 2 KB) and INT32 sums, one after the other
+inline size_t eig_codes_area(const CodesPlan &P) { return P.head_bytes + P.dig_bytes + P.part_bytes; }
+
+// ---- fastmode's FP64 panel products (fpca.hip): X A and X^T B of the power iterations, and
+// the finishing X^T U of a basis of r columns
+inline CodesPlan eig_fpca_plan(int num_cu, int mode, int32_t C, int64_t nrow, int64_t nblk) {
+  // splits whose sums stay within 2 GiB
+  const CodesPlan one = eig_codes_plan(num_cu, mode, C, nrow, nblk, 1);
+  const size_t b = one.part_bytes / (size_t)one.nsplit;
+  return eig_codes_plan(num_cu, mode, C, nrow, nblk,
+                        (int32_t)std::max<size_t>(1, std::min<size_t>(32, ((size_t)2 << 30) / b)));
+}
+struct FpcaPlans {
+  CodesPlan pa, pb;
+  size_t area;  // holds each of them and the finishing product at every rank the basis may have
+};
+inline CodesPlan eig_fpca_basis_plan(int num_cu, int64_t M, int32_t nst, int32_t r) {
+  return eig_fpca_plan(num_cu, kCdSum, r, (int64_t)nst * 128, (M + 127) / 128);
+}
+inline FpcaPlans eig_fpca_plans(int num_cu, int64_t M, int32_t nst, int32_t K, int32_t L, int32_t Ctot) {
+  FpcaPlans F;
+  F.pa = eig_fpca_plan(num_cu, kCdPair, L, M, nst);
+  F.pb = eig_fpca_plan(num_cu, kCdSum, L, (int64_t)nst * 128, (M + 127) / 128);
+  F.area = std::max(eig_codes_area(F.pa), eig_codes_area(F.pb));
+  // fewer columns can need more: their groups, and with them the row padding and the splits,
+  // are chosen anew
+  for (int32_t r = K; r <= Ctot; ++r)
+    F.area = std::max(F.area, eig_codes_area(eig_fpca_basis_plan(num_cu, M, nst, r)));
+  return F;
+}
