@@ -26,8 +26,8 @@ typedef unsigned long long u64;
 
 namespace {
 // ------------------------------------------------------------------ columns
-// The three FP64 values of column c at index k: v1 multiplies the code, v2 the missing
-// bit, v3 is summed alone.
+// The three FP64 values of column c at index k: v1 multiplies the code, v2 = -(3 v1 + v3) the
+// missing bit, v3 is summed alone.  (Columns over samples multiply both with one value.)
 struct ColArgs {
   const double *a;      // panel, axes or loadings
   int64_t ld;           // their leading dimension
@@ -163,8 +163,12 @@ __device__ __forceinline__ double col_quantum(u64 mx) {
 // dst[(((group * nblk + blk) * 2 + step a) * planes + plane) * NT + tile][1024]; lane l's 16
 // bytes of a step's operand: digit column l % 16 of the tile, word 2 (l / 16) + a, byte
 // 4 t + b = code slot 4 b + t.  Digit column s * Cg + c holds digit s (highest first) of the
-// group's column c.  sums[2 c], [2 c + 1]: the sums of v3 on the grid, in two parts of 28
-// low and the remaining high bits, so that they stay exact.
+// group's column c.  The missing bit's plane is formed from the other two on the grid, so
+// that a missing genotype (code 3, its bit, and its share of v3's sum) adds up to zero exactly:
+// v1, v2 and v3 rounded one by one left up to 2.5 steps each, 2e-13 of the right-hand side of
+// a sample with 99.9 % missing.  It is within 2 steps of v2, inside the seven digits' range.
+// sums[2 c], [2 c + 1]: the sums of v3 on the grid, in two parts of 28 low and the remaining
+// high bits, so that they stay exact.
 template <int KIND, int MODE>
 __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int64_t b0, int32_t C,
                                                   int32_t Cg, int32_t NT, const u64 *__restrict__ mx,
@@ -192,9 +196,7 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
     for (int b = 0; b < 4; ++b)
       v[b] = col_value<KIND>(A, code_elem(layout, 8 * (b0 + blk) + jl, 4 * b + u), c0 + c);
     const int at = (jl >> 1) * 256 + u * 4;
-    auto put = [&](double x0, double x1, double x2, double x3, int plane) {
-      int64_t q[4] = {llrint(scalbn(x0, sh)), llrint(scalbn(x1, sh)), llrint(scalbn(x2, sh)),
-                      llrint(scalbn(x3, sh))};
+    auto put = [&](int64_t (&q)[4], int plane) {
 #pragma unroll
       for (int s = kCdDig - 1; s >= 0; --s) {
         uint32_t w = 0;
@@ -208,18 +210,20 @@ __global__ __launch_bounds__(256) void k_cd_build(ColArgs A, int32_t layout, int
         *(uint32_t *)&img[((jl & 1) * planes * NT + plane * NT + (dc >> 4)) * kCdFrag + (dc & 15) * 16 + at] = w;
       }
     };
-    if (MODE == kCdMiss) {
-      put(v[0].v2, v[1].v2, v[2].v2, v[3].v2, 0);
-    } else {
-      put(v[0].v1, v[1].v1, v[2].v1, v[3].v1, 0);
-      if (MODE == kCdSum) put(v[0].v2, v[1].v2, v[2].v2, v[3].v2, 1);
-    }
-    int64_t lo = 0, hi = 0;
+    int64_t q1[4], q2[4], lo = 0, hi = 0;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       const int64_t q3 = llrint(scalbn(v[b].v3, sh));
+      q1[b] = llrint(scalbn(v[b].v1, sh));
+      q2[b] = -(3 * q1[b] + q3);
       lo += q3 & ((1 << 28) - 1);
       hi += q3 >> 28;
+    }
+    if (MODE == kCdMiss) {
+      put(q2, 0);
+    } else {
+      put(q1, 0);
+      if (MODE == kCdSum) put(q2, 1);
     }
     if (lo != 0) atomicAdd(&ssum[2 * c], (u64)lo);
     if (hi != 0) atomicAdd(&ssum[2 * c + 1], (u64)hi);
