@@ -21,6 +21,35 @@ int eig_set_err(eig_ctx *ctx, int code, const char *fmt, ...) {
   return code;
 }
 
+// What XTX and the eigensolver keep between calls and form anew in each (their results are in
+// buffers of their own) goes when memory runs short, unless the call under way is theirs.
+static bool release_idle(eig_ctx *ctx) {
+  std::vector<DevBuf *> idle;
+  if (!ctx->in_syrk) idle.insert(idle.end(), {&ctx->xdplanes, &ctx->xdtab, &ctx->xdpart, &ctx->part});
+  if (!ctx->in_eigh) idle.insert(idle.end(), {&ctx->ework, &ctx->tribuf, &ctx->evall});
+  bool any = false;
+  for (DevBuf *b : idle) {
+    if (!b->p) continue;
+    if (!any) hipStreamSynchronize(ctx->stream);
+    any = true;
+    hipFree(b->p);
+    *b = DevBuf();
+  }
+  return any;
+}
+
+hipError_t eig_malloc(eig_ctx *ctx, void **p, size_t bytes) {
+  hipError_t e = hipSuccess;
+  for (int i = 0; i < 2; ++i) {
+    e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    *p = nullptr;
+    (void)hipGetLastError();  // reported here, not by a later launch's check
+    if (!release_idle(ctx)) break;
+  }
+  return e;
+}
+
 int eig_ensure(eig_ctx *ctx, DevBuf &b, size_t bytes) {
   if (bytes == 0) bytes = 256;
   if (b.bytes >= bytes) return EIG_OK;
@@ -30,11 +59,9 @@ int eig_ensure(eig_ctx *ctx, DevBuf &b, size_t bytes) {
     b.p = nullptr;
     b.bytes = 0;
   }
-  hipError_t e = hipMalloc(&b.p, bytes);
-  if (e != hipSuccess) {
-    b.p = nullptr;
+  hipError_t e = eig_malloc(ctx, &b.p, bytes);
+  if (e != hipSuccess)
     return eig_set_err(ctx, EIG_E_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-  }
   b.bytes = bytes;
   return EIG_OK;
 }
@@ -261,10 +288,8 @@ extern "C" int eig_load_packed(eig_ctx *ctx, const uint8_t *rows, int64_t rlen, 
 extern "C" int eig_dev_alloc(eig_ctx *ctx, size_t bytes, void **ptr) {
   if (!ctx || !ptr || bytes == 0) return eig_set_err(ctx, EIG_E_ARG, "eig_dev_alloc: args");
   EIG_HIP(ctx, hipSetDevice(ctx->device));
-  if (hipMalloc(ptr, bytes) != hipSuccess) {
-    *ptr = nullptr;
+  if (eig_malloc(ctx, ptr, bytes) != hipSuccess)
     return eig_set_err(ctx, EIG_E_NOMEM, "eig_dev_alloc(%zu)", bytes);
-  }
   return EIG_OK;
 }
 

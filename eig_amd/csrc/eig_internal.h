@@ -74,6 +74,7 @@ struct eig_ctx {
   // FP64 form on the integer matrix cores: digit planes, tables, INT32 sums, pair list
   DevBuf xdplanes, xdtab, xdpart, xdmisc;
   bool have_xtx = false;
+  bool in_syrk = false, in_eigh = false;  // their workspaces are in use (eig_malloc)
 
   // eigensolver
   DevBuf ework;
@@ -97,6 +98,13 @@ struct eig_ctx {
 
 int eig_set_err(eig_ctx *ctx, int code, const char *fmt, ...);
 int eig_ensure(eig_ctx *ctx, DevBuf &b, size_t bytes);
+// device memory; where it does not fit, the workspaces that no call under way uses go first
+hipError_t eig_malloc(eig_ctx *ctx, void **p, size_t bytes);
+struct EigInUse {  // marks an entry point's workspaces in use while it lives
+  explicit EigInUse(bool &f) : flag(f) { flag = true; }
+  ~EigInUse() { flag = false; }
+  bool &flag;
+};
 // Results to the caller's (pageable) memory.  The runtime's own copies wait for each one,
 // and move 12 GB/s.  get() queues a small copy into pinned memory, and the caller's memory
 // is filled in wait(); a large one is done at once by several threads, each with two pinned

@@ -1962,6 +1962,7 @@ static int run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, do
 
 int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, double *evals,
                  double *evecs, bool internal) {
+  EigInUse busy(ctx->in_eigh);
   bool again = false;
   EIG_TRY(run_eigh(ctx, d_a, n, nvec, evals, evecs, internal, true, &again));
   // the resident part gave up waiting for blocks that were not scheduled: start over with

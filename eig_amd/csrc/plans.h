@@ -104,3 +104,55 @@ inline FpcaPlans eig_fpca_plans(int num_cu, int64_t M, int32_t nst, int32_t K, i
     F.area = std::max(F.area, eig_codes_area(eig_fpca_basis_plan(num_cu, M, nst, r)));
   return F;
 }
+
+// ---- the FP64 XTX on digit planes (xdigit.hip)
+constexpr int kXT = 256;          // samples per tile side
+constexpr int64_t kXMaxK = 131072;  // SNPs of one INT32 sum: 128 * (126 + 1) * 2^17 < 2^31
+// Workspace that stays with the context: 8 GiB of planes (SNP chunks; 5,000 samples fill it at
+// 600,000 SNPs) and 4 GiB of INT32 sums.  The sums of every tile pair at once are 1.4 GiB at
+// 5,000 samples, 28 at 46,000 and 117 GB at 85,000, which would leave the eigensolver no
+// room; past 4 GiB (2,340 pairs of 16,384 blocks, 64 rounds of the chip) the pairs run in bands.
+constexpr int64_t kXPlaneBytes = (int64_t)8 << 30, kXPartBytes = (int64_t)4 << 30;
+struct XdPlan {
+  int32_t nT, RT, npair, np;  // tiles of kXT, row tiles of 32, tile pairs, planes
+  int64_t K, nchunk;          // SNPs per chunk (a multiple of 128), chunks
+  int32_t nsplit, per;        // splits of a chunk, 64-SNP stages each (even)
+  int32_t band;               // tile pairs per pass
+  size_t plane_bytes, part_bytes;
+};
+// p1 and p2 digits of the two brackets
+inline XdPlan eig_xd_plan(int num_cu, int64_t M, int32_t nst, int32_t p1, int32_t p2) {
+  XdPlan X;
+  X.nT = (nst + 1) / 2;
+  X.RT = 8 * X.nT;
+  X.npair = X.nT * (X.nT + 1) / 2;
+  X.np = p1 + p2 + 2;
+  const int64_t rows = (int64_t)X.RT * 32;
+  const int64_t kmem = std::max<int64_t>(4096, kXPlaneBytes / (rows * X.np) / 128 * 128);
+  const int64_t kmax = std::min<int64_t>(kXMaxK, kmem);
+  X.nchunk = (M + kmax - 1) / kmax;
+  X.K = ((M + X.nchunk - 1) / X.nchunk + 127) / 128 * 128;
+  X.plane_bytes = (size_t)X.np * rows * X.K;
+  const int32_t nstage = (int32_t)(X.K / 64);
+  const int64_t one = (int64_t)p1 * kXT * kXT * 4;  // bytes of a pair's sums, per split
+  // the blocks run one per CU
+  const int64_t slots = std::max(num_cu, 1);
+  X.nsplit = 1;
+  X.per = nstage;
+  double best = 0.0;
+  for (int32_t s = 1; s <= std::min(nstage, 64); ++s) {
+    if (s > 1 && s * X.npair * one > kXPartBytes) break;
+    const int32_t pe = ((nstage + s - 1) / s + 1) & ~1, ns = (nstage + pe - 1) / pe;
+    if (ns != s) continue;
+    const double rounds = (double)(((int64_t)X.npair * p1 * ns + slots - 1) / slots);
+    const double cost = rounds * ((double)pe + 12.0) + 0.5 * (double)X.npair * p1 * ns / slots;
+    if (s == 1 || cost < best) {
+      best = cost;
+      X.nsplit = ns;
+      X.per = pe;
+    }
+  }
+  X.band = (int32_t)std::min<int64_t>(X.npair, kXPartBytes / (X.nsplit * one));
+  X.part_bytes = (size_t)(X.nsplit * X.band * one);
+  return X;
+}

@@ -360,16 +360,16 @@ static void srv_free(eig_server *s) {
   delete s;
 }
 
-static int srv_alloc_lane(eig_server *s, SrvLane &L) {
+static int srv_alloc_lane(eig_ctx *ctx, eig_server *s, SrvLane &L) {
   SRV_HIP(s, hipStreamCreateWithFlags(&L.stream, hipStreamNonBlocking));
   SRV_HIP(s, hipEventCreateWithFlags(&L.done, hipEventDisableTiming));
   SRV_HIP(s, hipHostMalloc((void **)&L.desc_h, sizeof(SrvDesc), hipHostMallocDefault));
   SRV_HIP(s, hipHostMalloc((void **)&L.out_h, sizeof(double) * s->max_batch * (s->K + 2),
                            hipHostMallocDefault));
-  SRV_HIP(s, hipMalloc((void **)&L.desc_d, sizeof(SrvDesc)));
-  SRV_HIP(s, hipMalloc((void **)&L.rows_d, (size_t)s->max_batch * s->rowpad));
-  SRV_HIP(s, hipMalloc((void **)&L.partial_d, s->part_bytes));
-  SRV_HIP(s, hipMalloc((void **)&L.sums_d, sizeof(double) * s->W * s->max_batch));
+  SRV_HIP(s, eig_malloc(ctx, (void **)&L.desc_d, sizeof(SrvDesc)));
+  SRV_HIP(s, eig_malloc(ctx, (void **)&L.rows_d, (size_t)s->max_batch * s->rowpad));
+  SRV_HIP(s, eig_malloc(ctx, (void **)&L.partial_d, s->part_bytes));
+  SRV_HIP(s, eig_malloc(ctx, (void **)&L.sums_d, sizeof(double) * s->W * s->max_batch));
   std::memset(L.desc_h, 0, sizeof(SrvDesc));
   return EIG_OK;
 }
@@ -424,8 +424,8 @@ extern "C" int eig_server_start(eig_ctx *ctx, const double *eigscale, int32_t nl
     s->pr = srv_plan(s, kCdSum, 16);
     s->pg = srv_plan(s, kCdMiss, 16);
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    if (hipMalloc((void **)&s->panel_d, s->pr.head_bytes + s->pg.head_bytes + up(s->pr.dig_bytes) +
-                                            s->pg.dig_bytes) != hipSuccess)
+    if (eig_malloc(ctx, (void **)&s->panel_d, s->pr.head_bytes + s->pg.head_bytes + up(s->pr.dig_bytes) +
+                                                  s->pg.dig_bytes) != hipSuccess)
       return fail(srv_err(s, EIG_E_NOMEM, "panel allocation"));
     s->head_r = s->panel_d;
     s->head_g = s->panel_d + s->pr.head_bytes;
@@ -449,7 +449,7 @@ extern "C" int eig_server_start(eig_ctx *ctx, const double *eigscale, int32_t nl
   }
   for (int l = 0; l < nlanes; ++l) {
     SrvLane &L = s->lane[l];
-    int rc = srv_alloc_lane(s, L);
+    int rc = srv_alloc_lane(ctx, s, L);
     if (rc != EIG_OK) return fail(rc);
     // a batch of each kind on the lane, so that the first request does not pay for the
     // stream's queue and the first touch of its memory (any byte is a valid row)

@@ -536,6 +536,7 @@ static int eig_ensure_selb(eig_ctx *ctx) {
 }
 
 int eig_run_syrk(eig_ctx *ctx, int form, int bf16_block, double *trace_scale) {
+  EigInUse busy(ctx->in_syrk);
   const int64_t M = ctx->nsnp;
   const int32_t T = ctx->nst;
   const int32_t P = T * (T + 1) / 2;

@@ -14,6 +14,7 @@
 // SNPs, seven plus six digits leave 2 to 25 times less error than FP64 accumulation of
 // the same products (an off-diagonal entry's rounding, 300,000 SNPs: 3.0e-12 against
 // 8.0e-11; 2,000 SNPs: 1.3e-13 against 2.3e-13).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -24,12 +25,10 @@ typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4;
 typedef __attribute__((__vector_size__(16 * sizeof(int)))) int i32x16;
 
 namespace {
-constexpr int kXT = 256;          // samples per tile side
 constexpr int kFrag = 1024;       // bytes of one MFMA operand: 32 samples x 32 SNPs
 constexpr int kQ = 63;            // the grid of the right side's integers
 constexpr int kXMaxP = 8;         // digits of the first bracket at most
 constexpr int kXPlanes = 2 * kXMaxP + 2;
-constexpr int64_t kXMaxK = 131072;  // SNPs of one INT32 sum: 128 * (126 + 1) * 2^17 < 2^31
 
 // ------------------------------------------------------------------ the panel's range
 // max over SNPs and genotypes of |f level|, as the bits of a non-negative double (the
@@ -338,8 +337,7 @@ int eig_syrk_digits(eig_ctx *ctx, double *dst, int *done) {
   const int32_t nst = ctx->nst;
   hipStream_t st = ctx->stream;
   const double *lev = (const double *)ctx->lev.p;
-  const int32_t nT = (nst + 1) / 2, RT = 8 * nT;
-  const int32_t npair = nT * (nT + 1) / 2;
+  const int32_t nT = (nst + 1) / 2, npair = nT * (nT + 1) / 2;
   // tile pairs in bands of four rows, column by column: 32 consecutive pairs touch
   // about four row strips and eight column strips
   std::vector<uint32_t> pairs;
@@ -370,33 +368,12 @@ int eig_syrk_digits(eig_ctx *ctx, double *dst, int *done) {
   // of 2,000 to 300,000 SNPs with E from 1 to 7); eight plus seven leave less than either
   const double r = std::ldexp(1.0, E) / std::sqrt((double)M);
   const int32_t p1 = r <= 0.4 ? 7 : 8, p2 = r <= 0.08 ? 6 : 7;
-  const int32_t np = p1 + p2 + 2;
-  // SNP chunks: bounded by the INT32 sums and by the planes' memory
-  const int64_t rows = (int64_t)RT * 32;
-  const int64_t kmem = std::max<int64_t>(4096, ((int64_t)8 << 30) / (rows * np) / 128 * 128);
-  const int64_t kmax = std::min<int64_t>(kXMaxK, kmem);
-  const int64_t nchunk = (M + kmax - 1) / kmax;
-  const int64_t K = ((M + nchunk - 1) / nchunk + 127) / 128 * 128;
-  const int32_t nstage = (int32_t)(K / 64);
-  // splits of a chunk: the blocks run one per CU
-  const int64_t slots = std::max(ctx->num_cu, 1);
-  int32_t nsplit = 1, per = nstage;
-  double best = 0.0;
-  for (int32_t s = 1; s <= std::min(nstage, 64); ++s) {
-    const int32_t pe = ((nstage + s - 1) / s + 1) & ~1, ns = (nstage + pe - 1) / pe;
-    if (ns != s) continue;
-    const double rounds = (double)(((int64_t)npair * p1 * ns + slots - 1) / slots);
-    const double cost = rounds * ((double)pe + 12.0) + 0.5 * (double)npair * p1 * ns / slots;
-    if (s == 1 || cost < best) {
-      best = cost;
-      nsplit = ns;
-      per = pe;
-    }
-  }
-  if (eig_ensure(ctx, ctx->xdplanes, (size_t)np * rows * K) != EIG_OK ||
+  const XdPlan X = eig_xd_plan(ctx->num_cu, M, nst, p1, p2);
+  const int32_t np = X.np, RT = X.RT;
+  const int64_t K = X.K;
+  if (eig_ensure(ctx, ctx->xdplanes, X.plane_bytes) != EIG_OK ||
       eig_ensure(ctx, ctx->xdtab, (size_t)np * K * 4) != EIG_OK ||
-      eig_ensure(ctx, ctx->xdpart, (size_t)nsplit * p1 * npair * kXT * kXT * 4) != EIG_OK) {
-    (void)hipGetLastError();
+      eig_ensure(ctx, ctx->xdpart, X.part_bytes) != EIG_OK) {
     for (DevBuf *b : {&ctx->xdplanes, &ctx->xdtab, &ctx->xdpart}) {
       if (b->p) hipFree(b->p);
       *b = DevBuf();
@@ -405,19 +382,22 @@ int eig_syrk_digits(eig_ctx *ctx, double *dst, int *done) {
   }
   const double s1 = std::ldexp(1.0, 8 * p1 - 1 - E), s2 = std::ldexp(1.0, 8 * p2 - 1 - E);
   const double grid = std::ldexp(1.0, E + 1 - 8 * p1);
-  XdArgs A{(const uint8_t *)ctx->xdplanes.p, d_pairs, (int32_t *)ctx->xdpart.p, K / 32, RT, npair,
-           p1, p2, nsplit, per};
-  const int64_t items = (int64_t)npair * p1 * nsplit;
-  for (int64_t c = 0; c < nchunk; ++c) {
+  for (int64_t c = 0; c < X.nchunk; ++c) {
     const int64_t m0 = c * K;
     hipLaunchKernelGGL(k_xd_tab, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, st, lev, m0, M, K, p1,
                        p2, s1, s2, (uint32_t *)ctx->xdtab.p);
     hipLaunchKernelGGL(k_xd_planes, dim3((unsigned)(K / 32), (unsigned)(RT / 4)), dim3(256), 0, st,
                        (const uint32_t *)ctx->sel.p, M, nst, m0, K, np, RT,
                        (const uint32_t *)ctx->xdtab.p, (uint8_t *)ctx->xdplanes.p);
-    hipLaunchKernelGGL(k_xd_gemm, dim3((unsigned)((items + 7) / 8 * 8)), dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_xd_sum, dim3((unsigned)npair * 64), dim3(256), 0, st, (const int32_t *)ctx->xdpart.p,
-                       d_pairs, npair, p1, nsplit, nst, grid, (int32_t)(c == 0), dst);
+    for (int32_t b = 0; b < npair; b += X.band) {
+      const int32_t nb = std::min(X.band, npair - b);
+      const XdArgs A{(const uint8_t *)ctx->xdplanes.p, d_pairs + b, (int32_t *)ctx->xdpart.p, K / 32, RT, nb,
+                     p1, p2, X.nsplit, X.per};
+      const int64_t items = (int64_t)nb * p1 * X.nsplit;
+      hipLaunchKernelGGL(k_xd_gemm, dim3((unsigned)((items + 7) / 8 * 8)), dim3(256), 0, st, A);
+      hipLaunchKernelGGL(k_xd_sum, dim3((unsigned)nb * 64), dim3(256), 0, st, (const int32_t *)ctx->xdpart.p,
+                         d_pairs + b, nb, p1, X.nsplit, nst, grid, (int32_t)(c == 0), dst);
+    }
     EIG_HIP(ctx, hipGetLastError());
   }
   *done = 1;

@@ -1,6 +1,6 @@
 """What the kernels write against what is allocated for it: the launch plans (plans.h, host
-arithmetic) enumerated on the CPU, and fastmode on panels whose Krylov basis has a lower rank
-than its panels have columns."""
+arithmetic) enumerated on the CPU, fastmode on panels whose Krylov basis has a lower rank
+than its panels have columns, and XTX where its workspace takes several passes."""
 import os
 import subprocess
 
@@ -59,6 +59,106 @@ int main() {
 }
 """)
     assert out == []
+
+
+def test_xtx_workspace_is_bounded(tmp_path):
+    # 8 GiB of planes (4,096 SNPs at least) and 4 of sums at every size, bands that cover the
+    # tile pairs, and all pairs at once where one pass holds them
+    out = run_plans(tmp_path, r"""
+int main() {
+  for (int64_t n : {1, 128, 129, 198, 1000, 5000, 10184, 17000, 17500, 46000, 85000, 92000, 200000})
+    for (int64_t m : {1, 127, 129, 2000, 131073, 600000, 5000000})
+      for (int p1 : {7, 8})
+        for (int p2 : {6, 7}) {
+          const XdPlan X = eig_xd_plan(256, m, (int)((n + 127) / 128), p1, p2);
+          const size_t pair = (size_t)X.nsplit * p1 * 256 * 256 * 4, rows = (size_t)X.RT * 32;
+          bool ok = X.part_bytes <= kXPartBytes && X.band >= 1 && X.band <= X.npair && X.part_bytes == X.band * pair;
+          ok = ok && (X.plane_bytes <= (size_t)kXPlaneBytes || X.K <= 4096) && X.plane_bytes == rows * X.np * X.K;
+          ok = ok && X.K % 128 == 0 && X.K <= kXMaxK && X.K * X.nchunk >= m && rows >= (size_t)n;
+          ok = ok && X.per % 2 == 0 && (int64_t)X.per * 64 * X.nsplit >= X.K;
+          ok = ok && (X.band == X.npair || (X.npair + 0.0) * pair > kXPartBytes);
+          if (!ok) printf("N=%ld M=%ld p1=%d p2=%d\n", n, m, p1, p2);
+        }
+}
+""")
+    assert out == []
+
+
+@pytest.mark.gpu
+def test_xtx_in_bands_of_tile_pairs():
+    """17,500 samples: 2,415 tile pairs, two bands of INT32 sums.  The digits' rounding stays
+    below FP64's own, so an entry is within M ulps of the largest diagonal entry, as is the
+    reference's."""
+    import eig_amd
+    rng = np.random.default_rng(1)
+    N, M = 17500, 200
+    g = rng.binomial(2, rng.uniform(0.05, 0.5, M)[:, None], size=(M, N)).astype(np.int32)
+    g[rng.random(g.shape) < 0.02] = -1
+    print(f"[gpu-case] XTX in bands N={N} M={M}", flush=True)
+    eng = eig_amd.Engine(0)
+    try:
+        eng.load_packed(O.pack_genotypes(g), N)
+        eng.select(np.arange(N, dtype=np.int32))
+        st = eng.snpstats()
+        scale, x = eng.xtx(eig_amd.FORM_FP64, 0, want_matrix=True)
+    finally:
+        eng.close()
+    z = (g - st["mean"][:, None]) * st["fancy"][:, None]
+    z[(g < 0) | (st["status"] != 0)[:, None]] = 0
+    d = (z * z).sum(axis=0)
+    y = d.sum() / (N - 1)
+    tol = 2 * (M + 16) * 2.0 ** -53 * d.max()
+    assert abs(scale - y) <= tol
+    worst = 0.0
+    for i in range(0, N, 2500):
+        ref = z[:, i:i + 2500].T @ z
+        worst = max(worst, np.abs(x[i:i + 2500] * scale - ref).max())
+    assert worst <= tol
+
+
+@pytest.mark.gpu
+def test_idle_workspaces_are_given_back():
+    """An allocation that does not fit frees what XTX and the eigensolver keep between calls;
+    their results stay, and the next calls give the same bits."""
+    import ctypes
+    import eig_amd
+    hip = ctypes.CDLL("/opt/rocm/lib/libamdhip64.so")
+
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value, t.value
+
+    rng = np.random.default_rng(2)
+    N, M = 700, 30000
+    g = rng.binomial(2, rng.uniform(0.05, 0.5, M)[:, None], size=(M, N)).astype(np.int32)
+    eng = eig_amd.Engine(0)
+    try:
+        eng.load_packed(O.pack_genotypes(g), N)
+        eng.select(np.arange(N, dtype=np.int32))
+        eng.snpstats()
+        s0, x0 = eng.xtx(eig_amd.FORM_FP64, 0)
+        e0, v0 = eng.eigh_xtx(N)
+        before, total = free()
+        with pytest.raises(eig_amd.EigError):
+            eng.dev_alloc(4 * total)
+        after, _ = free()
+        # 16 planes of 768 samples by 30,000 SNPs alone are 350 MB
+        assert after - before >= 300 << 20
+        # one that fits once they are gone: the card left with 200 MiB less than it takes
+        fill = eng.dev_alloc(after - (2 << 30))
+        eng.xtx(eig_amd.FORM_FP64, 0, want_matrix=False)
+        left, _ = free()
+        eng.dev_free(eng.dev_alloc(left + (200 << 20)))
+        eng.dev_free(fill)
+        e1, v1 = eng.eigh_xtx(N)
+        s1, x1 = eng.xtx(eig_amd.FORM_FP64, 0)
+        e2, v2 = eng.eigh_xtx(N)
+    finally:
+        eng.close()
+    assert s0 == s1 and np.array_equal(x0, x1)
+    for e, v in ((e1, v1), (e2, v2)):
+        assert np.array_equal(e, e0) and np.array_equal(v, v0)
 
 
 @pytest.mark.gpu
