@@ -12,10 +12,12 @@ constexpr int kCdStage = 128;    // k per stage
 constexpr int kCdFrag = 1024;    // bytes of a digit operand: 16 digit columns x 64 k
 constexpr int kCdMaxCols = 20;   // columns of a group of nine tiles (140 of 144 digit columns)
 constexpr int kCdMaxNT = 9;
-// one INT32 sum holds this many terms (digit 128, code 3)
-constexpr int64_t kCodesMaxK = (int64_t)5 << 20;
 
 enum { kCdPair, kCdSum, kCdMiss };
+// Terms that one INT32 sum holds.  A term is a digit (-128 .. 127) times a code of up to 3, and
+// with kCdSum, whose two planes meet in one sum, the missing bit's digit on top: 384 and 512.
+constexpr int64_t cd_max_k(int mode) { return mode == kCdSum ? (int64_t)4 << 20 : (int64_t)5 << 20; }
+static_assert(128 * 4 * cd_max_k(kCdSum) <= (int64_t)1 << 31 && 128 * 3 * cd_max_k(kCdPair) < (int64_t)1 << 31, "");
 struct CodesPlan {
   int mode;
   int32_t C, ngroup, Cg, NT, R, nrowblk, nsplit;
@@ -52,7 +54,7 @@ inline CodesPlan eig_codes_plan(int num_cu, int mode, int32_t C, int64_t nrow, i
   // splits: rounds of the blocks the chip holds (two per CU) times stages each, plus the
   // sums' way to memory and back, worth about two stages a block
   const int64_t slots = 2 * (int64_t)std::max(num_cu, 1);
-  const int64_t pmax = kCodesMaxK / kCdStage;  // stages of one INT32 sum
+  const int64_t pmax = cd_max_k(mode) / kCdStage;  // stages of one INT32 sum
   const int64_t smin = (nblk + pmax - 1) / pmax;
   double best = 0.0;
   P.nsplit = 1;

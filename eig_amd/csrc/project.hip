@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256) void k_regroup_geno(const uint8_t *__restrict_
 // individual's missing ones, so it needs the missing bits alone.  Individuals run in
 // chunks of whole tiles and SNPs in chunks of whole stages, as the workspace holds; the
 // sums within kLsqRange stages are exact, so the chunks do not change the result.
-constexpr int64_t kLsqRange = kCodesMaxK / 128 / 2;  // whole chunks of it stay within kCodesMaxK
+constexpr int64_t kLsqRange = ((int64_t)5 << 20) / 128 / 2;  // below cd_max_k of both products
 static int lsq_normal(eig_ctx *ctx, double *acc, char *ws, size_t bytes) {
   const int64_t M = ctx->nsnp;
   const int32_t nind = ctx->nind, K = ctx->last_K, nP = K * (K + 1) / 2, W = nP + K + 2;

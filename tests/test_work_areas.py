@@ -51,7 +51,7 @@ int main() {
         for (int64_t nblk : {1, 2, 3, 7, 40, 157, 4688, 40960, 40961, 100000})
           for (int smax : {1, 2, 5, 32, 512}) {
             const CodesPlan P = eig_codes_plan(256, mode, C, nrow, nblk, smax);
-            const int64_t pmax = kCodesMaxK / 128, least = (nblk + pmax - 1) / pmax;
+            const int64_t pmax = cd_max_k(mode) / 128, least = (nblk + pmax - 1) / pmax;
             const int64_t most = smax > least ? smax : least;
             if (P.nsplit > most || P.per > pmax || P.per * P.nsplit < nblk || P.per * (P.nsplit - 1) >= nblk)
               printf("mode %d C %d rows %ld stages %ld smax %d: %d splits of %ld\n", mode, C, nrow, nblk, smax, P.nsplit, P.per);
@@ -79,6 +79,25 @@ int main() {
           ok = ok && (X.band == X.npair || (X.npair + 0.0) * pair > kXPartBytes);
           if (!ok) printf("N=%ld M=%ld p1=%d p2=%d\n", n, m, p1, p2);
         }
+}
+""")
+    assert out == []
+
+
+def test_int32_sums_hold_their_splits(tmp_path):
+    # the worst term per code: digit -128 with code 3 (kCdPair), with code 3 and the missing
+    # bit's digit (kCdSum), with the missing bit (kCdMiss); -2^31 itself is an INT32
+    out = run_plans(tmp_path, r"""
+int main() {
+  const int64_t term[3] = {128 * 3, 128 * 3 + 128, 128};
+  for (int mode = 0; mode < 3; ++mode)
+    for (int C : {1, 20, 136})
+      for (int64_t nrow : {1, 5000, 200000})
+        for (int64_t nblk = 30000; nblk < 90000; nblk += 997)
+          for (int smax : {1, 16}) {
+            const CodesPlan P = eig_codes_plan(256, mode, C, nrow, nblk, smax);
+            if (P.per * 128 * term[mode] > (int64_t)1 << 31) printf("mode %d rows %ld stages %ld\n", mode, nrow, nblk);
+          }
 }
 """)
     assert out == []
