@@ -292,17 +292,29 @@ static void srv_finish(eig_server *s, SrvLane &L, int err) {
   L.busy = false;
 }
 
+// The worker looks for finished batches without a pause for this long after it last started or
+// finished one: a batch takes 0.1 to a few tenths of a millisecond, and a timed wait of 20 us
+// returns after 70 to 80.  Longer ones (large batches, host rows, a card that others use) are
+// waited for with such waits, not with the core.
+constexpr auto kSrvSpin = std::chrono::milliseconds(1);
+
 static void srv_worker(eig_server *s) {
   hipSetDevice(s->device);
   std::unique_lock<std::mutex> lk(s->mu);
+  auto spin_end = Clock::now();
   for (;;) {
     bool progressed = false;
-    // completions
+    // completions; the lanes are this thread's alone, so it asks without the lock that submit
+    // and poll need
+    hipError_t state[kSrvMaxLanes];
+    lk.unlock();
+    for (int l = 0; l < s->nlanes; ++l)
+      state[l] = s->lane[l].busy ? hipEventQuery(s->lane[l].done) : hipErrorNotReady;
+    lk.lock();
     for (int l = 0; l < s->nlanes; ++l) {
       SrvLane &L = s->lane[l];
-      if (!L.busy) continue;
-      hipError_t q = hipEventQuery(L.done);
-      if (q == hipErrorNotReady) continue;
+      const hipError_t q = state[l];
+      if (!L.busy || q == hipErrorNotReady) continue;
       srv_finish(s, L, q == hipSuccess ? EIG_OK : EIG_E_HIP);
       if (q != hipSuccess) s->err = hipGetErrorString(q);
       progressed = true;
@@ -332,15 +344,19 @@ static void srv_worker(eig_server *s) {
     bool any_busy = false;
     for (int l = 0; l < s->nlanes; ++l) any_busy |= s->lane[l].busy;
     if (s->stopping && !any_busy && s->pending.empty()) break;
-    if (progressed) continue;
-    if (any_busy) {
-      // a batch takes 0.1 to a few tenths of a millisecond; a timed wait of 20 us returns
-      // after 70 to 80
+    if (progressed) {
+      spin_end = Clock::now() + kSrvSpin;
+      continue;
+    }
+    if (!any_busy) {
+      s->cv_work.wait(lk, [s] { return s->stopping || !s->pending.empty(); });
+    } else if (Clock::now() < spin_end) {
       lk.unlock();
       std::this_thread::yield();
       lk.lock();
-    } else
-      s->cv_work.wait(lk, [s] { return s->stopping || !s->pending.empty(); });
+    } else {
+      s->cv_work.wait_for(lk, std::chrono::microseconds(20));
+    }
   }
 }
 

@@ -232,7 +232,9 @@ typedef struct eig_server eig_server;
  * (0 = 1024, at most 1024) -- together they bound the device memory admitted
  * requests may use.  chunk: SNPs at least per partial sum (multiple of 64; 0 =
  * 4,096); results do not depend on it.  The context may be used or closed
- * afterwards; the server owns its copies. */
+ * afterwards; the server owns its copies.  The server has one worker thread: it
+ * polls without a pause for up to a millisecond after it starts or finishes a
+ * batch, so a steady stream of short batches takes a core, and waits otherwise. */
 int eig_server_start(eig_ctx *ctx, const double *eigscale, int32_t nlanes, int32_t max_batch,
                      int32_t chunk, eig_server **out);
 /* Queue nq (1..max_batch) query rows of `stride` bytes.  on_device != 0: rows is
