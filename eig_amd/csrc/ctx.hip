@@ -22,11 +22,14 @@ int eig_set_err(eig_ctx *ctx, int code, const char *fmt, ...) {
 }
 
 // What XTX and the eigensolver keep between calls and form anew in each (their results are in
-// buffers of their own) goes when memory runs short, unless the call under way is theirs.
+// buffers of their own), and the regrouped copies of the selection, which are formed again when
+// needed, go when memory runs short, unless the call under way uses them.
 static bool release_idle(eig_ctx *ctx) {
   std::vector<DevBuf *> idle;
   if (!ctx->in_syrk) idle.insert(idle.end(), {&ctx->xdplanes, &ctx->xdtab, &ctx->xdpart, &ctx->part});
   if (!ctx->in_eigh) idle.insert(idle.end(), {&ctx->ework, &ctx->tribuf, &ctx->evall});
+  if (!ctx->in_syrk) idle.push_back(&ctx->selb), ctx->have_selb = false;
+  if (!ctx->in_selg) idle.push_back(&ctx->selg), ctx->have_selg = false;
   bool any = false;
   for (DevBuf *b : idle) {
     if (!b->p) continue;

@@ -74,7 +74,8 @@ struct eig_ctx {
   // FP64 form on the integer matrix cores: digit planes, tables, INT32 sums, pair list
   DevBuf xdplanes, xdtab, xdpart, xdmisc;
   bool have_xtx = false;
-  bool in_syrk = false, in_eigh = false;  // their workspaces are in use (eig_malloc)
+  // in use: XTX's workspaces, the eigensolver's, the regrouped codes (eig_malloc)
+  bool in_syrk = false, in_eigh = false, in_selg = false;
 
   // eigensolver
   DevBuf ework;
@@ -167,6 +168,7 @@ int eig_run_syrk(eig_ctx *ctx, int form, int bf16_block, double *trace_scale);
 // code of SNP 16 s + k of the group, h = (k >> 2) & 1, j = (k & 3) | ((k >> 3) << 2)
 constexpr int kGrp = 64;  // SNPs per group of the grouped code layout
 int eig_ensure_selg(eig_ctx *ctx);
+int eig_regroup(eig_ctx *ctx, int64_t g0, int64_t ng);  // a range of the groups, at ctx->selg
 // internal: a helper's own small problem -- the context's published eigenvectors
 // (used by the loadings) and its stage times are left untouched
 int eig_run_eigh(eig_ctx *ctx, const double *d_a, int32_t n, int32_t nvec, double *evals,
@@ -237,6 +239,8 @@ int eig_codes_mul(eig_ctx *ctx, const CodesPlan &P, const CodeView &v, const Cod
 int eig_codes_out_sum(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void *head, const void *part,
                       double scale, double *out, int64_t ldr, int64_t ldc, int32_t Cpad, bool add,
                       hipStream_t st);
+int eig_codes_samples(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, char *ws, int64_t nrow,
+                      double scale, double *out, int64_t ldr, int64_t ldc, int32_t Cpad, hipStream_t st);
 int eig_codes_out_pair(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void *head, const void *part,
                        const double *lev, const uint8_t *ignore, double scale, double *out, int64_t ldr,
                        int64_t ldc, hipStream_t st);

@@ -970,14 +970,17 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   const size_t o_ta = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxa * npad) : 0;
   const size_t o_tb = bf ? add(sizeof(uint16_t) * 2 * (size_t)cxb * Mpad) : 0;
   const size_t o_tab = bf ? add(sizeof(uint32_t) * 2 * kFpTab * (size_t)(Mpad / kGrp)) : 0;
-  EIG_TRY(eig_ensure_selg(ctx));
+  // the split form reads all of the regrouped codes; without room for them the FP64 form's
+  // products over SNPs take ranges of them
+  bool keep = false;
+  EigInUse using_selg(bf ? ctx->in_selg : keep);
+  const int rg = eig_ensure_selg(ctx);
+  if (rg != EIG_OK && (bf || rg != EIG_E_NOMEM)) return rg;
   // FP64 form: the code products' digit operands and INT32 sums (codes.hip), one area for
   // the X A, X^T B and finishing X^T U products
   const int64_t G64 = Mpad / kGrp;
   const CodeView vm{(const uint8_t *)ctx->sel.p, nullptr, 128 * 32, 32, M * 32, 16, M, (int64_t)nst * 8,
                     kCodeLinear};
-  const CodeView vs{(const uint8_t *)ctx->selg.p, nullptr, G64 * 2048, 16, 4096, 2048, npad, G64 * 4,
-                    kCodeGrouped};
   FpcaPlans F{};
   size_t o_cw = 0;
   if (!bf) {
@@ -1022,29 +1025,23 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
                        (const uint32_t *)lbf, M, G64, tabs);
     EIG_HIP(ctx, hipGetLastError());
   }
-  // X A and X^T B of the FP64 form: `plan`'s product of the codes with cols, its INT32 sums
-  // left in the work area
+  // X^T B and X A of the FP64 form, in the work area
   char *cw = base + o_cw;
-  auto code_mul = [&](const CodesPlan &plan, const CodeView &v, const CodeCols &cols) -> int {
-    if (eig_codes_area(plan) > F.area) return eig_set_err(ctx, EIG_E_STATE, "eig_fpca: work area");
-    EIG_TRY(eig_codes_scales(ctx, plan, cols, cw, st));
-    return eig_codes_mul(ctx, plan, v, cols, 0, cw, cw + plan.head_bytes,
-                         cw + plan.head_bytes + plan.dig_bytes, false, st);
-  };
   auto code_xtb = [&](const CodesPlan &plan, const double *B_, double scale, double *out, int64_t ldo,
                       int32_t Cpad) -> int {
+    if (eig_codes_area(plan) > F.area) return eig_set_err(ctx, EIG_E_STATE, "eig_fpca: work area");
     CodeCols c{kColLevB, B_, ldq, M};
     c.lev = lf;
-    EIG_TRY(code_mul(plan, vs, c));
-    return eig_codes_out_sum(ctx, plan, npad, cw, cw + plan.head_bytes + plan.dig_bytes, scale, out,
-                             ldo, 1, Cpad, false, st);
+    return eig_codes_samples(ctx, plan, c, cw, npad, scale, out, ldo, 1, Cpad, st);
   };
   auto xa = [&](const double *A_, double *Y_) -> int {
     if (bf)
       return launch_xa_bf16(ctx, P, lbf, fa, cxa, A_, lda, Y_, ldq, L, st);
-    EIG_TRY(code_mul(pa, vm, CodeCols{kColPanel, A_, lda, n}));
-    return eig_codes_out_pair(ctx, pa, M, cw, cw + pa.head_bytes + pa.dig_bytes, lf, nullptr, 1.0,
-                              Y_, ldq, 1, st);
+    const CodeCols c{kColPanel, A_, lda, n};
+    char *sums = cw + pa.head_bytes + pa.dig_bytes;
+    EIG_TRY(eig_codes_scales(ctx, pa, c, cw, st));
+    EIG_TRY(eig_codes_mul(ctx, pa, vm, c, 0, cw, cw + pa.head_bytes, sums, false, st));
+    return eig_codes_out_pair(ctx, pa, M, cw, sums, lf, nullptr, 1.0, Y_, ldq, 1, st);
   };
   auto xtb = [&](const double *B_, double *out_) -> int {
     if (bf)

@@ -76,6 +76,13 @@ inline CodesPlan eig_codes_plan(int num_cu, int mode, int32_t C, int64_t nrow, i
   P.part_bytes = (size_t)P.ngroup * P.nsplit * nacc * P.rowpad * P.NT * 16 * 4;
   return P;
 }
+// Where the regrouped codes of all SNPs (a copy of the selection) find no room, the products
+// over SNPs take this many stages of them at a time: a sixteenth, from 16 MiB to 1 GiB.
+inline int64_t eig_codes_chunk(int32_t nst, int64_t nblk) {
+  const int64_t stage = (int64_t)nst * 4096;
+  const int64_t b = std::min<int64_t>((int64_t)1 << 30, std::max<int64_t>((int64_t)16 << 20, stage * nblk / 16));
+  return std::max<int64_t>(1, std::min(nblk, b / stage));
+}
 // a plan's scales, digit operands (a multiple of 2 KB) and INT32 sums, one after the other
 inline size_t eig_codes_area(const CodesPlan &P) { return P.head_bytes + P.dig_bytes + P.part_bytes; }
 

@@ -237,7 +237,9 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
   EIG_TRY(eig_ensure(ctx, ctx->ffvecs, 8 * (size_t)K * M));
   EIG_TRY(eig_ensure(ctx, ctx->fxscal, 8 * (size_t)(kMaxK + M)));  // fxscal | xmean
   EIG_TRY(eig_ensure(ctx, ctx->projw, 8 * (size_t)K * n * 2));     // axes | fxvecs
-  EIG_TRY(eig_ensure_selg(ctx));
+  // without room for the regrouped codes the product over SNPs takes ranges of them
+  const int rg = eig_ensure_selg(ctx);
+  if (rg != EIG_OK && rg != EIG_E_NOMEM) return rg;
   double *d_fx = (double *)ctx->fxscal.p, *d_xm = d_fx + kMaxK;
   double *d_ev = (double *)ctx->projw.p, *d_fxv = d_ev + (size_t)K * n;
   double *d_ff = (double *)ctx->ffvecs.p;
@@ -248,21 +250,16 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
   // over the SNPs (rows = samples), on the code planes (codes.hip).  At 5,000 x 600,000,
   // K = 10, both read the codes once: 19.6 ms with per-code bins and FP64 sums on the
   // vector units, 1.45 now.
-  const int64_t G64 = (M + kGrp - 1) / kGrp;
   const CodeView vm{(const uint8_t *)ctx->sel.p, nullptr, 128 * 32, 32, M * 32, 16, M,
                     (int64_t)ctx->nst * 8, kCodeLinear};
-  const CodeView vs{(const uint8_t *)ctx->selg.p, nullptr, G64 * 2048, 16, 4096, 2048,
-                    (int64_t)ctx->nst * kTileS, G64 * 4, kCodeGrouped};
   CodeCols ax{kColAxes, d_ev, n, n};
   CodeCols fc{kColFx, d_ff, M, M};
   fc.fancy = (const double *)ctx->fancy.p;
   fc.xmean = d_xm;
   fc.ignore = d_ign;
   const CodesPlan pl = eig_codes_plan(ctx->num_cu, kCdPair, K, M, ctx->nst, 16);
-  const CodesPlan pf = eig_codes_plan(ctx->num_cu, kCdSum, K, vs.nrow, (G64 + 1) / 2, 32);
-  const size_t need = std::max(pl.head_bytes + pl.dig_bytes + pl.part_bytes,
-                               pf.head_bytes + pf.dig_bytes + pf.part_bytes);
-  EIG_TRY(eig_ensure(ctx, ctx->scratch2, need));
+  const CodesPlan pf = eig_codes_plan(ctx->num_cu, kCdSum, K, (int64_t)ctx->nst * kTileS, (M + 127) / 128, 32);
+  EIG_TRY(eig_ensure(ctx, ctx->scratch2, std::max(eig_codes_area(pl), eig_codes_area(pf))));
   char *ws = (char *)ctx->scratch2.p;
   eig_time_begin(ctx);
   hipLaunchKernelGGL(k_load_prep, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, st,
@@ -273,11 +270,7 @@ extern "C" int eig_loadings(eig_ctx *ctx, const double *evecs, int32_t K, const 
                         false, st));
   EIG_TRY(eig_codes_out_pair(ctx, pl, M, ws, ws + pl.head_bytes + pl.dig_bytes,
                              (const double *)ctx->lev.p, d_ign, 10.0, d_ff, 1, M, st));
-  EIG_TRY(eig_codes_scales(ctx, pf, fc, ws, st));
-  EIG_TRY(eig_codes_mul(ctx, pf, vs, fc, 0, ws, ws + pf.head_bytes, ws + pf.head_bytes + pf.dig_bytes,
-                        false, st));
-  EIG_TRY(eig_codes_out_sum(ctx, pf, n, ws, ws + pf.head_bytes + pf.dig_bytes, 1.0, d_fxv, 1, n, K,
-                            false, st));
+  EIG_TRY(eig_codes_samples(ctx, pf, fc, ws, n, 1.0, d_fxv, 1, n, K, st));
   hipLaunchKernelGGL(k_fxscal, dim3((unsigned)K), dim3(256), 0, st, (const double *)d_fxv, n, d_fx);
   EIG_HIP(ctx, hipGetLastError());
   eig_time_end(ctx, "loadings");

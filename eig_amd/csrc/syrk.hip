@@ -150,13 +150,13 @@ __global__ __launch_bounds__(256, 2) void k_syrk_f64(const uint32_t *__restrict_
 // word pair per group.
 
 __global__ __launch_bounds__(256) void k_regroup(const uint32_t *__restrict__ sel, int64_t M,
-                                                 int64_t G64, int64_t ngroups,
+                                                 int64_t g0, int64_t ng, int64_t ngroups,
                                                  uint4 *__restrict__ selg) {
   __shared__ uint32_t w[2][kGrp * kTileWords];
   const int half = threadIdx.x >> 7, i = threadIdx.x & 127;
-  const int64_t gid = (int64_t)blockIdx.x * 2 + half;  // over nst * G64 groups
+  const int64_t gid = (int64_t)blockIdx.x * 2 + half;  // over nst * ng groups, from group g0
   const bool live = gid < ngroups;
-  const int64_t st = live ? gid / G64 : 0, g = live ? gid % G64 : 0;
+  const int64_t st = live ? gid / ng : 0, g = live ? g0 + gid % ng : 0;
   const uint32_t *src = sel + (st * M + g * kGrp) * kTileWords;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -504,17 +504,22 @@ __global__ __launch_bounds__(256) void k_unpack_scale(const double *__restrict__
   }
 }
 
-// the per-64-SNP code layout of the current selection (built once per selection)
+// the per-64-SNP code layout of the current selection, groups g0 .. g0 + ng - 1
+int eig_regroup(eig_ctx *ctx, int64_t g0, int64_t ng) {
+  const int64_t ngroups = (int64_t)ctx->nst * ng;
+  hipLaunchKernelGGL(k_regroup, dim3((unsigned)((ngroups + 1) / 2)), dim3(256), 0, ctx->stream,
+                     (const uint32_t *)ctx->sel.p, ctx->nsnp, g0, ng, ngroups, (uint4 *)ctx->selg.p);
+  EIG_HIP(ctx, hipGetLastError());
+  return EIG_OK;
+}
+
+// all of them (built once per selection)
 int eig_ensure_selg(eig_ctx *ctx) {
   if (ctx->have_selg) return EIG_OK;
-  const int64_t M = ctx->nsnp;
-  const int64_t G64 = (M + kGrp - 1) / kGrp;
-  const int64_t ngroups = (int64_t)ctx->nst * G64;
-  EIG_TRY(eig_ensure(ctx, ctx->selg, (size_t)ngroups * kTileS * 16));
+  const int64_t G64 = (ctx->nsnp + kGrp - 1) / kGrp;
+  EIG_TRY(eig_ensure(ctx, ctx->selg, (size_t)ctx->nst * G64 * kTileS * 16));
   eig_time_begin(ctx);
-  hipLaunchKernelGGL(k_regroup, dim3((unsigned)((ngroups + 1) / 2)), dim3(256), 0, ctx->stream,
-                     (const uint32_t *)ctx->sel.p, M, G64, ngroups, (uint4 *)ctx->selg.p);
-  EIG_HIP(ctx, hipGetLastError());
+  EIG_TRY(eig_regroup(ctx, 0, G64));
   eig_time_end(ctx, "regroup");
   ctx->have_selg = true;
   return EIG_OK;

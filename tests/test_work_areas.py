@@ -1,6 +1,7 @@
 """What the kernels write against what is allocated for it: the launch plans (plans.h, host
 arithmetic) enumerated on the CPU, fastmode on panels whose Krylov basis has a lower rank
 than its panels have columns, and XTX where its workspace takes several passes."""
+import ctypes
 import os
 import subprocess
 
@@ -84,6 +85,24 @@ int main() {
     assert out == []
 
 
+def test_ranges_of_regrouped_codes_fit_their_area(tmp_path):
+    out = run_plans(tmp_path, r"""
+int main() {
+  for (int C : {1, 10, 11, 16, 20, 21, 64, 240})
+    for (int nst : {1, 2, 24, 157, 782, 4000})
+      for (int64_t m : {1, 300, 4096, 400000, 600000, 5000000})
+        for (int smax : {1, 2, 32}) {
+          const int64_t nblk = (m + 127) / 128, nb = eig_codes_chunk(nst, nblk);
+          const CodesPlan P = eig_codes_plan(256, kCdSum, C, (int64_t)nst * 128, nblk, smax);
+          const CodesPlan Q = eig_codes_plan(256, kCdSum, C, (int64_t)nst * 128, nb, P.nsplit);
+          if (nb < 1 || nb > nblk || eig_codes_area(Q) > eig_codes_area(P) || nb > cd_max_k(kCdSum) / 128)
+            printf("C=%d nst=%d M=%ld smax=%d\n", C, nst, m, smax);
+        }
+}
+""")
+    assert out == []
+
+
 def test_int32_sums_hold_their_splits(tmp_path):
     # the worst term per code: digit -128 with code 3 (kCdPair), with code 3 and the missing
     # bit's digit (kCdSum), with the missing bit (kCdMiss); -2^31 itself is an INT32
@@ -135,19 +154,75 @@ def test_xtx_in_bands_of_tile_pairs():
     assert worst <= tol
 
 
+def free():
+    """Free and total bytes of the card."""
+    hip = ctypes.CDLL("/opt/rocm/lib/libamdhip64.so")
+    f, t = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+    return f.value, t.value
+
+
+def fill(eng, left):
+    """Blocks of the card's memory until `left` bytes are free (an allocation may leave more
+    free than the count before it had said)."""
+    blocks = []
+    while (more := free()[0] - left) > 4 << 20:
+        blocks.append(eng.dev_alloc(more))
+    return blocks
+
+
+@pytest.mark.gpu
+def test_products_without_room_for_the_regrouped_codes():
+    """Loadings and FP64 fastmode where the card holds the genotypes and the selection but not
+    a third copy of them: ranges of it, the same bits."""
+    import eig_amd
+    rng = np.random.default_rng(4)
+    N, M, K, L = 3000, 400000, 4, 6
+    rows = rng.integers(0, 256, (M, N // 4), dtype=np.uint8)
+    vec = rng.standard_normal((K, N))
+    omega = rng.standard_normal((N, L))
+    every, half = np.arange(N, dtype=np.int32), np.arange(N // 2, dtype=np.int32)
+
+    def panel(eng, sel):
+        eng.select(sel)
+        eng.snpstats(fetch=False)
+
+    def results(eng, n):
+        ff, fx = eng.loadings(np.ascontiguousarray(vec[:, :n]))
+        ev, v = eng.fpca(2, L, 1, omega=np.ascontiguousarray(omega[:n]))
+        return ff, fx, ev, v
+
+    eng = eig_amd.Engine(0)
+    try:
+        eng.load_packed(rows, N)
+        panel(eng, every)
+        want = results(eng, N)
+    finally:
+        eng.close()
+    eng = eig_amd.Engine(0)
+    try:
+        eng.load_packed(rows, N)
+        panel(eng, every)  # its buffers, and those of the products for half of the samples
+        panel(eng, half)
+        results(eng, N // 2)
+        panel(eng, every)
+        # 24 tiles' codes take 307 MB: 154 are there, and 120 more are left free
+        blocks = fill(eng, 120 << 20)
+        print(f"[gpu-case] regrouped codes in ranges N={N} M={M}", flush=True)
+        got = results(eng, N)
+        for b in blocks:
+            eng.dev_free(b)
+    finally:
+        eng.close()
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.gpu
 def test_idle_workspaces_are_given_back():
     """An allocation that does not fit frees what XTX and the eigensolver keep between calls;
     their results stay, and the next calls give the same bits."""
-    import ctypes
     import eig_amd
-    hip = ctypes.CDLL("/opt/rocm/lib/libamdhip64.so")
-
-    def free():
-        f, t = ctypes.c_size_t(), ctypes.c_size_t()
-        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
-        return f.value, t.value
-
     rng = np.random.default_rng(2)
     N, M = 700, 30000
     g = rng.binomial(2, rng.uniform(0.05, 0.5, M)[:, None], size=(M, N)).astype(np.int32)
@@ -164,12 +239,11 @@ def test_idle_workspaces_are_given_back():
         after, _ = free()
         # 16 planes of 768 samples by 30,000 SNPs alone are 350 MB
         assert after - before >= 300 << 20
-        # one that fits once they are gone: the card left with 200 MiB less than it takes
-        fill = eng.dev_alloc(after - (2 << 30))
+        # one that fits once they are gone: 100 MiB free, and 200 to be had
         eng.xtx(eig_amd.FORM_FP64, 0, want_matrix=False)
-        left, _ = free()
-        eng.dev_free(eng.dev_alloc(left + (200 << 20)))
-        eng.dev_free(fill)
+        blocks = fill(eng, 100 << 20)
+        for b in blocks + [eng.dev_alloc(200 << 20)]:
+            eng.dev_free(b)
         e1, v1 = eng.eigh_xtx(N)
         s1, x1 = eng.xtx(eig_amd.FORM_FP64, 0)
         e2, v2 = eng.eigh_xtx(N)
