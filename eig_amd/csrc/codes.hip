@@ -688,40 +688,44 @@ int eig_codes_out_sum(eig_ctx *ctx, const CodesPlan &P, int64_t nrow, const void
   return EIG_OK;
 }
 
-// The selection's samples (a plan of kCdSum for all of their rows and all SNPs) times cols, in a
-// workspace of eig_codes_area(P): from the regrouped codes that the context keeps, or, without
-// them, from a range of them at a time.  The INT32 sums go on from range to range as long as
-// they hold (their bound in SNPs), so the results are the same bits up to there.
+// The selection's samples times cols, over all SNPs, in a workspace of eig_codes_area(P): P is
+// a plan of kCdSum for all of their rows and the stages of a pass (all, or as many as its
+// digits may take).  The codes come from the regrouped ones that the context keeps or, without
+// them, from a range of them at a time.  The INT32 sums go on from pass to pass as long as they
+// hold (their bound in SNPs), so the results are the same bits up to there.
 int eig_codes_samples(eig_ctx *ctx, const CodesPlan &P, const CodeCols &cols, char *ws, int64_t nrow,
                       double scale, double *out, int64_t ldr, int64_t ldc, int32_t Cpad, hipStream_t st) {
-  const int64_t rows = (int64_t)ctx->nst * kTileS, G64 = (ctx->nsnp + kGrp - 1) / kGrp;
-  EIG_TRY(eig_codes_scales(ctx, P, cols, ws, st));
-  if (ctx->have_selg) {
-    const CodeView v{(const uint8_t *)ctx->selg.p, nullptr, G64 * 2048, 16, 4096, 2048, rows, G64 * 4,
-                     kCodeGrouped};
-    EIG_TRY(eig_codes_mul(ctx, P, v, cols, 0, ws, ws + P.head_bytes, ws + P.head_bytes + P.dig_bytes, false, st));
-    return eig_codes_out_sum(ctx, P, nrow, ws, ws + P.head_bytes + P.dig_bytes, scale, out, ldr, ldc, Cpad,
-                             false, st);
+  const int64_t rows = (int64_t)ctx->nst * kTileS, G64 = (ctx->nsnp + kGrp - 1) / kGrp, nblk = (G64 + 1) / 2;
+  const bool kept = ctx->have_selg;
+  const int64_t most = cd_max_k(kCdSum) / kCdStage;
+  CodesPlan C = P;
+  if (!kept) {
+    const int64_t nb = std::min(P.nblk, eig_codes_chunk(ctx->nst, nblk));
+    C = eig_codes_plan(ctx->num_cu, kCdSum, P.C, rows, nb, P.nsplit);
+    EIG_TRY(eig_ensure(ctx, ctx->selg, (size_t)rows * nb * 32));
+    if (eig_codes_area(C) > eig_codes_area(P)) return eig_set_err(ctx, EIG_E_STATE, "code products: work area");
   }
-  const int64_t nb = eig_codes_chunk(ctx->nst, P.nblk), most = cd_max_k(kCdSum) / kCdStage;
-  EIG_TRY(eig_ensure(ctx, ctx->selg, (size_t)rows * nb * 32));
-  const CodesPlan C = eig_codes_plan(ctx->num_cu, kCdSum, P.C, rows, nb, P.nsplit);
-  if (eig_codes_area(C) > eig_codes_area(P)) return eig_set_err(ctx, EIG_E_STATE, "code products: work area");
   char *dig = ws + C.head_bytes, *part = dig + C.dig_bytes;
-  const CodeView v{(const uint8_t *)ctx->selg.p, nullptr, nb * 4096, 16, 4096, 2048, rows, nb * 8, kCodeGrouped};
-  int64_t held = 0;  // stages in the INT32 sums
+  EIG_TRY(eig_codes_scales(ctx, C, cols, ws, st));
+  int64_t held = 0;  // stages in an INT32 sum
   bool add = false;
-  for (int64_t b0 = 0; b0 < P.nblk; b0 += nb) {
-    const int64_t n = std::min(nb, P.nblk - b0);
-    if (held + n > most) {
+  for (int64_t b0 = 0; b0 < nblk; b0 += C.nblk) {
+    if (held > 0 && held + C.per > most) {
       EIG_TRY(eig_codes_out_sum(ctx, C, nrow, ws, part, scale, out, ldr, ldc, Cpad, add, st));
       EIG_TRY(eig_codes_restart(ctx, C, ws, st));
       add = true;
       held = 0;
     }
-    EIG_TRY(eig_regroup(ctx, 2 * b0, 2 * nb));
+    CodeView v{(const uint8_t *)ctx->selg.p, nullptr, C.nblk * 4096, 16, 4096, 2048, rows, C.nblk * 8, kCodeGrouped};
+    if (kept) {
+      v.base += b0 * 4096;
+      v.RT = G64 * 2048;
+      v.nword = (G64 - 2 * b0) * 4;
+    } else {
+      EIG_TRY(eig_regroup(ctx, 2 * b0, 2 * C.nblk));
+    }
     EIG_TRY(eig_codes_mul(ctx, C, v, cols, b0, ws, dig, part, held > 0, st));
-    held += n;
+    held += C.per;
   }
   return eig_codes_out_sum(ctx, C, nrow, ws, part, scale, out, ldr, ldc, Cpad, add, st);
 }

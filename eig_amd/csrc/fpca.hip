@@ -972,15 +972,13 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
   const size_t o_tab = bf ? add(sizeof(uint32_t) * 2 * kFpTab * (size_t)(Mpad / kGrp)) : 0;
   // the split form reads all of the regrouped codes; without room for them the FP64 form's
   // products over SNPs take ranges of them
-  bool keep = false;
-  EigInUse using_selg(bf ? ctx->in_selg : keep);
+  bool released = false;
+  EigInUse reads_selg(bf ? ctx->in_selg : released);
   const int rg = eig_ensure_selg(ctx);
   if (rg != EIG_OK && (bf || rg != EIG_E_NOMEM)) return rg;
   // FP64 form: the code products' digit operands and INT32 sums (codes.hip), one area for
   // the X A, X^T B and finishing X^T U products
   const int64_t G64 = Mpad / kGrp;
-  const CodeView vm{(const uint8_t *)ctx->sel.p, nullptr, 128 * 32, 32, M * 32, 16, M, (int64_t)nst * 8,
-                    kCodeLinear};
   FpcaPlans F{};
   size_t o_cw = 0;
   if (!bf) {
@@ -1040,8 +1038,15 @@ extern "C" int eig_fpca_form(eig_ctx *ctx, int32_t K, int32_t L, int32_t I, uint
     const CodeCols c{kColPanel, A_, lda, n};
     char *sums = cw + pa.head_bytes + pa.dig_bytes;
     EIG_TRY(eig_codes_scales(ctx, pa, c, cw, st));
-    EIG_TRY(eig_codes_mul(ctx, pa, vm, c, 0, cw, cw + pa.head_bytes, sums, false, st));
-    return eig_codes_out_pair(ctx, pa, M, cw, sums, lf, nullptr, 1.0, Y_, ldq, 1, st);
+    EIG_TRY(eig_codes_build(ctx, pa, c, kCodeLinear, 0, cw, cw + pa.head_bytes, st));
+    for (int64_t m = 0; m < M; m += F.arows) {
+      const int64_t rows = std::min(F.arows, M - m);
+      const CodeView v{(const uint8_t *)ctx->sel.p + m * 32, nullptr, 128 * 32, 32, M * 32, 16, rows,
+                       (int64_t)nst * 8, kCodeLinear};
+      EIG_HIP(ctx, eig_codes_product(pa, v, cw + pa.head_bytes, sums, false, st));
+      EIG_TRY(eig_codes_out_pair(ctx, pa, rows, cw, sums, lf + 4 * m, nullptr, 1.0, Y_ + m * ldq, ldq, 1, st));
+    }
+    return EIG_OK;
   };
   auto xtb = [&](const double *B_, double *out_) -> int {
     if (bf)

@@ -87,17 +87,28 @@ inline int64_t eig_codes_chunk(int32_t nst, int64_t nblk) {
 inline size_t eig_codes_area(const CodesPlan &P) { return P.head_bytes + P.dig_bytes + P.part_bytes; }
 
 // ---- fastmode's FP64 panel products (fpca.hip): X A and X^T B of the power iterations, and
-// the finishing X^T U of a basis of r columns
+// the finishing X^T U of a basis of r columns.  The digits of the products over SNPs and the
+// sums of X A grow with the SNPs (3.1 and 1.2 KB each, with 20 and 220 columns): a pass takes
+// as many SNPs as 4 GiB of either hold, which is all of them up to 1.4 and 3.7 million.
+constexpr int64_t kFpcaBytes = (int64_t)4 << 30;
 inline CodesPlan eig_fpca_plan(int num_cu, int mode, int32_t C, int64_t nrow, int64_t nblk) {
+  CodesPlan one = eig_codes_plan(num_cu, mode, C, nrow, 1, 1);
+  if (mode == kCdSum) {
+    nblk = std::min<int64_t>(nblk, kFpcaBytes / (int64_t)one.dig_bytes);
+  } else {
+    const int64_t row = (int64_t)one.part_bytes / one.rowpad;
+    nrow = std::min<int64_t>(nrow, kFpcaBytes / row / 128 * 128);
+  }
   // splits whose sums stay within 2 GiB
-  const CodesPlan one = eig_codes_plan(num_cu, mode, C, nrow, nblk, 1);
+  one = eig_codes_plan(num_cu, mode, C, nrow, nblk, 1);
   const size_t b = one.part_bytes / (size_t)one.nsplit;
   return eig_codes_plan(num_cu, mode, C, nrow, nblk,
                         (int32_t)std::max<size_t>(1, std::min<size_t>(32, ((size_t)2 << 30) / b)));
 }
 struct FpcaPlans {
   CodesPlan pa, pb;
-  size_t area;  // holds each of them and the finishing product at every rank the basis may have
+  int64_t arows;  // SNPs of a pass of X A
+  size_t area;    // holds each of them and the finishing product at every rank the basis may have
 };
 inline CodesPlan eig_fpca_basis_plan(int num_cu, int64_t M, int32_t nst, int32_t r) {
   return eig_fpca_plan(num_cu, kCdSum, r, (int64_t)nst * 128, (M + 127) / 128);
@@ -105,6 +116,7 @@ inline CodesPlan eig_fpca_basis_plan(int num_cu, int64_t M, int32_t nst, int32_t
 inline FpcaPlans eig_fpca_plans(int num_cu, int64_t M, int32_t nst, int32_t K, int32_t L, int32_t Ctot) {
   FpcaPlans F;
   F.pa = eig_fpca_plan(num_cu, kCdPair, L, M, nst);
+  F.arows = std::min<int64_t>(M, F.pa.rowpad);
   F.pb = eig_fpca_plan(num_cu, kCdSum, L, (int64_t)nst * 128, (M + 127) / 128);
   F.area = std::max(eig_codes_area(F.pa), eig_codes_area(F.pb));
   // fewer columns can need more: their groups, and with them the row padding and the splits,

@@ -35,6 +35,12 @@ int main() {
           const int L = l[0], Ct = (l[1] + 1) * L, nst = (int)((n + 127) / 128);
           const FpcaPlans F = eig_fpca_plans(cu, m, nst, 1, L, Ct);
           if (eig_codes_area(F.pa) > F.area || eig_codes_area(F.pb) > F.area) printf("panel L=%d N=%ld M=%ld\n", L, n, m);
+          // bounded whatever M: 4 GiB of digits and one split's or 2 GiB of sums
+          const CodesPlan u = eig_fpca_basis_plan(cu, m, nst, Ct);
+          if (F.pa.part_bytes > kFpcaBytes || F.pb.dig_bytes > kFpcaBytes || u.dig_bytes > kFpcaBytes ||
+              u.part_bytes > std::max<size_t>(u.part_bytes / u.nsplit, (size_t)2 << 30))
+            printf("bounds L=%d I=%d N=%ld M=%ld\n", L, l[1], n, m);
+          if (F.arows < 1 || F.arows > m || F.arows > F.pa.rowpad || (F.arows < m && F.arows % 128)) printf("rows L=%d N=%ld M=%ld\n", L, n, m);
           for (int r = 1; r <= Ct; ++r)
             if (eig_codes_area(eig_fpca_basis_plan(cu, m, nst, r)) > F.area) printf("L=%d I=%d N=%ld M=%ld r=%d\n", L, l[1], n, m, r);
         }
@@ -216,6 +222,36 @@ def test_products_without_room_for_the_regrouped_codes():
         eng.close()
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+def test_fastmode_in_passes():
+    """1,200,000 SNPs with 64 columns and a basis of 256: X A's sums and X^T U's digits take two
+    passes each.  The two leading eigenvalues stand twenty times above the rest, so seven
+    products with X and as many with its transpose leave less than 1e-17 of the rest beside
+    their axes, and both are XTX's to rounding."""
+    import eig_amd
+    rng = np.random.default_rng(6)
+    N, M, L, I = 300, 1200000, 64, 3
+    thr = rng.uniform(0.05, 0.95, (3, M))
+    thr = (np.clip(thr, 0.02, 0.98) * 2.0 ** 32).astype(np.uint32)
+    pop = np.searchsorted([0.5, 0.8], np.arange(N) / N, side="right").astype(np.int32)
+    print(f"[gpu-case] fastmode in passes N={N} M={M}", flush=True)
+    eng = eig_amd.Engine(0)
+    try:
+        eng.synth(M, N, thr, np.repeat(pop[:, None], 3, axis=1), np.full((N, 2), 0xFFFFFFFF, np.uint32),
+                  1 << 26, 9)
+        eng.select(np.arange(N, dtype=np.int32))
+        eng.snpstats(fetch=False)
+        scale, _ = eng.xtx(eig_amd.FORM_FP64, 0, want_matrix=False)
+        ex, vx = eng.eigh_xtx(3)
+        ev, vec = eng.fpca(2, L, I, omega=rng.standard_normal((N, L)))
+    finally:
+        eng.close()
+    want = ex * scale / (2 * M)
+    assert want[1] > 20 * want[2]
+    assert np.all(np.abs(ev - want[:2]) <= 1e-11 * want[0])
+    assert np.max(np.abs(vec - vx[:2])) <= 1e-9
 
 
 @pytest.mark.gpu
