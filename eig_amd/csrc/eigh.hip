@@ -796,15 +796,18 @@ __global__ __launch_bounds__(T) void k_tri(EigWs ws, int32_t n, int32_t c0, int3
     if (lane == 0) rnrm[wv] = s;
   };
   norm(0);
-  // the largest squared norm of a column so far, with those of the columns before this launch
-  double top = 0.0;
-  for (int32_t i = t; i < c0; i += T) top = fmax(top, ws.e2[i]);
+  // 2^-160 of the largest squared norm of a column, first of those before this launch
+  {
+    double top = 0.0;
+    for (int32_t i = t; i < c0; i += T) top = fmax(top, 0x1p-160 * ws.e2[i]);
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) top = fmax(top, xlane(top, o));
-  if (lane == 0) rdot[wv] = top;
+    for (int o = 32; o > 0; o >>= 1) top = fmax(top, xlane(top, o));
+    if (lane == 0) rdot[wv] = top;
+  }
   __syncthreads();
+  double drop = rdot[0];
 #pragma unroll
-  for (int u = 0; u < W; ++u) top = fmax(top, rdot[u]);
+  for (int u = 1; u < W; ++u) drop = fmax(drop, rdot[u]);
   for (int32_t c = 0; c < cols; ++c) {
     if (r0 + RS - 1 <= c) return;  // no live rows: nothing to give and nothing to keep
     const int cur = c & 1;
@@ -816,10 +819,10 @@ __global__ __launch_bounds__(T) void k_tri(EigWs ws, int32_t n, int32_t c0, int3
     double tau = 0.0, scale = 0.0, beta = al;
     // A matrix of constant blocks leaves a remainder of the same structure in every column,
     // each 1e-16 of the last, until its squares underflow and tau no longer fits v (vectors
-    // orthogonal to 1e-2 only).  A column below 2^-80 of an earlier one is far below the
+    // orthogonal to 1e-2 only).  What is below 2^-80 of an earlier column is far below the
     // matrix' rounding: it is dropped, as the Sturm counts do with such an e.
-    const double s2 = fma(al, al, xn2);
-    if (xn2 > 0.0 && s2 > 0x1p-160 * top) {
+    if (xn2 > drop) {
+      const double s2 = fma(al, al, xn2);
       if (s2 > 1e-280 && s2 < 1e280) {
         // 1 / sqrt and 1 / x by the hardware's approximations and two Newton steps each (a
         // few ulps, as rcp_nr's), whose chains are shorter than a square root's and division's
@@ -836,7 +839,6 @@ __global__ __launch_bounds__(T) void k_tri(EigWs ws, int32_t n, int32_t c0, int3
         scale = 1.0 / (al - beta);
       }
     }
-    top = fmax(top, s2);
     double vn[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -942,6 +944,7 @@ __global__ __launch_bounds__(T) void k_tri(EigWs ws, int32_t n, int32_t c0, int3
       sw[t + T * k] = w[k];
     }
     norm(c + 1);
+    drop = fmax(drop, 0x1p-160 * (beta * beta));
     // ---- results of column c, by the owner of row c + 1
     if (owner) {
       double *const out = A + (int64_t)c * lda;
