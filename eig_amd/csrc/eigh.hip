@@ -1176,6 +1176,42 @@ __device__ inline double rcp_nr(double a) {
   return fma(r, fma(-a, r, 1.0), r);
 }
 
+// The shift for eigenvalue i (ascending) of the n: the eigenvalue itself, unless it belongs to a
+// run of ones that stand closer than their own errors (8 ulps of the norm apart).  Shifts that
+// differ by such an error turn the run's vectors to whichever of its directions is nearest to
+// each, several to the same one, and orthogonalising them again leaves rounding errors
+// enlarged a hundred times and more: residuals of 1e-13 where an eigenvalue fills several batches of
+// vectors.  The whole run (at most 32 ulps wide) takes one shift instead, 16 of its widths off
+// its middle: a solve scales all of its directions alike, so vectors orthogonalised after the
+// first one stay so in the second.  Other directions shrink by 16 widths over the gap to the
+// next eigenvalue a solve; where that is above 1e-10 the eigenvalues keep their own shifts.
+// Every lane of a wave calls it with the same i.
+__device__ inline double invit_shift(const double *__restrict__ eval, int32_t n, int32_t i, double tnorm) {
+  const double ulp = 2.220446049250313e-16 * tnorm, lam = eval[i];
+  auto apart = [&](int32_t k) { return k < 0 || k + 1 >= n || !(eval[k + 1] - eval[k] <= 8.0 * ulp); };
+  if (apart(i - 1) && apart(i)) return lam;
+  const int lane = threadIdx.x & 63;
+  int32_t a = i, b = i;  // the run's ends, 64 steps at a time
+  for (;; a -= 64) {
+    const uint64_t m = __ballot(apart(a - 1 - lane));
+    if (m == 0) continue;
+    a -= __ffsll((unsigned long long)m) - 1;
+    break;
+  }
+  for (;; b += 64) {
+    const uint64_t m = __ballot(apart(b + lane));
+    if (m == 0) continue;
+    b += __ffsll((unsigned long long)m) - 1;
+    break;
+  }
+  const double width = fmax(eval[b] - eval[a], 2.0 * ulp);
+  double gap = tnorm;
+  if (a > 0) gap = fmin(gap, eval[a] - eval[a - 1]);
+  if (b + 1 < n) gap = fmin(gap, eval[b + 1] - eval[b]);
+  const double off = 16.0 * width;
+  return width <= 32.0 * ulp && off <= 1e-10 * gap ? 0.5 * (eval[a] + eval[b]) + off : lam;
+}
+
 // One inverse iteration for the eigenvalues j0 + blockIdx.x (descending order) of the
 // tridiagonal, one block per vector: with `first` from a fixed start vector, else from
 // X[j]; the pivoted LU of T - lambda I is formed with `factor`, else read back; the result is
@@ -1201,7 +1237,7 @@ __global__ __launch_bounds__(256) void k_invit_solve(EigWs ws, int32_t n, int32_
   __shared__ double red[4], sinv;
   const int tid = threadIdx.x;
   const int32_t j = j0 + (int32_t)blockIdx.x;
-  const double lam = ws.eval[n - 1 - j];
+  const double lam = factor ? invit_shift(ws.eval, n, n - 1 - j, ws.sc[S_TNORM]) : 0.0;
   const double tiny = 2.220446049250313e-16 * ws.sc[S_TNORM];
   double *x = X + (int64_t)j * n, *L = lu + (int64_t)blockIdx.x * kLuF * n;
   // start vectors: a fixed hash of index and vector
