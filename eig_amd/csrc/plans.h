@@ -128,6 +128,7 @@ inline FpcaPlans eig_fpca_plans(int num_cu, int64_t M, int32_t nst, int32_t K, i
 
 // ---- the FP64 XTX on digit planes (xdigit.hip)
 constexpr int kXT = 256;          // samples per tile side
+constexpr int kResSnps = 128;     // SNPs a step of the left-out parts' sums
 constexpr int64_t kXMaxK = 131072;  // SNPs of one INT32 sum: 128 * (126 + 1) * 2^17 < 2^31
 // Workspace that stays with the context: 8 GiB of planes (SNP chunks; 5,000 samples fill it at
 // 600,000 SNPs) and 4 GiB of INT32 sums.  The sums of every tile pair at once are 1.4 GiB at
@@ -139,7 +140,8 @@ struct XdPlan {
   int64_t K, nchunk;          // SNPs per chunk (a multiple of 128), chunks
   int32_t nsplit, per;        // splits of a chunk, 64-SNP stages each (even)
   int32_t band;               // tile pairs per pass
-  size_t plane_bytes, part_bytes;
+  int32_t rsplit, rstep;      // splits of the left-out parts' sums, steps of kResSnps in each
+  size_t plane_bytes, tab_bytes, part_bytes;
 };
 // p1 and p2 digits of the two brackets
 inline XdPlan eig_xd_plan(int num_cu, int64_t M, int32_t nst, int32_t p1, int32_t p2) {
@@ -175,5 +177,12 @@ inline XdPlan eig_xd_plan(int num_cu, int64_t M, int32_t nst, int32_t p1, int32_
   }
   X.band = (int32_t)std::min<int64_t>(X.npair, kXPartBytes / (X.nsplit * one));
   X.part_bytes = (size_t)(X.nsplit * X.band * one);
+  // about eight blocks a CU over the sample tiles
+  const int32_t steps = (int32_t)((X.K + kResSnps - 1) / kResSnps);
+  X.rsplit = std::min<int32_t>(steps, std::max<int32_t>(1, (int32_t)(8 * slots / nst)));
+  X.rstep = (steps + X.rsplit - 1) / X.rsplit;
+  X.rsplit = (steps + X.rstep - 1) / X.rstep;
+  // left-out parts [K][4], their splits' and the chunk's sums, the digit tables
+  X.tab_bytes = 64 * (size_t)X.K + 16 * (size_t)(X.rsplit + 1) * nst * 128 + 4 * (size_t)X.np * X.K;
   return X;
 }

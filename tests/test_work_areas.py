@@ -91,6 +91,24 @@ int main() {
     assert out == []
 
 
+def test_xtx_left_out_parts_cover_a_chunk(tmp_path):
+    out = run_plans(tmp_path, r"""
+int main() {
+  for (int cu : {1, 32, 256})
+    for (int64_t n : {2, 129, 257, 2503, 5000, 100000})
+      for (int64_t m : {1, 128, 129, 2000, 20011, 131073, 600000}) {
+        const int nst = (int)((n + 127) / 128);
+        const XdPlan X = eig_xd_plan(cu, m, nst, 7, 6);
+        // every SNP is in one split, none of which is empty
+        if ((int64_t)X.rsplit * X.rstep * kResSnps < X.K || (int64_t)(X.rsplit - 1) * X.rstep * kResSnps >= X.K) printf("split N=%ld M=%ld\n", n, m);
+        // table of 4 pairs a SNP, pairs of each split and of their sum, digit tables
+        if (X.tab_bytes < (size_t)X.K * 4 * 16 + (size_t)(X.rsplit + 1) * nst * 128 * 16 + (size_t)X.np * X.K * 4) printf("bytes N=%ld M=%ld\n", n, m);
+      }
+}
+""")
+    assert out == []
+
+
 def test_ranges_of_regrouped_codes_fit_their_area(tmp_path):
     out = run_plans(tmp_path, r"""
 int main() {
