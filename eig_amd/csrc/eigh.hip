@@ -741,7 +741,8 @@ __device__ __forceinline__ double rows_sum(const double (&z)[G]) {
   a += xlane(a, 32);
   return a;
 }
-__device__ __forceinline__ double tri_rcp(double a) {
+// 1/a by the hardware reciprocal and two Newton steps (error a few ulp)
+__device__ __forceinline__ double rcp_nr(double a) {
   double r = __builtin_amdgcn_rcp(a);
   r = fma(r, fma(-a, r, 1.0), r);
   return fma(r, fma(-a, r, 1.0), r);
@@ -832,7 +833,7 @@ __global__ __launch_bounds__(T) void k_tri(EigWs ws, int32_t n, int32_t c0, int3
         const double nb = copysign(s2 * h, al);  // -beta
         beta = -nb;
         tau = fma(fabs(al), h, 1.0);
-        scale = tri_rcp(al + nb);
+        scale = rcp_nr(al + nb);
       } else {
         beta = -copysign(sqrt(s2), al);
         tau = (beta - al) / beta;
@@ -1168,13 +1169,7 @@ __global__ __launch_bounds__(256) void k_multisect(EigWs ws, int32_t n,
 }
 
 // ---------------------------------------------------------------- inverse iteration
-// 1/a by the hardware reciprocal and two Newton steps (error a few ulp): the LU of
-// T - lambda I keeps pivot reciprocals, so no division sits on a serial chain
-__device__ inline double rcp_nr(double a) {
-  double r = __builtin_amdgcn_rcp(a);
-  r = fma(r, fma(-a, r, 1.0), r);
-  return fma(r, fma(-a, r, 1.0), r);
-}
+// The LU of T - lambda I keeps pivot reciprocals, so no division sits on a serial chain.
 
 // The shift for eigenvalue i (ascending) of the n: the eigenvalue itself, unless it belongs to a
 // run of ones that stand closer than their own errors (8 ulps of the norm apart).  Shifts that

@@ -279,10 +279,10 @@ __global__ __launch_bounds__(256) void k_xd_planes(const uint32_t *__restrict__ 
 // stores; a wave reads the next operands from LDS while the current MFMAs run.
 // Four waves of 128 x 128, one per SIMD with 384 registers: LDS traffic bounds smaller
 // wave tiles (eight waves of 128 x 64 read 96 and write 32 bytes per CU cycle of MFMA at
-// full rate, the LDS' own 128; here it is 94).  At 5,000 samples, 120,000 SNPs a chunk,
-// 13 products: 17.7 ms a chunk, 2.4 POP/s, the matrix units busy about 60 % of the cycles
-// at the clock that this load leaves (the eight-wave kernel took 19.5 ms scheduled alike,
-// 21 without the interleaving below).
+// full rate, the LDS' own 128; here it is 94).  At 5,000 samples x 600,000 SNPs,
+// six chunks of 13 products: 14.7 ms a chunk, 2.4 POP/s, the matrix units busy 72 % of the
+// cycles at the clock that this load leaves, 1.6 GHz (chunks of 120,000 SNPs took 17.7 ms,
+// and an eight-wave kernel 19.5 scheduled alike, 21 without the interleaving below).
 struct XdArgs {
   const uint8_t *planes;
   const uint32_t *pairs;  // tile pair list: row tile | column tile << 16

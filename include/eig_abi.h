@@ -250,8 +250,8 @@ int eig_server_submit(eig_server *s, const uint8_t *rows, int64_t stride, int32_
  * != 0 blocks).  A finished ticket is released by the poll that returns it. */
 int eig_server_poll(eig_server *s, int64_t ticket, int32_t wait, double *coords,
                     int32_t *status, double *latency_ms);
-/* Shape and counters: K, nsnp, padded device row bytes, the chunk and the largest
- * grid in use, batches launched and samples admitted so far.  Any may be NULL. */
+/* Shape and counters: K, nsnp, padded device row bytes, the chunk, the blocks that
+ * fill the device (two per CU), batches launched and samples admitted so far.  Any may be NULL. */
 int eig_server_info(eig_server *s, int32_t *K, int64_t *nsnp, int64_t *rowpad, int32_t *chunk,
                     int32_t *grid, int64_t *batches, int64_t *samples);
 const char *eig_server_error(const eig_server *s);
