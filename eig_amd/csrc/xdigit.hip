@@ -529,8 +529,9 @@ int eig_syrk_digits(eig_ctx *ctx, double *dst, int *done) {
                        (const int32_t *)ctx->nmiss.p, ctx->nrows, d_tab, d_res);
     hipLaunchKernelGGL(k_xd_res, dim3((unsigned)nst, (unsigned)X.rsplit), dim3(256), 0, st,
                        (const uint32_t *)ctx->sel.p, M, m0, K, X.rstep, (const double2 *)d_res, d_rpart);
-    // few splits are added up by k_xd_sum itself, which saves a launch
-    const bool few = X.rsplit <= 16;
+    // few splits are added up by k_xd_sum itself, which saves a launch, while its blocks are
+    // one round of the device: each adds them up again
+    const bool few = X.rsplit <= 16 && npair * 64 <= ctx->num_cu;
     if (!few)
       hipLaunchKernelGGL(k_xd_res_sum, dim3((unsigned)(nst * kTileS / 16)), dim3(256), 0, st,
                          (const double2 *)d_rpart, X.rsplit, nst * kTileS, d_rsum);
