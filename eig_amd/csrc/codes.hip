@@ -12,7 +12,9 @@
 // from a code word) are multiplied with the digit planes by v_mfma_i32_16x16x64_i8.  The
 // INT32 sums are exact, so the result has no rounding but the grid's and the final
 // conversion's: less than FP64 accumulation leaves, and the same bits however the sums are
-// split.
+// split.  The grid is the column's, though: where its largest entry stands far above the sum of
+// the others that a row sees (and the row lacks that entry), FP64 accumulation keeps more.  With
+// n entries seen, of mean size a, that is where the largest exceeds about n a.
 //
 // Used by fastmode's FP64 panel products (kjg_fpca.c:104-178), the SNP loadings and their
 // scales (smartpca.c:1438-1525) and lsqproject's normal equations (smartpca.c:4606-4757).
